@@ -1056,12 +1056,14 @@ c10::intrusive_ptr<c10d::Work> ProcessGroupMCCL::broadcast(std::vector<at::Tenso
                            "broadcast: ranks disagree on root or tensor count");
                 check_rc(mcclx_queue_wait_stream(shared->ctx, all[r].stream));
             }
+            std::vector<mcclx_copy_desc> copies;  // source by source: each is read once for all who get it
             for (size_t i = 0; i < all[0].dst.size(); ++i)
                 for (int r = 0; r < world; ++r) {
                     if (r == root) continue;
                     MCCL_CHECK(all[r].nbytes[i] == all[root].nbytes[i], "broadcast: size mismatch");
-                    check_rc(mcclx_copy(shared->ctx, all[r].dst[i], all[root].dst[i], all[root].nbytes[i]));
+                    copies.push_back(mcclx_copy_desc{all[r].dst[i], all[root].dst[i], all[root].nbytes[i]});
                 }
+            check_rc(mcclx_copy_batched(shared->ctx, copies.data(), static_cast<uint32_t>(copies.size())));
         });
     });
 }
@@ -1135,14 +1137,17 @@ c10::intrusive_ptr<c10d::Work> ProcessGroupMCCL::allgather(
             shared->begin_main_work();
             for (int r = 0; r < world; ++r) check_rc(mcclx_queue_wait_stream(shared->ctx, all[r].stream));
             const size_t nt = all[0].src.size();
-            for (size_t i = 0; i < nt; ++i)
-                for (int r = 0; r < world; ++r) {
+            std::vector<mcclx_copy_desc> copies;  // source by source: each is read once for all who get it
+            for (size_t i = 0; i < nt; ++i) {
+                for (int r = 0; r < world; ++r)
                     MCCL_CHECK(all[r].src.size() == nt && all[r].nbytes[i] == all[0].nbytes[i],
                                "allgather: ranks pass different tensors");
-                    for (int p = 0; p < world; ++p)
-                        check_rc(mcclx_copy(shared->ctx, all[r].dst[i * static_cast<size_t>(world) + p],
-                                            all[p].src[i], all[0].nbytes[i]));
-                }
+                for (int p = 0; p < world; ++p)
+                    for (int r = 0; r < world; ++r)
+                        copies.push_back(mcclx_copy_desc{all[r].dst[i * static_cast<size_t>(world) + p], all[p].src[i],
+                                                         all[0].nbytes[i]});
+            }
+            check_rc(mcclx_copy_batched(shared->ctx, copies.data(), static_cast<uint32_t>(copies.size())));
         });
     });
 }

@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "fold_launch.h"
 
 namespace mcclx {
@@ -22,39 +24,60 @@ template <> struct Packet<4> { typedef u32x4 type __attribute__((aligned(4))); }
 template <> struct Packet<2> { typedef u32x4 type __attribute__((aligned(2))); };
 template <> struct Packet<1> { typedef u32x4 type __attribute__((aligned(1))); };
 constexpr int kBlock = 256;
-constexpr int kU = 1;  // packets per lane
+
+constexpr int kOneWave = 64, kFourWaves = 256;  // threads per block of a launch by value, see kOneWaveBlocksFrom
+
+// One packet from its source to everybody who gets it.  FAN = false: one destination.
+template <bool FAN, typename V>
+__device__ __forceinline__ void deliver(MCCLX_GLOBAL uint8_t* const (&dst)[FAN ? kCopyDsts : 1], uint32_t n, uint64_t off, u32x4 v) {
+    COPY_ST((MCCLX_GLOBAL V*)(dst[0] + off), v);
+    if constexpr (FAN) {
+#pragma unroll
+        for (uint32_t f = 1; f < (uint32_t)kCopyDsts; ++f)
+            if (f < n) COPY_ST((MCCLX_GLOBAL V*)(dst[f] + off), v);
+    }
+}
 
 // Up to kFewCopies copies with their descriptors in the kernel arguments:
-// blockIdx.y picks the copy, blockIdx.x one tile of kU * kBlock packets of 16
-// bytes; block 0 of a copy also moves the bytes behind its last whole packet.
+// blockIdx.y picks the copy, blockIdx.x one tile of B packets of 16 bytes, one
+// per lane; block 0 of a copy also moves the bytes in front of its first and
+// behind its last whole packet.  Packets start on a 128-byte boundary of the
+// first destination: a stream of full lines, where an odd-sized chunk of an
+// allgather would otherwise write every line in two parts.
 // One tile per block and no loop, like the fold kernels: a uniform 64-bit base
 // plus a 32-bit lane offset per access, and a short path to the first load.
-template <int A>
-__global__ void __launch_bounds__(kBlock) copy_few_kernel(CopyFew a) {
+template <int A, bool FAN, int B>
+__global__ void __launch_bounds__(B) copy_few_kernel(CopyFew a) {
     typedef typename Packet<A>::type V;
-    const CopyDesc d = a.d[blockIdx.y];
-    const uint64_t P = d.nbytes / 16;
-    const uint64_t first = (uint64_t)blockIdx.x * (kU * kBlock);
+    constexpr int D = FAN ? kCopyDsts : 1;
+    const CopyDesc& d = a.d[blockIdx.y];
+    const uint64_t nbytes = d.nbytes;
+    const uint32_t n = FAN ? (uint32_t)d.n : 1u;
+    const uint32_t mis = (0u - (uint32_t)reinterpret_cast<uintptr_t>(d.dst[0])) & 127u;
+    const uint32_t head = nbytes < mis ? (uint32_t)nbytes : mis;
+    const uint64_t P = (nbytes - head) / 16;
+    const uint64_t first = (uint64_t)blockIdx.x * B;
+    const uint64_t at = head + first * 16;
     if (first < P) {
-        const MCCLX_GLOBAL uint8_t* gs = (const MCCLX_GLOBAL uint8_t*)d.src + first * 16;
-        MCCLX_GLOBAL uint8_t* gd = (MCCLX_GLOBAL uint8_t*)d.dst + first * 16;
-        const uint64_t left = P - first;
-        if (left >= (uint64_t)kU * kBlock) {
-            u32x4 v[kU];
+        const MCCLX_GLOBAL uint8_t* gs = (const MCCLX_GLOBAL uint8_t*)d.src + at;
+        MCCLX_GLOBAL uint8_t* gd[D];
 #pragma unroll
-            for (int u = 0; u < kU; ++u) v[u] = COPY_LD((const MCCLX_GLOBAL V*)(gs + ((uint32_t)u * kBlock + threadIdx.x) * 16u));
-#pragma unroll
-            for (int u = 0; u < kU; ++u) COPY_ST((MCCLX_GLOBAL V*)(gd + ((uint32_t)u * kBlock + threadIdx.x) * 16u), v[u]);
-        } else {
-            for (uint32_t p = threadIdx.x; p < (uint32_t)left; p += kBlock) {
-                u32x4 v = COPY_LD((const MCCLX_GLOBAL V*)(gs + p * 16u));
-                COPY_ST((MCCLX_GLOBAL V*)(gd + p * 16u), v);
-            }
+        for (int f = 0; f < D; ++f) gd[f] = (MCCLX_GLOBAL uint8_t*)d.dst[f] + at;
+        if (threadIdx.x < P - first) {
+            const uint32_t off = threadIdx.x * 16u;
+            deliver<FAN, V>(gd, n, off, COPY_LD((const MCCLX_GLOBAL V*)(gs + off)));
         }
     }
     if (blockIdx.x == 0) {
-        const uint64_t i = P * 16 + threadIdx.x;
-        if (i < d.nbytes) ((MCCLX_GLOBAL uint8_t*)d.dst)[i] = ((const MCCLX_GLOBAL uint8_t*)d.src)[i];
+        auto byte = [&](uint64_t i) {
+            const uint8_t x = ((const MCCLX_GLOBAL uint8_t*)d.src)[i];
+#pragma unroll
+            for (int f = 0; f < D; ++f)
+                if ((uint32_t)f < n) ((MCCLX_GLOBAL uint8_t*)d.dst[f])[i] = x;
+        };
+        for (uint32_t i = threadIdx.x; i < head; i += B) byte(i);
+        const uint64_t i = head + P * 16 + threadIdx.x;  // fewer than 16 bytes remain
+        if (i < nbytes) byte(i);
     }
 }
 
@@ -89,9 +112,10 @@ __device__ __forceinline__ uint64_t uni64(uint64_t v) {
 // bytes behind the last whole packet.  The loop bound is fixed at launch.
 constexpr int kManyU = 4;
 
-template <int A>
+template <int A, bool FAN>
 __global__ void __launch_bounds__(kBlock) copy_many_kernel(CopyTable t) {
     typedef typename Packet<A>::type V;
+    constexpr int D = FAN ? kCopyDsts : 1;
     const uint64_t span = (uint64_t)kManyU * kBlock;
     for (uint32_t w = blockIdx.x; w < t.total_items; w += gridDim.x) {
         uint32_t c, tile;
@@ -115,7 +139,10 @@ __global__ void __launch_bounds__(kBlock) copy_many_kernel(CopyTable t) {
         tile = uni32(tile);
         const CopyDesc* __restrict__ d = t.descs + c;
         const MCCLX_GLOBAL uint8_t* gs = (const MCCLX_GLOBAL uint8_t*)uni64(reinterpret_cast<uint64_t>(d->src));
-        MCCLX_GLOBAL uint8_t* gd = (MCCLX_GLOBAL uint8_t*)uni64(reinterpret_cast<uint64_t>(d->dst));
+        const uint32_t n = FAN ? uni32((uint32_t)d->n) : 1u;
+        MCCLX_GLOBAL uint8_t* gd[D];
+#pragma unroll
+        for (int f = 0; f < D; ++f) gd[f] = (MCCLX_GLOBAL uint8_t*)uni64(reinterpret_cast<uint64_t>(d->dst[f]));
         const uint64_t nbytes = uni64(d->nbytes);
         const uint64_t P = nbytes / 16;
         const uint64_t base = (uint64_t)tile * span;
@@ -125,17 +152,19 @@ __global__ void __launch_bounds__(kBlock) copy_many_kernel(CopyTable t) {
             for (int u = 0; u < kManyU; ++u)
                 v[u] = COPY_LD((const MCCLX_GLOBAL V*)(gs + (base + (uint64_t)u * kBlock + threadIdx.x) * 16));
 #pragma unroll
-            for (int u = 0; u < kManyU; ++u)
-                COPY_ST((MCCLX_GLOBAL V*)(gd + (base + (uint64_t)u * kBlock + threadIdx.x) * 16), v[u]);
+            for (int u = 0; u < kManyU; ++u) deliver<FAN, V>(gd, n, (base + (uint64_t)u * kBlock + threadIdx.x) * 16, v[u]);
         } else {
-            for (uint64_t p = base + threadIdx.x; p < P; p += kBlock) {
-                u32x4 v = COPY_LD((const MCCLX_GLOBAL V*)(gs + p * 16));
-                COPY_ST((MCCLX_GLOBAL V*)(gd + p * 16), v);
-            }
+            for (uint64_t p = base + threadIdx.x; p < P; p += kBlock)
+                deliver<FAN, V>(gd, n, p * 16, COPY_LD((const MCCLX_GLOBAL V*)(gs + p * 16)));
         }
         if (tile == 0) {
-            uint64_t i = P * 16 + threadIdx.x;
-            if (i < nbytes) gd[i] = gs[i];
+            const uint64_t i = P * 16 + threadIdx.x;
+            if (i < nbytes) {
+                const uint8_t x = gs[i];
+#pragma unroll
+                for (int f = 0; f < D; ++f)
+                    if ((uint32_t)f < n) gd[f][i] = x;
+            }
         }
     }
 }
@@ -147,15 +176,19 @@ uint64_t copy_items(uint64_t nbytes) {
     return n ? n : (nbytes ? 1 : 0);
 }
 
-hipError_t launch_copy_many(hipStream_t st, const CopyTable& t, int align, uint32_t max_blocks) {
+hipError_t launch_copy_many(hipStream_t st, const CopyTable& t, int align, int most, uint32_t max_blocks) {
     if (t.total_items == 0) return hipSuccess;
-    uint32_t g = t.total_items < max_blocks ? t.total_items : max_blocks;
-    if (align == 4)
-        copy_many_kernel<4><<<dim3(g), dim3(kBlock), 0, st>>>(t);
-    else if (align == 2)
-        copy_many_kernel<2><<<dim3(g), dim3(kBlock), 0, st>>>(t);
-    else
-        copy_many_kernel<1><<<dim3(g), dim3(kBlock), 0, st>>>(t);
+    const dim3 grid(t.total_items < max_blocks ? t.total_items : max_blocks), block(kBlock);
+    auto go = [&](auto fan) {
+        constexpr bool FAN = decltype(fan)::value;
+        if (align == 4)
+            copy_many_kernel<4, FAN><<<grid, block, 0, st>>>(t);
+        else if (align == 2)
+            copy_many_kernel<2, FAN><<<grid, block, 0, st>>>(t);
+        else
+            copy_many_kernel<1, FAN><<<grid, block, 0, st>>>(t);
+    };
+    if (most > 1) go(std::true_type{}); else go(std::false_type{});
     return hipGetLastError();
 }
 
@@ -171,30 +204,46 @@ hipError_t launch_stream_probe(hipStream_t st, void* buf, uint64_t nbytes, bool 
     return hipGetLastError();
 }
 
-hipError_t launch_copy_few(hipStream_t st, const CopyFew& a, int align) {
-    uint64_t longest = 0;
-    for (uint32_t i = 0; i < a.n; ++i) longest = a.d[i].nbytes > longest ? a.d[i].nbytes : longest;
+hipError_t launch_copy_few(hipStream_t st, const CopyFew& a, int align, int most) {
+    uint64_t longest = 0, moved = 0;
+    for (uint32_t i = 0; i < a.n; ++i) {
+        longest = a.d[i].nbytes > longest ? a.d[i].nbytes : longest;
+        moved += a.d[i].nbytes * (1 + a.d[i].n);
+    }
     if (a.n == 0 || longest == 0) return hipSuccess;
-    const uint64_t span = (uint64_t)kU * kBlock * 16;
-    uint64_t g = (longest + span - 1) / span;
+    const uint64_t waves = (longest + 1023) / 1024;
+    const bool four = waves * a.n < kOneWaveBlocksFrom;
+    const uint64_t g = four ? (waves + 3) / 4 : waves;
     if (g >> 31) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)g, a.n);
-    if (align == 4)
-        copy_few_kernel<4><<<grid, dim3(kBlock), 0, st>>>(a);
-    else if (align == 2)
-        copy_few_kernel<2><<<grid, dim3(kBlock), 0, st>>>(a);
-    else
-        copy_few_kernel<1><<<grid, dim3(kBlock), 0, st>>>(a);
+    const uint32_t lds = resident_lds(moved, 16 * (most + 1), most);
+    auto go = [&](auto fan, auto block) {
+        constexpr bool FAN = decltype(fan)::value;
+        constexpr int B = decltype(block)::value;
+        if (align == 4)
+            copy_few_kernel<4, FAN, B><<<grid, dim3(B), lds, st>>>(a);
+        else if (align == 2)
+            copy_few_kernel<2, FAN, B><<<grid, dim3(B), lds, st>>>(a);
+        else
+            copy_few_kernel<1, FAN, B><<<grid, dim3(B), lds, st>>>(a);
+    };
+    const std::integral_constant<int, kOneWave> one_wave;
+    const std::integral_constant<int, kFourWaves> four_waves;
+    if (most > 1) {
+        if (four) go(std::true_type{}, four_waves); else go(std::true_type{}, one_wave);
+    } else {
+        if (four) go(std::false_type{}, four_waves); else go(std::false_type{}, one_wave);
+    }
     return hipGetLastError();
 }
 
-hipError_t launch_copy(hipStream_t st, void* dst, const void* src, uint64_t nbytes, uint32_t) {
+hipError_t launch_copy(hipStream_t st, void* dst, const void* src, uint64_t nbytes) {
     if (nbytes == 0) return hipSuccess;
     CopyFew a;
-    a.d[0] = CopyDesc{dst, src, nbytes};
+    a.d[0] = CopyDesc{src, nbytes, 1, {dst}};
     a.n = 1;
     const uintptr_t both = reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src);
-    return launch_copy_few(st, a, both % 4 == 0 ? 4 : both % 2 == 0 ? 2 : 1);
+    return launch_copy_few(st, a, both % 4 == 0 ? 4 : both % 2 == 0 ? 2 : 1, 1);
 }
 
 }  // namespace mcclx

@@ -91,12 +91,50 @@ uint32_t items_for(const PlanKey& key, uint64_t count);
 // hipErrorInvalidValue = no kernel for this plan.
 hipError_t launch_fold(hipStream_t st, const PlanKey& key, const LaunchParams& lp);
 
-// Many copies in one launch: descriptors and nseg+1 work-item prefix sums in
-// device memory (mirrors mcclx_copy_desc).
+// How many one-wavefront blocks share a CU in a large launch of several streams.
+//
+// A full CU holds 32 of them, and a launch of k operands then has 32 * k KiB of loads per CU
+// under way, spread over a range of every stream that is wider than what the memory channels
+// keep open: the more streams, the more rows each channel switches between, and the slower
+// the launch (measured on 1-4 GB, TB/s at 32 waves: one stream in and one out 6.7, three in
+// one out 6.4, four tensors reduced in place 5.9, eight in place 5.5, one to eight 5.3).
+// With fewer waves resident the same launches run at 6.1-6.8 TB/s: what a channel sees at
+// one time shrinks with the bytes under way, and 70-80 KiB per CU (20 MB on the device) still
+// covers the latency.  The optimum, swept over 3..20 waves per CU, lies near one number of
+// bytes for every shape, waves x bytes a lane moves: 1150 (8 operands into one: 8 waves;
+// 4 into one: 14; 3 into one: 17; one source to 4 / 8 destinations: 11-14 / 7-8), a little
+// more where tensors are reduced in place, which opens each row once for both directions
+// (2 / 3 / 4 / 5 / 8 ranks: 18 / 12 / 8-10 / 8 / 5 waves).  A reservation of LDS nobody uses
+// sets the number: it is granted in units of 1280 bytes of a CU's 160 KiB.
+//
+// A launch that ends soon needs its waves to get going: the limit pays from 160 MB moved on
+// (200 MB, eight operands into one: 36.2 -> 35.4 us; 80 MB: 5.5 TB/s without it, 5.1 with),
+// and not where 20 waves or more would be left of a launch with one output.
+constexpr uint64_t kResidentMinBytes = 160'000'000;
+constexpr int kLaneBytes = 1150, kLaneBytesInPlace = 1280;
+inline uint32_t resident_lds(uint64_t launch_bytes, int lane_bytes, int outputs, int budget = kLaneBytes) {
+    int waves = budget / lane_bytes;
+    if (launch_bytes < kResidentMinBytes || (outputs == 1 && waves >= 20)) return 0;
+    waves = waves > 18 ? 18 : waves < 3 ? 3 : waves;  // three blocks reserve 53 KiB each: a launch may ask for 64 KiB
+    return 163840u / (uint32_t)waves / 1280u * 1280u;
+}
+
+// Launches that one generation of waves nearly covers (8192 on 256 CUs) start sooner in
+// blocks of four wavefronts: 4 MB copied in 2.5 us against 2.9, an encode of 4 MB 2.3 against
+// 2.7; larger ones stream faster in one-wavefront blocks, whose slots turn over one by one
+// (27 MB copied: 10.1 -> 9.2 us, a two-operand wire fold of a 25 MiB bucket: 12.5 -> 11.4 us).
+constexpr uint64_t kOneWaveBlocksFrom = 12288;
+
+// Many copies in one launch: descriptors and n+1 work-item prefix sums in
+// device memory.  A descriptor is one source and everybody who gets it: copies
+// that share a source (the allgather leg hands every chunk to every other rank)
+// read it once.
+constexpr int kCopyDsts = 8;
 struct CopyDesc {
-    void* dst;
     const void* src;
     uint64_t nbytes;
+    uint64_t n;  // destinations, 1..kCopyDsts
+    void* dst[kCopyDsts];
 };
 struct CopyTable {
     const CopyDesc* __restrict__ descs;
@@ -112,16 +150,16 @@ struct CopyFew {
     CopyDesc d[kFewCopies];
     uint32_t n;
 };
-hipError_t launch_copy_few(hipStream_t st, const CopyFew& copies, int align);
+// `most`: the largest number of destinations any descriptor of the launch has.
+hipError_t launch_copy_few(hipStream_t st, const CopyFew& copies, int align, int most);
 // Work items (tiles) one copy of nbytes splits into.
 uint64_t copy_items(uint64_t nbytes);
 // `align`: the widest of 4 / 2 / 1 bytes that every pointer in the table is aligned to.
-hipError_t launch_copy_many(hipStream_t st, const CopyTable& t, int align, uint32_t max_blocks);
+hipError_t launch_copy_many(hipStream_t st, const CopyTable& t, int align, int most, uint32_t max_blocks);
 
 // Plain device copy with the same packet shape (also the calibration kernel for
 // the memory counters): dst <- src, nbytes.
-hipError_t launch_copy(hipStream_t st, void* dst, const void* src, uint64_t nbytes,
-                       uint32_t max_blocks);
+hipError_t launch_copy(hipStream_t st, void* dst, const void* src, uint64_t nbytes);
 
 // Reads (write == false) or writes nbytes of `buf` once, one 16-byte packet per
 // lane like the copy kernel: the one-directional ceilings of a launch of that size.

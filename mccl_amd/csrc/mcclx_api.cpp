@@ -934,7 +934,7 @@ int mcclx_copy(mcclx_ctx* ctx, void* dst, const void* src, uint64_t nbytes) {
         if (int rc = check_range(dst, nbytes, "dst", 0)) return rc;
     }
     DeviceGuard guard(ctx->device);
-    hipError_t e = mcclx::launch_copy(ctx->stream, dst, src, nbytes, ctx->max_blocks);
+    hipError_t e = mcclx::launch_copy(ctx->stream, dst, src, nbytes);
     if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy launch failed: %s", hipGetErrorString(e));
     ++ctx->launches;
     return MCCLX_OK;
@@ -944,9 +944,12 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     if (n == 0) return MCCLX_OK;
     if (!descs) return fail(MCCLX_ERR_INVALID, "copy_batched: descriptor array is null");
+    // Consecutive copies of one source become one descriptor with several destinations
+    // (the schedules list them that way): the source is read once.
+    std::vector<mcclx::CopyDesc> groups;
     uintptr_t both = 0;
-    uint64_t bytes = 0;
-    uint32_t live = 0;
+    uint64_t bytes = 0;  // per destination: what decides the length of a grid
+    int most = 0;
     for (uint32_t i = 0; i < n; ++i) {
         const mcclx_copy_desc& d = descs[i];
         if (d.nbytes == 0 || d.dst == d.src) continue;
@@ -956,10 +959,17 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
             if (int rc = check_range(d.dst, d.nbytes, "dst", i)) return rc;
         }
         both |= reinterpret_cast<uintptr_t>(d.dst) | reinterpret_cast<uintptr_t>(d.src);
-        bytes += d.nbytes;
-        ++live;
+        mcclx::CopyDesc* last = groups.empty() ? nullptr : &groups.back();
+        if (last && last->src == d.src && last->nbytes == d.nbytes && last->n < (uint64_t)mcclx::kCopyDsts) {
+            last->dst[last->n++] = d.dst;
+        } else {
+            groups.push_back(mcclx::CopyDesc{d.src, d.nbytes, 1, {d.dst}});
+            bytes += d.nbytes;
+        }
+        if ((int)groups.back().n > most) most = (int)groups.back().n;
     }
-    if (live == 0) return MCCLX_OK;
+    if (groups.empty()) return MCCLX_OK;
+    const uint32_t live = (uint32_t)groups.size();
     DeviceGuard guard(ctx->device);
     if (!guard.ok) return fail(MCCLX_ERR_HIP, "hipSetDevice(%d) failed", ctx->device);
     const int align = (both % 4 == 0) ? 4 : (both % 2 == 0) ? 2 : 1;
@@ -974,22 +984,20 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
         uint64_t longest = 0, sum = 0;
         auto flush = [&]() -> int {
             if (few.n == 0) return MCCLX_OK;
-            hipError_t e = mcclx::launch_copy_few(ctx->stream, few, align);
+            hipError_t e = mcclx::launch_copy_few(ctx->stream, few, align, most);
             if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy_batched launch failed: %s", hipGetErrorString(e));
             ++ctx->launches;
             few.n = 0;
             longest = sum = 0;
             return MCCLX_OK;
         };
-        for (uint32_t i = 0; i < n; ++i) {
-            const mcclx_copy_desc& d = descs[i];
-            if (d.nbytes == 0 || d.dst == d.src) continue;
+        for (const mcclx::CopyDesc& d : groups) {
             const uint64_t lg = d.nbytes > longest ? d.nbytes : longest;
             // blocks with nothing to do: more than 3 in 4 -> start a new group
             if (few.n == (uint32_t)mcclx::kFewCopies || (few.n && lg * (few.n + 1) > 4 * (sum + d.nbytes) + (1u << 16)))
                 if (int rc = flush()) return rc;
-            few.d[few.n++] = mcclx::CopyDesc{d.dst, d.src, d.nbytes};
-            longest = d.nbytes > longest ? d.nbytes : longest;
+            few.d[few.n++] = d;
+            longest = lg;
             sum += d.nbytes;
         }
         return flush();
@@ -997,20 +1005,14 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
     std::lock_guard<std::mutex> lk(ctx->mu);
     const size_t desc_bytes = (size_t)live * sizeof(mcclx::CopyDesc);
     std::vector<char> host(desc_bytes + ((size_t)live + 1) * sizeof(uint64_t));
-    auto* hd = reinterpret_cast<mcclx::CopyDesc*>(host.data());
+    memcpy(host.data(), groups.data(), desc_bytes);
     auto* pre = reinterpret_cast<uint64_t*>(host.data() + desc_bytes);
-    uint64_t total = 0, uniform = 0;
-    uint32_t j = 0;
-    for (uint32_t i = 0; i < n; ++i) {
-        const mcclx_copy_desc& d = descs[i];
-        if (d.nbytes == 0 || d.dst == d.src) continue;
-        hd[j] = mcclx::CopyDesc{d.dst, d.src, d.nbytes};
+    uint64_t total = 0, uniform = mcclx::copy_items(groups[0].nbytes);
+    for (uint32_t j = 0; j < live; ++j) {
         pre[j] = total;
-        const uint64_t items = mcclx::copy_items(d.nbytes);
-        if (j == 0) uniform = items;
+        const uint64_t items = mcclx::copy_items(groups[j].nbytes);
         if (items != uniform) uniform = 0;
         total += items;
-        ++j;
     }
     pre[live] = total;
     if (total >> 31) return fail(MCCLX_ERR_INVALID, "copy_batched: more than 2^31 work items in one launch");
@@ -1033,7 +1035,7 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
     t.total_items = (uint32_t)total;
     t.uniform_items = (uint32_t)uniform;
     t.n = live;
-    hipError_t e = mcclx::launch_copy_many(ctx->stream, t, align, ctx->max_blocks);
+    hipError_t e = mcclx::launch_copy_many(ctx->stream, t, align, most, ctx->max_blocks);
     if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy_batched launch failed: %s", hipGetErrorString(e));
     ++ctx->launches;
     return MCCLX_OK;

@@ -1,0 +1,62 @@
+"""Batched copies of one source to several destinations: consecutive descriptors of one source
+travel as one, the source is read once.  Bytes must arrive unchanged and nothing around a
+destination may be touched, at every edge of the packet grid (16-byte packets that start on a
+128-byte boundary of the first destination), in both block shapes and with the resident waves
+limited (launches that move 160 MB and more)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def deliver(q, nbytes, fan, src_off, dst_offs, repeat=1):
+    rng = np.random.default_rng(nbytes * 31 + fan * 7 + src_off)
+    host = rng.integers(0, 256, repeat * nbytes + 64, dtype=np.uint8)
+    src = torch.from_numpy(host).cuda()
+    outs = [torch.full((repeat * nbytes + 512,), 0xA5, dtype=torch.uint8, device="cuda") for _ in range(fan)]
+    descs = [(outs[f].data_ptr() + 128 + dst_offs[f % len(dst_offs)] + s * nbytes, src.data_ptr() + src_off + s * nbytes, nbytes)
+             for s in range(repeat) for f in range(fan)]
+    torch.cuda.synchronize()
+    before = q.launch_count()
+    q.copy_batched(descs)
+    q.drain()
+    for f in range(fan):
+        lo = 128 + dst_offs[f % len(dst_offs)]
+        want = np.full(repeat * nbytes + 512, 0xA5, dtype=np.uint8)
+        want[lo:lo + repeat * nbytes] = host[src_off:src_off + repeat * nbytes]
+        assert np.array_equal(outs[f].cpu().numpy(), want), (nbytes, fan, src_off, f)
+    return q.launch_count() - before
+
+
+@pytest.mark.parametrize("fan", [1, 2, 7, 8, 9])
+@pytest.mark.parametrize("src_off,dst_offs", [(0, [0]), (4, [8, 100]), (2, [2]), (1, [3, 0, 77])])
+def test_one_source_to_several_destinations(fan, src_off, dst_offs):
+    from mccl_amd import kernels as K
+    q = K.hip_kernels_init(0)
+    for nbytes in (1, 15, 16, 17, 127, 128, 129, 255, 1023, 1024, 1025, 4096, 4097, 65_537):
+        assert deliver(q, nbytes, fan, src_off, dst_offs) == 1
+    assert deliver(q, 1021, fan, src_off, dst_offs, repeat=40) == 1      # 40 sources or more: the table launch
+    deliver(q, 9_000_001, fan, src_off, dst_offs)                        # from 12,288 wavefronts on: blocks of one
+    deliver(q, 13_000_003, fan, src_off, dst_offs)
+
+
+@pytest.mark.parametrize("fan,nbytes", [(8, 18_000_005), (4, 33_000_001), (2, 54_000_001), (1, 81_000_003)])
+def test_large_launches_with_fewer_waves_resident(fan, nbytes):
+    from mccl_amd import kernels as K
+    assert deliver(K.hip_kernels_init(0), nbytes, fan, 2, [6]) == 1
+
+
+@pytest.mark.parametrize("world", [2, 3, 8])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_allgather_of_odd_chunks(world, in_place):
+    """Chunks of an odd number of elements leave every destination but the first off the packet
+    grid; in place, a rank's own chunk is already where it belongs and is not copied."""
+    from mccl_amd import harness as H
+    for chunk in (1, 63, 4099, 300_001):
+        outs = [torch.zeros(world * chunk, dtype=torch.bfloat16, device="cuda") for _ in range(world)]
+        parts = [torch.randn(chunk, device="cuda").to(torch.bfloat16) for _ in range(world)]
+        ins = [outs[r][r * chunk:(r + 1) * chunk].copy_(parts[r]) for r in range(world)] if in_place else parts
+        H.allgather_replay(outs, ins)
+        want = torch.cat(parts)
+        assert all(torch.equal(o.view(torch.int16), want.view(torch.int16)) for o in outs), chunk
