@@ -202,6 +202,14 @@ typedef struct {
 #define MCCLX_PLAN_FANOUT_SHIFT 8
 #define MCCLX_PLAN_FANOUT_MASK 0x700
 #define MCCLX_PLAN_FANOUT(n) ((n) << MCCLX_PLAN_FANOUT_SHIFT)
+/* To all: the result goes back into every operand's own buffer -- a whole
+ * allreduce of k ranks in one pass, each rank's tensor being an operand and a
+ * destination (AllreduceAlgos.cpp:62-86: reduce and allgather legs together), in
+ * the form the operands have.  Unlike fan-out it names no further pointers, so it
+ * reaches MCCLX_MAX_INPUTS ranks, and it takes every op.  Per-step rounding only,
+ * io PURE or ALL_F32 (MIN, MAX and PRODUCT too), k >= 2; `out` must be in[0],
+ * `wire_out` NULL.  Not together with fan-out. */
+#define MCCLX_PLAN_TO_ALL 2
 
 typedef struct {
     int32_t dtype;      /* W: MCCLX_F32 / F16 / BF16                                  */

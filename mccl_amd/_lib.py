@@ -27,6 +27,7 @@ ACC_STEP, ACC_F32 = 0, 1
 ALGO_RING, ALGO_TREE, ALGO_BUTTERFLY = 0, 1, 2
 REPLAY_STEPWISE, REPLAY_FUSED, REPLAY_DIRECT = 0, 1, 2
 PLAN_ACC_IS_SRC = 1
+PLAN_TO_ALL = 2
 
 
 def PLAN_FANOUT(n: int) -> int:

@@ -33,6 +33,8 @@
 #include <stdint.h>
 #include <stdlib.h>
 
+#include <type_traits>
+
 #include "fold_launch.h"
 
 namespace mcclx {
@@ -163,6 +165,27 @@ template <int OP> __device__ __forceinline__ float apply(float a, float b) {
     else return (b < a) ? a : b;  // MCCLX_MAX_ACC_SRC
 }
 
+// `op` is C::OP, or the launch's own operator where C::OP is kAnyOp (MIN, MAX and PRODUCT
+// of the to-all form share one kernel: the choice is a uniform branch per operand, free in
+// a launch that waits for memory).
+constexpr int kAnyOp = 100;
+template <class C> __device__ __forceinline__ float apply_op(float a, float b, int op) {
+    if constexpr (C::OP != kAnyOp) return apply<C::OP>(a, b);
+    switch (op) {
+        case MCCLX_PRODUCT: return apply<MCCLX_PRODUCT>(a, b);
+        case MCCLX_MIN: return apply<MCCLX_MIN>(a, b);
+        case MCCLX_MAX: return apply<MCCLX_MAX>(a, b);
+        case MCCLX_MIN_ACC_SRC: return apply<MCCLX_MIN_ACC_SRC>(a, b);
+        default: return apply<MCCLX_MAX_ACC_SRC>(a, b);
+    }
+}
+
+// Where a result goes: to `out` / `wire_out`; also to the `fan` further destinations the
+// segment names behind its operands; or back into every operand's own buffer (an allreduce
+// in place: each rank's tensor is an operand and a destination, so the segment needs no
+// pointers beyond the operands' and eight ranks fit).
+enum { kOutOne = 0, kOutFan = 1, kOutAll = 2 };
+
 // ------------------------------------------------------------ configuration
 
 template <int W_, int IO_, int K_, int TOPO_, int OP_, int ACC_>
@@ -219,8 +242,8 @@ __device__ __forceinline__ void decode(const RawPack& r, float (&v)[C::E]) {
 }
 
 template <class C>
-__device__ __forceinline__ float step(float a, float b) {
-    float r = apply<C::OP>(a, b);
+__device__ __forceinline__ float step(float a, float b, int op = C::OP) {
+    float r = apply_op<C>(a, b, op);
     if constexpr (C::ACC == MCCLX_ACC_STEP) r = Num<C::W>::rnd(r);
     return r;
 }
@@ -245,9 +268,23 @@ __device__ __forceinline__ void load_all(const SegArgs& s, const uint32_t (&pk)[
 
 // acc = acc (op) v for one packet, rounded to W in STEP mode (NaNs not yet canonical).
 template <class C>
-__device__ __forceinline__ void step_pack(float (&acc)[C::E], const float (&v)[C::E]) {
+__device__ __forceinline__ void step_pack(float (&acc)[C::E], const float (&v)[C::E], int op = C::OP) {
+    if constexpr (C::OP == kAnyOp) {
+        auto all = [&](auto one) {
 #pragma unroll
-    for (int j = 0; j < C::E; ++j) acc[j] = apply<C::OP>(acc[j], v[j]);
+            for (int j = 0; j < C::E; ++j) acc[j] = apply<decltype(one)::value>(acc[j], v[j]);
+        };
+        switch (op) {
+            case MCCLX_PRODUCT: all(std::integral_constant<int, MCCLX_PRODUCT>{}); break;
+            case MCCLX_MIN: all(std::integral_constant<int, MCCLX_MIN>{}); break;
+            case MCCLX_MAX: all(std::integral_constant<int, MCCLX_MAX>{}); break;
+            case MCCLX_MIN_ACC_SRC: all(std::integral_constant<int, MCCLX_MIN_ACC_SRC>{}); break;
+            default: all(std::integral_constant<int, MCCLX_MAX_ACC_SRC>{}); break;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < C::E; ++j) acc[j] = apply<C::OP>(acc[j], v[j]);
+    }
     if constexpr (C::ACC == MCCLX_ACC_STEP) Num<C::W>::template round_mid<C::E>(acc);
 }
 
@@ -270,11 +307,11 @@ __device__ __forceinline__ void finish_pack(float (&acc)[C::E], float scale, boo
 }
 
 template <class C, int k>
-__device__ __forceinline__ void fold_from(const RawPack (&raw)[C::K], float (&acc)[C::E]) {
+__device__ __forceinline__ void fold_from(const RawPack (&raw)[C::K], float (&acc)[C::E], int op) {
     float v[C::E];
     decode<C, k>(raw[k], v);
-    step_pack<C>(acc, v);
-    if constexpr (k + 1 < C::K) fold_from<C, k + 1>(raw, acc);
+    step_pack<C>(acc, v, op);
+    if constexpr (k + 1 < C::K) fold_from<C, k + 1>(raw, acc, op);
 }
 
 template <class C, int k>
@@ -285,10 +322,10 @@ __device__ __forceinline__ void decode_all(const RawPack (&raw)[C::K], float (&v
 
 // Reduce one packet's K operands to acc[E].
 template <class C>
-__device__ __forceinline__ void combine(const RawPack (&raw)[C::K], float (&acc)[C::E]) {
+__device__ __forceinline__ void combine(const RawPack (&raw)[C::K], float (&acc)[C::E], int op = C::OP) {
     if constexpr (C::TOPO == MCCLX_TOPO_FOLD) {
         decode<C, 0>(raw[0], acc);
-        if constexpr (C::K > 1) fold_from<C, 1>(raw, acc);
+        if constexpr (C::K > 1) fold_from<C, 1>(raw, acc, op);
     } else {
         // allreduce_tree's reduce phase (AllreduceAlgos.cpp:100-114): at level
         // `mask` every surviving rank r (r % 2mask == 0) absorbs rank r+mask.
@@ -297,7 +334,7 @@ __device__ __forceinline__ void combine(const RawPack (&raw)[C::K], float (&acc)
 #pragma unroll
         for (int mask = 1; mask < C::K; mask <<= 1)
 #pragma unroll
-            for (int r = 0; r + mask < C::K; r += 2 * mask) step_pack<C>(v[r], v[r + mask]);
+            for (int r = 0; r + mask < C::K; r += 2 * mask) step_pack<C>(v[r], v[r + mask], op);
 #pragma unroll
         for (int j = 0; j < C::E; ++j) acc[j] = v[0][j];
     }
@@ -322,15 +359,29 @@ __device__ __forceinline__ void store16(void* base, uint32_t pack, const float (
 // `has_out` / `has_wire`: which outputs the segment names (the pointers in `s` have
 // been advanced to the tile, so they no longer tell).  `fan` (fan-out kernels): the
 // result also goes to in[K .. K+fan-1], in the form `out` has.
-template <class C, bool FAN = false>
+template <class C, int OUT = kOutOne>
 __device__ __forceinline__ void store_pack(const SegArgs& s, bool has_out, bool has_wire, uint32_t pack,
                                            const float (&y)[C::E], int fan = 0) {
+    if constexpr (OUT == kOutAll) {
+        if constexpr (C::W == MCCLX_F32 || C::kOutF32) {
+            u32x4 t;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) t[j] = __float_as_uint(y[j]);
+#pragma unroll
+            for (int k = 0; k < C::K; ++k)
+                MCCLX_STG(gptr<u32x4_a4>(static_cast<float*>(const_cast<void*>(s.in[k])) + pack * C::E), t);
+        } else {
+#pragma unroll
+            for (int k = 0; k < C::K; ++k) store16<C>(const_cast<void*>(s.in[k]), pack, y);
+        }
+        return;
+    }
     if constexpr (C::W == MCCLX_F32 || C::kOutF32) {
         u32x4 t;
 #pragma unroll
         for (int j = 0; j < 4; ++j) t[j] = __float_as_uint(y[j]);
         if (has_out) MCCLX_STG(gptr<u32x4_a4>(static_cast<float*>(s.out) + pack * C::E), t);
-        if constexpr (FAN) {
+        if constexpr (OUT == kOutFan) {
 #pragma unroll
             for (int f = 0; f < MCCLX_MAX_INPUTS - C::K; ++f)
                 if (f < fan)
@@ -343,7 +394,7 @@ __device__ __forceinline__ void store_pack(const SegArgs& s, bool has_out, bool 
         } else {
             if (has_out) store16<C>(s.out, pack, y);
             if (has_wire) store16<C>(s.wire_out, pack, y);
-            if constexpr (FAN) {
+            if constexpr (OUT == kOutFan) {
 #pragma unroll
                 for (int f = 0; f < MCCLX_MAX_INPUTS - C::K; ++f)
                     if (f < fan) store16<C>(const_cast<void*>(s.in[C::K + f]), pack, y);
@@ -365,23 +416,34 @@ __device__ __forceinline__ void load_elems(const SegArgs& s, uint64_t i, float (
     v[k] = load_elem<C, k>(s, i);
     if constexpr (k + 1 < C::K) load_elems<C, k + 1>(s, i, v);
 }
-template <class C, bool FAN = false>
-__device__ __forceinline__ void fold_elem(const SegArgs& s, uint64_t i, float scale, bool has_scale, int fan = 0) {
+template <class C, int OUT = kOutOne>
+__device__ __forceinline__ void fold_elem(const SegArgs& s, uint64_t i, float scale, bool has_scale, int fan = 0,
+                                          int op = C::OP) {
     float v[C::K];
     load_elems<C, 0>(s, i, v);
     if constexpr (C::TOPO == MCCLX_TOPO_FOLD) {
 #pragma unroll
-        for (int k = 1; k < C::K; ++k) v[0] = step<C>(v[0], v[k]);
+        for (int k = 1; k < C::K; ++k) v[0] = step<C>(v[0], v[k], op);
     } else {
 #pragma unroll
         for (int mask = 1; mask < C::K; mask <<= 1)
 #pragma unroll
-            for (int r = 0; r + mask < C::K; r += 2 * mask) v[r] = step<C>(v[r], v[r + mask]);
+            for (int r = 0; r + mask < C::K; r += 2 * mask) v[r] = step<C>(v[r], v[r + mask], op);
     }
     float y = finish<C>(v[0], scale, has_scale);
+    if constexpr (OUT == kOutAll) {
+#pragma unroll
+        for (int k = 0; k < C::K; ++k) {
+            if constexpr (C::W == MCCLX_F32 || C::kOutF32)
+                gptr<float>(const_cast<void*>(s.in[k]))[i] = y;
+            else
+                gptr<uint16_t>(const_cast<void*>(s.in[k]))[i] = (uint16_t)Num<C::W>::enc(y);
+        }
+        return;
+    }
     if constexpr (C::W == MCCLX_F32 || C::kOutF32) {
         if (s.out) gptr<float>(s.out)[i] = y;
-        if constexpr (FAN) {
+        if constexpr (OUT == kOutFan) {
 #pragma unroll
             for (int f = 0; f < MCCLX_MAX_INPUTS - C::K; ++f)
                 if (f < fan) gptr<float>(const_cast<void*>(s.in[C::K + f]))[i] = y;
@@ -394,7 +456,7 @@ __device__ __forceinline__ void fold_elem(const SegArgs& s, uint64_t i, float sc
         } else {
             if (s.out) gptr<uint16_t>(s.out)[i] = h;
             if (s.wire_out) gptr<uint16_t>(s.wire_out)[i] = h;
-            if constexpr (FAN) {
+            if constexpr (OUT == kOutFan) {
 #pragma unroll
                 for (int f = 0; f < MCCLX_MAX_INPUTS - C::K; ++f)
                     if (f < fan) gptr<uint16_t>(const_cast<void*>(s.in[C::K + f]))[i] = h;
@@ -406,9 +468,9 @@ __device__ __forceinline__ void fold_elem(const SegArgs& s, uint64_t i, float sc
 // U packets per lane: all loads first, then arithmetic, then stores.  `s` points
 // at the tile's first packet; pk[] are packet indices inside the tile, so every
 // address is a uniform 64-bit base plus a 32-bit lane offset.
-template <class C, int U, bool FAN = false>
+template <class C, int U, int OUT = kOutOne>
 __device__ __forceinline__ void fold_packs(const SegArgs& s, bool has_out, bool has_wire, const uint32_t (&pk)[U],
-                                           float scale, bool has_scale, int fan = 0) {
+                                           float scale, bool has_scale, int fan = 0, int op = C::OP) {
     RawPack raw[C::K][U];
     load_all<C, 0, U>(s, pk, raw);
 #pragma unroll
@@ -417,18 +479,19 @@ __device__ __forceinline__ void fold_packs(const SegArgs& s, bool has_out, bool 
 #pragma unroll
         for (int k = 0; k < C::K; ++k) col[k] = raw[k][u];
         float acc[C::E];
-        combine<C>(col, acc);
+        combine<C>(col, acc, op);
         finish_pack<C>(acc, scale, has_scale);
-        store_pack<C, FAN>(s, has_out, has_wire, pk[u], acc, fan);
+        store_pack<C, OUT>(s, has_out, has_wire, pk[u], acc, fan);
     }
 }
 
 // Elements in front of the packet grid: up to the 128-byte boundary of the
 // buffer the widest stores go to.
-template <class C>
+template <class C, int OUT = kOutOne>
 __device__ __forceinline__ uint32_t head_elems(const SegArgs& s) {
-    const bool wide_out = (C::W == MCCLX_F32 || C::kOutF32) && s.out;
-    const uint32_t a = (uint32_t)reinterpret_cast<uintptr_t>(s.out ? s.out : s.wire_out);
+    const bool wide_out = (C::W == MCCLX_F32 || C::kOutF32) && (OUT == kOutAll || s.out);
+    const void* first = OUT == kOutAll ? s.in[0] : s.out ? s.out : s.wire_out;
+    const uint32_t a = (uint32_t)reinterpret_cast<uintptr_t>(first);
     const uint32_t mis = a & 127u;
     const uint32_t h = mis ? (128u - mis) >> (wide_out ? 2 : 1) : 0u;
     return s.count < h ? (uint32_t)s.count : h;
@@ -436,7 +499,7 @@ __device__ __forceinline__ uint32_t head_elems(const SegArgs& s) {
 
 // Every pointer of the segment moved `elems` elements on (null outputs become
 // garbage: the caller keeps their presence in flags).
-template <class C, bool FAN = false>
+template <class C, int OUT = kOutOne>
 __device__ __forceinline__ SegArgs advanced(const SegArgs& s, uint64_t elems) {
     SegArgs t;
     const uint64_t b2 = elems * 2, b4 = elems * 4;
@@ -447,7 +510,7 @@ __device__ __forceinline__ SegArgs advanced(const SegArgs& s, uint64_t elems) {
     for (int k = 0; k < MCCLX_MAX_INPUTS; ++k) {
         if (k < C::K)
             t.in[k] = static_cast<const char*>(s.in[k]) + (C::in_is_f32(k) ? b4 : b2);
-        else if constexpr (FAN)
+        else if constexpr (OUT == kOutFan)
             t.in[k] = static_cast<const char*>(s.in[k]) + (out_f32 ? b4 : b2);  // a further destination
         else
             t.in[k] = nullptr;
@@ -462,34 +525,34 @@ __device__ __forceinline__ SegArgs advanced(const SegArgs& s, uint64_t elems) {
 // load is kept short -- a block lives for about 2 us and eight waves per SIMD
 // share one scalar unit, so every scalar instruction in front of the loads is
 // paid eight times over.
-template <class C, bool FAN = false>
+template <class C, int OUT = kOutOne>
 __device__ __forceinline__ void fold_tile(const SegArgs& s, float scale, bool has_scale, uint64_t first,
-                                          bool do_edges, int fan = 0) {
+                                          bool do_edges, int fan = 0, int op = C::OP) {
     constexpr int U = C::U;
     const uint32_t tid = threadIdx.x;
     constexpr int kB = C::BLOCK;
-    const uint32_t head = head_elems<C>(s);  // < 64 <= kB
+    const uint32_t head = head_elems<C, OUT>(s);  // < 64 <= kB
     const uint64_t P = (s.count - head) / C::E;
     const bool has_out = s.out != nullptr, has_wire = s.wire_out != nullptr;
     if (first < P) {
-        const SegArgs t = advanced<C, FAN>(s, head + first * C::E);
+        const SegArgs t = advanced<C, OUT>(s, head + first * C::E);
         const uint64_t left = P - first;
         if (left >= (uint64_t)U * kB) {
             uint32_t pk[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) pk[u] = (uint32_t)u * kB + tid;
-            fold_packs<C, U, FAN>(t, has_out, has_wire, pk, scale, has_scale, fan);
+            fold_packs<C, U, OUT>(t, has_out, has_wire, pk, scale, has_scale, fan, op);
         } else {
             for (uint32_t p = tid; p < (uint32_t)left; p += kB) {
                 uint32_t one[1] = {p};
-                fold_packs<C, 1, FAN>(t, has_out, has_wire, one, scale, has_scale, fan);
+                fold_packs<C, 1, OUT>(t, has_out, has_wire, one, scale, has_scale, fan, op);
             }
         }
     }
     if (do_edges) {
-        if (tid < head) fold_elem<C, FAN>(s, tid, scale, has_scale, fan);
+        if (tid < head) fold_elem<C, OUT>(s, tid, scale, has_scale, fan, op);
         const uint64_t i = head + P * C::E + tid;  // fewer than E <= 8 elements remain
-        if (i < s.count) fold_elem<C, FAN>(s, i, scale, has_scale, fan);
+        if (i < s.count) fold_elem<C, OUT>(s, i, scale, has_scale, fan, op);
     }
 }
 
@@ -504,9 +567,12 @@ __device__ __forceinline__ void fold_tile(const SegArgs& s, float scale, bool ha
 // blocks live for 2 us.  The empty asm makes every field live at one point.
 // Only the K operand pointers the plan reads are fetched: scalar registers are
 // what decides how many blocks a CU holds (see fold_few_kernel).
-template <int K>
+template <int K, int OUT>
 __device__ __forceinline__ void fetch_together(SegArgs& s, float& scale, int32_t& has_scale, uint32_t& grid) {
-    asm volatile("" : "+s"(s.out), "+s"(s.wire_out), "+s"(s.count), "+s"(scale), "+s"(has_scale), "+s"(grid));
+    if constexpr (OUT == kOutAll)
+        asm volatile("" : "+s"(s.count), "+s"(scale), "+s"(has_scale), "+s"(grid));
+    else
+        asm volatile("" : "+s"(s.out), "+s"(s.wire_out), "+s"(s.count), "+s"(scale), "+s"(has_scale), "+s"(grid));
 #pragma unroll
     for (int k = 0; k < K; ++k) asm volatile("" : "+s"(s.in[k]));
 }
@@ -519,7 +585,7 @@ __device__ __forceinline__ void fetch_together(SegArgs& s, float& scale, int32_t
 // kernel with more starts 768 blocks at launch instead of 1024 and streams
 // 2-4 % slower.  Six registers are set aside on top of what the code uses (VCC,
 // flat scratch, XNACK mask), so the code itself has 74.
-template <class C, bool FAN = false>
+template <class C, int OUT = kOutOne>
 __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
 #if MCCLX_TUNE_TIMELINE
     const uint64_t t_start = wall_clock64();
@@ -528,9 +594,9 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
     float scale = a.scale;
     int32_t has_scale = a.has_scale;
     uint32_t grid = gridDim.x;
-    fetch_together<FAN ? MCCLX_MAX_INPUTS : C::K>(s, scale, has_scale, grid);
+    fetch_together<OUT == kOutFan ? MCCLX_MAX_INPUTS : C::K, OUT>(s, scale, has_scale, grid);
     int32_t fan = 0;
-    if constexpr (FAN) fan = a.fan;
+    if constexpr (OUT == kOutFan) fan = a.fan;
 #if MCCLX_TUNE_TIMELINE
     const uint64_t t_args = wall_clock64();
 #endif
@@ -539,7 +605,9 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
     // dispatched in address order (giving each XCD one contiguous part of a segment instead was
     // level on a 25 MiB bucket and 3.5-9 % slower on large operands).
     (void)grid;
-    fold_tile<C, FAN>(s, scale, has_scale != 0, (uint64_t)blockIdx.x * span, blockIdx.x == 0, fan);
+    int op = C::OP;
+    if constexpr (C::OP == kAnyOp) op = a.op;
+    fold_tile<C, OUT>(s, scale, has_scale != 0, (uint64_t)blockIdx.x * span, blockIdx.x == 0, fan, op);
 #if MCCLX_TUNE_TIMELINE
     if (a.timeline && threadIdx.x == 0) {
         TimelineRecord r;
@@ -560,13 +628,16 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
 template <class C> constexpr bool kLightPlan = C::K <= 4;
 
 template <class C>
-__global__ void __launch_bounds__(C::BLOCK) MCCLX_SGPR_CAP fold_few_kernel(FewArgs a) { fold_few_body<C>(a); }
+__global__ void __launch_bounds__(C::BLOCK) MCCLX_SGPR_CAP fold_few_kernel(FewArgs a) { fold_few_body<C, kOutOne>(a); }
 template <class C>
-__global__ void __launch_bounds__(C::BLOCK) fold_few_wide_kernel(FewArgs a) { fold_few_body<C>(a); }
+__global__ void __launch_bounds__(C::BLOCK) fold_few_wide_kernel(FewArgs a) { fold_few_body<C, kOutOne>(a); }
 // Fan-out form: the result also goes to in[K .. K+fan-1] (the other ranks' tensors: the
 // allgather leg of an allreduce done by the reduce itself, stores instead of a second pass).
 template <class C>
-__global__ void __launch_bounds__(C::BLOCK) fold_few_fan_kernel(FewArgs a) { fold_few_body<C, true>(a); }
+__global__ void __launch_bounds__(C::BLOCK) fold_few_fan_kernel(FewArgs a) { fold_few_body<C, kOutFan>(a); }
+// To-all form: the result goes back into every operand's buffer.
+template <class C>
+__global__ void __launch_bounds__(C::BLOCK) fold_few_all_kernel(FewArgs a) { fold_few_body<C, kOutAll>(a); }
 
 #if MCCLX_TUNE_TIMELINE
 // Where the next by-value launches put their records (measurement build): a caller-provided
@@ -597,20 +668,20 @@ TimelineRecord* timeline_next(uint64_t blocks);
 // packets per lane would cover more, but from about 80 MB read on the plain
 // form has caught up (a 40 MiB bucket at T = 7: 21.0 us against 20.7 us); and
 // 256-lane blocks run the C2 fold in 14.3 us where 512-lane blocks take 13.1 us.
-template <class C, int T, int kHoldBlock, bool FAN>
+template <class C, int T, int kHoldBlock, int OUT>
 __global__ void __launch_bounds__(kHoldBlock) fold_few_hold_kernel(FewArgs a, uint32_t gate) {
     const uint64_t t_start = wall_clock64();
     SegArgs s = a.seg[blockIdx.y];
     float scale = a.scale;
     int32_t has_scale = a.has_scale;
     uint32_t grid = gridDim.x;
-    fetch_together<FAN ? MCCLX_MAX_INPUTS : C::K>(s, scale, has_scale, grid);
+    fetch_together<OUT == kOutFan ? MCCLX_MAX_INPUTS : C::K, OUT>(s, scale, has_scale, grid);
     int32_t fan = 0;
-    if constexpr (FAN) fan = a.fan;
-    const uint32_t head = head_elems<C>(s);
+    if constexpr (OUT == kOutFan) fan = a.fan;
+    const uint32_t head = head_elems<C, OUT>(s);
     const uint64_t P = (s.count - head) / C::E;
     const bool has_out = s.out != nullptr, has_wire = s.wire_out != nullptr;
-    const SegArgs t = advanced<C, FAN>(s, head);
+    const SegArgs t = advanced<C, OUT>(s, head);
     // packet u of lane l is packet u * L + l of the segment: consecutive lanes, consecutive packets
     const uint32_t L = grid * kHoldBlock;
     const uint32_t lane = blockIdx.x * kHoldBlock + threadIdx.x;
@@ -665,12 +736,18 @@ __global__ void __launch_bounds__(kHoldBlock) fold_few_hold_kernel(FewArgs a, ui
             if constexpr (C::E == 4) {
                 const float y[C::E] = {__uint_as_float(raw[0][u].x), __uint_as_float(raw[0][u].y), __uint_as_float(raw[0][u].z),
                                        __uint_as_float(raw[0][u].w)};
-                store_pack<C, FAN>(t, has_out, has_wire, p, y, fan);
+                store_pack<C, OUT>(t, has_out, has_wire, p, y, fan);
             } else {  // all streams 16-bit: the packed result goes out as it is
                 const u32x4 bits = raw[0][u];
+                if constexpr (OUT == kOutAll) {
+#pragma unroll
+                    for (int k = 0; k < C::K; ++k)
+                        MCCLX_STG(gptr<u32x4_a2>(static_cast<uint16_t*>(const_cast<void*>(t.in[k])) + p * C::E), bits);
+                    continue;
+                }
                 if (has_out) MCCLX_STG(gptr<u32x4_a2>(static_cast<uint16_t*>(t.out) + p * C::E), bits);
                 if (has_wire) MCCLX_STG(gptr<u32x4_a2>(static_cast<uint16_t*>(t.wire_out) + p * C::E), bits);
-                if constexpr (FAN) {
+                if constexpr (OUT == kOutFan) {
 #pragma unroll
                     for (int f = 0; f < MCCLX_MAX_INPUTS - C::K; ++f)
                         if (f < fan)
@@ -680,9 +757,9 @@ __global__ void __launch_bounds__(kHoldBlock) fold_few_hold_kernel(FewArgs a, ui
         }
     }
     if (blockIdx.x == 0) {  // the elements in front of and behind the packet grid
-        if (threadIdx.x < head) fold_elem<C, FAN>(s, threadIdx.x, scale, has_scale != 0, fan);
+        if (threadIdx.x < head) fold_elem<C, OUT>(s, threadIdx.x, scale, has_scale != 0, fan);
         const uint64_t i = head + P * C::E + threadIdx.x;
-        if (i < s.count) fold_elem<C, FAN>(s, i, scale, has_scale != 0, fan);
+        if (i < s.count) fold_elem<C, OUT>(s, i, scale, has_scale != 0, fan);
     }
 #if MCCLX_TUNE_TIMELINE
     if (a.timeline && threadIdx.x == 0) {
@@ -709,11 +786,11 @@ constexpr bool kHoldPlan = ((C::K >= 2 && C::K <= 4) || kHoldEncode<C>) && C::OP
                            C::ACC == MCCLX_ACC_STEP && C::TOPO == MCCLX_TOPO_FOLD;
 
 // Blocks of one generation: what the device holds at once of this kernel.
-template <class C, int T, int HB, bool FAN>
+template <class C, int T, int HB, int OUT>
 static uint32_t hold_capacity(int cus) {
     static const int per_cu = [] {
         int n = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fold_few_hold_kernel<C, T, HB, FAN>, HB, 0) != hipSuccess) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fold_few_hold_kernel<C, T, HB, OUT>, HB, 0) != hipSuccess) {
             (void)hipGetLastError();
             n = 0;
         }
@@ -722,9 +799,9 @@ static uint32_t hold_capacity(int cus) {
     return (uint32_t)(per_cu * cus);
 }
 
-template <class C, int T, int HB, bool FAN>
+template <class C, int T, int HB, int OUT>
 static bool hold_launch(hipStream_t st, FewArgs& a, uint64_t packets, uint32_t gate, const LaunchParams& lp) {
-    const uint32_t cap = hold_capacity<C, T, HB, FAN>(lp.cus);
+    const uint32_t cap = hold_capacity<C, T, HB, OUT>(lp.cus);
     if (cap < (uint32_t)a.nseg) return false;
     uint32_t hx = cap / (uint32_t)a.nseg;
     if (packets > (uint64_t)hx * HB * T) return false;
@@ -738,12 +815,12 @@ static bool hold_launch(hipStream_t st, FewArgs& a, uint64_t packets, uint32_t g
 #if MCCLX_TUNE_TIMELINE
     a.timeline = timeline_next((uint64_t)hx * (uint64_t)a.nseg);
 #endif
-    fold_few_hold_kernel<C, T, HB, FAN><<<dim3(hx, (uint32_t)a.nseg), dim3(HB), 0, st>>>(a, gate);
+    fold_few_hold_kernel<C, T, HB, OUT><<<dim3(hx, (uint32_t)a.nseg), dim3(HB), 0, st>>>(a, gate);
     return true;
 }
 
 // Takes the launch if it reads enough for the separation to pay and one generation covers it.
-template <class C, bool FAN>
+template <class C, int OUT>
 static bool try_hold(hipStream_t st, FewArgs& a, uint64_t maxc, const LaunchParams& lp) {
     if (!lp.hold_min_read_bytes || lp.cus <= 0) return false;
     uint64_t read_bytes = 0;
@@ -751,7 +828,7 @@ static bool try_hold(hipStream_t st, FewArgs& a, uint64_t maxc, const LaunchPara
         for (int k = 0; k < C::K; ++k) read_bytes += a.seg[i].count * (C::in_is_f32(k) ? 4 : 2);
     // measured break-even: 10 MiB read for a fold with one output, half as much again for one that
     // writes as much as it reads (fan-out)
-    if (read_bytes < (FAN ? lp.hold_min_read_bytes * 3 / 2 : lp.hold_min_read_bytes)) return false;
+    if (read_bytes < (OUT != kOutOne ? lp.hold_min_read_bytes * 3 / 2 : lp.hold_min_read_bytes)) return false;
     // The encode: measured on 1-8 tensors of 1-40 MiB, the form wins 4-10 % from three tensors and
     // 18 MiB read on (three of 25 MiB: 20.6 -> 19.0 us); on one or two tensors it ties or loses.
     if constexpr (kHoldEncode<C>)
@@ -760,7 +837,7 @@ static bool try_hold(hipStream_t st, FewArgs& a, uint64_t maxc, const LaunchPara
     // the encode writes half of what it reads and does best with its stores a little early
     if constexpr (kHoldEncode<C>) ticks = lp.hold_latency_ticks + read_bytes * 100 / (lp.hold_bytes_per_tick * kHoldEncodeEarlyPct);
     uint32_t gate5 = 0;  // a fan-out fold at five packets per lane (fewer waves, more loads each): its reads take 3 % longer
-    if constexpr (FAN) {
+    if constexpr (OUT == kOutFan) {
         const uint64_t t5 = lp.hold_latency_ticks + read_bytes * 100 / (lp.hold_bytes_per_tick * kHoldFanLatePct);
         gate5 = t5 > 100000 ? 100000u : (uint32_t)t5;
     }
@@ -771,9 +848,9 @@ static bool try_hold(hipStream_t st, FewArgs& a, uint64_t maxc, const LaunchPara
     // 26.7 us at five.)
     bool took;
     if constexpr (kHoldEncode<C>)
-        took = hold_launch<C, 10, 512, false>(st, a, packets, gate, lp);
+        took = hold_launch<C, 10, 512, kOutOne>(st, a, packets, gate, lp);
     else
-        took = hold_launch<C, 4, 512, FAN>(st, a, packets, gate, lp) || hold_launch<C, 5, 512, FAN>(st, a, packets, FAN ? gate5 : gate, lp);
+        took = hold_launch<C, 4, 512, OUT>(st, a, packets, gate, lp) || hold_launch<C, 5, 512, OUT>(st, a, packets, OUT != kOutOne ? gate5 : gate, lp);
     if (took && lp.held) *lp.held = true;
     return took;
 }
@@ -796,7 +873,7 @@ __device__ __forceinline__ P* uniptr(P* p) {
 // blockIdx.x + gridDim.x, ...  (one item per block unless the grid is capped).
 // The loop bound is fixed at launch, so every wave exits.  total_items < 2^31
 // (checked by the host).
-template <class C, bool FAN = false>
+template <class C, int OUT = kOutOne>
 __device__ __forceinline__ void fold_table_body(const TableArgs& a) {
     const uint64_t span = (uint64_t)C::U * C::BLOCK;
     const uint32_t total = (uint32_t)a.total_items;
@@ -824,13 +901,14 @@ __device__ __forceinline__ void fold_table_body(const TableArgs& a) {
         tile = uni32(tile);
         const SegArgs* __restrict__ d = a.segs + seg;
         SegArgs s;
-        s.out = uniptr(d->out);
-        s.wire_out = uniptr(d->wire_out);
+        s.out = OUT == kOutAll ? nullptr : uniptr(d->out);
+        s.wire_out = OUT == kOutAll ? nullptr : uniptr(d->wire_out);
 #pragma unroll
-        for (int k = 0; k < MCCLX_MAX_INPUTS; ++k) s.in[k] = (k < C::K || FAN) ? uniptr(d->in[k]) : nullptr;
+        for (int k = 0; k < MCCLX_MAX_INPUTS; ++k) s.in[k] = (k < C::K || OUT == kOutFan) ? uniptr(d->in[k]) : nullptr;
         s.count = uni64(d->count);
         // one tile: packets [tile*span, tile*span + span); tile 0 also owns the tail
-        fold_tile<C, FAN>(s, a.scale, a.has_scale != 0, (uint64_t)tile * span, tile == 0, FAN ? a.fan : 0);
+        fold_tile<C, OUT>(s, a.scale, a.has_scale != 0, (uint64_t)tile * span, tile == 0, OUT == kOutFan ? a.fan : 0,
+                          C::OP == kAnyOp ? a.op : C::OP);
     }
 }
 
@@ -839,7 +917,10 @@ __global__ void __launch_bounds__(C::BLOCK) MCCLX_SGPR_CAP fold_table_kernel(Tab
 template <class C>
 __global__ void __launch_bounds__(C::BLOCK) fold_table_wide_kernel(TableArgs a) { fold_table_body<C>(a); }
 template <class C>
-__global__ void __launch_bounds__(C::BLOCK) fold_table_fan_kernel(TableArgs a) { fold_table_body<C, true>(a); }
+__global__ void __launch_bounds__(C::BLOCK) fold_table_fan_kernel(TableArgs a) { fold_table_body<C, kOutFan>(a); }
+
+template <class C>
+__global__ void __launch_bounds__(C::BLOCK) fold_table_all_kernel(TableArgs a) { fold_table_body<C, kOutAll>(a); }
 
 // Plans with a fan-out form (host mirror: fan_plan_ok).
 template <class C>
@@ -848,66 +929,80 @@ constexpr bool kFanPlan = C::OP == MCCLX_SUM && C::ACC == MCCLX_ACC_STEP && C::K
 
 // ----------------------------------------------------------------- dispatch
 
+// A by-value launch: one block per tile of the longest segment, the hold form where it applies.
+template <class C, int OUT>
+static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchParams& lp) {
+    FewArgs a = args;
+    uint64_t maxc = 0;
+    for (int i = 0; i < a.nseg; ++i) maxc = a.seg[i].count > maxc ? a.seg[i].count : maxc;
+    if (maxc == 0) return hipSuccess;
+#if MCCLX_TUNE_TIMELINE
+    a.timeline = nullptr;
+#endif
+    if constexpr (kHoldPlan<C>)
+        if (try_hold<C, OUT>(st, a, maxc, lp)) return hipGetLastError();
+    const uint64_t span = (uint64_t)C::U * C::BLOCK * C::E;  // elements per block iteration
+    const uint64_t gx = (maxc + span - 1) / span;
+    if (gx >> 31) return hipErrorInvalidValue;
+    const dim3 grid((uint32_t)gx, (uint32_t)a.nseg), block(C::BLOCK);
+#if MCCLX_TUNE_TIMELINE
+    if (OUT == kOutOne) a.timeline = timeline_next(gx * (uint64_t)a.nseg);
+#endif
+    if constexpr (OUT == kOutAll)
+        fold_few_all_kernel<C><<<grid, block, 0, st>>>(a);
+    else if constexpr (OUT == kOutFan)
+        fold_few_fan_kernel<C><<<grid, block, 0, st>>>(a);
+    else if constexpr (kLightPlan<C>)
+        fold_few_kernel<C><<<grid, block, 0, st>>>(a);
+    else
+        fold_few_wide_kernel<C><<<grid, block, 0, st>>>(a);
+    return hipGetLastError();
+}
+
+template <class C, int OUT>
+static hipError_t launch_table(hipStream_t st, const TableArgs& a, const LaunchParams& lp) {
+    const dim3 grid((uint32_t)(a.total_items < lp.max_blocks ? a.total_items : lp.max_blocks)), block(C::BLOCK);
+    if (grid.x == 0) return hipSuccess;
+    if constexpr (OUT == kOutAll)
+        fold_table_all_kernel<C><<<grid, block, 0, st>>>(a);
+    else if constexpr (OUT == kOutFan)
+        fold_table_fan_kernel<C><<<grid, block, 0, st>>>(a);
+    else if constexpr (kLightPlan<C>)
+        fold_table_kernel<C><<<grid, block, 0, st>>>(a);
+    else
+        fold_table_wide_kernel<C><<<grid, block, 0, st>>>(a);
+    return hipGetLastError();
+}
+
+template <class C, int OUT>
+static hipError_t launch_out(hipStream_t st, const LaunchParams& lp, int op) {
+    if (lp.table) {
+        TableArgs a = *lp.table;
+        a.fan = lp.fan;
+        a.op = op;
+        return launch_table<C, OUT>(st, a, lp);
+    }
+    FewArgs a = *lp.few;
+    a.fan = lp.fan;
+    a.op = op;
+    return launch_few<C, OUT>(st, a, lp);
+}
 
 template <class C>
 static hipError_t launch_cfg(hipStream_t st, const LaunchParams& lp) {
-    const uint64_t span = (uint64_t)C::U * C::BLOCK * C::E;  // elements per block iteration
     if (lp.fan > 0) {
-        if constexpr (!kFanPlan<C>) {
-            return hipErrorInvalidValue;
-        } else {
-            if (lp.fan > MCCLX_MAX_INPUTS - C::K) return hipErrorInvalidValue;
-            if (lp.table) {
-                TableArgs a = *lp.table;
-                a.fan = lp.fan;
-                uint32_t grid = (uint32_t)(a.total_items < lp.max_blocks ? a.total_items : lp.max_blocks);
-                if (grid == 0) return hipSuccess;
-                fold_table_fan_kernel<C><<<dim3(grid), dim3(C::BLOCK), 0, st>>>(a);
-            } else {
-                FewArgs a = *lp.few;
-                a.fan = lp.fan;
-                uint64_t maxc = 0;
-                for (int i = 0; i < a.nseg; ++i) maxc = a.seg[i].count > maxc ? a.seg[i].count : maxc;
-                if (maxc == 0) return hipSuccess;
-                uint64_t gx = (maxc + span - 1) / span;
-                if (gx >> 31) return hipErrorInvalidValue;
-#if MCCLX_TUNE_TIMELINE
-                a.timeline = nullptr;
-#endif
-                if constexpr (kHoldPlan<C>)
-                    if (try_hold<C, true>(st, a, maxc, lp)) return hipGetLastError();
-                fold_few_fan_kernel<C><<<dim3((uint32_t)gx, (uint32_t)a.nseg), dim3(C::BLOCK), 0, st>>>(a);
-            }
-            return hipGetLastError();
+        if constexpr (kFanPlan<C>) {
+            if (lp.fan <= MCCLX_MAX_INPUTS - C::K) return launch_out<C, kOutFan>(st, lp, C::OP);
         }
+        return hipErrorInvalidValue;
     }
-    if (lp.table) {
-        TableArgs a = *lp.table;
-        uint32_t grid = (uint32_t)(a.total_items < lp.max_blocks ? a.total_items : lp.max_blocks);
-        if (grid == 0) return hipSuccess;
-        if constexpr (kLightPlan<C>)
-            fold_table_kernel<C><<<dim3(grid), dim3(C::BLOCK), 0, st>>>(a);
-        else
-            fold_table_wide_kernel<C><<<dim3(grid), dim3(C::BLOCK), 0, st>>>(a);
-    } else {
-        FewArgs a = *lp.few;
-        uint64_t maxc = 0;
-        for (int i = 0; i < a.nseg; ++i) maxc = a.seg[i].count > maxc ? a.seg[i].count : maxc;
-        if (maxc == 0) return hipSuccess;
-        // one block per tile of the longest segment (the by-value kernel does not loop)
-        uint64_t gx = (maxc + span - 1) / span;
-        if (gx >> 31) return hipErrorInvalidValue;
-        if constexpr (kHoldPlan<C>)
-            if (try_hold<C, false>(st, a, maxc, lp)) return hipGetLastError();
-#if MCCLX_TUNE_TIMELINE
-        a.timeline = timeline_next(gx * (uint64_t)a.nseg);
-#endif
-        if constexpr (kLightPlan<C>)
-            fold_few_kernel<C><<<dim3((uint32_t)gx, (uint32_t)a.nseg), dim3(C::BLOCK), 0, st>>>(a);
-        else
-            fold_few_wide_kernel<C><<<dim3((uint32_t)gx, (uint32_t)a.nseg), dim3(C::BLOCK), 0, st>>>(a);
-    }
-    return hipGetLastError();
+    return launch_out<C, kOutOne>(st, lp, C::OP);
+}
+
+// The to-all form of a plan (all operands and the result of one form; host mirror: all_plan_ok).
+template <class C>
+static hipError_t launch_all(hipStream_t st, const PlanKey& key, const LaunchParams& lp) {
+    return launch_out<C, kOutAll>(st, lp, key.op);
 }
 
 // The kernel template is instantiated for every supported plan.  To keep build
@@ -963,6 +1058,10 @@ bool fan_plan_ok(const PlanKey& key) {
            key.io != MCCLX_IO_OUT_F32;
 }
 
+bool all_plan_ok(const PlanKey& key) {
+    return key.acc == MCCLX_ACC_STEP && key.k >= 2 && (key.io == MCCLX_IO_PURE || key.io == MCCLX_IO_ALL_F32);
+}
+
 int plan_unroll(const PlanKey& key) {
     if (key_is_wide(key)) return kWideU;
     if (key.topo == MCCLX_TOPO_BINOMIAL) return 1;
@@ -1014,6 +1113,29 @@ int plan_unroll(const PlanKey& key) {
         default: return hipErrorInvalidValue;                                                      \
     }
 
+#define MCCLX_ALL_K(W, IO, TOPO, OP)                                                    \
+    switch (key.k) {                                                                    \
+        case 2: return launch_all<Cfg<W, IO, 2, MCCLX_TOPO_FOLD, OP, MCCLX_ACC_STEP>>(st, key, lp); \
+        case 3: return launch_all<Cfg<W, IO, 3, MCCLX_TOPO_FOLD, OP, MCCLX_ACC_STEP>>(st, key, lp); \
+        case 4: return launch_all<Cfg<W, IO, 4, TOPO, OP, MCCLX_ACC_STEP>>(st, key, lp); \
+        case 5: return launch_all<Cfg<W, IO, 5, TOPO, OP, MCCLX_ACC_STEP>>(st, key, lp); \
+        case 6: return launch_all<Cfg<W, IO, 6, TOPO, OP, MCCLX_ACC_STEP>>(st, key, lp); \
+        case 7: return launch_all<Cfg<W, IO, 7, TOPO, OP, MCCLX_ACC_STEP>>(st, key, lp); \
+        case 8: return launch_all<Cfg<W, IO, 8, TOPO, OP, MCCLX_ACC_STEP>>(st, key, lp); \
+        default: return hipErrorInvalidValue;                                           \
+    }
+#define MCCLX_ALL_CASES(W, IO)                                                          \
+    if (key.op == MCCLX_SUM) {                                                          \
+        if (key.topo == MCCLX_TOPO_BINOMIAL) MCCLX_ALL_K(W, IO, MCCLX_TOPO_BINOMIAL, MCCLX_SUM) \
+        MCCLX_ALL_K(W, IO, MCCLX_TOPO_FOLD, MCCLX_SUM)                                  \
+    }                                                                                   \
+    if (key.topo == MCCLX_TOPO_BINOMIAL) MCCLX_ALL_K(W, IO, MCCLX_TOPO_BINOMIAL, kAnyOp) \
+    MCCLX_ALL_K(W, IO, MCCLX_TOPO_FOLD, kAnyOp)
+
+hipError_t launch_part_all_f32(hipStream_t st, const PlanKey& key, const LaunchParams& lp);
+hipError_t launch_part_all_f16(hipStream_t st, const PlanKey& key, const LaunchParams& lp);
+hipError_t launch_part_all_bf16(hipStream_t st, const PlanKey& key, const LaunchParams& lp);
+hipError_t launch_part_all_bf16_f32(hipStream_t st, const PlanKey& key, const LaunchParams& lp);
 hipError_t launch_part_sum_f32_f16(hipStream_t st, const PlanKey& key, const LaunchParams& lp);
 hipError_t launch_part_sum_bf16_step(hipStream_t st, const PlanKey& key, const LaunchParams& lp);
 hipError_t launch_part_sum_bf16_f32acc(hipStream_t st, const PlanKey& key, const LaunchParams& lp);
@@ -1024,6 +1146,12 @@ hipError_t launch_part_ops_bf16(hipStream_t st, const PlanKey& key, const Launch
 
 #if MCCLX_HAS_PART(0)
 hipError_t launch_fold(hipStream_t st, const PlanKey& key, const LaunchParams& lp) {
+    if (lp.to_all) {
+        if (!all_plan_ok(key)) return hipErrorInvalidValue;
+        if (key.io == MCCLX_IO_ALL_F32) return launch_part_all_bf16_f32(st, key, lp);
+        return key.dtype == MCCLX_F32 ? launch_part_all_f32(st, key, lp)
+               : key.dtype == MCCLX_F16 ? launch_part_all_f16(st, key, lp) : launch_part_all_bf16(st, key, lp);
+    }
     if (key.op != MCCLX_SUM) {
         if (key.io != MCCLX_IO_PURE || key.acc != MCCLX_ACC_STEP) return hipErrorInvalidValue;
         switch (key.dtype) {
@@ -1087,6 +1215,24 @@ hipError_t launch_part_sum_bf16_all_f32(hipStream_t st, const PlanKey& key, cons
         MCCLX_TOPO_CASES(MCCLX_BF16, MCCLX_IO_ALL_F32, MCCLX_SUM, MCCLX_ACC_STEP)
     }
     MCCLX_TOPO_CASES(MCCLX_BF16, MCCLX_IO_ALL_F32, MCCLX_SUM, MCCLX_ACC_F32)
+}
+#endif
+
+#if MCCLX_HAS_PART(7)
+hipError_t launch_part_all_f32(hipStream_t st, const PlanKey& key, const LaunchParams& lp) {
+    MCCLX_ALL_CASES(MCCLX_F32, MCCLX_IO_PURE)
+}
+hipError_t launch_part_all_f16(hipStream_t st, const PlanKey& key, const LaunchParams& lp) {
+    MCCLX_ALL_CASES(MCCLX_F16, MCCLX_IO_PURE)
+}
+#endif
+
+#if MCCLX_HAS_PART(8)
+hipError_t launch_part_all_bf16(hipStream_t st, const PlanKey& key, const LaunchParams& lp) {
+    MCCLX_ALL_CASES(MCCLX_BF16, MCCLX_IO_PURE)
+}
+hipError_t launch_part_all_bf16_f32(hipStream_t st, const PlanKey& key, const LaunchParams& lp) {
+    MCCLX_ALL_CASES(MCCLX_BF16, MCCLX_IO_ALL_F32)
 }
 #endif
 

@@ -40,6 +40,7 @@ struct FewArgs {
     int32_t has_scale;
     int32_t nseg;
     int32_t fan;        // further destinations of the result, in[k .. k+fan-1] (fan-out kernels only)
+    int32_t op;         // the operator, where the kernel takes it from here (to-all kernels of MIN, MAX, PRODUCT)
 #if MCCLX_TUNE_TIMELINE
     TimelineRecord* timeline;  // this launch's records, one per block (x fastest, then y), or null
 #endif
@@ -55,6 +56,7 @@ struct TableArgs {
     float scale;
     int32_t has_scale;
     int32_t fan;                 // further destinations of the result, in[k .. k+fan-1] (fan-out kernels only)
+    int32_t op;                  // as FewArgs::op
 };
 
 // Kernel-side operator codes beyond the public MCCLX_* ones: MIN / MAX with the
@@ -70,6 +72,7 @@ struct LaunchParams {
     const TableArgs* table = nullptr;
     uint32_t max_blocks = 0;           // cap on the grid (persistent sizing)
     int fan = 0;                       // > 0: the fan-out form of the kernel (plans in fan_plan_ok only)
+    bool to_all = false;               // the to-all form: the result goes back into every operand (all_plan_ok only)
     // Reads-then-writes form of a by-value launch that one generation of blocks covers:
     // taken when the launch reads at least hold_min_read_bytes (0 = never); no lane stores
     // before hold_latency_ticks + read bytes / hold_bytes_per_tick ticks of the 100 MHz
@@ -82,6 +85,8 @@ struct LaunchParams {
 };
 // Plans that have a fan-out form: sums with per-step rounding, 2..7 operands.
 bool fan_plan_ok(const PlanKey& key);
+// Plans that have a to-all form: per-step rounding, every operand in the form of the result.
+bool all_plan_ok(const PlanKey& key);
 
 // Packets-per-lane unroll and threads per block the kernel template uses for this plan.
 int plan_unroll(const PlanKey& key);

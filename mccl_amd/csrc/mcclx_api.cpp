@@ -203,11 +203,15 @@ int normalize_op(int op, int* out) {
     }
 }
 
+constexpr int kToAll = -1;  // in the place of a number of further destinations: MCCLX_PLAN_TO_ALL
+
 int check_plan(const mcclx_plan* p, mcclx::PlanKey* key, float* scale_f, int* has_scale, int* fan) {
     if (!p) return fail(MCCLX_ERR_INVALID, "plan is null");
-    if (p->flags & ~(MCCLX_PLAN_ACC_IS_SRC | MCCLX_PLAN_FANOUT_MASK))
+    if (p->flags & ~(MCCLX_PLAN_ACC_IS_SRC | MCCLX_PLAN_TO_ALL | MCCLX_PLAN_FANOUT_MASK))
         return fail(MCCLX_ERR_INVALID, "plan.flags=%d has unknown bits", p->flags);
     *fan = (p->flags & MCCLX_PLAN_FANOUT_MASK) >> MCCLX_PLAN_FANOUT_SHIFT;
+    const bool to_all = p->flags & MCCLX_PLAN_TO_ALL;
+    if (to_all && *fan) return fail(MCCLX_ERR_INVALID, "plan.flags=%d: to-all excludes fan-out", p->flags);
     if (!dtype_ok(p->dtype))
         return fail(MCCLX_ERR_UNSUPPORTED, "No kernel for dtype code %d", p->dtype);
     if (p->k < 1 || p->k > MCCLX_MAX_INPUTS)
@@ -222,7 +226,7 @@ int check_plan(const mcclx_plan* p, mcclx::PlanKey* key, float* scale_f, int* ha
         return fail(MCCLX_ERR_INVALID, "plan.topo=%d unknown", p->topo);
     if (p->acc != MCCLX_ACC_STEP && p->acc != MCCLX_ACC_F32)
         return fail(MCCLX_ERR_INVALID, "plan.acc=%d unknown", p->acc);
-    if (op != MCCLX_SUM && (p->io != MCCLX_IO_PURE || p->acc != MCCLX_ACC_STEP))
+    if (op != MCCLX_SUM && ((p->io != MCCLX_IO_PURE && !(to_all && p->io == MCCLX_IO_ALL_F32)) || p->acc != MCCLX_ACC_STEP))
         return fail(MCCLX_ERR_UNSUPPORTED,
                     "MIN/MAX/PRODUCT fold same-dtype operands with per-step rounding only (PURE, STEP)");
     if (p->dtype == MCCLX_F16 && p->acc != MCCLX_ACC_STEP)
@@ -236,7 +240,12 @@ int check_plan(const mcclx_plan* p, mcclx::PlanKey* key, float* scale_f, int* ha
         op = (op == MCCLX_MIN) ? mcclx::MCCLX_MIN_ACC_SRC : mcclx::MCCLX_MAX_ACC_SRC;
     int acc = (p->dtype == MCCLX_F32) ? MCCLX_ACC_STEP : p->acc;  // fp32 has no rounding to skip
     *key = mcclx::PlanKey{p->dtype, p->io, p->k, (p->k >= 4) ? p->topo : MCCLX_TOPO_FOLD, op, acc};
-    if (*fan && (!mcclx::fan_plan_ok(*key) || p->k + *fan > MCCLX_MAX_INPUTS))
+    if (to_all) {
+        *fan = kToAll;
+        if (!mcclx::all_plan_ok(*key))
+            return fail(MCCLX_ERR_UNSUPPORTED,
+                        "to-all needs per-step rounding, two operands or more and operands in the form of the result");
+    } else if (*fan && (!mcclx::fan_plan_ok(*key) || p->k + *fan > MCCLX_MAX_INPUTS))
         return fail(MCCLX_ERR_UNSUPPORTED,
                     "fan-out (%d further destinations) needs a sum with per-step rounding, an output of the "
                     "operands' form or fp32 next to an fp32 operand, and k + fan <= %d (k=%d)",
@@ -302,6 +311,8 @@ int check_segs(mcclx_ctx* ctx, const mcclx::PlanKey& key, const mcclx_seg* segs,
         if (g.wire_out && (uintptr_t)g.wire_out % 2)
             return fail(MCCLX_ERR_INVALID, "segment %u: wire_out=%p is not element aligned", s,
                         g.wire_out);
+        if (fan == kToAll && (g.out != g.in[0] || g.wire_out))
+            return fail(MCCLX_ERR_INVALID, "segment %u: to-all needs `out` to be in[0] and no wire_out", s);
         if (fan && !g.out) return fail(MCCLX_ERR_INVALID, "segment %u: fan-out needs `out`", s);
         for (int f = 0; f < fan; ++f) {
             const void* d = g.in[key.k + f];
@@ -330,6 +341,15 @@ int check_segs(mcclx_ctx* ctx, const mcclx::PlanKey& key, const mcclx_seg* segs,
             for (int i = 0; i < key.k; ++i)
                 if (int rc = check_range(g.in[i], g.count * (in_is_f32(key, i) ? 4 : 2), "in", s))
                     return rc;
+            if (fan == kToAll)  // every operand is a destination: the fan-out rule on overlaps holds for each pair
+                for (int i = 0; i < key.k; ++i)
+                    for (int j = 0; j < i; ++j) {
+                        const uint64_t nb = g.count * (out_f32 ? 4 : 2);
+                        const char *a = static_cast<const char*>(g.in[i]), *b = static_cast<const char*>(g.in[j]);
+                        if (a != b && a < b + nb && b < a + nb)
+                            return fail(MCCLX_ERR_INVALID, "segment %u: to-all operands in[%d]=%p and in[%d]=%p overlap at different offsets",
+                                        s, j, g.in[j], i, g.in[i]);
+                    }
             if (g.out)
                 if (int rc = check_range(g.out, g.count * (out_f32 ? 4 : 2), "out", s)) return rc;
             if (g.wire_out)
@@ -419,7 +439,8 @@ int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, in
                     const mcclx_seg* segs, uint32_t nseg, int fan) {
     mcclx::LaunchParams lp;
     lp.max_blocks = ctx->max_blocks;
-    lp.fan = fan;
+    lp.fan = fan > 0 ? fan : 0;
+    lp.to_all = fan == kToAll;
     lp.cus = ctx->cus;
     bool held = false;
     lp.held = &held;
@@ -513,7 +534,8 @@ int fold_impl(mcclx_ctx* ctx, const mcclx_plan* plan, const mcclx_seg* segs, uin
     t.scale = scale_f;
     t.has_scale = has_scale;
     lp.table = &t;
-    lp.fan = fan;
+    lp.fan = fan > 0 ? fan : 0;
+    lp.to_all = fan == kToAll;
     hipError_t e = mcclx::launch_fold(ctx->stream, key, lp);
     if (e != hipSuccess) return launch_error(e, key);
     ++ctx->launches;
@@ -860,7 +882,8 @@ int mcclx_fold_batched_noalloc(mcclx_ctx* ctx, const mcclx_plan* plan, const mcc
     mcclx::LaunchParams lp;
     lp.max_blocks = ctx->max_blocks;
     lp.table = &t;
-    lp.fan = fan;
+    lp.fan = fan > 0 ? fan : 0;
+    lp.to_all = fan == kToAll;
     hipError_t e = mcclx::launch_fold(ctx->stream, key, lp);
     if (e != hipSuccess) return launch_error(e, key);
     ++ctx->launches;

@@ -17,6 +17,7 @@
 
 #include <cstdarg>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -66,6 +67,7 @@ struct Layout {
 };
 
 int fan_of(const mcclx_replay* r);
+bool to_all(const mcclx_replay* r);
 bool direct_applies(const mcclx_replay* r);
 
 Layout layout_of(const mcclx_replay* r) {
@@ -73,7 +75,7 @@ Layout layout_of(const mcclx_replay* r) {
     L.wire = r->wire_bf16 && r->dtype == MCCLX_F32;  // ProcessGroupMCCL.cpp:131
     L.wdtype = L.wire ? MCCLX_BF16 : r->dtype;
     // a DIRECT fold that also hands the result to every rank needs no bf16 copy at all
-    const bool no_copies = direct_applies(r) && fan_of(r) > 0;
+    const bool no_copies = direct_applies(r) && (fan_of(r) > 0 || to_all(r));
     L.wire_stride = (L.wire && !no_copies) ? align_up(r->numel * 2) : 0;
     L.scratch_off = L.wire_stride * (uint64_t)r->world;
     bool need_scratch = r->mode == MCCLX_REPLAY_STEPWISE || r->world > MCCLX_MAX_INPUTS;
@@ -219,6 +221,8 @@ struct Phases {
     std::vector<mcclx_seg> enc_segs, dec_segs;
     std::vector<FoldPass> folds;  // one pass, or a chain of passes when the world is wider than one fold
     std::vector<mcclx_copy_desc> copies;
+    bool all = false;  // the fold stores every reduced chunk back into every rank's tensor
+                       // (MCCLX_PLAN_TO_ALL): no allgather launch either
     int fan = 0;  // > 0: the fold itself stores every reduced chunk into the other ranks' tensors
                   // (in[k .. k+fan-1] of its segments); there is no allgather launch then
 };
@@ -252,11 +256,31 @@ bool all_on_wire(const mcclx_replay* r) {
     return (r->op != MCCLX_SUM && r->op != MCCLX_AVG) || r->world > MCCLX_MAX_INPUTS;
 }
 
-// DIRECT: a sum over the wire codec whose operands fit one fold reads every
+// DIRECT: a sum over the wire codec whose operands fit one fold (and any other op that takes
+// the to-all form) reads every
 // rank's fp32 tensor itself and encodes it in registers -- the bits of
 // `t.to(at::kBFloat16)` (ProcessGroupMCCL.cpp:131-132) without the bf16 copy.
 bool direct_applies(const mcclx_replay* r) {
-    return r->mode == MCCLX_REPLAY_DIRECT && r->wire_bf16 && r->dtype == MCCLX_F32 && !all_on_wire(r);
+    return r->mode == MCCLX_REPLAY_DIRECT && r->wire_bf16 && r->dtype == MCCLX_F32 && (!all_on_wire(r) || to_all(r));
+}
+
+// The fold stores the reduced chunk back into every rank's tensor (MCCLX_PLAN_TO_ALL) where
+// fan-out cannot name everybody -- five to eight ranks -- or does not take the op: the
+// tensors are the operands, so each is read once and written once, where the fold + copy
+// (or fold + cast) pair reads the result again for every rank.  In place of those two
+// launches, measured on the device: 8 x 12.5 M bf16 89 -> 71 us, 8 x 25 MiB fp32 over the
+// wire codec 93 -> 77 us, MAX of 3 x 25 MiB 33 -> 26 us (49 -> 26 us over the codec),
+// 8 x 4 KB 4.1 -> 2.4 us.
+// From 8 MiB of tensors on, and up to 1 MiB, where a call is all latency.  In between the
+// launch sequence of a fused replay stays what callers that count launches rely on; one
+// launch less is worth 2 us there, of some 25 a call takes.
+bool to_all(const mcclx_replay* r) {
+    const bool wire = r->wire_bf16 && r->dtype == MCCLX_F32;
+    const bool step = r->acc == MCCLX_ACC_STEP || (r->dtype == MCCLX_F32 && !wire);
+    if (r->mode == MCCLX_REPLAY_STEPWISE || (wire && r->mode != MCCLX_REPLAY_DIRECT)) return false;
+    if (!step || r->world < 2 || r->world > MCCLX_MAX_INPUTS || fan_of(r) > 0) return false;
+    const uint64_t bytes = r->numel * esize(r->dtype) * (uint64_t)r->world;
+    return bytes >= (8u << 20) || bytes <= (1u << 20);
 }
 
 // A fold takes MCCLX_MAX_INPUTS operands.  A wider world is folded by a chain
@@ -313,7 +337,9 @@ void plan_phases(const mcclx_replay* r, const Layout& L, Phases& ph) {
     }
     mcclx_plan& fold = ph.folds[0].plan;
     if (r->algo == MCCLX_ALGO_TREE) fold.topo = MCCLX_TOPO_BINOMIAL;
-    ph.fan = fan_of(r);
+    ph.all = to_all(r);
+    ph.fan = ph.all ? 0 : fan_of(r);
+    if (ph.all) fold.flags |= MCCLX_PLAN_TO_ALL;
     if (ph.fan) fold.flags |= MCCLX_PLAN_FANOUT(ph.fan);
     if (direct_applies(r)) {          // every operand is read as fp32 and encoded in registers
         fold.io = MCCLX_IO_ALL_F32;
@@ -341,8 +367,8 @@ void collect_fused(const mcclx_replay* r, const Layout& L, Phases& ph) {
     mcclx_seg z;
     memset(&z, 0, sizeof z);
 
-    const bool bf16_only = L.wire && all_on_wire(r);
     const bool direct = direct_applies(r);  // peers' fp32 tensors are the operands: nothing is encoded
+    const bool bf16_only = L.wire && all_on_wire(r) && !direct;
     if (r->algo == MCCLX_ALGO_TREE) {
         // allreduce_tree: rank 0 ends with the binomial combination of all
         // tensors (AllreduceAlgos.cpp:100-114), everyone else receives a copy.
@@ -396,12 +422,12 @@ void collect_fused(const mcclx_replay* r, const Layout& L, Phases& ph) {
             for (int q = 1; q < N; ++q) s.in[q] = (L.wire && !direct) ? wire_of(q) : r->tensors[q];
             if (ph.fan) {  // rank 0's fold hands the result to ranks 1..N-1 itself
                 for (int q = 1; q < N; ++q) s.in[N + q - 1] = r->tensors[q];
-            } else if (L.wire) {
+            } else if (L.wire && !ph.all) {
                 s.wire_out = wire_of(0);
             }
         }
         ph.folds[0].segs.push_back(s);
-        if (ph.fan) return;
+        if (ph.fan || ph.all) return;
         for (int q = bf16_only ? 0 : 1; q < N; ++q) {
             if (L.wire) {  // broadcast of the bf16 result + the final cast on every rank
                 mcclx_seg g = z;
@@ -458,7 +484,9 @@ void collect_fused(const mcclx_replay* r, const Layout& L, Phases& ph) {
             s.count = (uint64_t)c[ch].elem_count;
             s.out = dest;
             for (int j = 0; j < N; ++j) s.in[j] = ops[(size_t)j];
-            if (ph.fan) {  // the owner's fold hands the reduced chunk to every other rank itself
+            if (ph.all) {  // every operand is a rank's own tensor and gets the result back
+                s.out = const_cast<void*>(ops[0]);
+            } else if (ph.fan) {  // the owner's fold hands the reduced chunk to every other rank itself
                 int f = 0;
                 for (int q = 0; q < N; ++q)
                     if (q != o) s.in[N + f++] = at(r->tensors[q], (uint64_t)c[ch].elem_start * ts);
@@ -488,7 +516,7 @@ void collect_fused(const mcclx_replay* r, const Layout& L, Phases& ph) {
     // allgather leg (AllreduceAlgos.cpp:77-86,185-200): every other rank gets
     // the owner's reduced chunk; with the wire codec it arrives as bf16 and is
     // cast on arrival (ProcessGroupMCCL.cpp:179-183).
-    if (ph.fan) return;  // done by the folds
+    if (ph.fan || ph.all) return;  // done by the folds
     for (int ch = 0; ch < N; ++ch) {
         if (c[ch].elem_count == 0) continue;
         int o = owner_of(ch);
@@ -582,7 +610,7 @@ bool overlaps(const std::vector<Range>& a, const std::vector<Range>& b) {
 // Same plan for every phase?
 bool same_plan(const mcclx_replay* a, const mcclx_replay* b) {
     return a->world == b->world && a->algo == b->algo && a->op == b->op && a->dtype == b->dtype &&
-           (a->wire_bf16 != 0) == (b->wire_bf16 != 0) && a->acc == b->acc && a->mode == b->mode;
+           (a->wire_bf16 != 0) == (b->wire_bf16 != 0) && a->acc == b->acc && a->mode == b->mode && to_all(a) == to_all(b);
 }
 
 }  // namespace
