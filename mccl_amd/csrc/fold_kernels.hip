@@ -40,20 +40,23 @@
 namespace mcclx {
 namespace {
 
-// Launch shapes, each measured on MI355X.
-constexpr int kBlock = 512;  // threads per block of folds that mix fp32 and 16-bit streams, and of one-operand passes
-// Folds whose streams all have one element size -- all 16-bit (16 bytes per lane
-// and operand) or all fp32 -- run one-wavefront blocks with one packet per lane:
-// a 512-lane block keeps its wave slots until the last of its loads is back,
-// 64-lane blocks turn them over eight times as often (two to eight 16-bit
-// operands of 512 MiB: +5...9 %, fp32 operands: +3...4 %; launches of a few MB
-// are level; fp32 operands encoded in registers, MCCLX_IO_ALL_F32: +7 % on
-// 256 MiB tensors, +1.5 % on 25 MiB ones).
+// Launch shapes, each measured on MI355X.  By-value launches run one-wavefront blocks of one
+// packet per lane (Cfg::FEW_U, kTwoShapes): a block of eight wavefronts keeps its slots until
+// the last of its loads is back, one-wavefront blocks turn them over one by one (operands of
+// 128-512 MiB: one fp32 operand scaled 84.5 -> 80.9 us, own fp32 + one bf16 peer 106 -> 99.6,
+// + two peers 124 -> 119.5, copy 82.6 -> 80.6; 25 MiB operands: 10.3 -> 9.5, 12.5 -> 11.4,
+// 13.7 -> 13.1, 10.1 -> 9.2).  The table kernels keep blocks of eight for folds that mix fp32
+// and 16-bit streams and one-operand passes: a tile per wavefront would mean eight times the
+// work items, and with them eight times the item map a ragged launch uploads.
+constexpr int kBlock = 512;  // threads per block of those table launches
+// Table launches of folds whose streams all have one element size -- all 16-bit (16 bytes
+// per lane and operand) or all fp32 -- take one-wavefront blocks with one packet per lane too.
 constexpr int kWideBlock = 64;
 constexpr int kWideU = 1;
 constexpr int kWideMinK = 2;   // all-16-bit folds of this many operands or more take the one-wavefront shape
 constexpr int kF32Block = 64;
 constexpr int kAllF32Block = 64;
+constexpr int kOneWave = 64, kFourWaves = 256;  // by-value launches, see Cfg::kTwoShapes
 
 // Every operand lives in global memory (HBM or host memory mapped into the
 // device).  Pointers that reach a kernel through a descriptor table are
@@ -210,6 +213,20 @@ struct Cfg {
     static constexpr int BLOCK = kWide ? kWideBlock
                                  : ((W == MCCLX_F32 && K >= 2) || kDecode) ? kF32Block
                                  : (IO == MCCLX_IO_ALL_F32 && K >= 2) ? kAllF32Block : kBlock;  // threads per block
+    // By-value launches: one-wavefront blocks of one packet per lane (two for the bf16 -> fp32
+    // cast, whose lanes read 8 bytes: 67 M elements 63.5 -> 62.1 us), in blocks of four
+    // wavefronts where the launch is small (kOneWaveBlocksFrom) and the plan mixes fp32 and
+    // 16-bit streams or has one operand.
+    static constexpr int FEW_U = kDecode ? 2 : 1;
+    static constexpr bool kTwoShapes = BLOCK == kBlock || kDecode;
+    // (an encode's lanes move 24 bytes: four wavefronts still win at 16,384, 4.2 M elements in 5.5 us against 5.9)
+    static constexpr uint64_t kOneWaveFrom = (K == 1 && IO == MCCLX_IO_OWN_FIRST_F32) ? 20480 : kOneWaveBlocksFrom;
+    // bytes a lane reads per packet
+    static constexpr int kReadBytes = [] {
+        int b = 0;
+        for (int k = 0; k < K; ++k) b += (in_is_f32(k) || E == 8) ? 16 : 8;
+        return b;
+    }();
 };
 
 typedef u32x4 RawPack;  // one packet of one operand: 16 B, or 8 B in .xy (16-bit operand, E = 4)
@@ -525,12 +542,10 @@ __device__ __forceinline__ SegArgs advanced(const SegArgs& s, uint64_t elems) {
 // load is kept short -- a block lives for about 2 us and eight waves per SIMD
 // share one scalar unit, so every scalar instruction in front of the loads is
 // paid eight times over.
-template <class C, int OUT = kOutOne>
+template <class C, int OUT, int kB, int U>
 __device__ __forceinline__ void fold_tile(const SegArgs& s, float scale, bool has_scale, uint64_t first,
                                           bool do_edges, int fan = 0, int op = C::OP) {
-    constexpr int U = C::U;
     const uint32_t tid = threadIdx.x;
-    constexpr int kB = C::BLOCK;
     const uint32_t head = head_elems<C, OUT>(s);  // < 64 <= kB
     const uint64_t P = (s.count - head) / C::E;
     const bool has_out = s.out != nullptr, has_wire = s.wire_out != nullptr;
@@ -585,7 +600,7 @@ __device__ __forceinline__ void fetch_together(SegArgs& s, float& scale, int32_t
 // kernel with more starts 768 blocks at launch instead of 1024 and streams
 // 2-4 % slower.  Six registers are set aside on top of what the code uses (VCC,
 // flat scratch, XNACK mask), so the code itself has 74.
-template <class C, int OUT = kOutOne>
+template <class C, int OUT, int B>
 __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
 #if MCCLX_TUNE_TIMELINE
     const uint64_t t_start = wall_clock64();
@@ -600,14 +615,14 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
 #if MCCLX_TUNE_TIMELINE
     const uint64_t t_args = wall_clock64();
 #endif
-    const uint64_t span = (uint64_t)C::U * C::BLOCK;
+    const uint64_t span = (uint64_t)C::FEW_U * B;
     // one tile per block, no loop: the launch sizes the grid to the longest segment.  Blocks are
     // dispatched in address order (giving each XCD one contiguous part of a segment instead was
     // level on a 25 MiB bucket and 3.5-9 % slower on large operands).
     (void)grid;
     int op = C::OP;
     if constexpr (C::OP == kAnyOp) op = a.op;
-    fold_tile<C, OUT>(s, scale, has_scale != 0, (uint64_t)blockIdx.x * span, blockIdx.x == 0, fan, op);
+    fold_tile<C, OUT, B, C::FEW_U>(s, scale, has_scale != 0, (uint64_t)blockIdx.x * span, blockIdx.x == 0, fan, op);
 #if MCCLX_TUNE_TIMELINE
     if (a.timeline && threadIdx.x == 0) {
         TimelineRecord r;
@@ -627,17 +642,17 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
 #define MCCLX_SGPR_CAP __attribute__((amdgpu_num_sgpr(80)))
 template <class C> constexpr bool kLightPlan = C::K <= 4;
 
-template <class C>
-__global__ void __launch_bounds__(C::BLOCK) MCCLX_SGPR_CAP fold_few_kernel(FewArgs a) { fold_few_body<C, kOutOne>(a); }
-template <class C>
-__global__ void __launch_bounds__(C::BLOCK) fold_few_wide_kernel(FewArgs a) { fold_few_body<C, kOutOne>(a); }
+template <class C, int B>
+__global__ void __launch_bounds__(B) MCCLX_SGPR_CAP fold_few_kernel(FewArgs a) { fold_few_body<C, kOutOne, B>(a); }
+template <class C, int B>
+__global__ void __launch_bounds__(B) fold_few_wide_kernel(FewArgs a) { fold_few_body<C, kOutOne, B>(a); }
 // Fan-out form: the result also goes to in[K .. K+fan-1] (the other ranks' tensors: the
 // allgather leg of an allreduce done by the reduce itself, stores instead of a second pass).
-template <class C>
-__global__ void __launch_bounds__(C::BLOCK) fold_few_fan_kernel(FewArgs a) { fold_few_body<C, kOutFan>(a); }
+template <class C, int B>
+__global__ void __launch_bounds__(B) fold_few_fan_kernel(FewArgs a) { fold_few_body<C, kOutFan, B>(a); }
 // To-all form: the result goes back into every operand's buffer.
-template <class C>
-__global__ void __launch_bounds__(C::BLOCK) fold_few_all_kernel(FewArgs a) { fold_few_body<C, kOutAll>(a); }
+template <class C, int B>
+__global__ void __launch_bounds__(B) fold_few_all_kernel(FewArgs a) { fold_few_body<C, kOutAll, B>(a); }
 
 #if MCCLX_TUNE_TIMELINE
 // Where the next by-value launches put their records (measurement build): a caller-provided
@@ -907,7 +922,7 @@ __device__ __forceinline__ void fold_table_body(const TableArgs& a) {
         for (int k = 0; k < MCCLX_MAX_INPUTS; ++k) s.in[k] = (k < C::K || OUT == kOutFan) ? uniptr(d->in[k]) : nullptr;
         s.count = uni64(d->count);
         // one tile: packets [tile*span, tile*span + span); tile 0 also owns the tail
-        fold_tile<C, OUT>(s, a.scale, a.has_scale != 0, (uint64_t)tile * span, tile == 0, OUT == kOutFan ? a.fan : 0,
+        fold_tile<C, OUT, C::BLOCK, C::U>(s, a.scale, a.has_scale != 0, (uint64_t)tile * span, tile == 0, OUT == kOutFan ? a.fan : 0,
                           C::OP == kAnyOp ? a.op : C::OP);
     }
 }
@@ -933,44 +948,71 @@ constexpr bool kFanPlan = C::OP == MCCLX_SUM && C::ACC == MCCLX_ACC_STEP && C::K
 template <class C, int OUT>
 static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchParams& lp) {
     FewArgs a = args;
-    uint64_t maxc = 0;
-    for (int i = 0; i < a.nseg; ++i) maxc = a.seg[i].count > maxc ? a.seg[i].count : maxc;
+    uint64_t maxc = 0, total = 0;
+    for (int i = 0; i < a.nseg; ++i) {
+        maxc = a.seg[i].count > maxc ? a.seg[i].count : maxc;
+        total += a.seg[i].count;
+    }
     if (maxc == 0) return hipSuccess;
 #if MCCLX_TUNE_TIMELINE
     a.timeline = nullptr;
 #endif
     if constexpr (kHoldPlan<C>)
         if (try_hold<C, OUT>(st, a, maxc, lp)) return hipGetLastError();
-    const uint64_t span = (uint64_t)C::U * C::BLOCK * C::E;  // elements per block iteration
-    const uint64_t gx = (maxc + span - 1) / span;
+    const uint64_t lane_elems = (uint64_t)C::FEW_U * C::E;
+    const int outputs = OUT == kOutAll ? C::K : 1 + a.fan;
+    const int lane_bytes = C::FEW_U * (C::kReadBytes + outputs * ((C::W == MCCLX_F32 || C::kOutF32) ? 16 : 2 * C::E));
+    const uint32_t lds = resident_lds(total / lane_elems * (uint64_t)lane_bytes, lane_bytes, outputs,
+                                      OUT == kOutAll ? kLaneBytesInPlace : kLaneBytes);
+    const uint64_t waves = (maxc + 64 * lane_elems - 1) / (64 * lane_elems);
+    const bool four = C::kTwoShapes && waves * (uint64_t)a.nseg < C::kOneWaveFrom;
+    const uint64_t gx = four ? (waves + 3) / 4 : waves;
     if (gx >> 31) return hipErrorInvalidValue;
-    const dim3 grid((uint32_t)gx, (uint32_t)a.nseg), block(C::BLOCK);
+    const dim3 grid((uint32_t)gx, (uint32_t)a.nseg);
 #if MCCLX_TUNE_TIMELINE
     if (OUT == kOutOne) a.timeline = timeline_next(gx * (uint64_t)a.nseg);
 #endif
-    if constexpr (OUT == kOutAll)
-        fold_few_all_kernel<C><<<grid, block, 0, st>>>(a);
-    else if constexpr (OUT == kOutFan)
-        fold_few_fan_kernel<C><<<grid, block, 0, st>>>(a);
-    else if constexpr (kLightPlan<C>)
-        fold_few_kernel<C><<<grid, block, 0, st>>>(a);
-    else
-        fold_few_wide_kernel<C><<<grid, block, 0, st>>>(a);
+    auto go = [&](auto block) {
+        constexpr int B = decltype(block)::value;
+        if constexpr (OUT == kOutAll)
+            fold_few_all_kernel<C, B><<<grid, dim3(B), lds, st>>>(a);
+        else if constexpr (OUT == kOutFan)
+            fold_few_fan_kernel<C, B><<<grid, dim3(B), lds, st>>>(a);
+        else if constexpr (kLightPlan<C>)
+            fold_few_kernel<C, B><<<grid, dim3(B), lds, st>>>(a);
+        else
+            fold_few_wide_kernel<C, B><<<grid, dim3(B), lds, st>>>(a);
+    };
+    if constexpr (C::kTwoShapes) {
+        if (four) {
+            go(std::integral_constant<int, kFourWaves>{});
+            return hipGetLastError();
+        }
+    }
+    go(std::integral_constant<int, kOneWave>{});
     return hipGetLastError();
 }
 
 template <class C, int OUT>
-static hipError_t launch_table(hipStream_t st, const TableArgs& a, const LaunchParams& lp) {
-    const dim3 grid((uint32_t)(a.total_items < lp.max_blocks ? a.total_items : lp.max_blocks)), block(C::BLOCK);
-    if (grid.x == 0) return hipSuccess;
+static hipError_t launch_table(hipStream_t st, const TableArgs& args, const LaunchParams& lp) {
+    TableArgs a = args;
+    const uint32_t grid = (uint32_t)(a.total_items < lp.max_blocks ? a.total_items : lp.max_blocks);
+    if (grid == 0) return hipSuccess;
+    uint32_t lds = 0;
+    if constexpr (C::BLOCK == kOneWave) {
+        const int outputs = OUT == kOutAll ? C::K : 1 + a.fan;
+        const int lane_bytes = C::U * (C::kReadBytes + outputs * ((C::W == MCCLX_F32 || C::kOutF32) ? 16 : 2 * C::E));
+        lds = resident_lds(a.total_items * 64 * (uint64_t)lane_bytes, lane_bytes, outputs,
+                                      OUT == kOutAll ? kLaneBytesInPlace : kLaneBytes);
+    }
     if constexpr (OUT == kOutAll)
-        fold_table_all_kernel<C><<<grid, block, 0, st>>>(a);
+        fold_table_all_kernel<C><<<dim3(grid), dim3(C::BLOCK), lds, st>>>(a);
     else if constexpr (OUT == kOutFan)
-        fold_table_fan_kernel<C><<<grid, block, 0, st>>>(a);
+        fold_table_fan_kernel<C><<<dim3(grid), dim3(C::BLOCK), lds, st>>>(a);
     else if constexpr (kLightPlan<C>)
-        fold_table_kernel<C><<<grid, block, 0, st>>>(a);
+        fold_table_kernel<C><<<dim3(grid), dim3(C::BLOCK), lds, st>>>(a);
     else
-        fold_table_wide_kernel<C><<<grid, block, 0, st>>>(a);
+        fold_table_wide_kernel<C><<<dim3(grid), dim3(C::BLOCK), lds, st>>>(a);
     return hipGetLastError();
 }
 

@@ -106,8 +106,8 @@ hipError_t launch_fold(hipStream_t st, const PlanKey& key, const LaunchParams& l
 // With fewer waves resident the same launches run at 6.1-6.8 TB/s: what a channel sees at
 // one time shrinks with the bytes under way, and 70-80 KiB per CU (20 MB on the device) still
 // covers the latency.  The optimum, swept over 3..20 waves per CU, lies near one number of
-// bytes for every shape, waves x bytes a lane moves: 1150 (8 operands into one: 8 waves;
-// 4 into one: 14; 3 into one: 17; one source to 4 / 8 destinations: 11-14 / 7-8), a little
+// bytes for every shape, waves x bytes a lane moves: 1160 (8 operands into one: 8 waves;
+// 4 into one: 14; 3 into one: 18; one source to 4 / 8 destinations: 11-14 / 7-8), a little
 // more where tensors are reduced in place, which opens each row once for both directions
 // (2 / 3 / 4 / 5 / 8 ranks: 18 / 12 / 8-10 / 8 / 5 waves).  A reservation of LDS nobody uses
 // sets the number: it is granted in units of 1280 bytes of a CU's 160 KiB.
@@ -116,7 +116,7 @@ hipError_t launch_fold(hipStream_t st, const PlanKey& key, const LaunchParams& l
 // (200 MB, eight operands into one: 36.2 -> 35.4 us; 80 MB: 5.5 TB/s without it, 5.1 with),
 // and not where 20 waves or more would be left of a launch with one output.
 constexpr uint64_t kResidentMinBytes = 160'000'000;
-constexpr int kLaneBytes = 1150, kLaneBytesInPlace = 1280;
+constexpr int kLaneBytes = 1160, kLaneBytesInPlace = 1280;
 inline uint32_t resident_lds(uint64_t launch_bytes, int lane_bytes, int outputs, int budget = kLaneBytes) {
     int waves = budget / lane_bytes;
     if (launch_bytes < kResidentMinBytes || (outputs == 1 && waves >= 20)) return 0;
