@@ -7,8 +7,6 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-#include <type_traits>
-
 #include "fold_launch.h"
 
 namespace mcclx {
@@ -18,25 +16,11 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // every byte is touched once: non-temporal loads and stores
 #define COPY_LD(p) __builtin_nontemporal_load(p)
 #define COPY_ST(p, v) __builtin_nontemporal_store((v), (p))
-// the widest alignment both pointers share decides the packet type
-template <int A> struct Packet;
-template <> struct Packet<4> { typedef u32x4 type __attribute__((aligned(4))); };
-template <> struct Packet<2> { typedef u32x4 type __attribute__((aligned(2))); };
-template <> struct Packet<1> { typedef u32x4 type __attribute__((aligned(1))); };
+// 16-byte packets at any address (gfx950 global accesses are alignment-agnostic)
+typedef u32x4 Packet __attribute__((aligned(1)));
 constexpr int kBlock = 256;
 
 constexpr int kOneWave = 64, kFourWaves = 256;  // threads per block of a launch by value, see kOneWaveBlocksFrom
-
-// One packet from its source to everybody who gets it.  FAN = false: one destination.
-template <bool FAN, typename V>
-__device__ __forceinline__ void deliver(MCCLX_GLOBAL uint8_t* const (&dst)[FAN ? kCopyDsts : 1], uint32_t n, uint64_t off, u32x4 v) {
-    COPY_ST((MCCLX_GLOBAL V*)(dst[0] + off), v);
-    if constexpr (FAN) {
-#pragma unroll
-        for (uint32_t f = 1; f < (uint32_t)kCopyDsts; ++f)
-            if (f < n) COPY_ST((MCCLX_GLOBAL V*)(dst[f] + off), v);
-    }
-}
 
 // Up to kFewCopies copies with their descriptors in the kernel arguments:
 // blockIdx.y picks the copy, blockIdx.x one tile of B packets of 16 bytes, one
@@ -46,34 +30,42 @@ __device__ __forceinline__ void deliver(MCCLX_GLOBAL uint8_t* const (&dst)[FAN ?
 // allgather would otherwise write every line in two parts.
 // One tile per block and no loop, like the fold kernels: a uniform 64-bit base
 // plus a 32-bit lane offset per access, and a short path to the first load.
-template <int A, bool FAN, int B>
+// The number of destinations is a compile-time constant and every field a block
+// needs is fetched in one batch of scalar loads (as the fold kernels do): with few
+// waves on a CU what a wave waits for in front of its load is not hidden by others.
+// MIXED: copies of different numbers of destinations, up to N, share the launch.
+template <int N, int B, bool MIXED = false>
 __global__ void __launch_bounds__(B) copy_few_kernel(CopyFew a) {
-    typedef typename Packet<A>::type V;
-    constexpr int D = FAN ? kCopyDsts : 1;
     const CopyDesc& d = a.d[blockIdx.y];
-    const uint64_t nbytes = d.nbytes;
-    const uint32_t n = FAN ? (uint32_t)d.n : 1u;
-    const uint32_t mis = (0u - (uint32_t)reinterpret_cast<uintptr_t>(d.dst[0])) & 127u;
+    const void* src = d.src;
+    uint64_t nbytes = d.nbytes;
+    const int n = MIXED ? (int)d.n : N;
+    void* dst[N];
+#pragma unroll
+    for (int f = 0; f < N; ++f) dst[f] = d.dst[f];
+    asm volatile("" : "+s"(src), "+s"(nbytes));
+#pragma unroll
+    for (int f = 0; f < N; ++f) asm volatile("" : "+s"(dst[f]));
+    const uint32_t mis = (0u - (uint32_t)reinterpret_cast<uintptr_t>(dst[0])) & 127u;
     const uint32_t head = nbytes < mis ? (uint32_t)nbytes : mis;
     const uint64_t P = (nbytes - head) / 16;
     const uint64_t first = (uint64_t)blockIdx.x * B;
     const uint64_t at = head + first * 16;
     if (first < P) {
-        const MCCLX_GLOBAL uint8_t* gs = (const MCCLX_GLOBAL uint8_t*)d.src + at;
-        MCCLX_GLOBAL uint8_t* gd[D];
-#pragma unroll
-        for (int f = 0; f < D; ++f) gd[f] = (MCCLX_GLOBAL uint8_t*)d.dst[f] + at;
         if (threadIdx.x < P - first) {
             const uint32_t off = threadIdx.x * 16u;
-            deliver<FAN, V>(gd, n, off, COPY_LD((const MCCLX_GLOBAL V*)(gs + off)));
+            const u32x4 v = COPY_LD((const MCCLX_GLOBAL Packet*)((const MCCLX_GLOBAL uint8_t*)src + at + off));
+#pragma unroll
+            for (int f = 0; f < N; ++f)
+                if (!MIXED || f < n) COPY_ST((MCCLX_GLOBAL Packet*)((MCCLX_GLOBAL uint8_t*)dst[f] + at + off), v);
         }
     }
     if (blockIdx.x == 0) {
         auto byte = [&](uint64_t i) {
-            const uint8_t x = ((const MCCLX_GLOBAL uint8_t*)d.src)[i];
+            const uint8_t x = ((const MCCLX_GLOBAL uint8_t*)src)[i];
 #pragma unroll
-            for (int f = 0; f < D; ++f)
-                if ((uint32_t)f < n) ((MCCLX_GLOBAL uint8_t*)d.dst[f])[i] = x;
+            for (int f = 0; f < N; ++f)
+                if (!MIXED || f < n) ((MCCLX_GLOBAL uint8_t*)dst[f])[i] = x;
         };
         for (uint32_t i = threadIdx.x; i < head; i += B) byte(i);
         const uint64_t i = head + P * 16 + threadIdx.x;  // fewer than 16 bytes remain
@@ -87,7 +79,7 @@ __global__ void __launch_bounds__(B) copy_few_kernel(CopyFew a) {
 // word).
 template <bool WRITE>
 __global__ void __launch_bounds__(kBlock) stream_probe_kernel(uint8_t* buf, uint64_t nbytes, uint32_t magic) {
-    typedef typename Packet<4>::type V;
+    typedef Packet V;
     MCCLX_GLOBAL uint8_t* g = (MCCLX_GLOBAL uint8_t*)buf;
     const uint64_t P = nbytes / 16;
     const uint64_t p = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
@@ -112,9 +104,9 @@ __device__ __forceinline__ uint64_t uni64(uint64_t v) {
 // bytes behind the last whole packet.  The loop bound is fixed at launch.
 constexpr int kManyU = 4;
 
-template <int A, bool FAN>
+// Up to kCopyDsts destinations a copy (FAN), or one.
+template <bool FAN>
 __global__ void __launch_bounds__(kBlock) copy_many_kernel(CopyTable t) {
-    typedef typename Packet<A>::type V;
     constexpr int D = FAN ? kCopyDsts : 1;
     const uint64_t span = (uint64_t)kManyU * kBlock;
     for (uint32_t w = blockIdx.x; w < t.total_items; w += gridDim.x) {
@@ -143,6 +135,14 @@ __global__ void __launch_bounds__(kBlock) copy_many_kernel(CopyTable t) {
         MCCLX_GLOBAL uint8_t* gd[D];
 #pragma unroll
         for (int f = 0; f < D; ++f) gd[f] = (MCCLX_GLOBAL uint8_t*)uni64(reinterpret_cast<uint64_t>(d->dst[f]));
+        auto deliver = [&](uint64_t off, u32x4 v) {
+            COPY_ST((MCCLX_GLOBAL Packet*)(gd[0] + off), v);
+            if constexpr (FAN) {
+#pragma unroll
+                for (uint32_t f = 1; f < (uint32_t)kCopyDsts; ++f)
+                    if (f < n) COPY_ST((MCCLX_GLOBAL Packet*)(gd[f] + off), v);
+            }
+        };
         const uint64_t nbytes = uni64(d->nbytes);
         const uint64_t P = nbytes / 16;
         const uint64_t base = (uint64_t)tile * span;
@@ -150,12 +150,12 @@ __global__ void __launch_bounds__(kBlock) copy_many_kernel(CopyTable t) {
             u32x4 v[kManyU];
 #pragma unroll
             for (int u = 0; u < kManyU; ++u)
-                v[u] = COPY_LD((const MCCLX_GLOBAL V*)(gs + (base + (uint64_t)u * kBlock + threadIdx.x) * 16));
+                v[u] = COPY_LD((const MCCLX_GLOBAL Packet*)(gs + (base + (uint64_t)u * kBlock + threadIdx.x) * 16));
 #pragma unroll
-            for (int u = 0; u < kManyU; ++u) deliver<FAN, V>(gd, n, (base + (uint64_t)u * kBlock + threadIdx.x) * 16, v[u]);
+            for (int u = 0; u < kManyU; ++u) deliver((base + (uint64_t)u * kBlock + threadIdx.x) * 16, v[u]);
         } else {
             for (uint64_t p = base + threadIdx.x; p < P; p += kBlock)
-                deliver<FAN, V>(gd, n, p * 16, COPY_LD((const MCCLX_GLOBAL V*)(gs + p * 16)));
+                deliver(p * 16, COPY_LD((const MCCLX_GLOBAL Packet*)(gs + p * 16)));
         }
         if (tile == 0) {
             const uint64_t i = P * 16 + threadIdx.x;
@@ -176,19 +176,13 @@ uint64_t copy_items(uint64_t nbytes) {
     return n ? n : (nbytes ? 1 : 0);
 }
 
-hipError_t launch_copy_many(hipStream_t st, const CopyTable& t, int align, int most, uint32_t max_blocks) {
+hipError_t launch_copy_many(hipStream_t st, const CopyTable& t, int most, uint32_t max_blocks) {
     if (t.total_items == 0) return hipSuccess;
     const dim3 grid(t.total_items < max_blocks ? t.total_items : max_blocks), block(kBlock);
-    auto go = [&](auto fan) {
-        constexpr bool FAN = decltype(fan)::value;
-        if (align == 4)
-            copy_many_kernel<4, FAN><<<grid, block, 0, st>>>(t);
-        else if (align == 2)
-            copy_many_kernel<2, FAN><<<grid, block, 0, st>>>(t);
-        else
-            copy_many_kernel<1, FAN><<<grid, block, 0, st>>>(t);
-    };
-    if (most > 1) go(std::true_type{}); else go(std::false_type{});
+    if (most > 1)
+        copy_many_kernel<true><<<grid, block, 0, st>>>(t);
+    else
+        copy_many_kernel<false><<<grid, block, 0, st>>>(t);
     return hipGetLastError();
 }
 
@@ -204,46 +198,51 @@ hipError_t launch_stream_probe(hipStream_t st, void* buf, uint64_t nbytes, bool 
     return hipGetLastError();
 }
 
-hipError_t launch_copy_few(hipStream_t st, const CopyFew& a, int align, int most) {
+namespace {
+template <int N, bool MIXED = false>
+hipError_t launch_copy_few_n(hipStream_t st, const CopyFew& a) {
     uint64_t longest = 0, moved = 0;
     for (uint32_t i = 0; i < a.n; ++i) {
         longest = a.d[i].nbytes > longest ? a.d[i].nbytes : longest;
         moved += a.d[i].nbytes * (1 + a.d[i].n);
     }
-    if (a.n == 0 || longest == 0) return hipSuccess;
+    if (longest == 0) return hipSuccess;
     const uint64_t waves = (longest + 1023) / 1024;
     const bool four = waves * a.n < kOneWaveBlocksFrom;
     const uint64_t g = four ? (waves + 3) / 4 : waves;
     if (g >> 31) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)g, a.n);
-    const uint32_t lds = resident_lds(moved, 16 * (most + 1), most);
-    auto go = [&](auto fan, auto block) {
-        constexpr bool FAN = decltype(fan)::value;
-        constexpr int B = decltype(block)::value;
-        if (align == 4)
-            copy_few_kernel<4, FAN, B><<<grid, dim3(B), lds, st>>>(a);
-        else if (align == 2)
-            copy_few_kernel<2, FAN, B><<<grid, dim3(B), lds, st>>>(a);
-        else
-            copy_few_kernel<1, FAN, B><<<grid, dim3(B), lds, st>>>(a);
-    };
-    const std::integral_constant<int, kOneWave> one_wave;
-    const std::integral_constant<int, kFourWaves> four_waves;
-    if (most > 1) {
-        if (four) go(std::true_type{}, four_waves); else go(std::true_type{}, one_wave);
-    } else {
-        if (four) go(std::false_type{}, four_waves); else go(std::false_type{}, one_wave);
-    }
+    const uint32_t lds = resident_lds(moved, 16 * (N + 1), N, kLaneBytesCopy);
+    if (four)
+        copy_few_kernel<N, kFourWaves, MIXED><<<grid, dim3(kFourWaves), lds, st>>>(a);
+    else
+        copy_few_kernel<N, kOneWave, MIXED><<<grid, dim3(kOneWave), lds, st>>>(a);
     return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_copy_few(hipStream_t st, const CopyFew& a) {
+    if (a.n == 0 || a.n > (uint32_t)kFewCopies) return a.n ? hipErrorInvalidValue : hipSuccess;
+    for (uint32_t i = 1; i < a.n; ++i)
+        if (a.d[i].n != a.d[0].n) return launch_copy_few_n<kCopyDsts, true>(st, a);
+    switch (a.d[0].n) {
+        case 1: return launch_copy_few_n<1>(st, a);
+        case 2: return launch_copy_few_n<2>(st, a);
+        case 3: return launch_copy_few_n<3>(st, a);
+        case 4: return launch_copy_few_n<4>(st, a);
+        case 5: return launch_copy_few_n<5>(st, a);
+        case 6: return launch_copy_few_n<6>(st, a);
+        case 7: return launch_copy_few_n<7>(st, a);
+        case 8: return launch_copy_few_n<8>(st, a);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 hipError_t launch_copy(hipStream_t st, void* dst, const void* src, uint64_t nbytes) {
-    if (nbytes == 0) return hipSuccess;
     CopyFew a;
     a.d[0] = CopyDesc{src, nbytes, 1, {dst}};
     a.n = 1;
-    const uintptr_t both = reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src);
-    return launch_copy_few(st, a, both % 4 == 0 ? 4 : both % 2 == 0 ? 2 : 1, 1);
+    return launch_copy_few(st, a);
 }
 
 }  // namespace mcclx

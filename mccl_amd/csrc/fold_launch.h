@@ -107,16 +107,17 @@ hipError_t launch_fold(hipStream_t st, const PlanKey& key, const LaunchParams& l
 // one time shrinks with the bytes under way, and 70-80 KiB per CU (20 MB on the device) still
 // covers the latency.  The optimum, swept over 3..20 waves per CU, lies near one number of
 // bytes for every shape, waves x bytes a lane moves: 1160 (8 operands into one: 8 waves;
-// 4 into one: 14; 3 into one: 18; one source to 4 / 8 destinations: 11-14 / 7-8), a little
-// more where tensors are reduced in place, which opens each row once for both directions
-// (2 / 3 / 4 / 5 / 8 ranks: 18 / 12 / 8-10 / 8 / 5 waves).  A reservation of LDS nobody uses
+// 4 into one: 14; 3 into one: 18), a little less where one source is copied to several
+// destinations (4 / 6 / 8: 12 / 9 / 7 waves, 33 M elements to four 214 -> 206 us against 14)
+// and a little more where tensors are reduced in place (2 / 3 / 4 / 5 / 8 ranks: 18 / 12 /
+// 8-10 / 8 / 5 waves).  A reservation of LDS nobody uses
 // sets the number: it is granted in units of 1280 bytes of a CU's 160 KiB.
 //
 // A launch that ends soon needs its waves to get going: the limit pays from 160 MB moved on
 // (200 MB, eight operands into one: 36.2 -> 35.4 us; 80 MB: 5.5 TB/s without it, 5.1 with),
 // and not where 20 waves or more would be left of a launch with one output.
 constexpr uint64_t kResidentMinBytes = 160'000'000;
-constexpr int kLaneBytes = 1160, kLaneBytesInPlace = 1280;
+constexpr int kLaneBytes = 1160, kLaneBytesInPlace = 1280, kLaneBytesCopy = 1020;
 inline uint32_t resident_lds(uint64_t launch_bytes, int lane_bytes, int outputs, int budget = kLaneBytes) {
     int waves = budget / lane_bytes;
     if (launch_bytes < kResidentMinBytes || (outputs == 1 && waves >= 20)) return 0;
@@ -155,12 +156,11 @@ struct CopyFew {
     CopyDesc d[kFewCopies];
     uint32_t n;
 };
-// `most`: the largest number of destinations any descriptor of the launch has.
-hipError_t launch_copy_few(hipStream_t st, const CopyFew& copies, int align, int most);
+hipError_t launch_copy_few(hipStream_t st, const CopyFew& copies);
 // Work items (tiles) one copy of nbytes splits into.
 uint64_t copy_items(uint64_t nbytes);
-// `align`: the widest of 4 / 2 / 1 bytes that every pointer in the table is aligned to.
-hipError_t launch_copy_many(hipStream_t st, const CopyTable& t, int align, int most, uint32_t max_blocks);
+// `most`: the largest number of destinations any descriptor of the launch has.
+hipError_t launch_copy_many(hipStream_t st, const CopyTable& t, int most, uint32_t max_blocks);
 
 // Plain device copy with the same packet shape (also the calibration kernel for
 // the memory counters): dst <- src, nbytes.

@@ -970,7 +970,6 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
     // Consecutive copies of one source become one descriptor with several destinations
     // (the schedules list them that way): the source is read once.
     std::vector<mcclx::CopyDesc> groups;
-    uintptr_t both = 0;
     uint64_t bytes = 0;  // per destination: what decides the length of a grid
     int most = 0;
     for (uint32_t i = 0; i < n; ++i) {
@@ -981,7 +980,6 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
             if (int rc = check_range(d.src, d.nbytes, "src", i)) return rc;
             if (int rc = check_range(d.dst, d.nbytes, "dst", i)) return rc;
         }
-        both |= reinterpret_cast<uintptr_t>(d.dst) | reinterpret_cast<uintptr_t>(d.src);
         mcclx::CopyDesc* last = groups.empty() ? nullptr : &groups.back();
         if (last && last->src == d.src && last->nbytes == d.nbytes && last->n < (uint64_t)mcclx::kCopyDsts) {
             last->dst[last->n++] = d.dst;
@@ -995,7 +993,6 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
     const uint32_t live = (uint32_t)groups.size();
     DeviceGuard guard(ctx->device);
     if (!guard.ok) return fail(MCCLX_ERR_HIP, "hipSetDevice(%d) failed", ctx->device);
-    const int align = (both % 4 == 0) ? 4 : (both % 2 == 0) ? 2 : 1;
     // Few or large copies: descriptors in the kernel arguments, up to 32 copies per
     // grid (a block of the table kernel first has to fetch its descriptor from
     // memory, which costs large copies 5-10 %); the grid is as wide as the longest
@@ -1007,7 +1004,7 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
         uint64_t longest = 0, sum = 0;
         auto flush = [&]() -> int {
             if (few.n == 0) return MCCLX_OK;
-            hipError_t e = mcclx::launch_copy_few(ctx->stream, few, align, most);
+            hipError_t e = mcclx::launch_copy_few(ctx->stream, few);
             if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy_batched launch failed: %s", hipGetErrorString(e));
             ++ctx->launches;
             few.n = 0;
@@ -1058,7 +1055,7 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
     t.total_items = (uint32_t)total;
     t.uniform_items = (uint32_t)uniform;
     t.n = live;
-    hipError_t e = mcclx::launch_copy_many(ctx->stream, t, align, most, ctx->max_blocks);
+    hipError_t e = mcclx::launch_copy_many(ctx->stream, t, most, ctx->max_blocks);
     if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy_batched launch failed: %s", hipGetErrorString(e));
     ++ctx->launches;
     return MCCLX_OK;
