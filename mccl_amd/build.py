@@ -95,7 +95,7 @@ def build(force: bool = True, verbose: bool = False) -> str:
 
 
 BACKEND_DIR = os.path.join(CSRC, "backend")
-BACKEND_SOURCES = ["Progress.cpp", "LocalMesh.cpp", "WorkMCCL.cpp", "HostWire.cpp", "ProcessGroupMCCL.cpp", "bindings.cpp"]
+BACKEND_SOURCES = ["Progress.cpp", "LocalMesh.cpp", "WorkMCCL.cpp", "HostWire.cpp", "ProcessGroupMCCL.cpp", "Replays.cpp", "bindings.cpp"]
 
 
 def backend_path() -> str:

@@ -35,6 +35,7 @@
 #include "backend/Phases.hpp"
 #include "backend/ProcessGroupMCCL.hpp"
 #include "backend/Progress.hpp"
+#include "backend/Replays.hpp"
 #include "backend/WorkMCCL.hpp"
 
 namespace py = pybind11;
@@ -498,4 +499,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("_test_mesh", &mesh_probe, py::arg("world"), py::arg("rounds") = 3, py::arg("absent") = -1,
           py::arg("timeout_ms") = 2000, py::arg("leader_throws") = false, py::arg("late_ms") = -1,
           py::call_guard<py::gil_scoped_release>());
+    mccl::bind_replays(m);
 }

@@ -19,6 +19,8 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <iterator>
+#include <map>
 #include <string>
 #include <vector>
 
@@ -585,27 +587,48 @@ int run_stepwise(mcclx_ctx* ctx, const mcclx_replay* r) {
     return replay_stepwise(ctx, &s, Ls);
 }
 
-// Byte ranges one replay reads or writes: its rank tensors and its workspace.
-struct Range {
-    uintptr_t lo, hi;
+// The byte ranges the replays of a run read or write -- their rank tensors and workspaces --
+// as disjoint intervals, neighbours merged: the tensors of a list are usually views that
+// follow one another, and thousands of them make a handful of intervals.  (Held against
+// every earlier range instead, a list of 4096 messages cost 20 ms.)
+class Touched {
+public:
+    // Does the replay touch memory an earlier one has touched?  If not, its ranges are added.
+    bool add(const mcclx_replay* r) {
+        const uint64_t tb = r->numel * esize(r->dtype);
+        auto each = [&](auto&& f) {
+            for (int i = 0; i < r->world; ++i)
+                if (f(reinterpret_cast<uintptr_t>(r->tensors[i]), tb)) return true;
+            return r->workspace && r->workspace_bytes && f(reinterpret_cast<uintptr_t>(r->workspace), r->workspace_bytes);
+        };
+        if (each([&](uintptr_t p, uint64_t n) { return hits(p, p + n); })) return false;
+        each([&](uintptr_t p, uint64_t n) {
+            insert(p, p + n);
+            return false;
+        });
+        return true;
+    }
+
+private:
+    std::map<uintptr_t, uintptr_t> spans_;  // start -> end
+    bool hits(uintptr_t lo, uintptr_t hi) const {
+        auto it = spans_.upper_bound(lo);
+        if (it != spans_.end() && it->first < hi) return true;
+        return it != spans_.begin() && std::prev(it)->second > lo;
+    }
+    void insert(uintptr_t lo, uintptr_t hi) {  // a rank's tensors of one replay may overlap each other
+        auto it = spans_.upper_bound(lo);
+        if (it != spans_.begin() && std::prev(it)->second >= lo) {
+            --it;
+            lo = it->first;
+        }
+        while (it != spans_.end() && it->first <= hi) {
+            hi = hi > it->second ? hi : it->second;
+            it = spans_.erase(it);
+        }
+        spans_.emplace(lo, hi);
+    }
 };
-void ranges_of(const mcclx_replay* r, std::vector<Range>& out) {
-    const uint64_t tb = r->numel * esize(r->dtype);
-    for (int i = 0; i < r->world; ++i) {
-        const uintptr_t p = reinterpret_cast<uintptr_t>(r->tensors[i]);
-        out.push_back(Range{p, p + tb});
-    }
-    if (r->workspace && r->workspace_bytes) {
-        const uintptr_t p = reinterpret_cast<uintptr_t>(r->workspace);
-        out.push_back(Range{p, p + r->workspace_bytes});
-    }
-}
-bool overlaps(const std::vector<Range>& a, const std::vector<Range>& b) {
-    for (const Range& x : a)
-        for (const Range& y : b)
-            if (x.lo < y.hi && y.lo < x.hi) return true;
-    return false;
-}
 
 // Same plan for every phase?
 bool same_plan(const mcclx_replay* a, const mcclx_replay* b) {
@@ -685,17 +708,14 @@ int mcclx_allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t
         // earlier result, as in the reference's one-by-one loop (ProcessGroupMCCL.cpp:173-177).
         Phases ph;
         const mcclx_replay* first = &rs[i];
-        std::vector<Range> taken, mine;
+        Touched touched;
         while (i < n) {
             if (&rs[i] != first) {
                 if (!same_plan(first, &rs[i])) break;
                 TRY(check_replay(ctx, &rs[i], &fused, &nothing));
                 if (!fused || nothing) break;
             }
-            mine.clear();
-            ranges_of(&rs[i], mine);
-            if (overlaps(taken, mine)) break;
-            taken.insert(taken.end(), mine.begin(), mine.end());
+            if (!touched.add(&rs[i])) break;
             collect_fused(&rs[i], layout_of(&rs[i]), ph);
             ++i;
         }

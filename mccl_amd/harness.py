@@ -18,6 +18,11 @@ from . import _lib as L
 from ._lib import MCCLError
 from .kernels import ReduceQueue, _q, _check_tensor, dtype_code, op_code
 
+try:  # lists of tensors are read natively where the extension is built
+    from . import _C as _native
+except ImportError:
+    _native = None
+
 ALGO_NAMES = {"ring": L.ALGO_RING, "tree": L.ALGO_TREE, "butterfly": L.ALGO_BUTTERFLY}
 
 
@@ -93,6 +98,10 @@ def allreduce_replay(tensors: List[torch.Tensor], op, algo: int, wire_bf16: bool
                      workspace: Optional[Workspace] = None, sync: bool = True) -> None:
     """In-place allreduce over the virtual ranks' tensors with a fixed algorithm."""
     q = _q(queue)
+    if workspace is None and _native is not None:
+        rc = _native._allreduce_replay(q.handle.value, q.device, tensors, op_code(op), algo, bool(wire_bf16), mode, acc)
+        if rc is not None:
+            return L.check(rc)
     if not tensors:
         raise MCCLError("[MCCL] Check failed: !tensors.empty() — allreduce: empty tensor list")
     for t in tensors:
@@ -136,6 +145,11 @@ def allreduce_replay_many(groups: List[List[torch.Tensor]], op, algo: int, wire_
     c10d allreduce over a list of tensors: entries that share a plan go out together,
     one launch per phase for all of them."""
     q = _q(queue)
+    if _native is not None:
+        rc = _native._allreduce_replay_many(q.handle.value, q.device, groups, op_code(op), algo, bool(wire_bf16),
+                                            _in_place_mode(mode), acc)
+        if rc is not None:
+            return L.check(rc)
     reps = (L.Replay * len(groups))()
     keep = []
     needs = []
@@ -167,6 +181,12 @@ def allreduce_replay_many(groups: List[List[torch.Tensor]], op, algo: int, wire_
 
 def allreduce(tensors: List[torch.Tensor], op="sum", queue=None, mode: int = L.REPLAY_FUSED) -> int:
     """ProcessGroupMCCL::allreduce for N virtual ranks; returns the algorithm used."""
+    if _native is not None:
+        q = _q(queue)
+        done = _native._allreduce(q.handle.value, q.device, tensors, op_code(op), _in_place_mode(mode))
+        if done is not None:
+            L.check(done[0])
+            return done[1]
     wire, env_algo, tree_below = _env_config()
     t0 = tensors[0]
     use_wire = wire and t0.dtype == torch.float32
