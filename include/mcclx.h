@@ -260,6 +260,16 @@ MCCLX_API int mcclx_fold_batched_noalloc(mcclx_ctx* ctx, const mcclx_plan* plan,
  * ProcessGroupMCCL.cpp:232-273). */
 MCCLX_API int mcclx_copy(mcclx_ctx* ctx, void* dst, const void* src, uint64_t nbytes);
 
+/* The tensor forms: one launch at the end of `stream` (a HIP stream of the context's device), as
+ * mcclx_queue_wait_stream, the call above of the same name and mcclx_stream_wait_queue in a row
+ * give it -- behind everything enqueued so far on `stream` and on the queue, in front of what
+ * either is given next.  Where the queue is idle the kernel runs on `stream` itself. */
+MCCLX_API int mcclx_reduce_ordered(mcclx_ctx* ctx, void* stream, void* dst, const void* src, int dtype, uint64_t count, int op);
+MCCLX_API int mcclx_scale_ordered(mcclx_ctx* ctx, void* stream, void* buf, int dtype, uint64_t count, double scale, int scale_mode);
+MCCLX_API int mcclx_accumulate_scale_ordered(mcclx_ctx* ctx, void* stream, void* dst, const void* src, int dtype, uint64_t count, double scale);
+MCCLX_API int mcclx_encode_bf16_ordered(mcclx_ctx* ctx, void* stream, void* dst_bf16, const void* src_f32, uint64_t count);
+MCCLX_API int mcclx_decode_bf16_ordered(mcclx_ctx* ctx, void* stream, void* dst_f32, const void* src_bf16, uint64_t count);
+
 /* Many copies with one launch: the allgather leg of a schedule hands every
  * reduced chunk to every other rank (AllreduceAlgos.cpp:77-86, 185-200; the
  * tree's broadcast :119-126), N-1 sends per chunk in the reference.  Ranges of

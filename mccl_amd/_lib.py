@@ -88,6 +88,11 @@ SIGNATURES = {
     "mcclx_fold": (_i, [_vp, C.POINTER(Plan), C.POINTER(Seg)]),
     "mcclx_fold_batched": (_i, [_vp, C.POINTER(Plan), C.POINTER(Seg), C.c_uint32]),
     "mcclx_fold_batched_noalloc": (_i, [_vp, C.POINTER(Plan), C.POINTER(Seg), C.c_uint32]),
+    "mcclx_reduce_ordered": (_i, [_vp, _vp, _vp, _vp, _i, _u64, _i]),
+    "mcclx_scale_ordered": (_i, [_vp, _vp, _vp, _i, _u64, _d, _i]),
+    "mcclx_accumulate_scale_ordered": (_i, [_vp, _vp, _vp, _vp, _i, _u64, _d]),
+    "mcclx_encode_bf16_ordered": (_i, [_vp, _vp, _vp, _vp, _u64]),
+    "mcclx_decode_bf16_ordered": (_i, [_vp, _vp, _vp, _vp, _u64]),
     "mcclx_copy": (_i, [_vp, _vp, _vp, _u64]),
     "mcclx_copy_batched": (_i, [_vp, C.POINTER(CopyDesc), C.c_uint32]),
     "mcclx_queue_drain": (_i, [_vp]),

@@ -101,6 +101,15 @@ struct mcclx_ctx {
     // re-recorded until 15 later waits have been issued
     hipEvent_t xev[16] = {};
     int xnext = 0;
+    // The newest launch that ran on a caller's stream in the queue's place (ordered_launch) and that
+    // neither the queue nor the host has waited for yet.
+    std::mutex away_mu;
+    std::atomic<bool> away{false};
+    hipStream_t away_stream = nullptr;
+    uint64_t away_number = 0;  // counts those launches; launch i marks its end in away_ev[i % kAwayEvents]
+    static constexpr uint64_t kAwayEvents = 4;
+    hipEvent_t away_ev[kAwayEvents] = {};
+    std::atomic<bool> exposed{false};  // the caller holds the queue's HIP stream (mcclx_queue_stream)
     hipStream_t upload_stream = nullptr;  // blocking table uploads while the queue is recording
     // staging pool (MPSInterop.mm:47-204): one grow-only pinned buffer for sends,
     // two fixed pinned chunks + events for pipelined receives from pageable memory
@@ -127,6 +136,41 @@ struct DeviceGuard {
         if (prev >= 0) (void)hipSetDevice(prev);
     }
 };
+
+// The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its place.
+hipStream_t queue_of(mcclx_ctx* ctx) {
+    if (ctx->away.load(std::memory_order_acquire)) {
+        std::lock_guard<std::mutex> lk(ctx->away_mu);
+        if (ctx->away.load(std::memory_order_relaxed)) {
+            const hipEvent_t ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
+            if (hipStreamWaitEvent(ctx->stream, ev, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                (void)hipEventSynchronize(ev);
+            }
+            ctx->away.store(false, std::memory_order_release);
+        }
+    }
+    return ctx->stream;
+}
+
+// Blocks until everything issued through the context has finished.
+hipError_t drain(mcclx_ctx* ctx) {
+    if (ctx->away.load(std::memory_order_acquire)) {
+        hipEvent_t ev;
+        uint64_t number;
+        {
+            std::lock_guard<std::mutex> lk(ctx->away_mu);
+            number = ctx->away_number;
+            ev = ctx->away_ev[number % mcclx_ctx::kAwayEvents];
+        }
+        // (a thread that launches again meanwhile makes this wait longer, never shorter)
+        if (ev)
+            if (hipError_t e = hipEventSynchronize(ev); e != hipSuccess) return e;
+        std::lock_guard<std::mutex> lk(ctx->away_mu);
+        if (ctx->away_number == number) ctx->away.store(false, std::memory_order_release);
+    }
+    return hipStreamSynchronize(ctx->stream);
+}
 
 // binary16 <- binary64 in one rounding (the `(__fp16)scale` of
 // MetalKernels.mm:387,656): scale into the target's quantum, round to nearest
@@ -423,7 +467,7 @@ int stage_table(mcclx_ctx* ctx, const void* bytes, size_t nbytes, void** dev, Ta
     ctx->next_slot = (ctx->next_slot + 1) % kTableSlots;
     if (int rc = ensure_slot(ctx, sl, nbytes)) return rc;
     memcpy(sl.host, bytes, nbytes);
-    HIP_TRY(hipMemcpyAsync(sl.dev, sl.host, nbytes, hipMemcpyHostToDevice, ctx->stream));
+    HIP_TRY(hipMemcpyAsync(sl.dev, sl.host, nbytes, hipMemcpyHostToDevice, queue_of(ctx)));
     // The slot's pinned half is busy until this copy has run; its device half is only
     // touched on the queue, whose order keeps the next upload behind the launch that
     // reads this one.  Recorded here, so that no exit path of the caller can skip it.
@@ -434,9 +478,9 @@ int stage_table(mcclx_ctx* ctx, const void* bytes, size_t nbytes, void** dev, Ta
     return MCCLX_OK;
 }
 
-// Descriptors in the kernel arguments (nseg <= kFewSegs).
+// Descriptors in the kernel arguments (nseg <= kFewSegs), on the queue or on `st`.
 int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, int has_scale,
-                    const mcclx_seg* segs, uint32_t nseg, int fan) {
+                    const mcclx_seg* segs, uint32_t nseg, int fan, hipStream_t st) {
     mcclx::LaunchParams lp;
     lp.max_blocks = ctx->max_blocks;
     lp.fan = fan > 0 ? fan : 0;
@@ -455,7 +499,7 @@ int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, in
     a.has_scale = has_scale;
     a.nseg = (int32_t)nseg;
     lp.few = &a;
-    hipError_t e = mcclx::launch_fold(ctx->stream, key, lp);
+    hipError_t e = mcclx::launch_fold(st, key, lp);
     if (e != hipSuccess) return launch_error(e, key);
     ++ctx->launches;
     if (held) ++ctx->hold_launches;
@@ -490,7 +534,7 @@ int fold_impl(mcclx_ctx* ctx, const mcclx_plan* plan, const mcclx_seg* segs, uin
     mcclx::LaunchParams lp;
     lp.max_blocks = ctx->max_blocks;
     if (nseg <= ctx->few_max && even_enough(key, segs, nseg))
-        return launch_by_value(ctx, key, scale_f, has_scale, segs, nseg, fan);
+        return launch_by_value(ctx, key, scale_f, has_scale, segs, nseg, fan, queue_of(ctx));
 
     // descriptor table: segs, then nseg+1 work-item prefix sums
     std::lock_guard<std::mutex> lk(ctx->mu);
@@ -536,7 +580,7 @@ int fold_impl(mcclx_ctx* ctx, const mcclx_plan* plan, const mcclx_seg* segs, uin
     lp.table = &t;
     lp.fan = fan > 0 ? fan : 0;
     lp.to_all = fan == kToAll;
-    hipError_t e = mcclx::launch_fold(ctx->stream, key, lp);
+    hipError_t e = mcclx::launch_fold(queue_of(ctx), key, lp);
     if (e != hipSuccess) return launch_error(e, key);
     ++ctx->launches;
     return MCCLX_OK;
@@ -764,10 +808,12 @@ int mcclx_init_on_stream(int device, void* hip_stream, mcclx_ctx** out) {
 int mcclx_destroy(mcclx_ctx* ctx) {
     if (!ctx) return MCCLX_OK;
     DeviceGuard guard(ctx->device);
-    (void)hipStreamSynchronize(ctx->stream);
+    (void)drain(ctx);
     for (auto& kv : ctx->tickets) (void)hipEventDestroy(kv.second.ev);
     for (auto ev : ctx->free_events) (void)hipEventDestroy(ev);
     for (auto ev : ctx->xev)
+        if (ev) (void)hipEventDestroy(ev);
+    for (auto ev : ctx->away_ev)
         if (ev) (void)hipEventDestroy(ev);
     for (auto& sl : ctx->slots) {
         if (sl.host) (void)hipHostFree(sl.host);
@@ -786,7 +832,12 @@ int mcclx_destroy(mcclx_ctx* ctx) {
     return MCCLX_OK;
 }
 
-void* mcclx_queue_stream(mcclx_ctx* ctx) { return ctx ? (void*)ctx->stream : nullptr; }
+void* mcclx_queue_stream(mcclx_ctx* ctx) {
+    if (!ctx) return nullptr;
+    ctx->exposed.store(true);
+    DeviceGuard guard(ctx->device);
+    return (void*)queue_of(ctx);
+}
 int mcclx_device_cus(mcclx_ctx* ctx) { return ctx ? ctx->cus : 0; }
 uint64_t mcclx_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->launches.load() : 0; }
 uint64_t mcclx_hold_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->hold_launches.load() : 0; }
@@ -825,7 +876,7 @@ int mcclx_fold_batched_noalloc(mcclx_ctx* ctx, const mcclx_plan* plan, const mcc
     DeviceGuard guard(ctx->device);
     if (!guard.ok) return fail(MCCLX_ERR_HIP, "hipSetDevice(%d) failed", ctx->device);
     if (nseg <= (uint32_t)mcclx::kFewSegs && even_enough(key, segs, nseg))
-        return launch_by_value(ctx, key, scale_f, has_scale, segs, nseg, fan);
+        return launch_by_value(ctx, key, scale_f, has_scale, segs, nseg, fan, queue_of(ctx));
 
     // One table per GPU, shared by every context on it: a second call that enters while this
     // one is still writing its descriptors would mix the two tables.  (Calls on one context
@@ -866,7 +917,7 @@ int mcclx_fold_batched_noalloc(mcclx_ctx* ctx, const mcclx_plan* plan, const mcc
                 ++next_prefix;
             }
         }
-        hipError_t e = mcclx::launch_table_write(ctx->stream, table + off, buf, n);
+        hipError_t e = mcclx::launch_table_write(queue_of(ctx), table + off, buf, n);
         if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "table write launch failed: %s", hipGetErrorString(e));
         ++ctx->launches;
     }
@@ -884,68 +935,145 @@ int mcclx_fold_batched_noalloc(mcclx_ctx* ctx, const mcclx_plan* plan, const mcc
     lp.table = &t;
     lp.fan = fan > 0 ? fan : 0;
     lp.to_all = fan == kToAll;
-    hipError_t e = mcclx::launch_fold(ctx->stream, key, lp);
+    hipError_t e = mcclx::launch_fold(queue_of(ctx), key, lp);
     if (e != hipSuccess) return launch_error(e, key);
     ++ctx->launches;
     return MCCLX_OK;
 }
 
+// Each call comes as a launch on the queue and, with a stream, in its ordered form.
+struct OneLaunch {
+    mcclx_plan plan;
+    mcclx_seg seg;
+};
+static int issue(mcclx_ctx* ctx, const OneLaunch& l) { return fold_impl(ctx, &l.plan, &l.seg, 1); }
+static OneLaunch one_launch(int dtype, int io, int k, int op, int scale_mode, double scale, void* out, void* wire_out,
+                            const void* in0, const void* in1, uint64_t count) {
+    OneLaunch l;
+    l.plan = {dtype, io, k, MCCLX_TOPO_FOLD, op, MCCLX_ACC_STEP, scale_mode, 0, scale};
+    memset(&l.seg, 0, sizeof l.seg);
+    l.seg.out = out;
+    l.seg.wire_out = wire_out;
+    l.seg.in[0] = in0;
+    l.seg.in[1] = in1;
+    l.seg.count = count;
+    return l;
+}
+static OneLaunch reduce_launch(void* dst, const void* src, int dtype, uint64_t count, int op) {
+    return one_launch(dtype, MCCLX_IO_PURE, 2, op, MCCLX_SCALE_NONE, 0.0, dst, nullptr, dst, src, count);
+}
+static OneLaunch scale_launch(void* buf, int dtype, uint64_t count, double scale, int scale_mode) {
+    return one_launch(dtype, MCCLX_IO_PURE, 1, MCCLX_SUM, scale_mode, scale, buf, nullptr, buf, nullptr, count);
+}
+static OneLaunch accumulate_scale_launch(void* dst, const void* src, int dtype, uint64_t count, double scale) {
+    return one_launch(dtype, MCCLX_IO_PURE, 2, MCCLX_SUM, MCCLX_SCALE_TENSOR, scale, dst, nullptr, dst, src, count);
+}
+static OneLaunch encode_launch(void* dst_bf16, const void* src_f32, uint64_t count) {
+    return one_launch(MCCLX_BF16, MCCLX_IO_OWN_FIRST_F32, 1, MCCLX_SUM, MCCLX_SCALE_NONE, 0.0, nullptr, dst_bf16, src_f32, nullptr, count);
+}
+static OneLaunch decode_launch(void* dst_f32, const void* src_bf16, uint64_t count) {
+    return one_launch(MCCLX_BF16, MCCLX_IO_OUT_F32, 1, MCCLX_SUM, MCCLX_SCALE_NONE, 0.0, dst_f32, nullptr, src_bf16, nullptr, count);
+}
+
 int mcclx_reduce(mcclx_ctx* ctx, void* dst, const void* src, int dtype, uint64_t count, int op) {
-    mcclx_plan p = {dtype, MCCLX_IO_PURE, 2, MCCLX_TOPO_FOLD, op, MCCLX_ACC_STEP, MCCLX_SCALE_NONE, 0, 0.0};
-    mcclx_seg s;
-    memset(&s, 0, sizeof s);
-    s.out = dst;
-    s.in[0] = dst;
-    s.in[1] = src;
-    s.count = count;
-    return fold_impl(ctx, &p, &s, 1);
+    return issue(ctx, reduce_launch(dst, src, dtype, count, op));
 }
 
 int mcclx_scale(mcclx_ctx* ctx, void* buf, int dtype, uint64_t count, double scale, int scale_mode) {
     if (scale_mode != MCCLX_SCALE_VIEW && scale_mode != MCCLX_SCALE_TENSOR)
         return fail(MCCLX_ERR_INVALID, "scale_mode %d is not VIEW or TENSOR", scale_mode);
-    mcclx_plan p = {dtype, MCCLX_IO_PURE, 1, MCCLX_TOPO_FOLD, MCCLX_SUM, MCCLX_ACC_STEP, scale_mode, 0, scale};
-    mcclx_seg s;
-    memset(&s, 0, sizeof s);
-    s.out = buf;
-    s.in[0] = buf;
-    s.count = count;
-    return fold_impl(ctx, &p, &s, 1);
+    return issue(ctx, scale_launch(buf, dtype, count, scale, scale_mode));
 }
 
-int mcclx_accumulate_scale(mcclx_ctx* ctx, void* dst, const void* src, int dtype, uint64_t count,
-                           double scale) {
-    mcclx_plan p = {dtype, MCCLX_IO_PURE, 2, MCCLX_TOPO_FOLD, MCCLX_SUM, MCCLX_ACC_STEP,
-                    MCCLX_SCALE_TENSOR, 0, scale};
-    mcclx_seg s;
-    memset(&s, 0, sizeof s);
-    s.out = dst;
-    s.in[0] = dst;
-    s.in[1] = src;
-    s.count = count;
-    return fold_impl(ctx, &p, &s, 1);
+int mcclx_accumulate_scale(mcclx_ctx* ctx, void* dst, const void* src, int dtype, uint64_t count, double scale) {
+    return issue(ctx, accumulate_scale_launch(dst, src, dtype, count, scale));
 }
 
 int mcclx_encode_bf16(mcclx_ctx* ctx, void* dst_bf16, const void* src_f32, uint64_t count) {
-    mcclx_plan p = {MCCLX_BF16, MCCLX_IO_OWN_FIRST_F32, 1, MCCLX_TOPO_FOLD, MCCLX_SUM, MCCLX_ACC_STEP,
-                    MCCLX_SCALE_NONE, 0, 0.0};
-    mcclx_seg s;
-    memset(&s, 0, sizeof s);
-    s.wire_out = dst_bf16;
-    s.in[0] = src_f32;
-    s.count = count;
-    return fold_impl(ctx, &p, &s, 1);
+    return issue(ctx, encode_launch(dst_bf16, src_f32, count));
 }
 
 int mcclx_decode_bf16(mcclx_ctx* ctx, void* dst_f32, const void* src_bf16, uint64_t count) {
-    mcclx_plan p = {MCCLX_BF16, MCCLX_IO_OUT_F32, 1, MCCLX_TOPO_FOLD, MCCLX_SUM, MCCLX_ACC_STEP,
-                    MCCLX_SCALE_NONE, 0, 0.0};
-    mcclx_seg s;
-    memset(&s, 0, sizeof s);
-    s.out = dst_f32;
-    s.in[0] = src_bf16;
-    s.count = count;
-    return fold_impl(ctx, &p, &s, 1);
+    return issue(ctx, decode_launch(dst_f32, src_bf16, count));
+}
+
+// A launch between two orderings, "the queue waits for `stream`" and "`stream` waits for the
+// queue", is a launch at the end of `stream` that the queue's earlier work comes before and its
+// later work behind.  Where the queue is idle the first holds already and the launch runs on
+// `stream` itself, its end marked for whoever uses the queue next (queue_of, drain,
+// mcclx_stream_wait_queue): no cross-stream event and none of the two hand-overs between
+// hardware queues, which bound a sequence of such calls (events and launch 31 us a call, the
+// launch and its mark 7; 4097 bf16 values reduced through Python 48 -> 8 us, 25 MiB encoded and
+// decoded 110 -> 23 us).  The mark is an event record and not the kernel's own stop event: after
+// thousands of launches with one, the next calls on the stream took three times as long.
+// Everything else takes the two orderings: a queue with work in flight, a queue whose HIP stream
+// the caller holds (what they put there would not see a launch made elsewhere), a recording or a
+// `stream` that records, another caller's stream still at work in the queue's place.
+static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
+    if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    auto records = [](hipStream_t s) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+    };
+    if (l.seg.count && st != ctx->stream && !ctx->capturing && !ctx->exposed.load() && ctx->few_max >= 1) {
+        DeviceGuard guard(ctx->device);
+        if (!guard.ok) return fail(MCCLX_ERR_HIP, "hipSetDevice(%d) failed", ctx->device);
+        if (!records(st) && !records(ctx->stream) && hipStreamQuery(ctx->stream) == hipSuccess) {
+            std::lock_guard<std::mutex> lk(ctx->away_mu);
+            if (ctx->away.load(std::memory_order_relaxed) && ctx->away_stream != st &&
+                hipEventQuery(ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents]) == hipSuccess)
+                ctx->away.store(false, std::memory_order_release);
+            if (!ctx->away.load(std::memory_order_relaxed) || ctx->away_stream == st) {
+                mcclx::PlanKey key;
+                float scale_f;
+                int has_scale, fan;
+                if (int rc = check_plan(&l.plan, &key, &scale_f, &has_scale, &fan)) return rc;
+                if (int rc = check_segs(ctx, key, &l.seg, 1, fan)) return rc;
+                hipEvent_t& ev = ctx->away_ev[(ctx->away_number + 1) % mcclx_ctx::kAwayEvents];
+                if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+                if (int rc = launch_by_value(ctx, key, scale_f, has_scale, &l.seg, 1, fan, st)) return rc;
+                if (hipError_t e = hipEventRecord(ev, st); e != hipSuccess) {  // no mark to order by: the host waits
+                    HIP_TRY(hipStreamSynchronize(st));
+                    return MCCLX_OK;
+                }
+                ++ctx->away_number;
+                ctx->away_stream = st;
+                ctx->away.store(true, std::memory_order_release);
+                return MCCLX_OK;
+            }
+        }
+        (void)hipGetLastError();
+    }
+    if (int rc = mcclx_queue_wait_stream(ctx, stream)) return rc;
+    const int rc = issue(ctx, l);
+    const std::string why = rc ? g_err : std::string();
+    const int waited = mcclx_stream_wait_queue(ctx, stream);
+    if (rc) g_err = why;
+    return rc ? rc : waited;
+}
+
+int mcclx_reduce_ordered(mcclx_ctx* ctx, void* stream, void* dst, const void* src, int dtype, uint64_t count, int op) {
+    return ordered_launch(ctx, stream, reduce_launch(dst, src, dtype, count, op));
+}
+
+int mcclx_scale_ordered(mcclx_ctx* ctx, void* stream, void* buf, int dtype, uint64_t count, double scale, int scale_mode) {
+    if (scale_mode != MCCLX_SCALE_VIEW && scale_mode != MCCLX_SCALE_TENSOR)
+        return fail(MCCLX_ERR_INVALID, "scale_mode %d is not VIEW or TENSOR", scale_mode);
+    return ordered_launch(ctx, stream, scale_launch(buf, dtype, count, scale, scale_mode));
+}
+
+int mcclx_accumulate_scale_ordered(mcclx_ctx* ctx, void* stream, void* dst, const void* src, int dtype, uint64_t count,
+                                   double scale) {
+    return ordered_launch(ctx, stream, accumulate_scale_launch(dst, src, dtype, count, scale));
+}
+
+int mcclx_encode_bf16_ordered(mcclx_ctx* ctx, void* stream, void* dst_bf16, const void* src_f32, uint64_t count) {
+    return ordered_launch(ctx, stream, encode_launch(dst_bf16, src_f32, count));
+}
+
+int mcclx_decode_bf16_ordered(mcclx_ctx* ctx, void* stream, void* dst_f32, const void* src_bf16, uint64_t count) {
+    return ordered_launch(ctx, stream, decode_launch(dst_f32, src_bf16, count));
 }
 
 int mcclx_copy(mcclx_ctx* ctx, void* dst, const void* src, uint64_t nbytes) {
@@ -957,7 +1085,7 @@ int mcclx_copy(mcclx_ctx* ctx, void* dst, const void* src, uint64_t nbytes) {
         if (int rc = check_range(dst, nbytes, "dst", 0)) return rc;
     }
     DeviceGuard guard(ctx->device);
-    hipError_t e = mcclx::launch_copy(ctx->stream, dst, src, nbytes);
+    hipError_t e = mcclx::launch_copy(queue_of(ctx), dst, src, nbytes);
     if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy launch failed: %s", hipGetErrorString(e));
     ++ctx->launches;
     return MCCLX_OK;
@@ -1004,7 +1132,7 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
         uint64_t longest = 0, sum = 0;
         auto flush = [&]() -> int {
             if (few.n == 0) return MCCLX_OK;
-            hipError_t e = mcclx::launch_copy_few(ctx->stream, few);
+            hipError_t e = mcclx::launch_copy_few(queue_of(ctx), few);
             if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy_batched launch failed: %s", hipGetErrorString(e));
             ++ctx->launches;
             few.n = 0;
@@ -1055,7 +1183,7 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
     t.total_items = (uint32_t)total;
     t.uniform_items = (uint32_t)uniform;
     t.n = live;
-    hipError_t e = mcclx::launch_copy_many(ctx->stream, t, most, ctx->max_blocks);
+    hipError_t e = mcclx::launch_copy_many(queue_of(ctx), t, most, ctx->max_blocks);
     if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy_batched launch failed: %s", hipGetErrorString(e));
     ++ctx->launches;
     return MCCLX_OK;
@@ -1083,7 +1211,7 @@ int mcclx_queue_drain(mcclx_ctx* ctx) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     REFUSE_WHILE_RECORDING(ctx, "queue_drain");
     DeviceGuard guard(ctx->device);
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    HIP_TRY(drain(ctx));
     return MCCLX_OK;
 }
 
@@ -1113,7 +1241,14 @@ int mcclx_queue_wait_stream(mcclx_ctx* ctx, void* producer_stream) {
 
 int mcclx_stream_wait_queue(mcclx_ctx* ctx, void* consumer_stream) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
-    return stream_wait(ctx, static_cast<hipStream_t>(consumer_stream), ctx->stream);
+    const hipStream_t consumer = static_cast<hipStream_t>(consumer_stream);
+    if (ctx->away.load(std::memory_order_acquire) && !ctx->capturing) {
+        DeviceGuard guard(ctx->device);
+        std::lock_guard<std::mutex> lk(ctx->away_mu);
+        if (ctx->away.load(std::memory_order_relaxed) && ctx->away_stream != consumer)
+            HIP_TRY(hipStreamWaitEvent(consumer, ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents], 0));
+    }
+    return stream_wait(ctx, consumer, ctx->stream);
 }
 
 int mcclx_event_record(mcclx_ctx* ctx, uint64_t* ticket) {
@@ -1123,7 +1258,7 @@ int mcclx_event_record(mcclx_ctx* ctx, uint64_t* ticket) {
     std::lock_guard<std::mutex> lk(ctx->mu);
     hipEvent_t ev;
     if (int rc = get_event(ctx, &ev)) return rc;
-    HIP_TRY(hipEventRecord(ev, ctx->stream));
+    HIP_TRY(hipEventRecord(ev, queue_of(ctx)));
     *ticket = ctx->next_ticket++;
     ctx->tickets[*ticket].ev = ev;
     return MCCLX_OK;
@@ -1183,7 +1318,7 @@ int mcclx_graph_begin(mcclx_ctx* ctx) {
     if (ctx->capturing) return fail(MCCLX_ERR_STATE, "graph recording already active");
     DeviceGuard guard(ctx->device);
     // relaxed mode: the blocking table uploads above stay legal while recording
-    HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeRelaxed));
+    HIP_TRY(hipStreamBeginCapture(queue_of(ctx), hipStreamCaptureModeRelaxed));
     ctx->capturing = true;
     return MCCLX_OK;
 }
@@ -1214,7 +1349,7 @@ int mcclx_graph_launch(mcclx_ctx* ctx, mcclx_graph* graph) {
     if (!ctx || !graph) return fail(MCCLX_ERR_INVALID, "graph_launch: null argument");
     REFUSE_WHILE_RECORDING(ctx, "graph_launch");
     DeviceGuard guard(ctx->device);
-    HIP_TRY(hipGraphLaunch(graph->exec, ctx->stream));
+    HIP_TRY(hipGraphLaunch(graph->exec, queue_of(ctx)));
     return MCCLX_OK;
 }
 
@@ -1222,7 +1357,7 @@ int mcclx_graph_destroy(mcclx_ctx* ctx, mcclx_graph* graph) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     if (!graph) return MCCLX_OK;
     DeviceGuard guard(ctx->device);
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    HIP_TRY(drain(ctx));
     if (graph->exec) (void)hipGraphExecDestroy(graph->exec);
     if (graph->graph) (void)hipGraphDestroy(graph->graph);
     for (void* t : graph->tables) (void)hipFree(t);
@@ -1278,7 +1413,7 @@ int mcclx_stage_for_send(mcclx_ctx* ctx, const void* device_src, uint64_t nbytes
     DeviceGuard guard(ctx->device);
     void* alias = nullptr;
     if (host_visible(device_src, &alias)) {  // direct path: no copy
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        HIP_TRY(drain(ctx));
         *host_ptr = alias;
         return MCCLX_OK;
     }
@@ -1296,8 +1431,8 @@ int mcclx_stage_for_send(mcclx_ctx* ctx, const void* device_src, uint64_t nbytes
         }
         ctx->stage_send_cap = cap;
     }
-    HIP_TRY(hipMemcpyAsync(ctx->stage_send, device_src, nbytes, hipMemcpyDeviceToHost, ctx->stream));
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    HIP_TRY(hipMemcpyAsync(ctx->stage_send, device_src, nbytes, hipMemcpyDeviceToHost, queue_of(ctx)));
+    HIP_TRY(drain(ctx));
     *host_ptr = ctx->stage_send;
     return MCCLX_OK;
 }
@@ -1310,7 +1445,7 @@ int mcclx_unstage_from_recv(mcclx_ctx* ctx, void* device_dst, const void* host_s
     DeviceGuard guard(ctx->device);
     void* alias = nullptr;
     if (host_visible(host_src, &alias)) {  // pinned source: one asynchronous copy
-        HIP_TRY(hipMemcpyAsync(device_dst, alias, nbytes, hipMemcpyHostToDevice, ctx->stream));
+        HIP_TRY(hipMemcpyAsync(device_dst, alias, nbytes, hipMemcpyHostToDevice, queue_of(ctx)));
         return MCCLX_OK;
     }
     // pageable source: memcpy into one pinned chunk while the other is in flight
@@ -1335,7 +1470,7 @@ int mcclx_unstage_from_recv(mcclx_ctx* ctx, void* device_dst, const void* host_s
             ctx->stage_recv_pending[slot] = false;
         }
         memcpy(ctx->stage_recv[slot], src + off, n);
-        HIP_TRY(hipMemcpyAsync(dst + off, ctx->stage_recv[slot], n, hipMemcpyHostToDevice, ctx->stream));
+        HIP_TRY(hipMemcpyAsync(dst + off, ctx->stage_recv[slot], n, hipMemcpyHostToDevice, queue_of(ctx)));
         HIP_TRY(hipEventRecord(ctx->stage_recv_done[slot], ctx->stream));
         ctx->stage_recv_pending[slot] = true;
     }
@@ -1353,7 +1488,7 @@ int mcclx_host_free(mcclx_ctx* ctx, void* host_ptr) {
         ctx->host_allocs.erase(it);
     }
     DeviceGuard guard(ctx->device);
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    HIP_TRY(drain(ctx));
     HIP_TRY(hipHostFree(host_ptr));
     return MCCLX_OK;
 }

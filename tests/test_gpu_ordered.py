@@ -1,0 +1,112 @@
+"""The tensor variants' ordering: one launch behind everything on torch's stream and on the reduce
+queue, in front of what either gets next -- wherever the launch itself runs (on torch's stream where
+the queue is idle, on the queue otherwise).  Every consumer reads a result without further waits of
+its own, behind a producer that is still running when the call is made."""
+import pytest
+import torch
+
+from mccl_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+
+N = 8_000_003  # some 10 us of device time a launch, several times what a call takes the host
+
+
+def _produce(n=N):
+    """(dst, src) of small whole numbers, the last of a chain of passes still under way."""
+    base = torch.arange(n, device="cuda", dtype=torch.float32).remainder_(64)
+    dst, src = base.clone(), torch.zeros_like(base)
+    for _ in range(40):
+        src.add_(1)
+    return base, dst, src
+
+
+def _streams():
+    return [("default", torch.cuda.default_stream()), ("side", torch.cuda.Stream())]
+
+
+@pytest.mark.parametrize("which", [0, 1])
+@pytest.mark.parametrize("consumer", ["torch", "queue", "other_stream", "ticket", "drain", "other_caller"])
+@pytest.mark.parametrize("queue_state", ["idle", "busy", "exposed"])
+def test_result_is_seen_by_every_consumer(which, consumer, queue_state):
+    q = K.ReduceQueue(0)
+    if queue_state == "exposed":
+        assert q.stream
+    st = _streams()[which][1]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(st):
+        base, dst, src = _produce()
+        got = torch.zeros_like(dst)
+        filler = torch.zeros(64_000_000, device="cuda", dtype=torch.float32)
+        if queue_state == "busy":
+            for _ in range(4):
+                q.copy(filler.data_ptr(), filler.data_ptr() + 128_000_000, 128_000_000)
+        for _ in range(3):
+            K.hip_reduce_op(dst, src, "sum", queue=q)
+        want = base + 3 * 40
+        if consumer == "torch":
+            got.copy_(dst)
+        elif consumer == "queue":          # a raw launch on the queue, then the host waits for the queue
+            q.copy(got.data_ptr(), dst.data_ptr(), 4 * N)
+            q.drain()
+        elif consumer == "other_stream":
+            other = torch.cuda.Stream()
+            q.torch_stream_wait(other)
+            with torch.cuda.stream(other):
+                got.copy_(dst)
+            other.synchronize()
+        elif consumer == "ticket":
+            q.wait(q.record())
+            other = torch.cuda.Stream()
+            with torch.cuda.stream(other):
+                got.copy_(dst)
+            other.synchronize()
+        elif consumer == "drain":
+            q.drain()
+            other = torch.cuda.Stream()
+            with torch.cuda.stream(other):
+                got.copy_(dst)
+            other.synchronize()
+        else:                              # the same queue called from another stream: behind the first caller's launches
+            other = torch.cuda.Stream()
+            with torch.cuda.stream(other):
+                K.hip_reduce_op(got, dst, "sum", queue=q)
+            other.synchronize()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    q.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 4_097, 2_000_003])
+def test_codec_round_trips_on_an_idle_and_a_busy_queue(n):
+    q = K.ReduceQueue(0)
+    x = torch.randn(n, device="cuda")
+    want = x.to(torch.bfloat16)
+    big = torch.zeros(32_000_000, device="cuda")
+    torch.cuda.synchronize()
+    for busy in (False, True, False):
+        if busy:
+            q.copy(big.data_ptr(), big.data_ptr() + 64_000_000, 64_000_000)
+        w = K.encode_bf16(x, queue=q)
+        back = K.decode_bf16(w, queue=q)
+        assert torch.equal(w.view(torch.int16), want.view(torch.int16))
+        assert torch.equal(back, want.float())
+        q.drain()
+    K.hip_scale_inplace(back, 0.5, queue=q)
+    assert torch.equal(back, want.float() * 0.5)
+    q.close()
+
+
+def test_errors_are_the_same_on_either_route():
+    q = K.ReduceQueue(0)
+    a = torch.zeros(8, device="cuda")
+    for _ in range(2):
+        with pytest.raises(K.MCCLError, match="Unsupported ReduceOp"):
+            K.hip_reduce_op(a, a, 9, queue=q)
+        assert q.stream  # from here on through the queue
+    q.graph_begin()
+    with pytest.raises(K.MCCLError, match="not allowed between graph_begin and graph_end"):
+        K.hip_reduce_op(a, a, "sum", queue=q)
+    q.copy(a.data_ptr(), a.data_ptr() + 16, 16)
+    q.graph_destroy(q.graph_end())
+    q.close()
