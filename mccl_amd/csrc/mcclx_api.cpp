@@ -102,14 +102,13 @@ struct mcclx_ctx {
     hipEvent_t xev[16] = {};
     int xnext = 0;
     // The newest launch that ran on a caller's stream in the queue's place (ordered_launch) and that
-    // neither the queue nor the host has waited for yet.
-    std::mutex away_mu;
+    // neither the queue nor the host has waited for yet.  It comes behind every earlier one.
+    std::mutex away_mu;  // also held while something is enqueued on the queue (queue_of); taken after mu
     std::atomic<bool> away{false};
-    hipStream_t away_stream = nullptr;
     uint64_t away_number = 0;  // counts those launches; launch i marks its end in away_ev[i % kAwayEvents]
     static constexpr uint64_t kAwayEvents = 4;
     hipEvent_t away_ev[kAwayEvents] = {};
-    std::atomic<bool> exposed{false};  // the caller holds the queue's HIP stream (mcclx_queue_stream)
+    std::atomic<bool> exposed{false};  // the caller holds the queue's HIP stream (mcclx_queue_stream, mcclx_init_on_stream)
     hipStream_t upload_stream = nullptr;  // blocking table uploads while the queue is recording
     // staging pool (MPSInterop.mm:47-204): one grow-only pinned buffer for sends,
     // two fixed pinned chunks + events for pipelined receives from pageable memory
@@ -137,20 +136,25 @@ struct DeviceGuard {
     }
 };
 
-// The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its place.
-hipStream_t queue_of(mcclx_ctx* ctx) {
-    if (ctx->away.load(std::memory_order_acquire)) {
-        std::lock_guard<std::mutex> lk(ctx->away_mu);
-        if (ctx->away.load(std::memory_order_relaxed)) {
-            const hipEvent_t ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
-            if (hipStreamWaitEvent(ctx->stream, ev, 0) != hipSuccess) {
-                (void)hipGetLastError();
-                (void)hipEventSynchronize(ev);
-            }
-            ctx->away.store(false, std::memory_order_release);
+// The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its
+// place.  As an argument it lives until the call that enqueues the operation has returned, so that
+// no other thread finds the queue idle in between and launches beside it.
+struct QueueUse {
+    std::unique_lock<std::mutex> lk;
+    hipStream_t stream;
+    operator hipStream_t() const { return stream; }
+};
+QueueUse queue_of(mcclx_ctx* ctx) {
+    std::unique_lock<std::mutex> lk(ctx->away_mu);
+    if (ctx->away.load(std::memory_order_relaxed)) {
+        const hipEvent_t ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
+        if (hipStreamWaitEvent(ctx->stream, ev, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipEventSynchronize(ev);
         }
+        ctx->away.store(false, std::memory_order_release);
     }
-    return ctx->stream;
+    return {std::move(lk), ctx->stream};
 }
 
 // Blocks until everything issued through the context has finished.
@@ -755,6 +759,7 @@ int make_ctx(int device, hipStream_t borrowed, bool borrow, mcclx_ctx** out) {
     }
     if (borrow) {
         ctx->stream = borrowed;
+        ctx->exposed.store(true);
     } else {
         e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);  // default priority
         if (e != hipSuccess) {
@@ -836,7 +841,7 @@ void* mcclx_queue_stream(mcclx_ctx* ctx) {
     if (!ctx) return nullptr;
     ctx->exposed.store(true);
     DeviceGuard guard(ctx->device);
-    return (void*)queue_of(ctx);
+    return (void*)(hipStream_t)queue_of(ctx);
 }
 int mcclx_device_cus(mcclx_ctx* ctx) { return ctx ? ctx->cus : 0; }
 uint64_t mcclx_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->launches.load() : 0; }
@@ -1008,7 +1013,7 @@ int mcclx_decode_bf16(mcclx_ctx* ctx, void* dst_f32, const void* src_bf16, uint6
 // thousands of launches with one, the next calls on the stream took three times as long.
 // Everything else takes the two orderings: a queue with work in flight, a queue whose HIP stream
 // the caller holds (what they put there would not see a launch made elsewhere), a recording or a
-// `stream` that records, another caller's stream still at work in the queue's place.
+// `stream` that records.
 static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     const hipStream_t st = static_cast<hipStream_t>(stream);
@@ -1019,17 +1024,17 @@ static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
     if (l.seg.count && st != ctx->stream && !ctx->capturing && !ctx->exposed.load() && ctx->few_max >= 1) {
         DeviceGuard guard(ctx->device);
         if (!guard.ok) return fail(MCCLX_ERR_HIP, "hipSetDevice(%d) failed", ctx->device);
-        if (!records(st) && !records(ctx->stream) && hipStreamQuery(ctx->stream) == hipSuccess) {
+        if (!records(st) && !records(ctx->stream)) {
             std::lock_guard<std::mutex> lk(ctx->away_mu);
-            if (ctx->away.load(std::memory_order_relaxed) && ctx->away_stream != st &&
-                hipEventQuery(ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents]) == hipSuccess)
-                ctx->away.store(false, std::memory_order_release);
-            if (!ctx->away.load(std::memory_order_relaxed) || ctx->away_stream == st) {
+            if (hipStreamQuery(ctx->stream) == hipSuccess) {
                 mcclx::PlanKey key;
                 float scale_f;
                 int has_scale, fan;
                 if (int rc = check_plan(&l.plan, &key, &scale_f, &has_scale, &fan)) return rc;
                 if (int rc = check_segs(ctx, key, &l.seg, 1, fan)) return rc;
+                // (on the stream of the launch before, the wait costs nothing and changes nothing)
+                if (ctx->away.load(std::memory_order_relaxed))
+                    HIP_TRY(hipStreamWaitEvent(st, ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents], 0));
                 hipEvent_t& ev = ctx->away_ev[(ctx->away_number + 1) % mcclx_ctx::kAwayEvents];
                 if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
                 if (int rc = launch_by_value(ctx, key, scale_f, has_scale, &l.seg, 1, fan, st)) return rc;
@@ -1038,7 +1043,6 @@ static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
                     return MCCLX_OK;
                 }
                 ++ctx->away_number;
-                ctx->away_stream = st;
                 ctx->away.store(true, std::memory_order_release);
                 return MCCLX_OK;
             }
@@ -1245,7 +1249,7 @@ int mcclx_stream_wait_queue(mcclx_ctx* ctx, void* consumer_stream) {
     if (ctx->away.load(std::memory_order_acquire) && !ctx->capturing) {
         DeviceGuard guard(ctx->device);
         std::lock_guard<std::mutex> lk(ctx->away_mu);
-        if (ctx->away.load(std::memory_order_relaxed) && ctx->away_stream != consumer)
+        if (ctx->away.load(std::memory_order_relaxed))
             HIP_TRY(hipStreamWaitEvent(consumer, ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents], 0));
     }
     return stream_wait(ctx, consumer, ctx->stream);

@@ -110,3 +110,41 @@ def test_errors_are_the_same_on_either_route():
     q.copy(a.data_ptr(), a.data_ptr() + 16, 16)
     q.graph_destroy(q.graph_end())
     q.close()
+
+
+def test_a_borrowed_streams_own_later_work_is_behind_the_launch():
+    """A queue on a stream of the caller's: what they enqueue there themselves comes after the call."""
+    mine, other = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(mine):
+        q = K.ReduceQueue(0, on_torch_stream=True)
+        got = torch.zeros(N, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(other):
+        base, dst, src = _produce()
+        K.hip_reduce_op(dst, src, "sum", queue=q)
+    with torch.cuda.stream(mine):
+        got.copy_(dst)
+    torch.cuda.synchronize()
+    assert torch.equal(got, base + 40)
+    q.close()
+
+
+def test_callers_on_alternating_streams_come_one_after_the_other():
+    """Launches of one queue keep their order whichever streams they are called from."""
+    q = K.ReduceQueue(0)
+    streams = [torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.Stream()]
+    dst = torch.zeros(N, device="cuda")
+    one = torch.ones(N, device="cuda")
+    torch.cuda.synchronize()
+    for i in range(24):
+        with torch.cuda.stream(streams[i % 3]):
+            K.hip_reduce_op(dst, one, "sum", queue=q)
+            K.hip_scale_inplace(dst, 2.0, queue=q)
+            if i % 4 == 3:
+                K.hip_scale_inplace(dst, 2.0 ** -4, queue=q)
+    q.drain()
+    want = 0.0
+    for i in range(24):
+        want = (want + 1) * 2 * (2.0 ** -4 if i % 4 == 3 else 1)
+    assert torch.equal(dst, torch.full_like(dst, want))
+    q.close()
