@@ -88,6 +88,12 @@ bool fan_plan_ok(const PlanKey& key);
 // Plans that have a to-all form: per-step rounding, every operand in the form of the result.
 bool all_plan_ok(const PlanKey& key);
 
+// One launch that folds segments 0..nfold-1 of `few` (a fan-out plan of up to four operands over
+// the wire codec, the owner's operand fp32) and encodes the others (fp32 -> bf16), tile by tile in
+// turn.  fold_encode_ok: the plans there are.
+bool fold_encode_ok(const PlanKey& key);
+hipError_t launch_fold_encode(hipStream_t st, const PlanKey& key, const FewArgs& few, uint32_t nfold);
+
 // Packets-per-lane unroll and threads per block the kernel template uses for this plan.
 int plan_unroll(const PlanKey& key);
 int plan_block(const PlanKey& key);

@@ -946,6 +946,48 @@ int mcclx_fold_batched_noalloc(mcclx_ctx* ctx, const mcclx_plan* plan, const mcc
     return MCCLX_OK;
 }
 
+bool mcclx_in_host_memory(mcclx_ctx* ctx, const void* p) {
+    DeviceGuard guard(ctx->device);
+    hipPointerAttribute_t attr;
+    if (hipPointerGetAttributes(&attr, p) == hipSuccess) return attr.type == hipMemoryTypeHost;
+    (void)hipGetLastError();
+    return false;
+}
+
+bool mcclx_fold_encode_ok(mcclx_ctx* ctx, const mcclx_plan* plan, uint32_t nseg) {
+    mcclx::PlanKey key;
+    float scale_f;
+    int has_scale, fan;
+    return nseg <= (uint32_t)mcclx::kFewSegs && nseg <= ctx->few_max &&
+           check_plan(plan, &key, &scale_f, &has_scale, &fan) == MCCLX_OK && fan > 0 && mcclx::fold_encode_ok(key);
+}
+
+int mcclx_fold_encode(mcclx_ctx* ctx, const mcclx_plan* plan, const mcclx_seg* folds, uint32_t nfold,
+                      const mcclx_plan* enc, const mcclx_seg* encodes, uint32_t nenc) {
+    mcclx::PlanKey key, enc_key;
+    float scale_f, enc_scale;
+    int has_scale, fan, enc_has_scale, enc_fan;
+    if (int rc = check_plan(plan, &key, &scale_f, &has_scale, &fan)) return rc;
+    if (int rc = check_plan(enc, &enc_key, &enc_scale, &enc_has_scale, &enc_fan)) return rc;
+    if (nfold + nenc > (uint32_t)mcclx::kFewSegs) return fail(MCCLX_ERR_INVALID, "fold_encode: too many segments");
+    if (int rc = check_segs(ctx, key, folds, nfold, fan)) return rc;
+    if (int rc = check_segs(ctx, enc_key, encodes, nenc, enc_fan)) return rc;
+    DeviceGuard guard(ctx->device);
+    if (!guard.ok) return fail(MCCLX_ERR_HIP, "hipSetDevice(%d) failed", ctx->device);
+    mcclx::FewArgs a;
+    memset(&a, 0, sizeof a);
+    if (nfold) memcpy(&a.seg[0], folds, nfold * sizeof(mcclx_seg));
+    if (nenc) memcpy(&a.seg[nfold], encodes, nenc * sizeof(mcclx_seg));
+    a.scale = scale_f;
+    a.has_scale = has_scale;
+    a.nseg = (int32_t)(nfold + nenc);
+    a.fan = fan;
+    hipError_t e = mcclx::launch_fold_encode(queue_of(ctx), key, a, nfold);
+    if (e != hipSuccess) return launch_error(e, key);
+    ++ctx->launches;
+    return MCCLX_OK;
+}
+
 // Each call comes as a launch on the queue and, with a stream, in its ordered form.
 struct OneLaunch {
     mcclx_plan plan;

@@ -3,8 +3,9 @@
 // (csrc/backend/AllreduceAlgos.cpp) plus reduce_scatter / allgather
 // (csrc/backend/ProcessGroupMCCL.cpp) for N virtual ranks on one GPU.
 //
-// Host C++ on top of the public C ABI only (mcclx_reduce, mcclx_fold_batched,
-// mcclx_copy, ...): nothing here touches HIP directly.
+// Host C++ on top of the public C ABI (mcclx_reduce, mcclx_fold_batched,
+// mcclx_copy, ...) and of the library's own mcclx_fold_encode: nothing here
+// touches HIP directly.
 //
 // STEPWISE mode issues the reference's launches one for one -- every send/recv
 // pair becomes a device copy into the receiver's scratch, followed by the
@@ -219,6 +220,7 @@ struct FoldPass {
 
 struct Phases {
     bool planned = false;
+    bool over_link = false;  // every replay's wire copies lie in pinned host memory, clear of its tensors
     mcclx_plan enc, dec;
     std::vector<mcclx_seg> enc_segs, dec_segs;
     std::vector<FoldPass> folds;  // one pass, or a chain of passes when the world is wider than one fold
@@ -539,7 +541,83 @@ void collect_fused(const mcclx_replay* r, const Layout& L, Phases& ph) {
     }
 }
 
+// Nothing the replay reads or writes lies in two places of it.
+bool all_disjoint(const mcclx_replay* r) {
+    const uintptr_t tb = r->numel * esize(r->dtype), ws = reinterpret_cast<uintptr_t>(r->workspace);
+    for (int i = 0; i < r->world; ++i) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(r->tensors[i]);
+        if (a < ws + r->workspace_bytes && ws < a + tb) return false;
+        for (int j = 0; j < i; ++j) {
+            const uintptr_t b = reinterpret_cast<uintptr_t>(r->tensors[j]);
+            if (a < b + tb && b < a + tb) return false;
+        }
+    }
+    return true;
+}
+
+// The wire copies of a run in pinned host memory: the encodes write over the link what the
+// folds read back over it, and a link that carries 55 GB/s in one direction carries 1.5 times
+// that in both.  So the run is cut into pieces of every chunk, and the launch that folds piece
+// p encodes piece p + 1; the ranges the two touch have nothing in common (all_disjoint), and
+// the launches' order on the queue is what the folds wait for.
+//
+// The number of pieces: the first piece's encode and the last piece's fold have the link for
+// themselves, 2 S / P of S seconds a direction, what is in between takes 1.3 S, and a launch
+// costs its 20 us of ramp, link latency and drain: the sum is least at P^2 = 0.7 S / 20 us,
+// which is (bytes a direction) / 1.5 MB.  One piece is the two launches it always was.
+constexpr uint64_t kPieceBytes2 = 1'500'000;
+constexpr uint64_t kPieceUnit = 64;  // elements: pieces keep their chunk's alignment, on full lines
+
+uint64_t pieces_of(const Phases& ph) {
+    uint64_t bytes = 0;
+    for (const mcclx_seg& s : ph.enc_segs) bytes += 2 * s.count;
+    uint64_t p = 1;
+    while ((p + 1) * (p + 1) * kPieceBytes2 <= bytes) ++p;
+    return p;
+}
+
+int issue_in_pieces(mcclx_ctx* ctx, const Phases& ph, uint64_t pieces) {
+    const FoldPass& f = ph.folds[0];
+    const int own = f.plan.io == MCCLX_IO_OWN_FIRST_F32 ? 0 : f.plan.k - 1;
+    uint64_t longest = 0;
+    for (const mcclx_seg& s : f.segs) longest = s.count > longest ? s.count : longest;
+    const uint64_t len = ((longest + pieces - 1) / pieces + kPieceUnit - 1) / kPieceUnit * kPieceUnit;
+    auto moved = [](const void* p, uint64_t bytes) { return const_cast<char*>(static_cast<const char*>(p)) + bytes; };
+    auto cut = [&](const std::vector<mcclx_seg>& whole, uint64_t lo, bool encode, std::vector<mcclx_seg>& part) {
+        part.clear();
+        for (mcclx_seg s : whole) {
+            if (lo >= s.count) continue;
+            s.count = s.count - lo < len ? s.count - lo : len;
+            if (encode) {
+                s.in[0] = moved(s.in[0], 4 * lo);
+                s.wire_out = moved(s.wire_out, 2 * lo);
+            } else {
+                s.out = moved(s.out, 4 * lo);
+                for (int j = 0; j < f.plan.k + ph.fan; ++j)  // the operands, then the other ranks' tensors
+                    s.in[j] = moved(s.in[j], (j == own || j >= f.plan.k ? 4 : 2) * lo);
+            }
+            part.push_back(s);
+        }
+    };
+    std::vector<mcclx_seg> folds, encodes;
+    cut(ph.enc_segs, 0, true, encodes);
+    TRY(mcclx_fold_encode(ctx, &f.plan, nullptr, 0, &ph.enc, encodes.data(), (uint32_t)encodes.size()));
+    for (uint64_t lo = 0; lo < longest; lo += len) {
+        cut(f.segs, lo, false, folds);
+        cut(ph.enc_segs, lo + len, true, encodes);
+        TRY(mcclx_fold_encode(ctx, &f.plan, folds.data(), (uint32_t)folds.size(), &ph.enc, encodes.data(),
+                              (uint32_t)encodes.size()));
+    }
+    return MCCLX_OK;
+}
+
 int issue_phases(mcclx_ctx* ctx, Phases& ph) {
+    if (ph.over_link && ph.fan && ph.folds.size() == 1 && !ph.enc_segs.empty()) {
+        const uint64_t pieces = pieces_of(ph);
+        if (pieces > 1 &&
+            mcclx_fold_encode_ok(ctx, &ph.folds[0].plan, (uint32_t)(ph.folds[0].segs.size() + ph.enc_segs.size())))
+            return issue_in_pieces(ctx, ph, pieces);
+    }
     if (!ph.enc_segs.empty())
         TRY(mcclx_fold_batched(ctx, &ph.enc, ph.enc_segs.data(), (uint32_t)ph.enc_segs.size()));
     for (FoldPass& f : ph.folds)
@@ -716,6 +794,10 @@ int mcclx_allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t
                 if (!fused || nothing) break;
             }
             if (!touched.add(&rs[i])) break;
+            const bool link = rs[i].mode == MCCLX_REPLAY_FUSED && rs[i].wire_bf16 && rs[i].workspace &&
+                              rs[i].algo != MCCLX_ALGO_TREE && fan_of(&rs[i]) > 0 &&
+                              mcclx_in_host_memory(ctx, rs[i].workspace) && all_disjoint(&rs[i]);
+            ph.over_link = link && (&rs[i] == first || ph.over_link);
             collect_fused(&rs[i], layout_of(&rs[i]), ph);
             ++i;
         }

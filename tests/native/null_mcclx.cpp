@@ -246,6 +246,13 @@ int mcclx_decode_bf16(mcclx_ctx* c, void*, const void*, uint64_t) {
 int mcclx_batch_begin(mcclx_ctx*, const char*) { return MCCLX_OK; }
 int mcclx_batch_end(mcclx_ctx*) { return MCCLX_OK; }
 
+// The scheduler's pieces over the link: there is no link here.
+bool mcclx_in_host_memory(mcclx_ctx*, const void*) { return false; }
+bool mcclx_fold_encode_ok(mcclx_ctx*, const mcclx_plan*, uint32_t) { return false; }
+int mcclx_fold_encode(mcclx_ctx*, const mcclx_plan*, const mcclx_seg*, uint32_t, const mcclx_plan*, const mcclx_seg*, uint32_t) {
+    return mcclx_fail(MCCLX_ERR_STATE, "no fold_encode");
+}
+
 int mcclx_copy(mcclx_ctx* c, void* dst, const void* src, uint64_t nbytes) {
     if (!c) return mcclx_fail(MCCLX_ERR_STATE, "context is null");
     if (nbytes == 0 || dst == src) return MCCLX_OK;
