@@ -263,7 +263,8 @@ MCCLX_API int mcclx_copy(mcclx_ctx* ctx, void* dst, const void* src, uint64_t nb
 /* The tensor forms: one launch at the end of `stream` (a HIP stream of the context's device), as
  * mcclx_queue_wait_stream, the call above of the same name and mcclx_stream_wait_queue in a row
  * give it -- behind everything enqueued so far on `stream` and on the queue, in front of what
- * either is given next.  Where the queue is idle the kernel runs on `stream` itself. */
+ * either is given next.  Where the queue is idle and `stream` is the
+ * default one (NULL) the kernel runs on it. */
 MCCLX_API int mcclx_reduce_ordered(mcclx_ctx* ctx, void* stream, void* dst, const void* src, int dtype, uint64_t count, int op);
 MCCLX_API int mcclx_scale_ordered(mcclx_ctx* ctx, void* stream, void* buf, int dtype, uint64_t count, double scale, int scale_mode);
 MCCLX_API int mcclx_accumulate_scale_ordered(mcclx_ctx* ctx, void* stream, void* dst, const void* src, int dtype, uint64_t count, double scale);

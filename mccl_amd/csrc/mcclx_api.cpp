@@ -101,7 +101,7 @@ struct mcclx_ctx {
     // re-recorded until 15 later waits have been issued
     hipEvent_t xev[16] = {};
     int xnext = 0;
-    // The newest launch that ran on a caller's stream in the queue's place (ordered_launch) and that
+    // The newest launch that ran on the default stream in the queue's place (ordered_launch) and that
     // neither the queue nor the host has waited for yet.  It comes behind every earlier one.
     std::mutex away_mu;  // also held while something is enqueued on the queue (queue_of); taken after mu
     std::atomic<bool> away{false};
@@ -135,6 +135,11 @@ struct DeviceGuard {
         if (prev >= 0) (void)hipSetDevice(prev);
     }
 };
+
+bool records(hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
+}
 
 // The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its
 // place.  As an argument it lives until the call that enqueues the operation has returned, so that
@@ -1054,16 +1059,14 @@ int mcclx_decode_bf16(mcclx_ctx* ctx, void* dst_f32, const void* src_bf16, uint6
 // decoded 110 -> 23 us).  The mark is an event record and not the kernel's own stop event: after
 // thousands of launches with one, the next calls on the stream took three times as long.
 // Everything else takes the two orderings: a queue with work in flight, a queue whose HIP stream
-// the caller holds (what they put there would not see a launch made elsewhere), a recording or a
-// `stream` that records.
+// the caller holds (what they put there would not see a launch made elsewhere), a recording, and
+// every `stream` but the legacy default one.  That one cannot be recorded; of any other the caller
+// may begin a recording later, and while it lasts the runtime refuses to wait for an event that
+// was recorded on the stream before.
 static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    auto records = [](hipStream_t s) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
-    };
-    if (l.seg.count && st != ctx->stream && !ctx->capturing && !ctx->exposed.load() && ctx->few_max >= 1) {
+    if (l.seg.count && st == nullptr && st != ctx->stream && !ctx->capturing && !ctx->exposed.load() && ctx->few_max >= 1) {
         DeviceGuard guard(ctx->device);
         if (!guard.ok) return fail(MCCLX_ERR_HIP, "hipSetDevice(%d) failed", ctx->device);
         if (!records(st) && !records(ctx->stream)) {
@@ -1074,9 +1077,7 @@ static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
                 int has_scale, fan;
                 if (int rc = check_plan(&l.plan, &key, &scale_f, &has_scale, &fan)) return rc;
                 if (int rc = check_segs(ctx, key, &l.seg, 1, fan)) return rc;
-                // (on the stream of the launch before, the wait costs nothing and changes nothing)
-                if (ctx->away.load(std::memory_order_relaxed))
-                    HIP_TRY(hipStreamWaitEvent(st, ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents], 0));
+                // (a launch before this one that is still away lies on the same stream, in front of it)
                 hipEvent_t& ev = ctx->away_ev[(ctx->away_number + 1) % mcclx_ctx::kAwayEvents];
                 if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
                 if (int rc = launch_by_value(ctx, key, scale_f, has_scale, &l.seg, 1, fan, st)) return rc;
@@ -1291,8 +1292,19 @@ int mcclx_stream_wait_queue(mcclx_ctx* ctx, void* consumer_stream) {
     if (ctx->away.load(std::memory_order_acquire) && !ctx->capturing) {
         DeviceGuard guard(ctx->device);
         std::lock_guard<std::mutex> lk(ctx->away_mu);
-        if (ctx->away.load(std::memory_order_relaxed))
-            HIP_TRY(hipStreamWaitEvent(consumer, ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents], 0));
+        if (ctx->away.load(std::memory_order_relaxed)) {
+            const hipEvent_t ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
+            if (records(consumer)) {  // it cannot wait for what its recording does not hold: the host does
+                hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (a blocking call beside a recording)
+                HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+                const hipError_t done = hipEventSynchronize(ev);
+                HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+                HIP_TRY(done);
+                ctx->away.store(false, std::memory_order_release);
+            } else {
+                HIP_TRY(hipStreamWaitEvent(consumer, ev, 0));
+            }
+        }
     }
     return stream_wait(ctx, consumer, ctx->stream);
 }

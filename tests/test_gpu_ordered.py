@@ -148,3 +148,29 @@ def test_callers_on_alternating_streams_come_one_after_the_other():
         want = (want + 1) * 2 * (2.0 ** -4 if i % 4 == 3 else 1)
     assert torch.equal(dst, torch.full_like(dst, want))
     q.close()
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_a_recording_stream_may_wait_for_an_idle_queue(which):
+    """The wait has nothing to record where the queue's work is done -- also when the newest launch
+    ran in the queue's place, on a stream of which, or beside which, the caller now records."""
+    q = K.ReduceQueue(0)
+    side = torch.cuda.Stream()
+    dst, src = torch.zeros(4_097, device="cuda"), torch.ones(4_097, device="cuda")
+    torch.cuda.synchronize()
+    with torch.cuda.stream(torch.cuda.default_stream() if which == 0 else side):
+        K.hip_reduce_op(dst, src, "sum", queue=q)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=side, capture_error_mode="relaxed"):
+            q.torch_stream_wait()
+            dst.add_(src)
+            q.drain()
+        for rep in range(3):
+            g.replay()
+            side.synchronize()
+            assert torch.equal(dst, torch.full_like(dst, 2.0 + rep)), rep
+        K.hip_reduce_op(dst, src, "sum", queue=q)
+        assert torch.equal(dst, torch.full_like(dst, 5.0))
+    q.close()
