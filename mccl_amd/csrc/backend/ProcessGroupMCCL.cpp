@@ -19,6 +19,7 @@
 #include "backend/Phases.hpp"
 #include "backend/Progress.hpp"
 #include "backend/WorkMCCL.hpp"
+#include "spans.h"
 
 namespace mccl {
 
@@ -33,6 +34,61 @@ c10::intrusive_ptr<c10d::Work> make_completed(c10d::OpType op, std::vector<at::T
     w->finish();
     return w;
 }
+
+// The copies of a list collective.  Entries go out together in one batch, whose copies have no
+// order, as long as none touches what another one writes; the entries of a list that do -- a
+// tensor named twice, an input that is an earlier entry's output -- run one behind the other,
+// as separate calls would.
+class ListCopies {
+public:
+    explicit ListCopies(mcclx_ctx* ctx) : ctx_(ctx) {}
+    // One entry, in the order the reference's loops have; copy j reads source j % sources.
+    void entry(const std::vector<mcclx_copy_desc>& copies, size_t sources) {
+        if (!apart(copies)) {
+            issue();
+            for (const mcclx_copy_desc& c : copies) check_rc(mcclx_copy(ctx_, c.dst, c.src, c.nbytes));
+            return;
+        }
+        for (const mcclx_copy_desc& c : copies)
+            if (writes_.hits(lo(c.src), hi(c.src, c)) ||
+                (moves(c) && (writes_.hits(lo(c.dst), hi(c.dst, c)) || reads_.hits(lo(c.dst), hi(c.dst, c))))) {
+                issue();
+                break;
+            }
+        for (size_t s = 0; s < sources; ++s)  // source by source: each is read once for all who get it
+            for (size_t j = s; j < copies.size(); j += sources) {
+                batch_.push_back(copies[j]);
+                reads_.insert(lo(copies[j].src), hi(copies[j].src, copies[j]));
+                if (moves(copies[j])) writes_.insert(lo(copies[j].dst), hi(copies[j].dst, copies[j]));
+            }
+    }
+    void issue() {
+        if (!batch_.empty()) check_rc(mcclx_copy_batched(ctx_, batch_.data(), static_cast<uint32_t>(batch_.size())));
+        batch_.clear();
+        reads_.clear();
+        writes_.clear();
+    }
+
+private:
+    mcclx_ctx* ctx_;
+    std::vector<mcclx_copy_desc> batch_;
+    mcclx::Spans reads_, writes_;
+    static bool moves(const mcclx_copy_desc& c) { return c.nbytes && c.dst != c.src; }  // (in place: nothing is written)
+    static uintptr_t lo(const void* p) { return reinterpret_cast<uintptr_t>(p); }
+    static uintptr_t hi(const void* p, const mcclx_copy_desc& c) { return lo(p) + c.nbytes; }
+    // Does no copy of the entry write what another one reads or writes?
+    static bool apart(const std::vector<mcclx_copy_desc>& copies) {
+        mcclx::Spans writes;
+        for (const mcclx_copy_desc& c : copies) {
+            if (!moves(c)) continue;
+            if (writes.hits(lo(c.dst), hi(c.dst, c))) return false;
+            writes.insert(lo(c.dst), hi(c.dst, c));
+        }
+        for (const mcclx_copy_desc& c : copies)
+            if (writes.hits(lo(c.src), hi(c.src, c))) return false;
+        return true;
+    }
+};
 
 // check_mps_ (ProcessGroupMCCL.cpp:72-79) for ROCm tensors.
 void check_gpu_(const at::Tensor& t, const char* op) {
@@ -1056,14 +1112,18 @@ c10::intrusive_ptr<c10d::Work> ProcessGroupMCCL::broadcast(std::vector<at::Tenso
                            "broadcast: ranks disagree on root or tensor count");
                 check_rc(mcclx_queue_wait_stream(shared->ctx, all[r].stream));
             }
-            std::vector<mcclx_copy_desc> copies;  // source by source: each is read once for all who get it
-            for (size_t i = 0; i < all[0].dst.size(); ++i)
+            ListCopies list(shared->ctx);
+            std::vector<mcclx_copy_desc> copies;
+            for (size_t i = 0; i < all[0].dst.size(); ++i) {
+                copies.clear();
                 for (int r = 0; r < world; ++r) {
                     if (r == root) continue;
                     MCCL_CHECK(all[r].nbytes[i] == all[root].nbytes[i], "broadcast: size mismatch");
                     copies.push_back(mcclx_copy_desc{all[r].dst[i], all[root].dst[i], all[root].nbytes[i]});
                 }
-            check_rc(mcclx_copy_batched(shared->ctx, copies.data(), static_cast<uint32_t>(copies.size())));
+                list.entry(copies, 1);
+            }
+            list.issue();
         });
     });
 }
@@ -1137,17 +1197,20 @@ c10::intrusive_ptr<c10d::Work> ProcessGroupMCCL::allgather(
             shared->begin_main_work();
             for (int r = 0; r < world; ++r) check_rc(mcclx_queue_wait_stream(shared->ctx, all[r].stream));
             const size_t nt = all[0].src.size();
-            std::vector<mcclx_copy_desc> copies;  // source by source: each is read once for all who get it
+            ListCopies list(shared->ctx);
+            std::vector<mcclx_copy_desc> copies;
             for (size_t i = 0; i < nt; ++i) {
                 for (int r = 0; r < world; ++r)
                     MCCL_CHECK(all[r].src.size() == nt && all[r].nbytes[i] == all[0].nbytes[i],
                                "allgather: ranks pass different tensors");
-                for (int p = 0; p < world; ++p)
-                    for (int r = 0; r < world; ++r)
+                copies.clear();
+                for (int r = 0; r < world; ++r)
+                    for (int p = 0; p < world; ++p)
                         copies.push_back(mcclx_copy_desc{all[r].dst[i * static_cast<size_t>(world) + p], all[p].src[i],
                                                          all[0].nbytes[i]});
+                list.entry(copies, static_cast<size_t>(world));
             }
-            check_rc(mcclx_copy_batched(shared->ctx, copies.data(), static_cast<uint32_t>(copies.size())));
+            list.issue();
         });
     });
 }

@@ -20,13 +20,12 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <iterator>
-#include <map>
 #include <string>
 #include <vector>
 
 #include "mcclx.h"
 #include "mcclx_internal.h"
+#include "spans.h"
 
 namespace {
 
@@ -665,10 +664,9 @@ int run_stepwise(mcclx_ctx* ctx, const mcclx_replay* r) {
     return replay_stepwise(ctx, &s, Ls);
 }
 
-// The byte ranges the replays of a run read or write -- their rank tensors and workspaces --
-// as disjoint intervals, neighbours merged: the tensors of a list are usually views that
-// follow one another, and thousands of them make a handful of intervals.  (Held against
-// every earlier range instead, a list of 4096 messages cost 20 ms.)
+// The byte ranges the replays of a run read or write: their rank tensors and workspaces.
+// (Held against every earlier range instead of merged intervals, a list of 4096 messages
+// cost 20 ms.)
 class Touched {
 public:
     // Does the replay touch memory an earlier one has touched?  If not, its ranges are added.
@@ -679,33 +677,16 @@ public:
                 if (f(reinterpret_cast<uintptr_t>(r->tensors[i]), tb)) return true;
             return r->workspace && r->workspace_bytes && f(reinterpret_cast<uintptr_t>(r->workspace), r->workspace_bytes);
         };
-        if (each([&](uintptr_t p, uint64_t n) { return hits(p, p + n); })) return false;
+        if (each([&](uintptr_t p, uint64_t n) { return spans_.hits(p, p + n); })) return false;
         each([&](uintptr_t p, uint64_t n) {
-            insert(p, p + n);
+            spans_.insert(p, p + n);  // (a rank's tensors of one replay may overlap each other)
             return false;
         });
         return true;
     }
 
 private:
-    std::map<uintptr_t, uintptr_t> spans_;  // start -> end
-    bool hits(uintptr_t lo, uintptr_t hi) const {
-        auto it = spans_.upper_bound(lo);
-        if (it != spans_.end() && it->first < hi) return true;
-        return it != spans_.begin() && std::prev(it)->second > lo;
-    }
-    void insert(uintptr_t lo, uintptr_t hi) {  // a rank's tensors of one replay may overlap each other
-        auto it = spans_.upper_bound(lo);
-        if (it != spans_.begin() && std::prev(it)->second >= lo) {
-            --it;
-            lo = it->first;
-        }
-        while (it != spans_.end() && it->first <= hi) {
-            hi = hi > it->second ? hi : it->second;
-            it = spans_.erase(it);
-        }
-        spans_.emplace(lo, hi);
-    }
+    mcclx::Spans spans_;
 };
 
 // Same plan for every phase?

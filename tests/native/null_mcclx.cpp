@@ -260,10 +260,14 @@ int mcclx_copy(mcclx_ctx* c, void* dst, const void* src, uint64_t nbytes) {
     return MCCLX_OK;
 }
 int mcclx_copy_batched(mcclx_ctx* c, const mcclx_copy_desc* d, uint32_t n) {
+    // The copies of one batch have no order: every source is read before anything is written, and
+    // the first copy is written last, so that a batch that needed an order shows in the result.
     std::vector<mcclx_copy_desc> v(d, d + n);
     c->launch([v] {
-        for (auto& x : v)
-            if (x.nbytes && x.dst != x.src) memmove(x.dst, x.src, x.nbytes);
+        std::vector<std::vector<char>> read;
+        for (auto& x : v) read.emplace_back(static_cast<const char*>(x.src), static_cast<const char*>(x.src) + x.nbytes);
+        for (size_t i = v.size(); i-- > 0;)
+            if (v[i].nbytes && v[i].dst != v[i].src) memcpy(v[i].dst, read[i].data(), v[i].nbytes);
     });
     return MCCLX_OK;
 }

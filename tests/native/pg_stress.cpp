@@ -44,6 +44,48 @@ void expect(const at::Tensor& t, float want) {
 }
 
 void settled(const c10::intrusive_ptr<c10d::Work>& w) { w->getFuture()->wait(); }  // untimed, and the Work has settled after it
+// Lists whose entries depend on each other run entry by entry, in the order of the list, as
+// separate calls would: an entry that reads what an earlier one writes sees it, and of several
+// copies into one tensor the last one stays.
+void lists(ProcessGroupMCCL& pg, int rank, int world) {
+    auto full = [](float v) { return at::full({19}, v); };
+    auto outputs = [&] {
+        std::vector<at::Tensor> t;
+        for (int p = 0; p < world; ++p) t.push_back(full(-1.0f));
+        return t;
+    };
+    // entry 1's input is entry 0's first output: everybody ends with rank 0's value
+    std::vector<std::vector<at::Tensor>> chain = {outputs(), outputs()};
+    std::vector<at::Tensor> in = {full(float(rank + 10)), chain[0][0]};
+    pg.allgather(chain, in)->wait();
+    for (int p = 0; p < world; ++p) {
+        expect(chain[0][size_t(p)], float(p + 10));
+        expect(chain[1][size_t(p)], 10.0f);
+    }
+    // one tensor in the place of every output: the last rank's value
+    at::Tensor one = full(-1.0f);
+    std::vector<std::vector<at::Tensor>> same = {std::vector<at::Tensor>(size_t(world), one)};
+    std::vector<at::Tensor> mine = {full(float(rank + 20))};
+    pg.allgather(same, mine)->wait();
+    expect(one, float(world + 19));
+    // in place: an output is the input itself, twice in the list
+    std::vector<std::vector<at::Tensor>> own = {outputs(), outputs()};
+    std::vector<at::Tensor> ins;
+    for (int e = 0; e < 2; ++e) {
+        own[size_t(e)][size_t(rank)].fill_(float(rank + 30 + 100 * e));
+        ins.push_back(own[size_t(e)][size_t(rank)]);
+    }
+    pg.allgather(own, ins)->wait();
+    for (int e = 0; e < 2; ++e)
+        for (int p = 0; p < world; ++p) expect(own[size_t(e)][size_t(p)], float(p + 30 + 100 * e));
+    // a tensor named twice where the root has two
+    at::Tensor a = full(float(rank)), b = full(float(rank + 40));
+    std::vector<at::Tensor> list = {a, rank == 0 ? b : a};
+    c10d::BroadcastOptions root;
+    root.rootRank = 0;
+    pg.broadcast(list, root)->wait();
+    expect(a, rank == 0 ? 0.0f : 40.0f);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -89,6 +131,7 @@ int main(int argc, char** argv) {
                 wb->wait();
                 for (int p = 0; p < world; ++p)
                     if (all.data_ptr<float>()[33 * p] != float(p)) ++g_bad;
+                lists(*pg, r, world);
                 // the last reference to the group goes with a Future callback: on the completer
                 // thread (event-based allreduce) or on the group's own engine thread (barrier)
                 std::vector<at::Tensor> last = {at::full({257}, float(r + 1))};

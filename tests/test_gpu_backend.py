@@ -242,6 +242,48 @@ def test_reduce_scatter_allgather_broadcast_barrier_threads(CX, U, world):
         assert torch.equal(out[r]["bcast"], torch.full((1001,), float(world - 1), device="cuda"))
 
 
+@pytest.mark.parametrize("world", [2, 3, 9])
+def test_allgather_and_broadcast_lists_run_in_the_order_of_the_list(CX, world):
+    """Entries of a list that depend on each other -- an input that is an earlier entry's output,
+    a tensor named twice -- give what separate calls give; independent ones too."""
+    n = 70_001  # odd: packets, heads and tails
+
+    def fn(r, pg):
+        full = lambda v, c=n: torch.full((c,), float(v), device="cuda")  # noqa: E731
+        outs = lambda c=n: [full(-1, c) for _ in range(world)]  # noqa: E731
+        res = {}
+        apart = [outs(), outs(333)]
+        assert pg.allgather(apart, [full(r + 1), full(r + 101, 333)]).wait()
+        res["apart"] = apart
+        chain = [outs(), outs()]
+        assert pg.allgather(chain, [full(r + 10), chain[0][0]]).wait()
+        res["chain"] = chain
+        one = full(-1)
+        assert pg.allgather([[one] * world], [full(r + 20)]).wait()
+        res["one"] = one
+        a, b = full(r), full(r + 40)
+        o = dist.BroadcastOptions()
+        o.rootRank = 0
+        assert pg.broadcast([a, b if r == 0 else a], o).wait()
+        res["twice"] = a
+        c, d = full(r), full(r + 50, 77)
+        o.rootRank = world - 1
+        assert pg.broadcast([c, d], o).wait()
+        res["pair"] = (c, d)
+        return res
+
+    out, errs = run_ranks(CX, world, fn)
+    assert errs == [None] * world, errs
+    is_all = lambda t, v: bool((t == float(v)).all())  # noqa: E731
+    for r in range(world):
+        for p in range(world):
+            assert is_all(out[r]["apart"][0][p], p + 1) and is_all(out[r]["apart"][1][p], p + 101)
+            assert is_all(out[r]["chain"][0][p], p + 10) and is_all(out[r]["chain"][1][p], 10)
+        assert is_all(out[r]["one"], world + 19)
+        assert is_all(out[r]["twice"], 0 if r == 0 else 40)
+        assert is_all(out[r]["pair"][0], world - 1) and is_all(out[r]["pair"][1], world + 49)
+
+
 def test_error_paths(CX, U):
     world = 2
 
