@@ -2,8 +2,8 @@
 // per tensor: addresses, sizes and types are read here, the workspace comes from torch's
 // allocator, and the calls into libmcclx run with the interpreter lock released.
 //
-// What is not a plain list of contiguous ROCm tensors is left to the Python form (the
-// functions return None and have done nothing), which words the error.
+// What is not a plain list of contiguous ROCm tensors, of one type and size within a group, is
+// left to the Python form (the functions return None and have done nothing), which words the error.
 #include "backend/Replays.hpp"
 
 #include <torch/extension.h>
@@ -38,7 +38,7 @@ struct How {
 
 // One group: `tensors` is a list or tuple of the virtual ranks' tensors; their addresses go to
 // `ptrs` (r->tensors is set by the caller, once `ptrs` has stopped growing).
-bool read_group(PyObject* tensors, const How& how, bool same_shapes, mcclx_replay* r, std::vector<void*>& ptrs) {
+bool read_group(PyObject* tensors, const How& how, mcclx_replay* r, std::vector<void*>& ptrs) {
     if (!PyList_Check(tensors) && !PyTuple_Check(tensors)) return false;
     const Py_ssize_t world = PySequence_Fast_GET_SIZE(tensors);
     if (world < 1) return false;
@@ -52,7 +52,7 @@ bool read_group(PyObject* tensors, const How& how, bool same_shapes, mcclx_repla
             r->dtype = dtype_code(t);
             r->numel = static_cast<uint64_t>(t.numel());
             if (r->dtype < 0) return false;
-        } else if (same_shapes && (dtype_code(t) != r->dtype || static_cast<uint64_t>(t.numel()) != r->numel)) {
+        } else if (dtype_code(t) != r->dtype || static_cast<uint64_t>(t.numel()) != r->numel) {
             return false;
         }
         ptrs.push_back(t.data_ptr());
@@ -101,7 +101,7 @@ py::object replay_many(uintptr_t ctx, int device, py::handle groups, int op, int
     std::vector<mcclx_replay> reps(static_cast<size_t>(n));
     std::vector<void*> ptrs;
     for (Py_ssize_t i = 0; i < n; ++i) {
-        if (!read_group(items[i], how, false, &reps[static_cast<size_t>(i)], ptrs)) return py::none();
+        if (!read_group(items[i], how, &reps[static_cast<size_t>(i)], ptrs)) return py::none();
         if (i == 0) ptrs.reserve(static_cast<size_t>(n) * static_cast<size_t>(reps[0].world));
     }
     size_t at = 0;
@@ -116,7 +116,7 @@ py::object replay_many(uintptr_t ctx, int device, py::handle groups, int op, int
 py::object replay_one(uintptr_t ctx, int device, py::handle tensors, int op, int algo, bool wire, int mode, int acc) {
     std::vector<mcclx_replay> reps(1);
     std::vector<void*> ptrs;
-    if (!read_group(tensors.ptr(), How{op, algo, wire ? 1 : 0, mode, acc}, true, &reps[0], ptrs)) return py::none();
+    if (!read_group(tensors.ptr(), How{op, algo, wire ? 1 : 0, mode, acc}, &reps[0], ptrs)) return py::none();
     reps[0].tensors = ptrs.data();
     return py::int_(run(reinterpret_cast<mcclx_ctx*>(ctx), device, reps));
 }
@@ -135,7 +135,7 @@ py::object allreduce(uintptr_t ctx, int device, py::handle tensors, int op, int 
     std::vector<mcclx_replay> reps(1);
     std::vector<void*> ptrs;
     mcclx_replay& r = reps[0];
-    if (!read_group(tensors.ptr(), How{op, 0, wire, mode, MCCLX_ACC_STEP}, true, &r, ptrs)) return py::none();
+    if (!read_group(tensors.ptr(), How{op, 0, wire, mode, MCCLX_ACC_STEP}, &r, ptrs)) return py::none();
     r.tensors = ptrs.data();
     const bool use_wire = wire && r.dtype == MCCLX_F32;
     r.algo = mcclx_select_algo(std::getenv("MCCL_ALLREDUCE_ALGO"), below, r.numel * (use_wire || r.dtype != MCCLX_F32 ? 2u : 4u),

@@ -156,6 +156,8 @@ def allreduce_replay_many(groups: List[List[torch.Tensor]], op, algo: int, wire_
     for i, tensors in enumerate(groups):
         for t in tensors:
             _check_tensor(t, "allreduce")
+            if t.dtype != tensors[0].dtype or t.numel() != tensors[0].numel():
+                raise MCCLError("[MCCL] allreduce: virtual ranks must hold same-shaped tensors")
         r = reps[i]
         r.world = len(tensors)
         r.algo, r.op, r.dtype = algo, op_code(op), dtype_code(tensors[0])

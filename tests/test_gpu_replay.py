@@ -341,6 +341,27 @@ def test_list_replay_with_a_tensor_named_twice_runs_in_order(H, U):
             U.assert_same_bits(db[r], wb[r], dtype, f"tensor reduced once, rank {r}")
 
 
+def test_a_list_group_of_mixed_sizes_or_types_is_refused(H, U):
+    """Every rank's tensor of a group is read and written with the first one's size and type:
+    another size or type is refused before anything is launched, as by the single call."""
+    from mccl_amd import kernels as K
+    ones = lambda n, dt=torch.float32: torch.ones(n, dtype=dt, device="cuda")  # noqa: E731
+    good = [ones(64), ones(64)]
+    before = K._q(None).launch_count()
+    for bad in ([ones(64), ones(63)], [ones(64), ones(65)], [ones(64), ones(64, torch.bfloat16)], [ones(1 << 20), ones(1)]):
+        for mode in (FUSED, DIRECT, STEPWISE):
+            with pytest.raises(Exception, match="same-shaped"):
+                H.allreduce_replay_many([good, bad], "sum", RING, mode=mode)
+            with pytest.raises(Exception, match="same-shaped"):
+                H.allreduce_replay(bad, "sum", RING, mode=mode)
+        with pytest.raises(Exception, match="same-shaped"):
+            H.allreduce(bad, "sum")
+    assert K._q(None).launch_count() == before
+    assert bool((good[0] == 1).all())
+    H.allreduce_replay_many([good, [ones((8, 8)), ones(64)]], "sum", RING)  # shapes may differ, sizes not
+    assert bool((good[1] == 2).all())
+
+
 def test_copy_batched_many_small_and_a_few_large(K, U):
     rng = np.random.default_rng(3)
     q = K._q(None)
