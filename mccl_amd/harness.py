@@ -84,15 +84,6 @@ class Workspace:
         self._tensor = None
 
 
-def _in_place_mode(mode: int) -> int:
-    """FUSED where the caller leaves the workspace to this module: the wire is HBM then, and the
-    virtual ranks' fp32 tensors are read where they lie instead of through bf16 copies -- the same
-    bits, 8 instead of 10.7 bytes per element and rank with three ranks (3 x 25 MiB over the codec 35 ->
-    26 us, 4 x 110 M elements 800 -> 530 us on the device).  `allreduce_replay`, which takes a
-    workspace that may be pinned host memory, runs the mode it is given."""
-    return L.REPLAY_DIRECT if mode == L.REPLAY_FUSED else mode
-
-
 def allreduce_replay(tensors: List[torch.Tensor], op, algo: int, wire_bf16: bool = False,
                      mode: int = L.REPLAY_FUSED, acc: int = L.ACC_STEP, queue=None,
                      workspace: Optional[Workspace] = None, sync: bool = True) -> None:
@@ -140,14 +131,13 @@ def allreduce_replay(tensors: List[torch.Tensor], op, algo: int, wire_bf16: bool
 
 
 def allreduce_replay_many(groups: List[List[torch.Tensor]], op, algo: int, wire_bf16: bool = False,
-                          mode: int = L.REPLAY_FUSED, acc: int = L.ACC_STEP, queue=None) -> None:
+                          mode: int = L.REPLAY_DIRECT, acc: int = L.ACC_STEP, queue=None) -> None:
     """A list of allreduces (groups[i] = the virtual ranks' tensors of message i), as a
     c10d allreduce over a list of tensors: entries that share a plan go out together,
-    one launch per phase for all of them."""
+    one launch per phase for all of them.  DIRECT by default, see `allreduce`."""
     q = _q(queue)
     if _native is not None:
-        rc = _native._allreduce_replay_many(q.handle.value, q.device, groups, op_code(op), algo, bool(wire_bf16),
-                                            _in_place_mode(mode), acc)
+        rc = _native._allreduce_replay_many(q.handle.value, q.device, groups, op_code(op), algo, bool(wire_bf16), mode, acc)
         if rc is not None:
             return L.check(rc)
     reps = (L.Replay * len(groups))()
@@ -161,7 +151,7 @@ def allreduce_replay_many(groups: List[List[torch.Tensor]], op, algo: int, wire_
         r = reps[i]
         r.world = len(tensors)
         r.algo, r.op, r.dtype = algo, op_code(op), dtype_code(tensors[0])
-        r.wire_bf16, r.mode, r.acc, r.reserved = int(wire_bf16), _in_place_mode(mode), acc, 0
+        r.wire_bf16, r.mode, r.acc, r.reserved = int(wire_bf16), mode, acc, 0
         r.numel = tensors[0].numel()
         ptrs = _ptr_array([t.data_ptr() for t in tensors])
         keep.append(ptrs)
@@ -181,11 +171,17 @@ def allreduce_replay_many(groups: List[List[torch.Tensor]], op, algo: int, wire_
         ws.free()
 
 
-def allreduce(tensors: List[torch.Tensor], op="sum", queue=None, mode: int = L.REPLAY_FUSED) -> int:
-    """ProcessGroupMCCL::allreduce for N virtual ranks; returns the algorithm used."""
+def allreduce(tensors: List[torch.Tensor], op="sum", queue=None, mode: int = L.REPLAY_DIRECT) -> int:
+    """ProcessGroupMCCL::allreduce for N virtual ranks; returns the algorithm used.
+
+    DIRECT by default: the workspace is this module's own and lies in HBM, so the ranks' fp32
+    tensors are read where they lie instead of through the bf16 copies of FUSED -- the same bits, 8
+    instead of 10.7 bytes per element and rank with three ranks (3 x 25 MiB over the codec 35 ->
+    26 us, 4 x 110 M elements 800 -> 530 us on the device).  `allreduce_replay`, whose workspace may
+    be pinned host memory, runs FUSED by default."""
     if _native is not None:
         q = _q(queue)
-        done = _native._allreduce(q.handle.value, q.device, tensors, op_code(op), _in_place_mode(mode))
+        done = _native._allreduce(q.handle.value, q.device, tensors, op_code(op), mode)
         if done is not None:
             L.check(done[0])
             return done[1]
@@ -194,7 +190,7 @@ def allreduce(tensors: List[torch.Tensor], op="sum", queue=None, mode: int = L.R
     use_wire = wire and t0.dtype == torch.float32
     wire_nbytes = t0.numel() * (2 if use_wire else t0.element_size())
     algo = select_algo(env_algo, tree_below, wire_nbytes, t0.numel(), len(tensors))
-    allreduce_replay(tensors, op, algo, wire_bf16=wire, mode=_in_place_mode(mode), queue=queue)
+    allreduce_replay(tensors, op, algo, wire_bf16=wire, mode=mode, queue=queue)
     return algo
 
 

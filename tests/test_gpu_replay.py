@@ -341,6 +341,63 @@ def test_list_replay_with_a_tensor_named_twice_runs_in_order(H, U):
             U.assert_same_bits(db[r], wb[r], dtype, f"tensor reduced once, rank {r}")
 
 
+@pytest.mark.parametrize("algo", [RING, TREE, BUTTERFLY])
+@pytest.mark.parametrize("world", [3, 6])
+def test_lists_over_the_wire_codec_run_the_mode_they_are_given(H, K, U, algo, world):
+    """FUSED encodes what travels into bf16 copies (encode, fold and, from five ranks on, the casts
+    on arrival, each one launch for the whole list); DIRECT reads the ranks' fp32 tensors in one.
+    Both give the oracle's bits, for more segments than fit the kernel arguments, and DIRECT is
+    what a caller gets who names no mode."""
+    q = K._q(None)
+    rng = np.random.default_rng(70 + algo + world)
+    sizes = [world, 64, 997, 4099, 16384] + [int(n) for n in rng.integers(world, 3000, 35)]
+    host = [[U.rand_values(rng, n, F32, scale=1e-2, specials=(n > 64)) for _ in range(world)] for n in sizes]
+    env = {RING: "ring", TREE: "tree", BUTTERFLY: "butterfly"}[algo]
+    wants = []
+    for msg in host:
+        want = [x.copy() for x in msg]
+        assert orc.pg_allreduce(want, F32, AVG, wire_bf16=True, env_algo=env)[0] == 0
+        wants.append(want)
+    fused, direct = (2, 1) if world <= 4 else (3, 1)
+    for kw, launches in (({"mode": FUSED}, fused), ({"mode": DIRECT}, direct), ({}, direct)):
+        groups = [[U.to_dev(x, F32) for x in msg] for msg in host]
+        before = q.launch_count()
+        H.allreduce_replay_many(groups, "avg", algo, wire_bf16=True, **kw)
+        assert q.launch_count() - before == launches, kw
+        for n, want, g in zip(sizes, wants, groups):
+            for r in range(world):
+                U.assert_same_bits(g[r], want[r], F32, f"algo {algo} n {n} rank {r} {kw}")
+
+
+@pytest.mark.parametrize("mode", [FUSED, DIRECT])
+def test_a_tensor_named_twice_over_the_wire_codec(H, U, mode):
+    world, n = 3, 5003
+    rng = np.random.default_rng(45)
+    a = [U.rand_values(rng, n, F32, scale=1e-2) for _ in range(world)]
+    da = [U.to_dev(x, F32) for x in a]
+    H.allreduce_replay_many([da, da, da], "sum", BUTTERFLY, wire_bf16=True, mode=mode)
+    for _ in range(3):
+        assert orc.pg_allreduce(a, F32, SUM, wire_bf16=True, env_algo="butterfly")[0] == 0
+    for r in range(world):
+        U.assert_same_bits(da[r], a[r], F32, f"rank {r}")
+
+
+@pytest.mark.parametrize("mode", [FUSED, DIRECT])
+def test_allreduce_runs_the_mode_it_is_given(H, K, U, monkeypatch, mode):
+    monkeypatch.setenv("MCCL_WIRE_DTYPE", "bf16")
+    monkeypatch.setenv("MCCL_ALLREDUCE_ALGO", "ring")
+    rng = np.random.default_rng(46)
+    a = [U.rand_values(rng, 4099, F32) for _ in range(3)]
+    da = [U.to_dev(x, F32) for x in a]
+    q = K._q(None)
+    before = q.launch_count()
+    assert H.allreduce(da, "avg", mode=mode) == RING
+    assert q.launch_count() - before == (2 if mode == FUSED else 1)
+    assert orc.pg_allreduce(a, F32, AVG, wire_bf16=True, env_algo="ring")[0] == 0
+    for r in range(3):
+        U.assert_same_bits(da[r], a[r], F32, f"rank {r}")
+
+
 def test_a_list_group_of_mixed_sizes_or_types_is_refused(H, U):
     """Every rank's tensor of a group is read and written with the first one's size and type:
     another size or type is refused before anything is launched, as by the single call."""
