@@ -23,6 +23,13 @@ try:  # lists of tensors are read natively where the extension is built
 except ImportError:
     _native = None
 
+
+def _reader():
+    """The native reader, or None where it is not built or the queues are another library's
+    (MCCLX_LIBRARY): it calls the libmcclx.so it is linked against."""
+    return _native if _native is not None and L.in_tree() else None
+
+
 ALGO_NAMES = {"ring": L.ALGO_RING, "tree": L.ALGO_TREE, "butterfly": L.ALGO_BUTTERFLY}
 
 
@@ -89,8 +96,9 @@ def allreduce_replay(tensors: List[torch.Tensor], op, algo: int, wire_bf16: bool
                      workspace: Optional[Workspace] = None, sync: bool = True) -> None:
     """In-place allreduce over the virtual ranks' tensors with a fixed algorithm."""
     q = _q(queue)
-    if workspace is None and _native is not None:
-        rc = _native._allreduce_replay(q.handle.value, q.device, tensors, op_code(op), algo, bool(wire_bf16), mode, acc)
+    native = _reader()
+    if workspace is None and native is not None:
+        rc = native._allreduce_replay(q.handle.value, q.device, tensors, op_code(op), algo, bool(wire_bf16), mode, acc)
         if rc is not None:
             return L.check(rc)
     if not tensors:
@@ -136,8 +144,9 @@ def allreduce_replay_many(groups: List[List[torch.Tensor]], op, algo: int, wire_
     c10d allreduce over a list of tensors: entries that share a plan go out together,
     one launch per phase for all of them.  DIRECT by default, see `allreduce`."""
     q = _q(queue)
-    if _native is not None:
-        rc = _native._allreduce_replay_many(q.handle.value, q.device, groups, op_code(op), algo, bool(wire_bf16), mode, acc)
+    native = _reader()
+    if native is not None:
+        rc = native._allreduce_replay_many(q.handle.value, q.device, groups, op_code(op), algo, bool(wire_bf16), mode, acc)
         if rc is not None:
             return L.check(rc)
     reps = (L.Replay * len(groups))()
@@ -179,9 +188,10 @@ def allreduce(tensors: List[torch.Tensor], op="sum", queue=None, mode: int = L.R
     instead of 10.7 bytes per element and rank with three ranks (3 x 25 MiB over the codec 35 ->
     26 us, 4 x 110 M elements 800 -> 530 us on the device).  `allreduce_replay`, whose workspace may
     be pinned host memory, runs FUSED by default."""
-    if _native is not None:
+    native = _reader()
+    if native is not None:
         q = _q(queue)
-        done = _native._allreduce(q.handle.value, q.device, tensors, op_code(op), mode)
+        done = native._allreduce(q.handle.value, q.device, tensors, op_code(op), mode)
         if done is not None:
             L.check(done[0])
             return done[1]

@@ -165,3 +165,21 @@ def test_header_is_strict_c99_and_a_plain_c_client_links_and_runs():
         raise AssertionError(e.stderr)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stderr
+
+
+@pytest.mark.parametrize("other", [False, True])
+def test_queues_of_another_library_are_not_handed_to_the_extension(tmp_path, other):
+    """mccl_amd/_C is linked against the in-tree libmcclx.so.  With MCCLX_LIBRARY the contexts are
+    another build's, so lists of tensors are read by the ctypes form."""
+    import shutil
+    import subprocess
+    from mccl_amd import _lib
+    env = dict(os.environ)
+    env.pop("MCCLX_LIBRARY", None)
+    if other:
+        env["MCCLX_LIBRARY"] = str(tmp_path / "libmcclx.so")
+        shutil.copy(_lib.LIB_PATH, env["MCCLX_LIBRARY"])
+    code = "from mccl_amd import harness as H; assert H._native is not None; print('native', H._reader() is not None)"
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, env=env, cwd=ROOT)
+    assert r.returncode == 0, r.stderr
+    assert r.stdout.strip() == f"native {not other}"
