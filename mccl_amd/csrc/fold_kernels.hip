@@ -754,12 +754,6 @@ __global__ void __launch_bounds__(kHoldBlock) fold_few_hold_kernel(FewArgs a, ui
                 store_pack<C, OUT>(t, has_out, has_wire, p, y, fan);
             } else {  // all streams 16-bit: the packed result goes out as it is
                 const u32x4 bits = raw[0][u];
-                if constexpr (OUT == kOutAll) {
-#pragma unroll
-                    for (int k = 0; k < C::K; ++k)
-                        MCCLX_STG(gptr<u32x4_a2>(static_cast<uint16_t*>(const_cast<void*>(t.in[k])) + p * C::E), bits);
-                    continue;
-                }
                 if (has_out) MCCLX_STG(gptr<u32x4_a2>(static_cast<uint16_t*>(t.out) + p * C::E), bits);
                 if (has_wire) MCCLX_STG(gptr<u32x4_a2>(static_cast<uint16_t*>(t.wire_out) + p * C::E), bits);
                 if constexpr (OUT == kOutFan) {
@@ -843,7 +837,7 @@ static bool try_hold(hipStream_t st, FewArgs& a, uint64_t maxc, const LaunchPara
         for (int k = 0; k < C::K; ++k) read_bytes += a.seg[i].count * (C::in_is_f32(k) ? 4 : 2);
     // measured break-even: 10 MiB read for a fold with one output, half as much again for one that
     // writes as much as it reads (fan-out)
-    if (read_bytes < (OUT != kOutOne ? lp.hold_min_read_bytes * 3 / 2 : lp.hold_min_read_bytes)) return false;
+    if (read_bytes < (OUT == kOutFan ? lp.hold_min_read_bytes * 3 / 2 : lp.hold_min_read_bytes)) return false;
     // The encode: measured on 1-8 tensors of 1-40 MiB, the form wins 4-10 % from three tensors and
     // 18 MiB read on (three of 25 MiB: 20.6 -> 19.0 us); on one or two tensors it ties or loses.
     if constexpr (kHoldEncode<C>)
@@ -865,7 +859,7 @@ static bool try_hold(hipStream_t st, FewArgs& a, uint64_t maxc, const LaunchPara
     if constexpr (kHoldEncode<C>)
         took = hold_launch<C, 10, 512, kOutOne>(st, a, packets, gate, lp);
     else
-        took = hold_launch<C, 4, 512, OUT>(st, a, packets, gate, lp) || hold_launch<C, 5, 512, OUT>(st, a, packets, OUT != kOutOne ? gate5 : gate, lp);
+        took = hold_launch<C, 4, 512, OUT>(st, a, packets, gate, lp) || hold_launch<C, 5, 512, OUT>(st, a, packets, OUT == kOutFan ? gate5 : gate, lp);
     if (took && lp.held) *lp.held = true;
     return took;
 }
@@ -957,7 +951,7 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
 #if MCCLX_TUNE_TIMELINE
     a.timeline = nullptr;
 #endif
-    if constexpr (kHoldPlan<C>)
+    if constexpr (kHoldPlan<C> && OUT != kOutAll)  // (the schedules give sums of two to four ranks to fan-out)
         if (try_hold<C, OUT>(st, a, maxc, lp)) return hipGetLastError();
     const uint64_t lane_elems = (uint64_t)C::FEW_U * C::E;
     const int outputs = OUT == kOutAll ? C::K : 1 + a.fan;

@@ -2,6 +2,7 @@
 of five to eight ranks, or of any op, in one launch) against the oracle's replay of the
 reference, bit for bit: every dtype, op, algorithm and number of ranks, sizes at the edges of
 packets and tiles, tensors off the 16-byte grid, and the sizes from which large replays take it."""
+import ctypes as C
 import re
 
 import numpy as np
@@ -68,3 +69,92 @@ def test_to_all_validation():
             (K.make_plan(L.F32, 2, flags=L.PLAN_TO_ALL), seg(pa, [pa, pa + 16]), "overlap")):
         with pytest.raises(Exception, match=re.escape(frag)):
             q.fold(plan, segs)
+
+
+KINDS = ["f32", "bf16", "f16", "all_f32"]
+
+
+def to_all_against_one_output(L, K, U, q, kind, k, op, counts, seed, noalloc=False, topo=0, scale=None):
+    """The to-all launch over `counts` against the same operands folded into buffers of their own
+    (the one-output form, which the oracle's tests hold): every operand becomes the result, and
+    what lies between the segments stays."""
+    W = {"f32": F32, "bf16": BF16, "f16": F16, "all_f32": BF16}[kind]
+    io = L.IO_ALL_F32 if kind == "all_f32" else L.IO_PURE
+    stored = F32 if kind == "all_f32" else W
+    es = 4 if stored == F32 else 2
+    gap = 5  # elements behind every segment: odd starts, and a guard
+    starts = np.concatenate([[0], np.cumsum([c + gap for c in counts])])
+    rng = np.random.default_rng(seed)
+    tdt = U.TORCH_DT[stored]
+    full = [torch.from_numpy(rng.standard_normal(int(starts[-1])).astype(np.float32)).cuda().to(tdt) for _ in range(k)]
+    out = torch.zeros_like(full[0])
+    kw = dict(io=io, op=op, topo=topo)
+    if scale is not None:
+        kw.update(scale_mode=L.SCALE_VIEW, scale=scale)
+    at = lambda t, i: t.data_ptr() + es * int(starts[i])  # noqa: E731
+    fn = L.lib().mcclx_fold_batched_noalloc if noalloc else L.lib().mcclx_fold_batched
+
+    def launch(flags, out_of):
+        arr = (L.Seg * len(counts))(*[K.make_seg(out_of(i), 0, [at(t, i) for t in full], c) for i, c in enumerate(counts)])
+        plan = K.make_plan(W, k, flags=flags, **kw)
+        L.check(fn(q.handle, C.byref(plan), arr, len(counts)))
+
+    torch.cuda.synchronize()
+    want = [f.clone() for f in full]
+    torch.cuda.synchronize()
+    launch(0, lambda i: at(out, i))
+    held = q.hold_launch_count()
+    launch(L.PLAN_TO_ALL, lambda i: at(full[0], i))
+    assert q.hold_launch_count() == held, "to-all has no hold form"
+    q.drain()
+    bits = torch.int32 if es == 4 else torch.int16
+    inside = torch.zeros(int(starts[-1]), dtype=torch.bool, device="cuda")
+    for i, c in enumerate(counts):
+        inside[int(starts[i]):int(starts[i]) + c] = True
+    for j in range(k):
+        expect = torch.where(inside, out.view(bits), want[j].view(bits))
+        assert torch.equal(full[j].view(bits), expect), f"{kind} k={k} op={op} operand {j} segs {len(counts)} noalloc {noalloc}"
+
+
+@pytest.fixture(scope="module")
+def env():
+    import gpu_util as U
+    from mccl_amd import _lib as L, kernels as K
+    return L, K, U, K.hip_kernels_init(0)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("k", [2, 3, 4, 8])
+def test_to_all_launches_by_value(env, kind, k):
+    """One to 32 segments in the kernel arguments, through both entry points: a size of a few
+    elements, tiles and their edges, and sums from where other plans take the hold form to where
+    fewer waves stay resident (160 MB moved)."""
+    L, K, U, q = env
+    es = 2 if kind in ("bf16", "f16") else 4
+    for noalloc in (False, True):
+        for counts in ([1], [7, 63, 64, 65], [4097, 5000, 4099], [1023] * 32):
+            to_all_against_one_output(L, K, U, q, kind, k, SUM, counts, 11 + k, noalloc, scale=1 / 3)
+    for bytes_read in (20 << 20, 34 << 20, 110_000_000):
+        n = bytes_read // (es * k) // 3
+        to_all_against_one_output(L, K, U, q, kind, k, SUM, [n, n, n + 1], 12 + k)
+    if kind != "all_f32":
+        to_all_against_one_output(L, K, U, q, kind, k, MAX, [4097, 5000, 4099], 13 + k)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("k", [2, 5, 8])
+def test_to_all_launches_over_a_table(env, kind, k):
+    """More segments than fit the kernel arguments, ragged ones and equal ones, from a table the
+    library uploads and from the one it writes with kernels."""
+    L, K, U, q = env
+    rng = np.random.default_rng(k)
+    ragged = [int(c) for c in rng.integers(1, 9000, size=90)] + [40_001, 1]
+    for noalloc in (False, True):
+        for counts in (ragged, [2048] * 100, [513] * 33):
+            to_all_against_one_output(L, K, U, q, kind, k, SUM, counts, 21 + k, noalloc, scale=0.25)
+        if kind != "all_f32":
+            to_all_against_one_output(L, K, U, q, kind, k, PRODUCT, ragged, 22 + k, noalloc)
+    n = 260_000_000 // (2 * k * (2 if kind in ("bf16", "f16") else 4)) // 200  # enough bytes for the residency limit
+    to_all_against_one_output(L, K, U, q, kind, k, SUM, [n] * 200, 23 + k)
+    if k >= 4:
+        to_all_against_one_output(L, K, U, q, kind, k, SUM, ragged, 24 + k, topo=L.TOPO_BINOMIAL)
