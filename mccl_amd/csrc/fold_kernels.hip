@@ -221,6 +221,12 @@ struct Cfg {
     static constexpr bool kTwoShapes = BLOCK == kBlock || kDecode;
     // (an encode's lanes move 24 bytes: four wavefronts still win at 16,384, 4.2 M elements in 5.5 us against 5.9)
     static constexpr uint64_t kOneWaveFrom = (K == 1 && IO == MCCLX_IO_OWN_FIRST_F32) ? 20480 : kOneWaveBlocksFrom;
+    // the first 16-bit operand next to an fp32 output, or -1
+    static constexpr int kWireIn = [] {
+        for (int k = 0; k < K; ++k)
+            if (W != MCCLX_F32 && IO != MCCLX_IO_PURE && !in_is_f32(k)) return k;
+        return -1;
+    }();
     // bytes a lane reads per packet
     static constexpr int kReadBytes = [] {
         int b = 0;
@@ -503,14 +509,22 @@ __device__ __forceinline__ void fold_packs(const SegArgs& s, bool has_out, bool 
 }
 
 // Elements in front of the packet grid: up to the 128-byte boundary of the
-// buffer the widest stores go to.
+// buffer the widest stores go to.  A line holds 32 fp32 or 64 16-bit elements: of the
+// two line starts of an fp32 output the grid takes the one at which the first 16-bit
+// operand starts a line too, if either does (a chunk of a tensor and the same chunk of
+// its wire copy, at any element).  A wavefront reads 512 bytes of such an operand: off
+// the line it fetches five lines for four, the fifth a second time for its neighbour on
+// another XCD (four segments of 27.5 M elements, every other one off the line, own fp32
+// + three bf16 peers: 257 -> 241 us, the peers in pinned host memory 13.1 -> 11.7 ms).
 template <class C, int OUT = kOutOne>
-__device__ __forceinline__ uint32_t head_elems(const SegArgs& s) {
+__host__ __device__ __forceinline__ uint32_t head_elems(const SegArgs& s) {
     const bool wide_out = (C::W == MCCLX_F32 || C::kOutF32) && (OUT == kOutAll || s.out);
     const void* first = OUT == kOutAll ? s.in[0] : s.out ? s.out : s.wire_out;
     const uint32_t a = (uint32_t)reinterpret_cast<uintptr_t>(first);
     const uint32_t mis = a & 127u;
-    const uint32_t h = mis ? (128u - mis) >> (wide_out ? 2 : 1) : 0u;
+    uint32_t h = mis ? (128u - mis) >> (wide_out ? 2 : 1) : 0u;
+    if constexpr (C::kWireIn >= 0)
+        if (wide_out && (((uint32_t)reinterpret_cast<uintptr_t>(s.in[C::kWireIn]) + 2 * h) & 127u) == 64u) h += 32;
     return s.count < h ? (uint32_t)s.count : h;
 }
 
@@ -600,7 +614,7 @@ __device__ __forceinline__ void fetch_together(SegArgs& s, float& scale, int32_t
 // kernel with more starts 768 blocks at launch instead of 1024 and streams
 // 2-4 % slower.  Six registers are set aside on top of what the code uses (VCC,
 // flat scratch, XNACK mask), so the code itself has 74.
-template <class C, int OUT, int B>
+template <class C, int OUT, int B, int U>
 __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
 #if MCCLX_TUNE_TIMELINE
     const uint64_t t_start = wall_clock64();
@@ -615,14 +629,14 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
 #if MCCLX_TUNE_TIMELINE
     const uint64_t t_args = wall_clock64();
 #endif
-    const uint64_t span = (uint64_t)C::FEW_U * B;
+    const uint64_t span = (uint64_t)U * B;
     // one tile per block, no loop: the launch sizes the grid to the longest segment.  Blocks are
     // dispatched in address order (giving each XCD one contiguous part of a segment instead was
     // level on a 25 MiB bucket and 3.5-9 % slower on large operands).
     (void)grid;
     int op = C::OP;
     if constexpr (C::OP == kAnyOp) op = a.op;
-    fold_tile<C, OUT, B, C::FEW_U>(s, scale, has_scale != 0, (uint64_t)blockIdx.x * span, blockIdx.x == 0, fan, op);
+    fold_tile<C, OUT, B, U>(s, scale, has_scale != 0, (uint64_t)blockIdx.x * span, blockIdx.x == 0, fan, op);
 #if MCCLX_TUNE_TIMELINE
     if (a.timeline && threadIdx.x == 0) {
         TimelineRecord r;
@@ -642,17 +656,17 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
 #define MCCLX_SGPR_CAP __attribute__((amdgpu_num_sgpr(80)))
 template <class C> constexpr bool kLightPlan = C::K <= 4;
 
-template <class C, int B>
-__global__ void __launch_bounds__(B) MCCLX_SGPR_CAP fold_few_kernel(FewArgs a) { fold_few_body<C, kOutOne, B>(a); }
-template <class C, int B>
-__global__ void __launch_bounds__(B) fold_few_wide_kernel(FewArgs a) { fold_few_body<C, kOutOne, B>(a); }
+template <class C, int B, int U>
+__global__ void __launch_bounds__(B) MCCLX_SGPR_CAP fold_few_kernel(FewArgs a) { fold_few_body<C, kOutOne, B, U>(a); }
+template <class C, int B, int U>
+__global__ void __launch_bounds__(B) fold_few_wide_kernel(FewArgs a) { fold_few_body<C, kOutOne, B, U>(a); }
 // Fan-out form: the result also goes to in[K .. K+fan-1] (the other ranks' tensors: the
 // allgather leg of an allreduce done by the reduce itself, stores instead of a second pass).
-template <class C, int B>
-__global__ void __launch_bounds__(B) fold_few_fan_kernel(FewArgs a) { fold_few_body<C, kOutFan, B>(a); }
+template <class C, int B, int U>
+__global__ void __launch_bounds__(B) fold_few_fan_kernel(FewArgs a) { fold_few_body<C, kOutFan, B, U>(a); }
 // To-all form: the result goes back into every operand's buffer.
-template <class C, int B>
-__global__ void __launch_bounds__(B) fold_few_all_kernel(FewArgs a) { fold_few_body<C, kOutAll, B>(a); }
+template <class C, int B, int U>
+__global__ void __launch_bounds__(B) fold_few_all_kernel(FewArgs a) { fold_few_body<C, kOutAll, B, U>(a); }
 
 #if MCCLX_TUNE_TIMELINE
 // Where the next by-value launches put their records (measurement build): a caller-provided
@@ -938,6 +952,25 @@ constexpr bool kFanPlan = C::OP == MCCLX_SUM && C::ACC == MCCLX_ACC_STEP && C::K
 
 // ----------------------------------------------------------------- dispatch
 
+// Does a stream of the launch start off the lines that its tiles start on?  Every wavefront's
+// first and last line is then its neighbour's too, and in one-wavefront blocks the neighbour is
+// on another XCD.  In blocks of eight it is on the same CU seven times in eight.  Large launches
+// with a peer one element off, one-wavefront blocks and blocks of eight: own fp32 + two bf16
+// peers of 60 M elements 121 and 113 us, + three 144 and 131, an encode of them 64.8 and 62.0,
+// one peer in pinned host memory 2650 and 2216 us.  (Further fp32 destinations may lie as they
+// will: 134 us against 147.)
+template <class C, int OUT>
+static bool off_lines(const FewArgs& a) {
+    for (int i = 0; i < a.nseg; ++i) {
+        const SegArgs& s = a.seg[i];
+        const uintptr_t h = head_elems<C, OUT>(s);
+        for (int k = 0; k < C::K; ++k)
+            if ((reinterpret_cast<uintptr_t>(s.in[k]) + h * (C::in_is_f32(k) ? 4 : 2)) & 127u) return true;
+        if (s.out && s.wire_out && ((reinterpret_cast<uintptr_t>(s.wire_out) + 2 * h) & 127u)) return true;
+    }
+    return false;
+}
+
 // A by-value launch: one block per tile of the longest segment, the hold form where it applies.
 template <class C, int OUT>
 static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchParams& lp) {
@@ -958,33 +991,35 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
     const int lane_bytes = C::FEW_U * (C::kReadBytes + outputs * ((C::W == MCCLX_F32 || C::kOutF32) ? 16 : 2 * C::E));
     const uint32_t lds = resident_lds(total / lane_elems * (uint64_t)lane_bytes, lane_bytes, outputs,
                                       OUT == kOutAll ? kLaneBytesInPlace : kLaneBytes);
-    const uint64_t waves = (maxc + 64 * lane_elems - 1) / (64 * lane_elems);
-    const bool four = C::kTwoShapes && waves * (uint64_t)a.nseg < C::kOneWaveFrom;
-    const uint64_t gx = four ? (waves + 3) / 4 : waves;
-    if (gx >> 31) return hipErrorInvalidValue;
-    const dim3 grid((uint32_t)gx, (uint32_t)a.nseg);
+    auto go = [&](auto block, auto packets, uint32_t reserve) -> hipError_t {
+        constexpr int B = decltype(block)::value, U = decltype(packets)::value;
+        constexpr uint64_t span = (uint64_t)B * U * C::E;
+        const uint64_t gx = (maxc + span - 1) / span;
+        if (gx >> 31) return hipErrorInvalidValue;
+        const dim3 grid((uint32_t)gx, (uint32_t)a.nseg);
 #if MCCLX_TUNE_TIMELINE
-    if (OUT == kOutOne) a.timeline = timeline_next(gx * (uint64_t)a.nseg);
+        if (OUT == kOutOne) a.timeline = timeline_next(gx * (uint64_t)a.nseg);
 #endif
-    auto go = [&](auto block) {
-        constexpr int B = decltype(block)::value;
         if constexpr (OUT == kOutAll)
-            fold_few_all_kernel<C, B><<<grid, dim3(B), lds, st>>>(a);
+            fold_few_all_kernel<C, B, U><<<grid, dim3(B), reserve, st>>>(a);
         else if constexpr (OUT == kOutFan)
-            fold_few_fan_kernel<C, B><<<grid, dim3(B), lds, st>>>(a);
+            fold_few_fan_kernel<C, B, U><<<grid, dim3(B), reserve, st>>>(a);
         else if constexpr (kLightPlan<C>)
-            fold_few_kernel<C, B><<<grid, dim3(B), lds, st>>>(a);
+            fold_few_kernel<C, B, U><<<grid, dim3(B), reserve, st>>>(a);
         else
-            fold_few_wide_kernel<C, B><<<grid, dim3(B), lds, st>>>(a);
+            fold_few_wide_kernel<C, B, U><<<grid, dim3(B), reserve, st>>>(a);
+        return hipGetLastError();
     };
+    using Few = std::integral_constant<int, C::FEW_U>;
     if constexpr (C::kTwoShapes) {
-        if (four) {
-            go(std::integral_constant<int, kFourWaves>{});
-            return hipGetLastError();
-        }
+        const uint64_t waves = (maxc + 64 * lane_elems - 1) / (64 * lane_elems);
+        if (waves * (uint64_t)a.nseg < C::kOneWaveFrom) return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
+        // (a grid may have 2^32 threads: an encode of more than 2^34 elements needs its two packets per lane)
+        if constexpr (C::BLOCK == kBlock)
+            if (waves * 64 >> 32 || off_lines<C, OUT>(a))
+                return go(std::integral_constant<int, kBlock>{}, std::integral_constant<int, C::U>{}, 0);
     }
-    go(std::integral_constant<int, kOneWave>{});
-    return hipGetLastError();
+    return go(std::integral_constant<int, kOneWave>{}, Few{}, lds);
 }
 
 // Folds and encodes in one launch, their tiles taken in turn, for wire copies in pinned host

@@ -76,3 +76,72 @@ def test_wire_folds_with_fewer_waves_resident(K, world, fan):
     want = (want * 0.25).float()
     for o in outs:
         assert same(o[:n], want) and bool((o[n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("n", [1, 40, 300, 70_003, 3_200_017])
+@pytest.mark.parametrize("own_off,wire_off", [(0, 32), (32, 0), (1, 1), (33, 1), (0, 7), (31, 63), (5, 4)])
+def test_wire_operands_on_and_off_the_lines_of_the_output(K, n, own_off, wire_off):
+    """The packet grid starts where the fp32 output and the first 16-bit operand both start a line
+    of memory, if they ever do (elements off it are done one by one), and a large launch takes
+    larger blocks if they do not."""
+    from mccl_amd import _lib as L
+    q = K._q(None)
+    for k, last in ((2, False), (3, True), (4, False)):
+        own, = operands(1, n, torch.float32, own_off)
+        peers = operands(k - 1, n, torch.bfloat16, wire_off)
+        outs = [torch.full((n + own_off + wire_off + 8,), 7.0, device="cuda") for _ in range(2)]
+        wire = torch.full((n + wire_off + 8,), 7.0, dtype=torch.bfloat16, device="cuda")
+        ops = peers + [own] if last else [own] + peers
+        want = ops[0].to(torch.bfloat16)
+        for t in ops[1:]:
+            want = want + t.to(torch.bfloat16)
+        want = want * 0.25
+        kw = dict(io=L.IO_OWN_LAST_F32 if last else L.IO_OWN_FIRST_F32, scale_mode=L.SCALE_VIEW, scale=0.25)
+        ins = [t.data_ptr() for t in ops]
+        at = [o.data_ptr() + 4 * own_off for o in outs]
+        torch.cuda.synchronize()
+        q.fold(K.make_plan(L.BF16, k, **kw), [K.make_seg(at[0], wire.data_ptr() + 2 * wire_off, ins, n)])
+        q.drain()
+        assert same(outs[0][own_off:own_off + n], want.float()) and same(wire[wire_off:wire_off + n], want)
+        for o in outs:
+            o.fill_(7.0)
+        torch.cuda.synchronize()
+        q.fold(K.make_plan(L.BF16, k, fanout=1, **kw), [K.make_seg(at[0], 0, ins + [outs[1].data_ptr() + 4 * wire_off], n)])
+        q.drain()
+        for o, off in ((outs[0], own_off), (outs[1], wire_off)):
+            assert same(o[off:off + n], want.float()) and bool((o[:off] == 7.0).all()) and bool((o[off + n:] == 7.0).all())
+        assert bool((wire[:wire_off] == 7.0).all()) and bool((wire[wire_off + n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("n", [70_003, 5_300_021])
+@pytest.mark.parametrize("f_off,h_off", [(0, 1), (1, 0), (32, 33), (3, 64)])
+def test_codec_passes_on_and_off_the_lines(K, n, f_off, h_off):
+    x, = operands(1, n, torch.float32, f_off)
+    full = torch.full((n + h_off + 8,), 7.0, dtype=torch.bfloat16, device="cuda")
+    K.encode_bf16(x, out=full[h_off:h_off + n])
+    want = x.to(torch.bfloat16)
+    assert same(full[h_off:h_off + n], want) and bool((full[:h_off] == 7.0).all()) and bool((full[h_off + n:] == 7.0).all())
+    back = torch.full((n + f_off + 8,), 7.0, device="cuda")
+    K.decode_bf16(full[h_off:h_off + n], out=back[f_off:f_off + n])
+    assert same(back[f_off:f_off + n], want.float()) and bool((back[:f_off] == 7.0).all()) and bool((back[f_off + n:] == 7.0).all())
+
+
+def test_an_encode_of_more_elements_than_a_grid_has_threads_for(K):
+    """A grid has at most 2^32 threads: one packet of four elements per lane ends at 2^34 elements."""
+    n = 2**34 + 4099
+    if torch.cuda.mem_get_info()[0] < 120 * 2**30:
+        pytest.skip("needs 100 GB of device memory")
+    x = torch.full((n,), 1.25, device="cuda")
+    marks = [0, 1, 2**33 + 5, 2**34 - 1, 2**34, 2**34 + 4097, n - 1]
+    for i, at in enumerate(marks):
+        x[at] = float(i + 3)
+    out = torch.zeros(n, dtype=torch.bfloat16, device="cuda")
+    K.encode_bf16(x, out=out)
+    del x
+    assert [float(out[at]) for at in marks] == [float(i + 3) for i in range(len(marks))]
+    for at in marks:
+        out[at] = 1.25
+    for lo in range(0, n, 2**31):
+        assert bool((out[lo:lo + 2**31] == 1.25).all()), lo
+    del out
+    torch.cuda.empty_cache()
