@@ -216,7 +216,7 @@ hipError_t launch_copy_few_n(hipStream_t st, const CopyFew& a) {
             off |= ((reinterpret_cast<uintptr_t>(a.d[i].src) ^ reinterpret_cast<uintptr_t>(a.d[i].dst[0])) & 127u) != 0;
     const bool four = off || waves * a.n < kOneWaveBlocksFrom;
     const uint64_t g = four ? (waves + 3) / 4 : waves;
-    if (g >> 31) return hipErrorInvalidValue;
+    if (g * (four ? kFourWaves : kOneWave) >> 32) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)g, a.n);
     const uint32_t lds = resident_lds(moved, 16 * (N + 1), N, kLaneBytesCopy);
     if (four)

@@ -995,7 +995,7 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
         constexpr int B = decltype(block)::value, U = decltype(packets)::value;
         constexpr uint64_t span = (uint64_t)B * U * C::E;
         const uint64_t gx = (maxc + span - 1) / span;
-        if (gx >> 31) return hipErrorInvalidValue;
+        if (gx * B >> 32) return hipErrorInvalidValue;  // (see few_fits)
         const dim3 grid((uint32_t)gx, (uint32_t)a.nseg);
 #if MCCLX_TUNE_TIMELINE
         if (OUT == kOutOne) a.timeline = timeline_next(gx * (uint64_t)a.nseg);
@@ -1014,9 +1014,8 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
     if constexpr (C::kTwoShapes) {
         const uint64_t waves = (maxc + 64 * lane_elems - 1) / (64 * lane_elems);
         if (waves * (uint64_t)a.nseg < C::kOneWaveFrom) return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
-        // (a grid may have 2^32 threads: an encode of more than 2^34 elements needs its two packets per lane)
         if constexpr (C::BLOCK == kBlock)
-            if (waves * 64 >> 32 || off_lines<C, OUT>(a))
+            if (off_lines<C, OUT>(a))
                 return go(std::integral_constant<int, kBlock>{}, std::integral_constant<int, C::U>{}, 0);
     }
     return go(std::integral_constant<int, kOneWave>{}, Few{}, lds);
@@ -1049,7 +1048,7 @@ static hipError_t launch_both(hipStream_t st, const FewArgs& a, uint32_t nfold) 
     const uint64_t tile = kFourWaves * C::E;
     const uint64_t blocks = (maxc + tile - 1) / tile * (uint64_t)a.nseg;
     if (blocks == 0) return hipSuccess;
-    if (blocks >> 31) return hipErrorInvalidValue;
+    if (blocks * kFourWaves >> 32) return hipErrorInvalidValue;
     fold_encode_kernel<C, kFourWaves><<<dim3((uint32_t)blocks), dim3(kFourWaves), 0, st>>>(a, nfold);
     return hipGetLastError();
 }
@@ -1145,6 +1144,11 @@ uint32_t items_for(const PlanKey& k, uint64_t count) {
     uint64_t span = (uint64_t)plan_unroll(k) * plan_block(k) * key_pack_elems(k);
     uint64_t n = (count + span - 1) / span;
     return (uint32_t)(n ? n : (count ? 1 : 0));
+}
+
+bool few_fits(const PlanKey& key, uint64_t count) {
+    const bool decode = key.k == 1 && key.io == MCCLX_IO_OUT_F32;
+    return count / (uint64_t)((decode ? 2 : 1) * key_pack_elems(key)) + kBlock < (1ull << 32);
 }
 
 static bool key_is_wide(const PlanKey& key) { return key_pack_elems(key) == 8 && key.k >= kWideMinK; }

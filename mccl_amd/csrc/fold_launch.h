@@ -94,6 +94,10 @@ bool all_plan_ok(const PlanKey& key);
 bool fold_encode_ok(const PlanKey& key);
 hipError_t launch_fold_encode(hipStream_t st, const PlanKey& key, const FewArgs& few, uint32_t nfold);
 
+// Can a segment of `count` elements be launched by value?  A grid has at most 2^32 threads, one
+// per packet there (more are dropped without an error); the table kernels loop.
+bool few_fits(const PlanKey& key, uint64_t count);
+
 // Packets-per-lane unroll and threads per block the kernel template uses for this plan.
 int plan_unroll(const PlanKey& key);
 int plan_block(const PlanKey& key);

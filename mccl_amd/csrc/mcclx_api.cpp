@@ -517,8 +517,11 @@ int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, in
 
 // By value the grid is (tiles of the longest segment) x (segments), so a launch whose
 // segments differ wildly in length would consist mostly of blocks with nothing to do;
-// such a launch takes a table, which has one block per tile.
+// such a launch takes a table, which has one block per tile.  So does one with a segment
+// that is too long for a grid.
 bool even_enough(const mcclx::PlanKey& key, const mcclx_seg* segs, uint32_t nseg) {
+    for (uint32_t s = 0; s < nseg; ++s)
+        if (!mcclx::few_fits(key, segs[s].count)) return false;
     if (nseg <= 4) return true;
     uint64_t longest = 0, total = 0;
     for (uint32_t s = 0; s < nseg; ++s) {
@@ -1066,7 +1069,7 @@ int mcclx_decode_bf16(mcclx_ctx* ctx, void* dst_f32, const void* src_bf16, uint6
 static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    if (l.seg.count && st == nullptr && st != ctx->stream && !ctx->capturing && !ctx->exposed.load() && ctx->few_max >= 1) {
+    if (l.seg.count && l.seg.count < (1ull << 33) && st == nullptr && st != ctx->stream && !ctx->capturing && !ctx->exposed.load() && ctx->few_max >= 1) {
         DeviceGuard guard(ctx->device);
         if (!guard.ok) return fail(MCCLX_ERR_HIP, "hipSetDevice(%d) failed", ctx->device);
         if (!records(st) && !records(ctx->stream)) {
@@ -1123,6 +1126,9 @@ int mcclx_decode_bf16_ordered(mcclx_ctx* ctx, void* stream, void* dst_f32, const
     return ordered_launch(ctx, stream, decode_launch(dst_f32, src_bf16, count));
 }
 
+// Longer copies are cut: a grid has at most 2^32 threads, each of which moves 16 bytes.
+constexpr uint64_t kCopyRange = 1ull << 35;
+
 int mcclx_copy(mcclx_ctx* ctx, void* dst, const void* src, uint64_t nbytes) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     if (nbytes == 0 || dst == src) return MCCLX_OK;
@@ -1132,9 +1138,12 @@ int mcclx_copy(mcclx_ctx* ctx, void* dst, const void* src, uint64_t nbytes) {
         if (int rc = check_range(dst, nbytes, "dst", 0)) return rc;
     }
     DeviceGuard guard(ctx->device);
-    hipError_t e = mcclx::launch_copy(queue_of(ctx), dst, src, nbytes);
-    if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy launch failed: %s", hipGetErrorString(e));
-    ++ctx->launches;
+    for (uint64_t at = 0; at < nbytes; at += kCopyRange) {
+        const uint64_t len = nbytes - at < kCopyRange ? nbytes - at : kCopyRange;
+        hipError_t e = mcclx::launch_copy(queue_of(ctx), static_cast<char*>(dst) + at, static_cast<const char*>(src) + at, len);
+        if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy launch failed: %s", hipGetErrorString(e));
+        ++ctx->launches;
+    }
     return MCCLX_OK;
 }
 
@@ -1155,14 +1164,19 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
             if (int rc = check_range(d.src, d.nbytes, "src", i)) return rc;
             if (int rc = check_range(d.dst, d.nbytes, "dst", i)) return rc;
         }
-        mcclx::CopyDesc* last = groups.empty() ? nullptr : &groups.back();
-        if (last && last->src == d.src && last->nbytes == d.nbytes && last->n < (uint64_t)mcclx::kCopyDsts) {
-            last->dst[last->n++] = d.dst;
-        } else {
-            groups.push_back(mcclx::CopyDesc{d.src, d.nbytes, 1, {d.dst}});
-            bytes += d.nbytes;
+        for (uint64_t at = 0; at < d.nbytes; at += kCopyRange) {
+            const uint64_t len = d.nbytes - at < kCopyRange ? d.nbytes - at : kCopyRange;
+            const void* src = static_cast<const char*>(d.src) + at;
+            void* dst = static_cast<char*>(d.dst) + at;
+            mcclx::CopyDesc* last = groups.empty() ? nullptr : &groups.back();
+            if (last && last->src == src && last->nbytes == len && last->n < (uint64_t)mcclx::kCopyDsts) {
+                last->dst[last->n++] = dst;
+            } else {
+                groups.push_back(mcclx::CopyDesc{src, len, 1, {dst}});
+                bytes += len;
+            }
+            if ((int)groups.back().n > most) most = (int)groups.back().n;
         }
-        if ((int)groups.back().n > most) most = (int)groups.back().n;
     }
     if (groups.empty()) return MCCLX_OK;
     const uint32_t live = (uint32_t)groups.size();

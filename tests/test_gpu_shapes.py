@@ -145,3 +145,39 @@ def test_an_encode_of_more_elements_than_a_grid_has_threads_for(K):
         assert bool((out[lo:lo + 2**31] == 1.25).all()), lo
     del out
     torch.cuda.empty_cache()
+
+
+def test_a_fold_and_a_copy_longer_than_a_grid(K):
+    from mccl_amd import _lib as L
+    if torch.cuda.mem_get_info()[0] < 160 * 2**30:
+        pytest.skip("needs 140 GB of device memory")
+    q = K._q(None)
+    n = 2**34 + 4099  # 64 GiB of fp32
+    marks = [0, 1, 2**33 + 5, 2**34 - 1, 2**34, n - 1]
+    a, b = torch.full((n,), 1.25, device="cuda"), torch.full((n,), 0.5, device="cuda")
+    for i, at in enumerate(marks):
+        a[at] = float(i + 3)
+
+    def check(t, base, plus):
+        assert [float(t[at]) for at in marks] == [i + 3 + plus for i in range(len(marks))]
+        keep = [float(t[at]) for at in marks]
+        for at in marks:
+            t[at] = base
+        for lo in range(0, n, 2**31):
+            assert bool((t[lo:lo + 2**31] == base).all()), lo
+        for at, v in zip(marks, keep):
+            t[at] = v
+
+    K.hip_reduce_op(a, b, "sum")
+    check(a, 1.75, 0.5)
+    torch.cuda.synchronize()
+    q.copy(b.data_ptr(), a.data_ptr(), 4 * n)
+    q.drain()
+    check(b, 1.75, 0.5)
+    b.zero_()
+    torch.cuda.synchronize()
+    q.copy_batched([(b.data_ptr(), a.data_ptr(), 4 * n)])
+    q.drain()
+    check(b, 1.75, 0.5)
+    del a, b
+    torch.cuda.empty_cache()
