@@ -1058,12 +1058,18 @@ static hipError_t launch_table(hipStream_t st, const TableArgs& args, const Laun
     TableArgs a = args;
     const uint32_t grid = (uint32_t)(a.total_items < lp.max_blocks ? a.total_items : lp.max_blocks);
     if (grid == 0) return hipSuccess;
+    // Fewer waves resident (resident_lds) only for launches that write to four places or more, or
+    // back into all operands: a block fetches its work item and its descriptor before its operands,
+    // and with one output or two the waves that are left do not hide that.  Without the limit and
+    // with it, 4096 messages of 64 KB: three operands into one 167 and 181 us, eight 393 and 414,
+    // two operands to two 172 and 192, three to three 266 and 267; four to four 377 and 351.
+    // In place, 1024 messages: three ranks 72 and 68 us, five 123 and 113, eight 206 and 187.
     uint32_t lds = 0;
-    if constexpr (C::BLOCK == kOneWave) {
-        const int outputs = OUT == kOutAll ? C::K : 1 + a.fan;
+    const int outputs = OUT == kOutAll ? C::K : 1 + a.fan;
+    if (C::BLOCK == kOneWave && (OUT == kOutAll || outputs >= 4)) {
         const int lane_bytes = C::U * (C::kReadBytes + outputs * ((C::W == MCCLX_F32 || C::kOutF32) ? 16 : 2 * C::E));
         lds = resident_lds(a.total_items * 64 * (uint64_t)lane_bytes, lane_bytes, outputs,
-                                      OUT == kOutAll ? kLaneBytesInPlace : kLaneBytes);
+                           OUT == kOutAll ? kLaneBytesInPlace : kLaneBytes);
     }
     if constexpr (OUT == kOutAll)
         fold_table_all_kernel<C><<<dim3(grid), dim3(C::BLOCK), lds, st>>>(a);

@@ -106,7 +106,8 @@ uint32_t items_for(const PlanKey& key, uint64_t count);
 // hipErrorInvalidValue = no kernel for this plan.
 hipError_t launch_fold(hipStream_t st, const PlanKey& key, const LaunchParams& lp);
 
-// How many one-wavefront blocks share a CU in a large launch of several streams.
+// How many one-wavefront blocks share a CU in a large launch of several streams (by value; what
+// launch_table takes of it is said there).
 //
 // A full CU holds 32 of them, and a launch of k operands then has 32 * k KiB of loads per CU
 // under way, spread over a range of every stream that is wider than what the memory channels
