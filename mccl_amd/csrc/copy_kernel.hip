@@ -218,7 +218,11 @@ hipError_t launch_copy_few_n(hipStream_t st, const CopyFew& a) {
     const uint64_t g = four ? (waves + 3) / 4 : waves;
     if (g * (four ? kFourWaves : kOneWave) >> 32) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)g, a.n);
-    const uint32_t lds = resident_lds(moved, 16 * (N + 1), N, kLaneBytesCopy);
+    // Where copies of different numbers of destinations share the launch, few blocks have all N: the
+    // waves that copies of three destinations get are right for every mixture tried (67 MB from nine
+    // ranks to all nine, eight destinations and one in turn, 1465 -> 1065 us; twelve ranks, eight and
+    // four, 609 -> 450).
+    const uint32_t lds = resident_lds(moved, MIXED ? 16 * (3 + 1) : 16 * (N + 1), N, kLaneBytesCopy);
     if (four)
         copy_few_kernel<N, kFourWaves, MIXED><<<grid, dim3(kFourWaves), lds, st>>>(a);
     else
