@@ -386,8 +386,9 @@ typedef struct {
 
 /* Scratch a replay needs: the recv scratch of ProcessGroupMCCL.cpp:152-162 per
  * virtual rank plus, with the wire codec, one bf16 copy per rank.  0 for a
- * DIRECT replay whose fold also hands the result to every rank (a sum of up to
- * four ranks): `workspace` may then be NULL. */
+ * DIRECT replay whose fold also hands the result to every rank (up to
+ * MCCLX_MAX_INPUTS ranks, any op, per-step rounding): `workspace` may then be
+ * NULL.  For the same other fields it does not fall as `numel` grows. */
 MCCLX_API uint64_t mcclx_replay_workspace_bytes(const mcclx_replay* r);
 
 /* Single-process replay of allreduce_ring / _tree / _butterfly

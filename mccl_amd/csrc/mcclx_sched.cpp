@@ -273,17 +273,13 @@ bool direct_applies(const mcclx_replay* r) {
 // (or fold + cast) pair reads the result again for every rank.  In place of those two
 // launches, measured on the device: 8 x 12.5 M bf16 89 -> 71 us, 8 x 25 MiB fp32 over the
 // wire codec 93 -> 77 us, MAX of 3 x 25 MiB 33 -> 26 us (49 -> 26 us over the codec),
-// 8 x 4 KB 4.1 -> 2.4 us.
-// From 8 MiB of tensors on, and up to 1 MiB, where a call is all latency.  In between the
-// launch sequence of a fused replay stays what callers that count launches rely on; one
-// launch less is worth 2 us there, of some 25 a call takes.
+// 8 x 4 KB 4.1 -> 2.4 us; whole calls of 1.5 to 8 MB of tensors 18-21 -> 14-17 us, MAX over the
+// codec 23-45 -> 15-18 us.
 bool to_all(const mcclx_replay* r) {
     const bool wire = r->wire_bf16 && r->dtype == MCCLX_F32;
     const bool step = r->acc == MCCLX_ACC_STEP || (r->dtype == MCCLX_F32 && !wire);
     if (r->mode == MCCLX_REPLAY_STEPWISE || (wire && r->mode != MCCLX_REPLAY_DIRECT)) return false;
-    if (!step || r->world < 2 || r->world > MCCLX_MAX_INPUTS || fan_of(r) > 0) return false;
-    const uint64_t bytes = r->numel * esize(r->dtype) * (uint64_t)r->world;
-    return bytes >= (8u << 20) || bytes <= (1u << 20);
+    return step && r->world >= 2 && r->world <= MCCLX_MAX_INPUTS && fan_of(r) == 0;
 }
 
 // A fold takes MCCLX_MAX_INPUTS operands.  A wider world is folded by a chain
@@ -692,7 +688,7 @@ private:
 // Same plan for every phase?
 bool same_plan(const mcclx_replay* a, const mcclx_replay* b) {
     return a->world == b->world && a->algo == b->algo && a->op == b->op && a->dtype == b->dtype &&
-           (a->wire_bf16 != 0) == (b->wire_bf16 != 0) && a->acc == b->acc && a->mode == b->mode && to_all(a) == to_all(b);
+           (a->wire_bf16 != 0) == (b->wire_bf16 != 0) && a->acc == b->acc && a->mode == b->mode;
 }
 
 }  // namespace

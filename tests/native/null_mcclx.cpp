@@ -5,7 +5,7 @@
 // A context is a reduce queue as the library's is: launches return at once and run later, in order,
 // on a thread of the context's own (the "device"); tickets, drains and cross-queue waits order the
 // host and other queues against it.  Arithmetic is done on host memory for what the stress test
-// checks -- fp32 sums with scale and fan-out, copies -- and skipped for everything else.  This is
+// checks -- fp32 sums with scale, fan-out and to-all, copies -- and skipped for everything else.  This is
 // test infrastructure: nothing in the product builds or loads it.
 #include <atomic>
 #include <chrono>
@@ -184,6 +184,8 @@ int mcclx_fold_batched(mcclx_ctx* c, const mcclx_plan* plan, const mcclx_seg* se
                 if (p.scale_mode != MCCLX_SCALE_NONE) acc *= scale;
                 if (g.out) static_cast<float*>(g.out)[i] = acc;
                 for (int f = 0; f < fan; ++f) static_cast<float*>(const_cast<void*>(g.in[p.k + f]))[i] = acc;
+                if (p.flags & MCCLX_PLAN_TO_ALL)
+                    for (int k = 0; k < p.k; ++k) static_cast<float*>(const_cast<void*>(g.in[k]))[i] = acc;
             }
     });
     return MCCLX_OK;

@@ -1,7 +1,7 @@
 // pg_stress.cpp -- the ownership side of the c10d backend under a sanitizer, without a GPU: the real
 // ProcessGroupMCCL, WorkMCCL, Progress, LocalMesh, HostWire and chunk scheduler, compiled with
 // -DMCCL_NULL_DEVICE (backend/Device.hpp) over a host stand-in of the kernel layer
-// (null_mcclx.cpp).  Groups of 2-4 rank threads come and go; every second group completes its
+// (null_mcclx.cpp).  Groups of 2-5 rank threads come and go; every second group completes its
 // allreduces event-based (completer thread, two queues, parked buckets).  What the test is after
 // is who lets go of what, where:
 //   * the registry of meshes and shared contexts while ranks join and leave at different times;
@@ -91,7 +91,7 @@ void lists(ProcessGroupMCCL& pg, int rank, int world) {
 int main(int argc, char** argv) {
     const int groups = argc > 1 ? atoi(argv[1]) : 60;
     for (int g = 0; g < groups; ++g) {
-        const int world = 2 + g % 3;
+        const int world = g % 10 == 9 ? 5 : 2 + g % 3;  // (five: sums go back into every operand)
         const bool async = (g & 1) != 0;
         if (async)
             setenv("MCCL_ALLREDUCE_ASYNC", "1", 1);

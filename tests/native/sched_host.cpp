@@ -1,0 +1,105 @@
+// sched_host.cpp -- the chunk scheduler (mccl_amd/csrc/mcclx_sched.cpp) over the host stand-in of
+// the kernel layer (null_mcclx.cpp): launches per list, results of fp32 sums, workspace sizes.
+#include <cstdio>
+#include <cstring>
+#include <vector>
+
+#include "mcclx.h"
+
+namespace {
+int g_bad = 0;
+
+mcclx_replay replay(int world, int algo, int op, int wire, int mode, uint64_t numel, void* const* tensors) {
+    mcclx_replay r;
+    memset(&r, 0, sizeof r);
+    r.world = world;
+    r.algo = algo;
+    r.op = op;
+    r.dtype = MCCLX_F32;
+    r.wire_bf16 = wire;
+    r.mode = mode;
+    r.acc = MCCLX_ACC_STEP;
+    r.numel = numel;
+    r.tensors = const_cast<void**>(tensors);
+    return r;
+}
+
+// A list of `entries` allreduces whose sizes alternate; returns the launches it took.
+unsigned long long list(mcclx_ctx* ctx, const char* what, int world, int algo, int op, int wire, int mode,
+                        uint64_t small, uint64_t large, int entries, unsigned long long want) {
+    std::vector<std::vector<float>> data;
+    std::vector<std::vector<void*>> ptrs(static_cast<size_t>(entries));
+    std::vector<std::vector<char>> ws;
+    std::vector<mcclx_replay> reps;
+    for (int e = 0; e < entries; ++e) {
+        const uint64_t n = e % 2 ? large : small;
+        for (int r = 0; r < world; ++r) data.emplace_back(n, static_cast<float>(r + 1 + e));
+    }
+    for (int e = 0; e < entries; ++e) {
+        const uint64_t n = e % 2 ? large : small;
+        for (int r = 0; r < world; ++r) ptrs[size_t(e)].push_back(data[size_t(e * world + r)].data());
+        mcclx_replay rp = replay(world, algo, op, wire, mode, n, ptrs[size_t(e)].data());
+        ws.emplace_back(mcclx_replay_workspace_bytes(&rp) + 1);
+        rp.workspace = ws.back().data();
+        rp.workspace_bytes = ws.back().size() - 1;
+        reps.push_back(rp);
+    }
+    const unsigned long long before = mcclx_launch_count(ctx);
+    if (mcclx_allreduce_replay_many(ctx, reps.data(), static_cast<uint32_t>(entries)) != MCCLX_OK) {
+        printf("FAILED: %s: %s\n", what, mcclx_last_error());
+        ++g_bad;
+    }
+    const unsigned long long launches = mcclx_launch_count(ctx) - before;
+    mcclx_queue_drain(ctx);
+    if (launches != want) {
+        printf("FAILED: %s: %llu launches, expected %llu\n", what, launches, want);
+        ++g_bad;
+    }
+    if (!wire && op == MCCLX_SUM)  // what the stand-in computes
+        for (int e = 0; e < entries; ++e)
+            for (int r = 0; r < world; ++r)
+                for (float v : data[size_t(e * world + r)])
+                    if (v != static_cast<float>(world * (world + 1) / 2 + world * e)) {
+                        printf("FAILED: %s: entry %d rank %d holds %g\n", what, e, r, static_cast<double>(v));
+                        ++g_bad;
+                        return launches;
+                    }
+    return launches;
+}
+}  // namespace
+
+int main() {
+    mcclx_ctx* ctx = nullptr;
+    if (mcclx_init(0, &ctx) != MCCLX_OK) return 1;
+    // one plan for the whole list, however its entries' sizes alternate: one launch
+    list(ctx, "8 ranks, AVG, tree", 8, MCCLX_ALGO_TREE, MCCLX_AVG, 0, MCCLX_REPLAY_FUSED, 1024, 65536, 100, 1);
+    list(ctx, "8 ranks, AVG over the codec, ring", 8, MCCLX_ALGO_RING, MCCLX_AVG, 1, MCCLX_REPLAY_DIRECT, 1024, 65536, 100, 1);
+    list(ctx, "3 ranks, MAX, ring", 3, MCCLX_ALGO_RING, MCCLX_MAX, 0, MCCLX_REPLAY_FUSED, 1024, 200000, 100, 1);
+    list(ctx, "3 ranks, MAX over the codec, tree", 3, MCCLX_ALGO_TREE, MCCLX_MAX, 1, MCCLX_REPLAY_DIRECT, 1024, 200000, 10, 1);
+    list(ctx, "5 ranks, SUM over the codec through copies", 5, MCCLX_ALGO_RING, MCCLX_SUM, 1, MCCLX_REPLAY_FUSED, 1024, 65536, 10, 3);
+    for (int world = 2; world <= 8; ++world)
+        for (int algo : {MCCLX_ALGO_RING, MCCLX_ALGO_TREE, MCCLX_ALGO_BUTTERFLY})
+            list(ctx, "SUM", world, algo, MCCLX_SUM, 0, MCCLX_REPLAY_FUSED, 37, 70001, 6, 1);
+    // what a replay needs does not fall as it grows: sized once for the largest, enough for all
+    for (int world = 2; world <= 20; ++world)
+        for (int algo : {MCCLX_ALGO_RING, MCCLX_ALGO_TREE, MCCLX_ALGO_BUTTERFLY})
+            for (int op : {MCCLX_SUM, MCCLX_MAX})
+                for (int wire : {0, 1})
+                    for (int mode : {MCCLX_REPLAY_STEPWISE, MCCLX_REPLAY_FUSED, MCCLX_REPLAY_DIRECT}) {
+                        uint64_t last = 0;
+                        for (uint64_t n = 32; n < (1u << 24); n = n * 5 / 4) {
+                            mcclx_replay r = replay(world, algo, op, wire, mode, n, nullptr);
+                            const uint64_t need = mcclx_replay_workspace_bytes(&r);
+                            if (need < last || (mode == MCCLX_REPLAY_DIRECT && world <= 8 && need)) {
+                                printf("FAILED: workspace of world %d algo %d op %d wire %d mode %d numel %llu\n", world, algo,
+                                       op, wire, mode, static_cast<unsigned long long>(n));
+                                ++g_bad;
+                                break;
+                            }
+                            last = need;
+                        }
+                    }
+    mcclx_destroy(ctx);
+    if (!g_bad) printf("ok\n");
+    return g_bad ? 1 : 0;
+}

@@ -443,8 +443,10 @@ def test_copy_batched_many_small_and_a_few_large(K, U):
 def test_launch_counts_of_the_fused_schedules(H, K, U):
     """What "fused" means in launches.  Up to four ranks a sum needs no allgather launch: the
     owner's fold stores the reduced chunk into every rank's tensor, so butterfly over the wire =
-    encode + fold (2) and without the wire one fold (1); the other reduce ops, and five ranks or
-    more, keep the separate cast / copy launch (3, or 1 fold + the allgather copies); a list of
+    encode + fold (2) and without the wire one fold (1); so do the other reduce ops and five to
+    eight ranks, whose fold stores back into its operands, where the operands are the ranks' own
+    tensors (1, without the wire or DIRECT); over bf16 copies (FUSED with the wire) and beyond
+    eight ranks the cast / copy launch stays separate (3 over the wire); a list of
     200 tree messages = 1 launch; the stepwise replay of the same butterfly issues the
     reference's sequence."""
     from mccl_amd import _lib as L
@@ -464,17 +466,17 @@ def test_launch_counts_of_the_fused_schedules(H, K, U):
     t = mk()
     assert launches(lambda: H.allreduce_replay(t, "sum", BUTTERFLY, mode=FUSED)) == 1
     t = mk()
-    assert launches(lambda: H.allreduce_replay(t, "max", BUTTERFLY, mode=FUSED)) == 1 + 1   # 6 copies of 400 KB: one launch
+    assert launches(lambda: H.allreduce_replay(t, "max", BUTTERFLY, mode=FUSED)) == 1
     # DIRECT: the fold reads the ranks' fp32 tensors itself -- the whole wire allreduce of up to
-    # four ranks is one launch, of five to eight a fold and the casts on arrival
+    # eight ranks is one launch, whatever the op
     for algo in (RING, TREE, BUTTERFLY):
         t = mk()
         assert launches(lambda: H.allreduce_replay(t, "avg", algo, wire_bf16=True, mode=DIRECT)) == 1
     t = mk()
-    assert launches(lambda: H.allreduce_replay(t, "max", BUTTERFLY, wire_bf16=True, mode=DIRECT)) == 3
+    assert launches(lambda: H.allreduce_replay(t, "max", BUTTERFLY, wire_bf16=True, mode=DIRECT)) == 1
     five = [U.to_dev(U.rand_values(rng, n, F32), F32) for _ in range(5)]
-    assert launches(lambda: H.allreduce_replay(five, "avg", RING, wire_bf16=True, mode=DIRECT)) == 2
-    assert launches(lambda: H.allreduce_replay(five, "sum", RING, mode=FUSED)) == 1 + 1
+    assert launches(lambda: H.allreduce_replay(five, "avg", RING, wire_bf16=True, mode=DIRECT)) == 1
+    assert launches(lambda: H.allreduce_replay(five, "sum", RING, mode=FUSED)) == 1
     assert launches(lambda: H.allreduce_replay(five, "avg", RING, wire_bf16=True, mode=FUSED)) == 3
     t = mk()
     stepwise = launches(lambda: H.allreduce_replay(t, "avg", BUTTERFLY, wire_bf16=True, mode=STEPWISE))

@@ -1,7 +1,7 @@
 """The to-all form of a fold (the result goes back into every operand's buffer: a whole allreduce
 of five to eight ranks, or of any op, in one launch) against the oracle's replay of the
 reference, bit for bit: every dtype, op, algorithm and number of ranks, sizes at the edges of
-packets and tiles, tensors off the 16-byte grid, and the sizes from which large replays take it."""
+packets and tiles, tensors off the 16-byte grid, and large replays."""
 import ctypes as C
 import re
 
@@ -46,6 +46,8 @@ def test_small_replays_against_the_oracle(dtype, wire, algo, op):
 
 
 @pytest.mark.parametrize("world,n,dtype,op,algo,wire", [
+    (5, 60_001, F32, SUM, RING, False), (8, 100_003, F32, AVG, RING, True), (3, 300_007, F32, MAX, BUTTERFLY, True),
+    (6, 200_001, BF16, AVG, TREE, False), (7, 150_001, F16, MIN, RING, False), (4, 400_003, F32, PRODUCT, TREE, False),
     (8, 524_288, BF16, AVG, RING, False), (8, 262_147, F32, SUM, BUTTERFLY, True), (5, 419_431, F32, AVG, TREE, False),
     (3, 699_053, F32, MAX, RING, True), (2, 2_097_153, F16, MIN, BUTTERFLY, False),
     (8, 5_000_011, BF16, AVG, RING, False), (6, 3_500_003, F32, AVG, RING, True)])  # the last two: fewer waves resident
