@@ -219,7 +219,7 @@ struct FoldPass {
 
 struct Phases {
     bool planned = false;
-    bool over_link = false;  // every replay's wire copies lie in pinned host memory, clear of its tensors
+    uint64_t pieces = 1;  // > 1: the wire copies lie in pinned host memory, see issue_in_pieces
     mcclx_plan enc, dec;
     std::vector<mcclx_seg> enc_segs, dec_segs;
     std::vector<FoldPass> folds;  // one pass, or a chain of passes when the world is wider than one fold
@@ -607,12 +607,9 @@ int issue_in_pieces(mcclx_ctx* ctx, const Phases& ph, uint64_t pieces) {
 }
 
 int issue_phases(mcclx_ctx* ctx, Phases& ph) {
-    if (ph.over_link && ph.fan && ph.folds.size() == 1 && !ph.enc_segs.empty()) {
-        const uint64_t pieces = pieces_of(ph);
-        if (pieces > 1 &&
-            mcclx_fold_encode_ok(ctx, &ph.folds[0].plan, (uint32_t)(ph.folds[0].segs.size() + ph.enc_segs.size())))
-            return issue_in_pieces(ctx, ph, pieces);
-    }
+    if (ph.pieces > 1 &&
+        mcclx_fold_encode_ok(ctx, &ph.folds[0].plan, (uint32_t)(ph.folds[0].segs.size() + ph.enc_segs.size())))
+        return issue_in_pieces(ctx, ph, ph.pieces);
     if (!ph.enc_segs.empty())
         TRY(mcclx_fold_batched(ctx, &ph.enc, ph.enc_segs.data(), (uint32_t)ph.enc_segs.size()));
     for (FoldPass& f : ph.folds)
@@ -771,12 +768,16 @@ int mcclx_allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t
                 if (!fused || nothing) break;
             }
             if (!touched.add(&rs[i])) break;
-            const bool link = rs[i].mode == MCCLX_REPLAY_FUSED && rs[i].wire_bf16 && rs[i].workspace &&
-                              rs[i].algo != MCCLX_ALGO_TREE && fan_of(&rs[i]) > 0 &&
-                              mcclx_in_host_memory(ctx, rs[i].workspace) && all_disjoint(&rs[i]);
-            ph.over_link = link && (&rs[i] == first || ph.over_link);
             collect_fused(&rs[i], layout_of(&rs[i]), ph);
             ++i;
+        }
+        if (first->mode == MCCLX_REPLAY_FUSED && first->algo != MCCLX_ALGO_TREE && ph.fan && !ph.enc_segs.empty()) {
+            // where the copies lie is asked only of a run that is long enough to be cut
+            const uint64_t pieces = pieces_of(ph);
+            bool link = pieces > 1;
+            for (const mcclx_replay* r = first; link && r != &rs[i]; ++r)
+                link = mcclx_in_host_memory(ctx, r->workspace) && all_disjoint(r);
+            if (link) ph.pieces = pieces;
         }
         TRY(issue_phases(ctx, ph));
     }

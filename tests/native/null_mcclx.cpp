@@ -249,7 +249,11 @@ int mcclx_batch_begin(mcclx_ctx*, const char*) { return MCCLX_OK; }
 int mcclx_batch_end(mcclx_ctx*) { return MCCLX_OK; }
 
 // The scheduler's pieces over the link: there is no link here.
-bool mcclx_in_host_memory(mcclx_ctx*, const void*) { return false; }
+std::atomic<long> null_memory_questions{0};  // for tests of when the scheduler asks
+bool mcclx_in_host_memory(mcclx_ctx*, const void*) {
+    ++null_memory_questions;
+    return false;
+}
 bool mcclx_fold_encode_ok(mcclx_ctx*, const mcclx_plan*, uint32_t) { return false; }
 int mcclx_fold_encode(mcclx_ctx*, const mcclx_plan*, const mcclx_seg*, uint32_t, const mcclx_plan*, const mcclx_seg*, uint32_t) {
     return mcclx_fail(MCCLX_ERR_STATE, "no fold_encode");

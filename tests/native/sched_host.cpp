@@ -1,10 +1,13 @@
 // sched_host.cpp -- the chunk scheduler (mccl_amd/csrc/mcclx_sched.cpp) over the host stand-in of
 // the kernel layer (null_mcclx.cpp): launches per list, results of fp32 sums, workspace sizes.
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <vector>
 
 #include "mcclx.h"
+
+extern "C" std::atomic<long> null_memory_questions;
 
 namespace {
 int g_bad = 0;
@@ -80,6 +83,15 @@ int main() {
     for (int world = 2; world <= 8; ++world)
         for (int algo : {MCCLX_ALGO_RING, MCCLX_ALGO_TREE, MCCLX_ALGO_BUTTERFLY})
             list(ctx, "SUM", world, algo, MCCLX_SUM, 0, MCCLX_REPLAY_FUSED, 37, 70001, 6, 1);
+    // where a workspace lies is asked of runs that are long enough to be cut into pieces only
+    null_memory_questions = 0;
+    list(ctx, "3 ranks, AVG over the codec through copies", 3, MCCLX_ALGO_RING, MCCLX_AVG, 1, MCCLX_REPLAY_FUSED, 1024, 8192, 40, 2);
+    const long asked = null_memory_questions;
+    list(ctx, "the same, large", 3, MCCLX_ALGO_RING, MCCLX_AVG, 1, MCCLX_REPLAY_FUSED, 4000000, 4000000, 2, 2);
+    if (asked || !null_memory_questions) {
+        printf("FAILED: %ld questions about small workspaces, %ld in all\n", asked, null_memory_questions.load());
+        ++g_bad;
+    }
     // what a replay needs does not fall as it grows: sized once for the largest, enough for all
     for (int world = 2; world <= 20; ++world)
         for (int algo : {MCCLX_ALGO_RING, MCCLX_ALGO_TREE, MCCLX_ALGO_BUTTERFLY})
