@@ -129,19 +129,14 @@ class MCCLError(RuntimeError):
 
 
 _lib = None
-_in_tree = False
-
-
-def in_tree() -> bool:
-    """Is the loaded library the in-tree one, which the extension mccl_amd/_C is linked against?
-    (A context belongs to the library that made it.)"""
-    lib()
-    return _in_tree
+# Is the loaded library the in-tree one, which the extension mccl_amd/_C is linked against?
+# (A context belongs to the library that made it.)
+in_tree = False
 
 
 def lib() -> C.CDLL:
     """Load libmcclx.so (once) and type every entry point.  Raises if absent."""
-    global _lib, _in_tree
+    global _lib, in_tree
     if _lib is None:
         # One HIP runtime per process.  PyTorch-ROCm wheels bundle their own
         # libamdhip64 (file "libamdhip64.so", soname "libamdhip64.so.N") next to the
@@ -160,7 +155,7 @@ def lib() -> C.CDLL:
             fn = getattr(L, name)  # AttributeError if the symbol is not exported
             fn.restype = res
             fn.argtypes = args
-        _in_tree = os.path.exists(LIB_PATH) and os.path.samefile(path, LIB_PATH)
+        in_tree = os.path.exists(LIB_PATH) and os.path.samefile(path, LIB_PATH)
         _lib = L
     return _lib
 

@@ -27,7 +27,7 @@ except ImportError:
 def _reader():
     """The native reader, or None where it is not built or the queues are another library's
     (MCCLX_LIBRARY): it calls the libmcclx.so it is linked against."""
-    return _native if _native is not None and L.in_tree() else None
+    return _native if L.in_tree else None
 
 
 ALGO_NAMES = {"ring": L.ALGO_RING, "tree": L.ALGO_TREE, "butterfly": L.ALGO_BUTTERFLY}

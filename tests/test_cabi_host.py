@@ -179,7 +179,8 @@ def test_queues_of_another_library_are_not_handed_to_the_extension(tmp_path, oth
     if other:
         env["MCCLX_LIBRARY"] = str(tmp_path / "libmcclx.so")
         shutil.copy(_lib.LIB_PATH, env["MCCLX_LIBRARY"])
-    code = "from mccl_amd import harness as H; assert H._native is not None; print('native', H._reader() is not None)"
+    code = ("from mccl_amd import _lib, harness as H; _lib.lib(); assert H._native is not None; "
+            "print('native', H._reader() is not None)")
     r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=300, env=env, cwd=ROOT)
     assert r.returncode == 0, r.stderr
     assert r.stdout.strip() == f"native {not other}"
