@@ -106,7 +106,11 @@ MCCLX_API int mcclx_init(int device, mcclx_ctx** out);
  * caller, e.g. PyTorch's current stream); nothing is created or destroyed. */
 MCCLX_API int mcclx_init_on_stream(int device, void* hip_stream, mcclx_ctx** out);
 MCCLX_API int mcclx_destroy(mcclx_ctx* ctx);
-/* The queue's hipStream_t, for callers that enqueue their own work on it. */
+/* The queue's hipStream_t, for callers that enqueue their own work on it.  From
+ * then on every launch of the context goes through that stream, also the
+ * mcclx_*_ordered calls, which otherwise run on the default stream where they can
+ * (about 11 us a call through Python instead of 50): a caller that wants those
+ * short takes the stream of a context of its own. */
 MCCLX_API void* mcclx_queue_stream(mcclx_ctx* ctx);
 /* Number of compute units of the context's device (sizing of persistent grids). */
 MCCLX_API int mcclx_device_cus(mcclx_ctx* ctx);
@@ -263,8 +267,9 @@ MCCLX_API int mcclx_copy(mcclx_ctx* ctx, void* dst, const void* src, uint64_t nb
 /* The tensor forms: one launch at the end of `stream` (a HIP stream of the context's device), as
  * mcclx_queue_wait_stream, the call above of the same name and mcclx_stream_wait_queue in a row
  * give it -- behind everything enqueued so far on `stream` and on the queue, in front of what
- * either is given next.  Where the queue is idle and `stream` is the
- * default one (NULL) the kernel runs on it. */
+ * either is given next.  Where the queue is idle, its HIP stream has not been
+ * handed out (mcclx_queue_stream) and `stream` is the default one (NULL) the
+ * kernel runs on it. */
 MCCLX_API int mcclx_reduce_ordered(mcclx_ctx* ctx, void* stream, void* dst, const void* src, int dtype, uint64_t count, int op);
 MCCLX_API int mcclx_scale_ordered(mcclx_ctx* ctx, void* stream, void* buf, int dtype, uint64_t count, double scale, int scale_mode);
 MCCLX_API int mcclx_accumulate_scale_ordered(mcclx_ctx* ctx, void* stream, void* dst, const void* src, int dtype, uint64_t count, double scale);
@@ -275,8 +280,10 @@ MCCLX_API int mcclx_decode_bf16_ordered(mcclx_ctx* ctx, void* stream, void* dst_
  * reduced chunk to every other rank (AllreduceAlgos.cpp:77-86, 185-200; the
  * tree's broadcast :119-126), N-1 sends per chunk in the reference.  Ranges of
  * different descriptors must not overlap each other's destinations; a
- * descriptor with nbytes == 0 or dst == src is skipped.  A few large copies are
- * issued one launch each (that streams best); many small ones go out together. */
+ * descriptor with nbytes == 0 or dst == src is skipped.  Consecutive descriptors
+ * of one source and length read it once.  Up to 32 sources share a launch, or
+ * many small ones (below 1 MiB each); copies of very different lengths get
+ * launches of their own. */
 typedef struct mcclx_copy_desc {
     void* dst;
     const void* src;

@@ -41,14 +41,16 @@ namespace mcclx {
 namespace {
 
 // Launch shapes, each measured on MI355X.  By-value launches run one-wavefront blocks of one
-// packet per lane (Cfg::FEW_U, kTwoShapes): a block of eight wavefronts keeps its slots until
+// packet per lane (Cfg::FEW_U, kSmallShape): a block of eight wavefronts keeps its slots until
 // the last of its loads is back, one-wavefront blocks turn them over one by one (operands of
 // 128-512 MiB: one fp32 operand scaled 84.5 -> 80.9 us, own fp32 + one bf16 peer 106 -> 99.6,
 // + two peers 124 -> 119.5, copy 82.6 -> 80.6; 25 MiB operands: 10.3 -> 9.5, 12.5 -> 11.4,
 // 13.7 -> 13.1, 10.1 -> 9.2).  The table kernels keep blocks of eight for folds that mix fp32
 // and 16-bit streams and one-operand passes: a tile per wavefront would mean eight times the
-// work items, and with them eight times the item map a ragged launch uploads.
-constexpr int kBlock = 512;  // threads per block of those table launches
+// work items, and with them eight times the item map a ragged launch uploads.  Large by-value
+// launches of those plans take blocks of eight as well where their streams start off each other's
+// lines (off_lines).
+constexpr int kBlock = 512;  // threads per block of those launches
 // Table launches of folds whose streams all have one element size -- all 16-bit (16 bytes
 // per lane and operand) or all fp32 -- take one-wavefront blocks with one packet per lane too.
 constexpr int kWideBlock = 64;
@@ -56,7 +58,7 @@ constexpr int kWideU = 1;
 constexpr int kWideMinK = 2;   // all-16-bit folds of this many operands or more take the one-wavefront shape
 constexpr int kF32Block = 64;
 constexpr int kAllF32Block = 64;
-constexpr int kOneWave = 64, kFourWaves = 256;  // by-value launches, see Cfg::kTwoShapes
+constexpr int kOneWave = 64, kFourWaves = 256;  // by-value launches, see Cfg::kSmallShape
 
 // Every operand lives in global memory (HBM or host memory mapped into the
 // device).  Pointers that reach a kernel through a descriptor table are
@@ -216,9 +218,9 @@ struct Cfg {
     // By-value launches: one-wavefront blocks of one packet per lane (two for the bf16 -> fp32
     // cast, whose lanes read 8 bytes: 67 M elements 63.5 -> 62.1 us), in blocks of four
     // wavefronts where the launch is small (kOneWaveBlocksFrom) and the plan mixes fp32 and
-    // 16-bit streams or has one operand.
+    // 16-bit streams or has one operand; BLOCK and U again where such a plan's streams are off_lines.
     static constexpr int FEW_U = kDecode ? 2 : 1;
-    static constexpr bool kTwoShapes = BLOCK == kBlock || kDecode;
+    static constexpr bool kSmallShape = BLOCK == kBlock || kDecode;
     // (an encode's lanes move 24 bytes: four wavefronts still win at 16,384, 4.2 M elements in 5.5 us against 5.9)
     static constexpr uint64_t kOneWaveFrom = (K == 1 && IO == MCCLX_IO_OWN_FIRST_F32) ? 20480 : kOneWaveBlocksFrom;
     // the first 16-bit operand next to an fp32 output, or -1
@@ -1011,7 +1013,7 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
         return hipGetLastError();
     };
     using Few = std::integral_constant<int, C::FEW_U>;
-    if constexpr (C::kTwoShapes) {
+    if constexpr (C::kSmallShape) {
         const uint64_t waves = (maxc + 64 * lane_elems - 1) / (64 * lane_elems);
         if (waves * (uint64_t)a.nseg < C::kOneWaveFrom) return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
         if constexpr (C::BLOCK == kBlock)

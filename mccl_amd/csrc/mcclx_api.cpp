@@ -1058,12 +1058,13 @@ int mcclx_decode_bf16(mcclx_ctx* ctx, void* dst_f32, const void* src_bf16, uint6
 // `stream` itself, its end marked for whoever uses the queue next (queue_of, drain,
 // mcclx_stream_wait_queue): no cross-stream event and none of the two hand-overs between
 // hardware queues, which bound a sequence of such calls (events and launch 31 us a call, the
-// launch and its mark 7; 4097 bf16 values reduced through Python 48 -> 8 us, 25 MiB encoded and
-// decoded 110 -> 23 us).  The mark is an event record and not the kernel's own stop event: after
+// launch and its mark 7; 4097 bf16 values reduced through Python 50 -> 11 us, 25 MiB encoded and
+// decoded 110 -> 25 us).  The mark is an event record and not the kernel's own stop event: after
 // thousands of launches with one, the next calls on the stream took three times as long.
 // Everything else takes the two orderings: a queue with work in flight, a queue whose HIP stream
 // the caller holds (what they put there would not see a launch made elsewhere), a recording, and
-// every `stream` but the legacy default one.  That one cannot be recorded; of any other the caller
+// every `stream` but the legacy default one.  (Once handed out, the HIP stream stays the caller's to
+// use, so `exposed` is never taken back.)  That one cannot be recorded; of any other the caller
 // may begin a recording later, and while it lasts the runtime refuses to wait for an event that
 // was recorded on the stream before.
 static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
