@@ -223,10 +223,10 @@ struct Cfg {
     static constexpr bool kSmallShape = BLOCK == kBlock || kDecode;
     // (an encode's lanes move 24 bytes: four wavefronts still win at 16,384, 4.2 M elements in 5.5 us against 5.9)
     static constexpr uint64_t kOneWaveFrom = (K == 1 && IO == MCCLX_IO_OWN_FIRST_F32) ? 20480 : kOneWaveBlocksFrom;
-    // the first 16-bit operand next to an fp32 output, or -1
+    // the first 16-bit operand of a fold with an fp32 output, or -1
     static constexpr int kWireIn = [] {
         for (int k = 0; k < K; ++k)
-            if (W != MCCLX_F32 && IO != MCCLX_IO_PURE && !in_is_f32(k)) return k;
+            if (K > 1 && W != MCCLX_F32 && IO != MCCLX_IO_PURE && !in_is_f32(k)) return k;
         return -1;
     }();
     // bytes a lane reads per packet
@@ -518,14 +518,16 @@ __device__ __forceinline__ void fold_packs(const SegArgs& s, bool has_out, bool 
 // the line it fetches five lines for four, the fifth a second time for its neighbour on
 // another XCD (four segments of 27.5 M elements, every other one off the line, own fp32
 // + three bf16 peers: 257 -> 241 us, the peers in pinned host memory 13.1 -> 11.7 ms).
-template <class C, int OUT = kOutOne>
+// Not in small launches (ALIGN), where the few scalar instructions in front of the first load
+// cost more (0.05 us of 2.4), nor in casts (4 M elements 4.8 -> 4.9 us).
+template <class C, int OUT = kOutOne, bool ALIGN = true>
 __host__ __device__ __forceinline__ uint32_t head_elems(const SegArgs& s) {
     const bool wide_out = (C::W == MCCLX_F32 || C::kOutF32) && (OUT == kOutAll || s.out);
     const void* first = OUT == kOutAll ? s.in[0] : s.out ? s.out : s.wire_out;
     const uint32_t a = (uint32_t)reinterpret_cast<uintptr_t>(first);
     const uint32_t mis = a & 127u;
     uint32_t h = mis ? (128u - mis) >> (wide_out ? 2 : 1) : 0u;
-    if constexpr (C::kWireIn >= 0)
+    if constexpr (ALIGN && C::kWireIn >= 0)
         if (wide_out && (((uint32_t)reinterpret_cast<uintptr_t>(s.in[C::kWireIn]) + 2 * h) & 127u) == 64u) h += 32;
     return s.count < h ? (uint32_t)s.count : h;
 }
@@ -558,11 +560,11 @@ __device__ __forceinline__ SegArgs advanced(const SegArgs& s, uint64_t elems) {
 // load is kept short -- a block lives for about 2 us and eight waves per SIMD
 // share one scalar unit, so every scalar instruction in front of the loads is
 // paid eight times over.
-template <class C, int OUT, int kB, int U>
+template <class C, int OUT, int kB, int U, bool ALIGN = true>
 __device__ __forceinline__ void fold_tile(const SegArgs& s, float scale, bool has_scale, uint64_t first,
                                           bool do_edges, int fan = 0, int op = C::OP) {
     const uint32_t tid = threadIdx.x;
-    const uint32_t head = head_elems<C, OUT>(s);  // < 64 <= kB
+    const uint32_t head = head_elems<C, OUT, ALIGN>(s);  // < 64 <= kB
     const uint64_t P = (s.count - head) / C::E;
     const bool has_out = s.out != nullptr, has_wire = s.wire_out != nullptr;
     if (first < P) {
@@ -638,7 +640,7 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
     (void)grid;
     int op = C::OP;
     if constexpr (C::OP == kAnyOp) op = a.op;
-    fold_tile<C, OUT, B, U>(s, scale, has_scale != 0, (uint64_t)blockIdx.x * span, blockIdx.x == 0, fan, op);
+    fold_tile<C, OUT, B, U, B != kFourWaves>(s, scale, has_scale != 0, (uint64_t)blockIdx.x * span, blockIdx.x == 0, fan, op);
 #if MCCLX_TUNE_TIMELINE
     if (a.timeline && threadIdx.x == 0) {
         TimelineRecord r;
