@@ -296,6 +296,12 @@ MCCLX_API int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, u
 /* Block until every launch on the queue has finished.  Replaces
  * mccl_queue_drain (MPSInterop.mm:312-318) and metal_sync (MetalKernels.mm:552). */
 MCCLX_API int mcclx_queue_drain(mcclx_ctx* ctx);
+/* The same for results in device memory, without the runtime's completion signal: once the call
+ * returns, every launch issued before it has run and any kernel or copy issued from now on, on any stream, finds
+ * what it wrote.  (What the launches wrote to host memory needs mcclx_queue_drain.)  The host
+ * polls a word that the queue's end writes, for spin_us microseconds; if it has not come by then, or with
+ * spin_us = 0, the call drains. */
+MCCLX_API int mcclx_queue_wait(mcclx_ctx* ctx, uint32_t spin_us);
 /* The queue waits (on the device, host not blocked) for everything enqueued so
  * far on `producer_stream`.  Replaces mps_stream_sync (MPSInterop.mm:308-310)
  * and mps_event_sync_nonblocking + wait_for_mps (:336-356, EventSync.mm:112-132). */

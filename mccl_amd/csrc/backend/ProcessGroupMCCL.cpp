@@ -247,10 +247,6 @@ struct ProcessGroupMCCL::Shared : std::enable_shared_from_this<ProcessGroupMCCL:
         if (completer) completer->shutdown();  // settles what is still in flight
         workspace_pool.clear();
         drop_graphs();
-        if (drain_word.host && ctx) {
-            (void)mcclx_queue_drain(ctx);  // the last copy into the word has landed
-            (void)mcclx_host_free(ctx, drain_word.host);
-        }
         if (alt) mcclx_destroy(alt);
         if (ctx) mcclx_destroy(ctx);
     }
@@ -468,72 +464,18 @@ struct ProcessGroupMCCL::Shared : std::enable_shared_from_this<ProcessGroupMCCL:
         check_rc(mcclx_set_hold(ctx, 1));
     }
 
-    // The drain of a synchronous allreduce.  hipStreamSynchronize hands the host back 9-10 us
-    // after the launch's last wave has gone (the completion signal's way through the runtime);
-    // a 4-byte copy queued behind the launch that writes a number into pinned host memory,
-    // and a host that watches that word, gets there 4 us sooner (a 26 us launch: 36.2 -> 32.2 us
-    // from launch call to return).  The copy is issued while the launch runs, so its own launch
-    // cost is hidden.  The word only says that the queue has got that far: the results are in
-    // device memory, where the ranks' next kernels (launched after this returns) find them,
-    // exactly as after the blocking drain.  If the word has not come after MCCL_DRAIN_SPIN_US
-    // (default 1000; 0 = always the blocking drain) the blocking drain takes over, which is also
-    // what reports a launch that failed.  Caller is the last arrival of a collective (one at a time).
-    struct DrainWord {
-        void* host = nullptr;       // pinned: the word at offset 0, the numbers 1..kNumbers from offset 1024 on
-        void* alias = nullptr;      // the same memory as the device addresses it
-        at::Tensor numbers;         // the numbers again, in device memory (the copy's source)
-        uint32_t next = 0;
-        long spin_us = -1;
-        static constexpr uint32_t kNumbers = 512;
-    } drain_word;
+    // The drain of a synchronous allreduce: its tensors are device memory, so the host need not wait
+    // for the queue's completion signal (a 26 us launch: 36.2 -> 32.2 us from launch call to return).
+    // If the queue's end is not seen within MCCL_DRAIN_SPIN_US (default 1000; 0 = always the blocking
+    // drain) the blocking drain takes over.  Caller is the last arrival of a collective (one at a time).
+    long drain_spin_us = -1;
     void drain_main() {
-#ifdef MCCL_NULL_DEVICE
-        check_rc(mcclx_queue_drain(ctx));  // (the host stand-in of the queue has no device to write the word)
-#else
-        DrainWord& w = drain_word;
-        if (w.spin_us < 0) {
+        if (drain_spin_us < 0) {
             const char* e = std::getenv("MCCL_DRAIN_SPIN_US");
-            w.spin_us = e ? std::strtol(e, nullptr, 10) : 1000;
-            if (w.spin_us < 0) w.spin_us = 0;
-            if (w.spin_us > 0) {
-                try {
-                    check_rc(mcclx_host_alloc(ctx, 4096, &w.host, &w.alias));
-                    auto* h = static_cast<uint32_t*>(w.host);
-                    h[0] = 0;
-                    for (uint32_t i = 0; i < DrainWord::kNumbers; ++i) h[256 + i] = i + 1;
-                    w.numbers = dev::empty_bytes(4 * DrainWord::kNumbers, device);
-                    order_after_allocator(ctx, device);
-                    check_rc(mcclx_copy(ctx, w.numbers.data_ptr(), static_cast<char*>(w.alias) + 1024, 4 * DrainWord::kNumbers));
-                    check_rc(mcclx_queue_drain(ctx));
-                } catch (const std::exception& e) {  // no pinned memory to be had: the blocking drain serves
-                    MCCL_WARN("the synchronous allreduce keeps the blocking drain: %s", e.what());
-                    if (w.host) (void)mcclx_host_free(ctx, w.host);
-                    w.host = w.alias = nullptr;
-                    w.numbers = at::Tensor();
-                    w.spin_us = 0;
-                }
-            }
+            const long v = e ? std::strtol(e, nullptr, 10) : 1000;
+            drain_spin_us = v < 0 ? 0 : v > 1000000 ? 1000000 : v;
         }
-        if (w.spin_us == 0) {
-            check_rc(mcclx_queue_drain(ctx));
-            return;
-        }
-        const uint32_t i = w.next++ % DrainWord::kNumbers;
-        check_rc(mcclx_copy(ctx, w.alias, static_cast<char*>(w.numbers.data_ptr()) + 4 * i, 4));
-        const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(w.spin_us);
-        const volatile uint32_t* word = static_cast<const volatile uint32_t*>(w.host);
-        for (;;) {
-            for (int k = 0; k < 64; ++k) {
-                if (*word == i + 1) {
-                    std::atomic_thread_fence(std::memory_order_acquire);
-                    return;
-                }
-                __builtin_ia32_pause();
-            }
-            if (std::chrono::steady_clock::now() >= until) break;
-        }
-        check_rc(mcclx_queue_drain(ctx));
-#endif
+        check_rc(mcclx_queue_wait(ctx, static_cast<uint32_t>(drain_spin_us)));
     }
 
     // Host-blocking: nothing of the event-based mode is left on the device.

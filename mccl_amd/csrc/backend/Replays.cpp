@@ -66,6 +66,8 @@ bool read_group(PyObject* tensors, const How& how, mcclx_replay* r, std::vector<
     return true;
 }
 
+constexpr uint32_t kWaitSpinUs = 1000;
+
 uint64_t aligned(uint64_t n) { return (n + 255) / 256 * 256; }
 
 // Orders the queue behind torch's current stream, issues the replays in a workspace of
@@ -89,8 +91,9 @@ int run(mcclx_ctx* ctx, int device, std::vector<mcclx_replay>& reps) {
     py::gil_scoped_release unlocked;
     int rc = mcclx_queue_wait_stream(ctx, stream);
     if (rc == MCCLX_OK) rc = mcclx_allreduce_replay_many(ctx, reps.data(), static_cast<uint32_t>(reps.size()));
-    const int drained = mcclx_queue_drain(ctx);  // in any case: the workspace goes back to the allocator
-    return rc == MCCLX_OK ? drained : rc;
+    // in any case: the workspace goes back to the allocator.  (Tensors and workspace are device memory.)
+    const int waited = mcclx_queue_wait(ctx, kWaitSpinUs);
+    return rc == MCCLX_OK ? waited : rc;
 }
 
 py::object replay_many(uintptr_t ctx, int device, py::handle groups, int op, int algo, bool wire, int mode, int acc) {

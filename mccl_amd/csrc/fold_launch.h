@@ -177,6 +177,9 @@ hipError_t launch_copy_many(hipStream_t st, const CopyTable& t, int most, uint32
 // the memory counters): dst <- src, nbytes.
 hipError_t launch_copy(hipStream_t st, void* dst, const void* src, uint64_t nbytes);
 
+// Behind everything on the stream: *word = number, in pinned host memory (`word` as the device addresses it).
+hipError_t launch_word(hipStream_t st, uint64_t* word, uint64_t number);
+
 // Reads (write == false) or writes nbytes of `buf` once, one 16-byte packet per
 // lane like the copy kernel: the one-directional ceilings of a launch of that size.
 hipError_t launch_stream_probe(hipStream_t st, void* buf, uint64_t nbytes, bool write);

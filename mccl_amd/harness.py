@@ -220,7 +220,7 @@ def reduce_scatter_replay(outs: List[torch.Tensor], ins: List[torch.Tensor], op=
         q.handle, world, _ptr_array([o.data_ptr() for o in outs]),
         _ptr_array([i.data_ptr() for i in ins]), dtype_code(outs[0]), outs[0].numel(), op_code(op),
         mode, acc))
-    q.drain()
+    q.wait_results()
 
 
 def allgather_replay(outs: List[torch.Tensor], ins: List[torch.Tensor], queue=None) -> None:
@@ -237,4 +237,4 @@ def allgather_replay(outs: List[torch.Tensor], ins: List[torch.Tensor], queue=No
     L.check(L.lib().mcclx_allgather_replay(
         q.handle, world, _ptr_array([o.data_ptr() for o in outs]),
         _ptr_array([i.data_ptr() for i in ins]), chunk))
-    q.drain()
+    q.wait_results()

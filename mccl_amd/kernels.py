@@ -109,6 +109,10 @@ class ReduceQueue:
         """mccl_queue_drain (MPSInterop.mm:312-318)."""
         L.check(L.lib().mcclx_queue_drain(self.handle))
 
+    def wait_results(self) -> None:
+        """The same for results in device memory, sooner (mcclx_queue_wait)."""
+        L.check(L.lib().mcclx_queue_wait(self.handle, 1000))
+
     def wait_torch_stream(self, stream: Optional[torch.cuda.Stream] = None) -> None:
         """Device-side replacement of mps_stream_sync (MPSInterop.mm:308-310)."""
         s = stream or torch.cuda.current_stream(self.device)

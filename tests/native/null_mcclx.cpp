@@ -283,6 +283,7 @@ int mcclx_queue_drain(mcclx_ctx* c) {
     c->marker()->wait();
     return MCCLX_OK;
 }
+int mcclx_queue_wait(mcclx_ctx* c, uint32_t) { return mcclx_queue_drain(c); }
 int mcclx_queue_wait_stream(mcclx_ctx* c, void* producer) {
     mcclx_ctx* p = nullptr;
     if (!producer || producer == c || !known_stream(producer, &p)) return MCCLX_OK;  // the null stream: host code, already done
