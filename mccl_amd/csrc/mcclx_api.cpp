@@ -111,6 +111,12 @@ struct mcclx_ctx {
     // Operations enqueued on the queue, and how many of them are known to have finished (counted while
     // away_mu is held).  Equal: the queue is idle, and nothing has to be asked of the runtime.
     std::atomic<uint64_t> issued{0}, finished{0};
+    std::atomic<uint64_t> marked{0};  // `issued` when an event was last recorded on the queue
+    // The stream that was last asked whether it is idle and was not, and for how many further waits it
+    // is taken to be busy without being asked (under mu).  A hint: a wait is right either way.
+    hipStream_t busy_stream = nullptr;
+    int busy_for = 0;
+    std::atomic<bool> host_caught_up{false};  // the queue has been drained since
     // mcclx_queue_wait: the last number the device has written, in pinned host memory
     uint64_t* word = nullptr;
     uint64_t* word_dev = nullptr;  // the same memory as the device addresses it
@@ -173,9 +179,15 @@ QueueUse queue_of(mcclx_ctx* ctx) {
 }
 
 // Is nothing in flight on the queue?  Not asked of the runtime where the library has seen the end
-// of what it enqueued, which is most of the time after a mcclx_queue_wait.
+// of what it enqueued, nor where a kernel is the newest of it: a stream whose last operation carries no
+// event answers "busy" however long ago that ended, after 16-22 us in which the runtime puts
+// one there (0.1 us where there is one).
 bool queue_idle(mcclx_ctx* ctx) {
-    if (!ctx->exposed.load() && ctx->issued.load(std::memory_order_acquire) == ctx->finished.load(std::memory_order_acquire)) return true;
+    if (!ctx->exposed.load()) {
+        const uint64_t issued = ctx->issued.load(std::memory_order_acquire);
+        if (issued == ctx->finished.load(std::memory_order_acquire)) return true;
+        if (issued != ctx->marked.load(std::memory_order_acquire)) return false;
+    }
     if (hipStreamQuery(ctx->stream) == hipSuccess) return true;
     (void)hipGetLastError();  // hipErrorNotReady, or a state that what follows reports properly
     return false;
@@ -210,7 +222,10 @@ hipError_t drain(mcclx_ctx* ctx) {
         if (ctx->away_number == number) ctx->away.store(false, std::memory_order_release);
     }
     const hipError_t e = hipStreamSynchronize(ctx->stream);
-    if (e == hipSuccess) note_finished(ctx, upto);
+    if (e == hipSuccess) {
+        note_finished(ctx, upto);
+        ctx->host_caught_up.store(true, std::memory_order_relaxed);
+    }
     return e;
 }
 
@@ -1343,7 +1358,10 @@ int mcclx_queue_wait(mcclx_ctx* ctx, uint32_t spin_us) {
             // its own, 6 us sooner if one is under way already.  Calls in quick succession leave it out:
             // it would be in front of the next launch (metrics of 4 KB, back to back, 11.5 -> 12..16.5 us).
             const auto now = std::chrono::steady_clock::now();
-            if (now - ctx->last_wait > std::chrono::microseconds(200)) HIP_TRY(hipEventRecord(ctx->word_ev, use));
+            if (now - ctx->last_wait > std::chrono::microseconds(200)) {
+                HIP_TRY(hipEventRecord(ctx->word_ev, use));
+                ctx->marked.store(upto, std::memory_order_release);
+            }
             ctx->last_wait = now;
         }
         const volatile uint64_t* word = ctx->word;
@@ -1353,6 +1371,7 @@ int mcclx_queue_wait(mcclx_ctx* ctx, uint32_t spin_us) {
                 if (*word >= number) {  // numbers are written in the order they are handed out
                     std::atomic_thread_fence(std::memory_order_acquire);
                     note_finished(ctx, upto);
+                    ctx->host_caught_up.store(true, std::memory_order_relaxed);
                     return MCCLX_OK;
                 }
                 __builtin_ia32_pause();
@@ -1369,18 +1388,33 @@ static int stream_wait(mcclx_ctx* ctx, hipStream_t waiter, hipStream_t producer)
     DeviceGuard guard(ctx->device);
     // A producer that has nothing in flight needs no event: everything enqueued on it so far is
     // complete, which is all the wait would establish (an event record plus a stream wait cost
-    // the host 10-20 us on torch's legacy stream, a query a fraction of that).
-    if (producer == ctx->stream) {
-        if (queue_idle(ctx)) return MCCLX_OK;
-    } else {
-        if (hipStreamQuery(producer) == hipSuccess) return MCCLX_OK;
-        (void)hipGetLastError();  // hipErrorNotReady, or a state the record below reports properly
-    }
+    // the host 10-20 us on torch's legacy stream, a query of an idle stream 0.1 us).  The query costs as
+    // much where the newest operation is a kernel (queue_idle), and a caller that runs ahead of the device
+    // finds the stream busy every time: one that was is not asked again for the next seven waits,
+    // unless the host has caught up with the queue in between (the two orderings around a fold of 12 us,
+    // back to back: 44.6 us a pass with both queries, 33.4 with neither).
+    if (producer == ctx->stream && queue_idle(ctx)) return MCCLX_OK;
     std::lock_guard<std::mutex> lk(ctx->mu);
+    if (producer != ctx->stream) {
+        if (ctx->host_caught_up.exchange(false, std::memory_order_relaxed)) ctx->busy_for = 0;
+        if (ctx->busy_for > 0 && ctx->busy_stream == producer) {
+            --ctx->busy_for;
+        } else {
+            if (hipStreamQuery(producer) == hipSuccess) return MCCLX_OK;
+            (void)hipGetLastError();  // hipErrorNotReady, or a state the record below reports properly
+            ctx->busy_stream = producer;
+            ctx->busy_for = 7;
+        }
+    }
     hipEvent_t& ev = ctx->xev[ctx->xnext];
     ctx->xnext = (ctx->xnext + 1) % 16;
     if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    HIP_TRY(hipEventRecord(ev, producer));
+    {
+        std::unique_lock<std::mutex> use(ctx->away_mu, std::defer_lock);
+        if (producer == ctx->stream) use.lock();
+        HIP_TRY(hipEventRecord(ev, producer));
+        if (producer == ctx->stream) ctx->marked.store(ctx->issued.load(std::memory_order_relaxed), std::memory_order_release);
+    }
     std::unique_lock<std::mutex> use(ctx->away_mu, std::defer_lock);
     if (waiter == ctx->stream) {  // (the wait is an operation on the queue like any other: queue_idle)
         use.lock();
@@ -1425,7 +1459,11 @@ int mcclx_event_record(mcclx_ctx* ctx, uint64_t* ticket) {
     std::lock_guard<std::mutex> lk(ctx->mu);
     hipEvent_t ev;
     if (int rc = get_event(ctx, &ev)) return rc;
-    HIP_TRY(hipEventRecord(ev, queue_of(ctx)));
+    {
+        QueueUse use = queue_of(ctx);
+        HIP_TRY(hipEventRecord(ev, use));
+        ctx->marked.store(ctx->issued.load(std::memory_order_relaxed), std::memory_order_release);
+    }
     *ticket = ctx->next_ticket++;
     ctx->tickets[*ticket].ev = ev;
     return MCCLX_OK;

@@ -118,3 +118,35 @@ def test_refused_while_recording_and_usable_after(env):
 def test_without_a_context(env):
     L, _ = env
     assert L.lib().mcclx_queue_wait(C.c_void_p(None), 1000) == L.ERR_STATE
+
+
+@pytest.mark.parametrize("streams", [1, 2])
+@pytest.mark.parametrize("drain_every", [0, 5])
+def test_every_wait_holds_whether_or_not_the_stream_was_asked(env, streams, drain_every):
+    """Waits for a stream that was busy are not preceded by a query for a while: in a run of them, with
+    the host catching up in between or not, each orders the queue behind what the stream was given last."""
+    _, K = env
+    q = K.ReduceQueue(0)
+    sides = [torch.cuda.Stream() for _ in range(streams)]
+    n = 200_003
+    xs = [torch.zeros(n, device="cuda") for _ in range(24)]
+    seen = [torch.zeros(n, device="cuda") for _ in range(24)]
+    torch.cuda.synchronize()
+    try:
+        for i, (x, y) in enumerate(zip(xs, seen)):
+            side = sides[i % streams]
+            with torch.cuda.stream(side):
+                torch.cuda._sleep(200_000)
+                x.fill_(i + 1)
+            q.wait_torch_stream(side)
+            q.copy(y.data_ptr(), x.data_ptr(), 4 * n)
+            q.torch_stream_wait(side)   # the queue's newest operation is a kernel: not asked either
+            with torch.cuda.stream(side):
+                y.mul_(2)
+            if drain_every and i % drain_every == drain_every - 1:
+                q.wait_results()
+        torch.cuda.synchronize()
+        for i, y in enumerate(seen):
+            assert y.cpu().eq(2 * (i + 1)).all(), i
+    finally:
+        q.close()
