@@ -682,6 +682,13 @@ private:
     mcclx::Spans spans_;
 };
 
+// Preparing an entry of a list takes the host some 50 ns (its descriptor, checks, the table), what
+// the device needs for an entry of more than 100 KB moved.  So a list is not prepared whole: every
+// kPieceEntries entries go out as a run of their own while the next are prepared, if they keep the
+// device busy for longer than the two launches of a run (table and fold) cost.
+constexpr long kPieceEntries = 512;
+constexpr uint64_t kPieceBytes = 64'000'000;
+
 // Same plan for every phase?
 bool same_plan(const mcclx_replay* a, const mcclx_replay* b) {
     return a->world == b->world && a->algo == b->algo && a->op == b->op && a->dtype == b->dtype &&
@@ -761,14 +768,18 @@ int mcclx_allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t
         Phases ph;
         const mcclx_replay* first = &rs[i];
         Touched touched;
+        uint64_t moved = 0;  // bytes the run reads and writes, at least
         while (i < n) {
             if (&rs[i] != first) {
+                // a long list goes out in pieces: see kPieceEntries
+                if (&rs[i] - first >= kPieceEntries && moved >= kPieceBytes) break;
                 if (!same_plan(first, &rs[i])) break;
                 TRY(check_replay(ctx, &rs[i], &fused, &nothing));
                 if (!fused || nothing) break;
             }
             if (!touched.add(&rs[i])) break;
             collect_fused(&rs[i], layout_of(&rs[i]), ph);
+            moved += 2 * (uint64_t)rs[i].world * rs[i].numel * esize(rs[i].dtype);
             ++i;
         }
         if (first->mode == MCCLX_REPLAY_FUSED && first->algo != MCCLX_ALGO_TREE && ph.fan && !ph.enc_segs.empty()) {
