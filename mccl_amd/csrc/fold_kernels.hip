@@ -41,7 +41,7 @@ namespace mcclx {
 namespace {
 
 // Launch shapes, each measured on MI355X.  By-value launches run one-wavefront blocks of one
-// packet per lane (Cfg::FEW_U, kSmallShape): a block of eight wavefronts keeps its slots until
+// packet per lane (Cfg::FEW_U, kSmallShape, four_waves): a block of eight wavefronts keeps its slots until
 // the last of its loads is back, one-wavefront blocks turn them over one by one (operands of
 // 128-512 MiB: one fp32 operand scaled 84.5 -> 80.9 us, own fp32 + one bf16 peer 106 -> 99.6,
 // + two peers 124 -> 119.5, copy 82.6 -> 80.6; 25 MiB operands: 10.3 -> 9.5, 12.5 -> 11.4,
@@ -229,6 +229,18 @@ struct Cfg {
             if (K > 1 && W != MCCLX_F32 && IO != MCCLX_IO_PURE && !in_is_f32(k)) return k;
         return -1;
     }();
+    // Bytes under way per CU that a large launch is held to (resident_lds).  The longer a wave computes
+    // between its loads and its stores, the more waves it takes to keep as many under way: bf16 rounds
+    // after every operand, fp16 in one instruction, the wire form once more on the way in, fp32 never.
+    // Eight ranks in place, 3 / 4 / 5 waves per CU (us): bf16 12.5 M 80.5 / 71.3 / 67.8, fp16 50 M 249 / 252 /
+    // 263, the wire form 8 M 86.8 / 80.9 / 83.4, fp32 40 M 407 / 414 / 425; five ranks of 40 M, 5 / 6 / 7 / 8:
+    // the wire form 261 / 249 / 249 / 251, fp32 246 / 250 / 252 / 254.
+    static constexpr int kInPlaceBudget = W == MCCLX_F32 ? (K >= 5 ? 800 : kLaneBytesInPlace)
+                                          : W == MCCLX_F16 ? 1024
+                                          : IO == MCCLX_IO_ALL_F32 ? 1130 : kLaneBytesInPlace;
+    // (fan-out of 100 M elements, 7 / 8 / 9 / 10 / 12 waves: four ranks over the wire form 496 / 496 / 504 / 513 / 511,
+    // three 398 / 378 / 367 / 367 / 375, four of bf16 268 / 251 / 246 / 248 / 257)
+    static constexpr int kFanBudget = (W == MCCLX_F32 || IO == MCCLX_IO_ALL_F32) ? 1024 : kLaneBytes;
     // bytes a lane reads per packet
     static constexpr int kReadBytes = [] {
         int b = 0;
@@ -975,6 +987,19 @@ static bool off_lines(const FewArgs& a) {
     return false;
 }
 
+// Blocks of four wavefronts for a by-value launch of `waves` one-wavefront tiles whose streams share one
+// element size?  Such launches take one-wavefront blocks (C::BLOCK) because those turn their slots over
+// one by one; one that one generation of waves covers turns nothing over, and four waves of a block spread over a
+// CU's four SIMDs where blocks of one pile up on some.  Cold, blocks of one and of four (us): 8 ranks of
+// 1 M bf16 in place (1950 waves) 9.3 and 7.8, of 0.5 M fp32 9.1 and 7.6, eight bf16 operands into one (4000)
+// 9.0 and 8.0, (6000) 11.6 and 10.8; two operands into one (5000) 4.6 and 4.1, two ranks in place (5500) 5.7 and
+// 5.0; four ranks (1400) 4.5 and 4.1, (5000) 9.2 and 8.9.  In between and above, blocks of one again: three or four
+// ranks (2500) 5.5 and 5.7, eight (8000) 26.4 and 27.8, two operands into one (12000) 7.7 and 8.1.
+static bool four_waves(uint64_t waves, int k) {
+    if (k >= 5) return waves >= 480 && waves < 6144;
+    return (waves >= 960 && waves < 2048) || (waves >= 4608 && waves < (k == 2 ? 7680u : 6144u));
+}
+
 // A by-value launch: one block per tile of the longest segment, the hold form where it applies.
 template <class C, int OUT>
 static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchParams& lp) {
@@ -994,7 +1019,7 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
     const int outputs = OUT == kOutAll ? C::K : 1 + a.fan;
     const int lane_bytes = C::FEW_U * (C::kReadBytes + outputs * ((C::W == MCCLX_F32 || C::kOutF32) ? 16 : 2 * C::E));
     const uint32_t lds = resident_lds(total / lane_elems * (uint64_t)lane_bytes, lane_bytes, outputs,
-                                      OUT == kOutAll ? kLaneBytesInPlace : kLaneBytes);
+                                      OUT == kOutAll ? C::kInPlaceBudget : OUT == kOutFan ? C::kFanBudget : kLaneBytes);
     auto go = [&](auto block, auto packets, uint32_t reserve) -> hipError_t {
         constexpr int B = decltype(block)::value, U = decltype(packets)::value;
         constexpr uint64_t span = (uint64_t)B * U * C::E;
@@ -1015,12 +1040,14 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
         return hipGetLastError();
     };
     using Few = std::integral_constant<int, C::FEW_U>;
+    const uint64_t waves = (maxc + 64 * lane_elems - 1) / (64 * lane_elems) * (uint64_t)a.nseg;
     if constexpr (C::kSmallShape) {
-        const uint64_t waves = (maxc + 64 * lane_elems - 1) / (64 * lane_elems);
-        if (waves * (uint64_t)a.nseg < C::kOneWaveFrom) return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
+        if (waves < C::kOneWaveFrom) return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
         if constexpr (C::BLOCK == kBlock)
             if (off_lines<C, OUT>(a))
                 return go(std::integral_constant<int, kBlock>{}, std::integral_constant<int, C::U>{}, 0);
+    } else if (four_waves(waves, C::K)) {
+        return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
     }
     return go(std::integral_constant<int, kOneWave>{}, Few{}, lds);
 }

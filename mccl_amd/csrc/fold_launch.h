@@ -120,8 +120,7 @@ hipError_t launch_fold(hipStream_t st, const PlanKey& key, const LaunchParams& l
 // bytes for every shape, waves x bytes a lane moves: 1160 (8 operands into one: 8 waves;
 // 4 into one: 14; 3 into one: 18), a little less where one source is copied to several
 // destinations (4 / 6 / 8: 12 / 9 / 7 waves, 33 M elements to four 214 -> 206 us against 14)
-// and a little more where tensors are reduced in place (2 / 3 / 4 / 5 / 8 ranks: 18 / 12 /
-// 8-10 / 8 / 5 waves).  A reservation of LDS nobody uses
+// and a little more or less where tensors are reduced in place or to several (Cfg::kInPlaceBudget, kFanBudget).  A reservation of LDS nobody uses
 // sets the number: it is granted in units of 1280 bytes of a CU's 160 KiB.
 //
 // A launch that ends soon needs its waves to get going: the limit pays from 160 MB moved on
