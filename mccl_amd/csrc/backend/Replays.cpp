@@ -74,9 +74,12 @@ uint64_t aligned(uint64_t n) { return (n + 255) / 256 * 256; }
 // their own and waits for them.
 int run(mcclx_ctx* ctx, int device, std::vector<mcclx_replay>& reps) {
     uint64_t total = 0;
-    for (mcclx_replay& r : reps) {
-        r.workspace_bytes = aligned(mcclx_replay_workspace_bytes(&r));
+    const mcclx_replay* before = nullptr;
+    for (mcclx_replay& r : reps) {  // (operation, algorithm, mode and wire form are the call's)
+        const bool alike = before && r.world == before->world && r.dtype == before->dtype && r.numel == before->numel;
+        r.workspace_bytes = alike ? before->workspace_bytes : aligned(mcclx_replay_workspace_bytes(&r));
         total += r.workspace_bytes;
+        before = &r;
     }
     at::Tensor ws;
     if (total) {

@@ -492,27 +492,22 @@ int ensure_slot(mcclx_ctx* ctx, TableSlot& sl, size_t need) {
 
 // Puts a descriptor table where a kernel can read it (caller holds ctx->mu).
 // Outside a recording: the next slot of the pinned staging ring, copied to its
-// device twin on the queue (`*slot` names it) by a launch that reads it over the link: 360 KB
+// device twin on the queue by a launch that reads it over the link: 360 KB
 // are there 14 us sooner than from a copy engine, whose hand-over to the launch behind it costs more
 // than the bytes do.  While recording: the launch needs a table that outlives this
 // call, so it gets its own device buffer, filled now with a blocking copy
-// (outside the recording) and owned by the graph; `*slot` stays null.
-int stage_table(mcclx_ctx* ctx, const void* bytes, size_t nbytes, void** dev, TableSlot** slot) {
-    *slot = nullptr;
+// (outside the recording) and owned by the graph.
+// The caller writes the table where stage_room says (nowhere else first: a list's is hundreds of KB)
+// and uploads it with stage_upload.
+struct Staged {
+    char* host = nullptr;
+    TableSlot* slot = nullptr;
+    std::vector<char> own;  // while recording
+};
+int stage_room(mcclx_ctx* ctx, size_t nbytes, Staged* s) {
     if (ctx->capturing) {
-        void* d = nullptr;
-        HIP_TRY(hipMalloc(&d, nbytes));
-        // not the legacy stream: that one may not be touched while another stream records
-        if (!ctx->upload_stream)
-            HIP_TRY(hipStreamCreateWithFlags(&ctx->upload_stream, hipStreamNonBlocking));
-        hipError_t ce = hipMemcpyAsync(d, bytes, nbytes, hipMemcpyHostToDevice, ctx->upload_stream);
-        if (ce == hipSuccess) ce = hipStreamSynchronize(ctx->upload_stream);
-        if (ce != hipSuccess) {
-            (void)hipFree(d);
-            return fail(MCCLX_ERR_HIP, "table upload failed: %s", hipGetErrorString(ce));
-        }
-        ctx->capture_tables.push_back(d);
-        *dev = d;
+        s->own.resize(nbytes);
+        s->host = s->own.data();
         return MCCLX_OK;
     }
     // The queue may be a stream the caller owns (mcclx_init_on_stream) and is recording
@@ -528,7 +523,28 @@ int stage_table(mcclx_ctx* ctx, const void* bytes, size_t nbytes, void** dev, Ta
     TableSlot& sl = ctx->slots[ctx->next_slot];
     ctx->next_slot = (ctx->next_slot + 1) % kTableSlots;
     if (int rc = ensure_slot(ctx, sl, nbytes)) return rc;
-    memcpy(sl.host, bytes, nbytes);
+    s->host = static_cast<char*>(sl.host);
+    s->slot = &sl;
+    return MCCLX_OK;
+}
+int stage_upload(mcclx_ctx* ctx, Staged* s, size_t nbytes, void** dev) {
+    if (!s->slot) {
+        void* d = nullptr;
+        HIP_TRY(hipMalloc(&d, nbytes));
+        // not the legacy stream: that one may not be touched while another stream records
+        if (!ctx->upload_stream)
+            HIP_TRY(hipStreamCreateWithFlags(&ctx->upload_stream, hipStreamNonBlocking));
+        hipError_t ce = hipMemcpyAsync(d, s->host, nbytes, hipMemcpyHostToDevice, ctx->upload_stream);
+        if (ce == hipSuccess) ce = hipStreamSynchronize(ctx->upload_stream);
+        if (ce != hipSuccess) {
+            (void)hipFree(d);
+            return fail(MCCLX_ERR_HIP, "table upload failed: %s", hipGetErrorString(ce));
+        }
+        ctx->capture_tables.push_back(d);
+        *dev = d;
+        return MCCLX_OK;
+    }
+    TableSlot& sl = *s->slot;
     {
         QueueUse use = queue_of(ctx);
         sl.upto = ctx->issued.load(std::memory_order_relaxed);
@@ -540,7 +556,6 @@ int stage_table(mcclx_ctx* ctx, const void* bytes, size_t nbytes, void** dev, Ta
     HIP_TRY(hipEventRecord(sl.done, ctx->stream));
     sl.pending = true;
     *dev = sl.dev;
-    *slot = &sl;
     return MCCLX_OK;
 }
 
@@ -605,42 +620,48 @@ int fold_impl(mcclx_ctx* ctx, const mcclx_plan* plan, const mcclx_seg* segs, uin
     if (nseg <= ctx->few_max && even_enough(key, segs, nseg))
         return launch_by_value(ctx, key, scale_f, has_scale, segs, nseg, fan, queue_of(ctx));
 
-    // descriptor table: segs, then nseg+1 work-item prefix sums
+    // Descriptor table: segs; then, where a block cannot work out its segment by division, (segment, tile)
+    // per work item, so that it finds its work with one load instead of a binary search through
+    // device memory (measured on 4096 ragged messages: 3.9 -> 6.3 TB/s), or nseg+1 work-item prefix
+    // sums where there are too many items for that.
     std::lock_guard<std::mutex> lk(ctx->mu);
-    size_t seg_bytes = (size_t)nseg * sizeof(mcclx_seg);
-    size_t pre_bytes = ((size_t)nseg + 1) * sizeof(uint64_t);
-    std::vector<char> host(seg_bytes + pre_bytes);
-    memcpy(host.data(), segs, seg_bytes);
-    uint64_t* pre = reinterpret_cast<uint64_t*>(host.data() + seg_bytes);
+    const size_t seg_bytes = (size_t)nseg * sizeof(mcclx_seg);
     uint64_t total = 0, uniform = mcclx::items_for(key, segs[0].count);
+    uint64_t count = segs[0].count, items = uniform;  // of the segment before
+    auto items_of = [&](uint32_t s) {
+        if (segs[s].count != count) {
+            count = segs[s].count;
+            items = mcclx::items_for(key, count);
+        }
+        return items;
+    };
     for (uint32_t s = 0; s < nseg; ++s) {
-        pre[s] = total;
-        uint64_t n = mcclx::items_for(key, segs[s].count);
+        const uint64_t n = items_of(s);
         if (n != uniform) uniform = 0;
         total += n;
     }
-    pre[nseg] = total;
     if (total == 0) return MCCLX_OK;
     if (total >> 31) return fail(MCCLX_ERR_INVALID, "fold: more than 2^31 work items in one launch");
-    // Ragged segments: spell out (segment, tile) per work item, so that a block finds
-    // its work with one load instead of a binary search through device memory
-    // (measured on 4096 ragged messages: 3.9 -> 6.3 TB/s).
     const bool mapped = uniform == 0 && total <= kMaxMappedItems;
-    const size_t map_off = host.size();
+    const size_t nbytes = seg_bytes + (mapped ? (size_t)total * sizeof(uint2) : uniform ? 0 : ((size_t)nseg + 1) * sizeof(uint64_t));
+    Staged st;
+    if (int rc = stage_room(ctx, nbytes, &st)) return rc;
+    memcpy(st.host, segs, seg_bytes);
     if (mapped) {
-        host.resize(map_off + (size_t)total * sizeof(uint2));
-        pre = reinterpret_cast<uint64_t*>(host.data() + seg_bytes);
-        uint2* map = reinterpret_cast<uint2*>(host.data() + map_off);
+        uint2* map = reinterpret_cast<uint2*>(st.host + seg_bytes);
         for (uint32_t s = 0; s < nseg; ++s)
-            for (uint64_t w = pre[s]; w < pre[s + 1]; ++w) map[w] = make_uint2(s, (uint32_t)(w - pre[s]));
+            for (uint64_t n = items_of(s), w = 0; w < n; ++w) *map++ = make_uint2(s, (uint32_t)w);
+    } else if (!uniform) {
+        uint64_t* pre = reinterpret_cast<uint64_t*>(st.host + seg_bytes);
+        pre[0] = 0;
+        for (uint32_t s = 0; s < nseg; ++s) pre[s + 1] = pre[s] + items_of(s);
     }
     void* dev = nullptr;
-    TableSlot* slot = nullptr;
-    if (int rc = stage_table(ctx, host.data(), host.size(), &dev, &slot)) return rc;
+    if (int rc = stage_upload(ctx, &st, nbytes, &dev)) return rc;
     mcclx::TableArgs t;
     t.segs = static_cast<const mcclx::SegArgs*>(dev);
-    t.first_item = reinterpret_cast<const uint64_t*>(static_cast<char*>(dev) + seg_bytes);
-    t.item_map = mapped ? reinterpret_cast<const uint2*>(static_cast<char*>(dev) + map_off) : nullptr;
+    t.first_item = mapped || uniform ? nullptr : reinterpret_cast<const uint64_t*>(static_cast<char*>(dev) + seg_bytes);
+    t.item_map = mapped ? reinterpret_cast<const uint2*>(static_cast<char*>(dev) + seg_bytes) : nullptr;
     t.total_items = total;
     t.uniform_items = uniform;
     t.nseg = nseg;
@@ -1284,34 +1305,33 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
     }
     std::lock_guard<std::mutex> lk(ctx->mu);
     const size_t desc_bytes = (size_t)live * sizeof(mcclx::CopyDesc);
-    std::vector<char> host(desc_bytes + ((size_t)live + 1) * sizeof(uint64_t));
-    memcpy(host.data(), groups.data(), desc_bytes);
-    auto* pre = reinterpret_cast<uint64_t*>(host.data() + desc_bytes);
     uint64_t total = 0, uniform = mcclx::copy_items(groups[0].nbytes);
     for (uint32_t j = 0; j < live; ++j) {
-        pre[j] = total;
         const uint64_t items = mcclx::copy_items(groups[j].nbytes);
         if (items != uniform) uniform = 0;
         total += items;
     }
-    pre[live] = total;
     if (total >> 31) return fail(MCCLX_ERR_INVALID, "copy_batched: more than 2^31 work items in one launch");
     const bool mapped = uniform == 0 && total <= kMaxMappedItems;
-    const size_t map_off = host.size();
+    const size_t nbytes = desc_bytes + (mapped ? (size_t)total * sizeof(uint2) : uniform ? 0 : ((size_t)live + 1) * sizeof(uint64_t));
+    Staged st;
+    if (int rc = stage_room(ctx, nbytes, &st)) return rc;
+    memcpy(st.host, groups.data(), desc_bytes);
     if (mapped) {
-        host.resize(map_off + (size_t)total * sizeof(uint2));
-        pre = reinterpret_cast<uint64_t*>(host.data() + desc_bytes);
-        uint2* map = reinterpret_cast<uint2*>(host.data() + map_off);
+        uint2* map = reinterpret_cast<uint2*>(st.host + desc_bytes);
         for (uint32_t c = 0; c < live; ++c)
-            for (uint64_t w = pre[c]; w < pre[c + 1]; ++w) map[w] = make_uint2(c, (uint32_t)(w - pre[c]));
+            for (uint64_t n = mcclx::copy_items(groups[c].nbytes), w = 0; w < n; ++w) *map++ = make_uint2(c, (uint32_t)w);
+    } else if (!uniform) {
+        uint64_t* pre = reinterpret_cast<uint64_t*>(st.host + desc_bytes);
+        pre[0] = 0;
+        for (uint32_t c = 0; c < live; ++c) pre[c + 1] = pre[c] + mcclx::copy_items(groups[c].nbytes);
     }
     void* dev = nullptr;
-    TableSlot* slot = nullptr;
-    if (int rc = stage_table(ctx, host.data(), host.size(), &dev, &slot)) return rc;
+    if (int rc = stage_upload(ctx, &st, nbytes, &dev)) return rc;
     mcclx::CopyTable t;
     t.descs = static_cast<const mcclx::CopyDesc*>(dev);
-    t.first_item = reinterpret_cast<const uint64_t*>(static_cast<char*>(dev) + desc_bytes);
-    t.item_map = mapped ? reinterpret_cast<const uint2*>(static_cast<char*>(dev) + map_off) : nullptr;
+    t.first_item = mapped || uniform ? nullptr : reinterpret_cast<const uint64_t*>(static_cast<char*>(dev) + desc_bytes);
+    t.item_map = mapped ? reinterpret_cast<const uint2*>(static_cast<char*>(dev) + desc_bytes) : nullptr;
     t.total_items = (uint32_t)total;
     t.uniform_items = (uint32_t)uniform;
     t.n = live;

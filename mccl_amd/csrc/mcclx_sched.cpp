@@ -410,7 +410,7 @@ void collect_fused(const mcclx_replay* r, const Layout& L, Phases& ph) {
             }
             return;
         }
-        mcclx_seg s = z;
+        mcclx_seg& s = ph.folds[0].segs.emplace_back(z);
         s.count = r->numel;
         if (bf16_only) {
             s.out = wire_of(0);
@@ -425,7 +425,6 @@ void collect_fused(const mcclx_replay* r, const Layout& L, Phases& ph) {
                 s.wire_out = wire_of(0);
             }
         }
-        ph.folds[0].segs.push_back(s);
         if (ph.fan || ph.all) return;
         for (int q = bf16_only ? 0 : 1; q < N; ++q) {
             if (L.wire) {  // broadcast of the bf16 result + the final cast on every rank
@@ -620,8 +619,15 @@ int issue_phases(mcclx_ctx* ctx, Phases& ph) {
     return MCCLX_OK;
 }
 
+int check_memory(const mcclx_replay* r, const Layout& L) {
+    for (int i = 0; i < r->world; ++i)
+        if (!r->tensors[i]) return bad("replay: null tensor");
+    if (L.total > 0 && (!r->workspace || r->workspace_bytes < L.total)) return bad("workspace too small");
+    return MCCLX_OK;
+}
+
 // Argument checks of one replay; *fused says whether the fused schedule can run it.
-int check_replay(mcclx_ctx* ctx, const mcclx_replay* r, bool* fused, bool* nothing_to_do) {
+int check_replay(mcclx_ctx* ctx, const mcclx_replay* r, Layout* L, bool* fused, bool* nothing_to_do) {
     *fused = false;
     *nothing_to_do = false;
     if (!ctx || !r || !r->tensors) return bad("replay: null argument");
@@ -639,10 +645,8 @@ int check_replay(mcclx_ctx* ctx, const mcclx_replay* r, bool* fused, bool* nothi
     if (r->numel == 0) return bad("replay: empty tensor");  // TensorChecks.hpp:31-34
     // AllreduceAlgos.cpp:55,137
     if (r->algo != MCCLX_ALGO_TREE && r->numel < (uint64_t)r->world) return bad("numel must be >= world");
-    for (int i = 0; i < r->world; ++i)
-        if (!r->tensors[i]) return bad("replay: null tensor");
-    Layout L = layout_of(r);
-    if (L.total > 0 && (!r->workspace || r->workspace_bytes < L.total)) return bad("workspace too small");
+    *L = layout_of(r);
+    TRY(check_memory(r, *L));
     // the tree is fused as a tree of 8-rank trees: up to 8 x 8 ranks
     *fused = r->mode != MCCLX_REPLAY_STEPWISE &&
              (r->algo != MCCLX_ALGO_TREE || r->world <= MCCLX_MAX_INPUTS * MCCLX_MAX_INPUTS);
@@ -665,6 +669,18 @@ public:
     // Does the replay touch memory an earlier one has touched?  If not, its ranges are added.
     bool add(const mcclx_replay* r) {
         const uint64_t tb = r->numel * esize(r->dtype);
+        // The usual list: each rank's tensor begins where its last one ended.
+        if (!r->workspace_bytes && (int)last_.size() == r->world) {
+            int i = 0;
+            for (; i < r->world; ++i) {
+                const uintptr_t p = reinterpret_cast<uintptr_t>(r->tensors[i]);
+                if (!spans_.follows(last_[(size_t)i], p, p + tb)) break;
+            }
+            if (i == r->world) {
+                for (i = 0; i < r->world; ++i) mcclx::Spans::grow(last_[(size_t)i], reinterpret_cast<uintptr_t>(r->tensors[i]) + tb);
+                return true;
+            }
+        }
         auto each = [&](auto&& f) {
             for (int i = 0; i < r->world; ++i)
                 if (f(reinterpret_cast<uintptr_t>(r->tensors[i]), tb)) return true;
@@ -675,18 +691,22 @@ public:
             spans_.insert(p, p + n);  // (a rank's tensors of one replay may overlap each other)
             return false;
         });
+        last_.clear();
+        for (int i = 0; i < r->world; ++i) last_.push_back(spans_.cursor(reinterpret_cast<uintptr_t>(r->tensors[i])));
         return true;
     }
 
 private:
     mcclx::Spans spans_;
+    std::vector<mcclx::Spans::Cursor> last_;  // the intervals the last replay's tensors lie in
 };
 
-// Preparing an entry of a list takes the host some 50 ns (its descriptor, checks, the table), what
-// the device needs for an entry of more than 100 KB moved.  So a list is not prepared whole: every
-// kPieceEntries entries go out as a run of their own while the next are prepared, if they keep the
-// device busy for longer than the two launches of a run (table and fold) cost.
-constexpr long kPieceEntries = 512;
+// Preparing an entry of a list takes the host some 25 ns (its descriptor, checks, the table).  A long
+// list is not prepared whole: every kPieceEntries entries go out as a run of their own while the next
+// are prepared, if they keep the device busy meanwhile.  A further run costs 8 us (a table's way over the
+// link, two gaps between launches, a ramp): 4096 messages of 64 KiB, three ranks, in pieces of 512 / 1024 /
+// 2048 436 / 415 / 390 us, of 20 KB 262 / 237 / 215.
+constexpr long kPieceEntries = 2048;
 constexpr uint64_t kPieceBytes = 64'000'000;
 
 // Same plan for every phase?
@@ -750,7 +770,8 @@ int mcclx_allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t
     uint32_t i = 0;
     while (i < n) {
         bool fused, nothing;
-        TRY(check_replay(ctx, &rs[i], &fused, &nothing));
+        Layout L;
+        TRY(check_replay(ctx, &rs[i], &L, &fused, &nothing));
         if (nothing) {
             ++i;
             continue;
@@ -774,11 +795,18 @@ int mcclx_allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t
                 // a long list goes out in pieces: see kPieceEntries
                 if (&rs[i] - first >= kPieceEntries && moved >= kPieceBytes) break;
                 if (!same_plan(first, &rs[i])) break;
-                TRY(check_replay(ctx, &rs[i], &fused, &nothing));
-                if (!fused || nothing) break;
+                if (rs[i].tensors && rs[i].reserved == 0 && rs[i].numel == rs[i - 1].numel) {
+                    TRY(check_memory(&rs[i], L));  // all else is as in the entry before
+                } else {
+                    TRY(check_replay(ctx, &rs[i], &L, &fused, &nothing));
+                    if (!fused || nothing) break;
+                }
+            } else if (first->algo == MCCLX_ALGO_TREE) {
+                plan_phases(first, L, ph);
+                ph.folds[0].segs.reserve(n - i < (uint32_t)kPieceEntries ? n - i : (uint32_t)kPieceEntries);
             }
             if (!touched.add(&rs[i])) break;
-            collect_fused(&rs[i], layout_of(&rs[i]), ph);
+            collect_fused(&rs[i], L, ph);
             moved += 2 * (uint64_t)rs[i].world * rs[i].numel * esize(rs[i].dtype);
             ++i;
         }

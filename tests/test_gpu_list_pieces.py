@@ -1,4 +1,4 @@
-"""Lists of many large enough messages go out in pieces of 512, one run of launches each: results
+"""Lists of many large enough messages go out in pieces of 2048, one run of launches each: results
 and the order of entries that share tensors are those of the whole list."""
 import pytest
 import torch
@@ -22,11 +22,11 @@ def _average(ts):
 
 
 @pytest.mark.parametrize("messages,numel,world,launches", [
-    (511, 20_001, 2, 1),      # just below a piece
-    (512, 20_001, 2, 1),      # one piece, whole
-    (513, 20_001, 2, 2),      # and one entry left over
-    (1_300, 8_192, 3, 3),
-    (1_300, 64, 3, 1),        # too little to keep the device busy: one launch
+    (2_047, 4_001, 2, 1),     # just below a piece
+    (2_048, 4_001, 2, 1),     # one piece, whole
+    (2_049, 4_001, 2, 2),     # and one entry left over
+    (5_000, 2_731, 3, 3),
+    (5_000, 64, 3, 1),        # too little to keep the device busy: one launch
 ])
 def test_pieces_of_a_list(env, messages, numel, world, launches):
     L, H, K = env
@@ -46,11 +46,11 @@ def test_pieces_of_a_list(env, messages, numel, world, launches):
 
 def test_an_entry_named_in_two_pieces_and_twice_in_one(env):
     L, H, K = env
-    n, messages, world = 20_000, 1_100, 2
+    n, messages, world = 5_000, 4_200, 2
     g = torch.Generator(device="cuda").manual_seed(6)
     ts = [[torch.randn(n, generator=g, device="cuda") for _ in range(world)] for _ in range(messages)]
-    order = list(range(messages)) + [3, 700, 700]
-    order.insert(600, 5)
+    order = list(range(messages)) + [3, 2_700, 2_700]
+    order.insert(2_500, 5)
     state = [[t.cpu() for t in pair] for pair in ts]
     for i in order:
         mean = _average(state[i])
@@ -82,3 +82,24 @@ def test_more_table_launches_than_staging_slots_without_a_drain(env):
         assert torch.equal(y, torch.ones_like(y))
     finally:
         q.close()
+
+
+@pytest.mark.parametrize("layout", ["in_order", "reversed", "interleaved", "scattered"])
+def test_entries_of_any_layout_and_one_that_overlaps(env, layout):
+    """What a run has touched is kept as intervals that usually just grow: lists whose tensors lie the other
+    way round, rank by rank in one buffer, or anywhere, and an entry that shares half of an earlier one's tensor."""
+    L, H, _ = env
+    n, messages, world = 1_000, 700, 3
+    g = torch.Generator(device="cuda").manual_seed(7)
+    buf = torch.randint(-50, 50, (messages * world * n,), generator=g, device="cuda").float()
+    at = {"in_order": lambda i, r: r * messages + i, "reversed": lambda i, r: r * messages + messages - 1 - i,
+          "interleaved": lambda i, r: i * world + r, "scattered": lambda i, r: (i * 389 + 7) % messages * world + r}[layout]
+    starts = [[at(i, r) * n for r in range(world)] for i in range(messages)]
+    starts.append([starts[400][0], starts[10][1] + n // 2, starts[20][2]])  # half of an earlier tensor, half of its neighbour
+    host = buf.cpu()
+    for s in starts:
+        total = sum(host[a:a + n].clone() for a in s)
+        for a in s:
+            host[a:a + n] = total
+    H.allreduce_replay_many([[buf[a:a + n] for a in s] for s in starts], "sum", L.ALGO_TREE)
+    assert torch.equal(buf.cpu(), host)
