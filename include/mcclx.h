@@ -418,6 +418,10 @@ MCCLX_API int mcclx_allreduce_replay(mcclx_ctx* ctx, const mcclx_replay* r);
  * become a handful of launches.  Results are those of n single replays. */
 MCCLX_API int mcclx_allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* replays, uint32_t n);
 
+/* mcclx_allreduce_replay_many and mcclx_queue_wait in one call: a last launch of few blocks writes the
+ * word itself.  The call waits whatever the replays return, which is what it returns. */
+MCCLX_API int mcclx_allreduce_replay_wait(mcclx_ctx* ctx, const mcclx_replay* replays, uint32_t n, uint32_t spin_us);
+
 /* _reduce_scatter_base (ProcessGroupMCCL.cpp:331-390): ins[r] holds
  * world*chunk_numel elements, outs[r] receives chunk_numel.  FUSED: one
  * k=world fold per rank in one batched launch. */

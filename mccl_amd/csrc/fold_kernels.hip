@@ -59,6 +59,7 @@ constexpr int kWideMinK = 2;   // all-16-bit folds of this many operands or more
 constexpr int kF32Block = 64;
 constexpr int kAllF32Block = 64;
 constexpr int kOneWave = 64, kFourWaves = 256;  // by-value launches, see Cfg::kSmallShape
+constexpr uint64_t kMarkBlocks = 32;  // most blocks of a launch that tells of its own end (fold_few_body)
 
 // Every operand lives in global memory (HBM or host memory mapped into the
 // device).  Pointers that reach a kernel through a descriptor table are
@@ -642,6 +643,11 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
     fetch_together<OUT == kOutFan ? MCCLX_MAX_INPUTS : C::K, OUT>(s, scale, has_scale, grid);
     int32_t fan = 0;
     if constexpr (OUT == kOutFan) fan = a.fan;
+    uint64_t* mark_word = nullptr;
+    if constexpr (OUT != kOutOne) {
+        mark_word = a.mark_word;
+        asm volatile("" : "+s"(mark_word));
+    }
 #if MCCLX_TUNE_TIMELINE
     const uint64_t t_args = wall_clock64();
 #endif
@@ -653,6 +659,22 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
     int op = C::OP;
     if constexpr (C::OP == kAnyOp) op = a.op;
     fold_tile<C, OUT, B, U, B != kFourWaves>(s, scale, has_scale != 0, (uint64_t)blockIdx.x * span, blockIdx.x == 0, fan, op);
+    // A launch of few blocks tells the host of its end itself: every block publishes what it has written
+    // (the next kernel of another stream may start before this one's own end does it) and counts itself,
+    // the last one writes the number.  Blocks that count themselves one after another cost 30 ns each, a
+    // launch behind this one 2 us: 16 blocks 7.8 us from launch call to word against 9.2, 64 blocks 9.2 and 9.4,
+    // 256 blocks 14.9 and 9.4 (kMarkBlocks).
+    if constexpr (OUT != kOutOne)
+        if (mark_word) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            if constexpr (B > kOneWave) __syncthreads();
+            if (threadIdx.x == 0 &&
+                __hip_atomic_fetch_add(a.mark_count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.mark_blocks - 1) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                __hip_atomic_store(a.mark_count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(mark_word, a.mark_number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
 #if MCCLX_TUNE_TIMELINE
     if (a.timeline && threadIdx.x == 0) {
         TimelineRecord r;
@@ -1026,6 +1048,13 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
         const uint64_t gx = (maxc + span - 1) / span;
         if (gx * B >> 32) return hipErrorInvalidValue;  // (see few_fits)
         const dim3 grid((uint32_t)gx, (uint32_t)a.nseg);
+        if (OUT != kOutOne && lp.mark && gx * (uint64_t)a.nseg <= kMarkBlocks) {
+            a.mark_word = lp.mark->word;
+            a.mark_count = lp.mark->count;
+            a.mark_number = lp.mark->number;
+            a.mark_blocks = (uint32_t)(gx * (uint64_t)a.nseg);
+            lp.mark->taken = true;
+        }
 #if MCCLX_TUNE_TIMELINE
         if (OUT == kOutOne) a.timeline = timeline_next(gx * (uint64_t)a.nseg);
 #endif
@@ -1046,7 +1075,7 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
         if constexpr (C::BLOCK == kBlock)
             if (off_lines<C, OUT>(a))
                 return go(std::integral_constant<int, kBlock>{}, std::integral_constant<int, C::U>{}, 0);
-    } else if (four_waves(waves, C::K)) {
+    } else if (four_waves(waves, C::K) || (OUT != kOutOne && lp.mark && waves > kMarkBlocks && waves <= 4 * kMarkBlocks)) {
         return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
     }
     return go(std::integral_constant<int, kOneWave>{}, Few{}, lds);
@@ -1095,8 +1124,12 @@ static hipError_t launch_table(hipStream_t st, const TableArgs& args, const Laun
     // with it, 4096 messages of 64 KB: three operands into one 167 and 181 us, eight 393 and 414,
     // two operands to two 172 and 192, three to three 266 and 267; four to four 377 and 351.
     // In place, 1024 messages: three ranks 72 and 68 us, five 123 and 113, eight 206 and 187.
+    // Three operands to three, 16 waves resident: 1.6 GB 261 and 248 us, 0.8 GB 130 and 126, 0.5 GB 86 and 86.
     uint32_t lds = 0;
     const int outputs = OUT == kOutAll ? C::K : 1 + a.fan;
+    if (C::BLOCK == kOneWave && OUT == kOutFan && outputs == 3 && C::E == 4 && C::K == 3 &&
+        a.total_items * 64 * (uint64_t)(C::U * (C::kReadBytes + 48)) >= 600'000'000)
+        lds = 163840u / 16u / 1280u * 1280u;
     if (C::BLOCK == kOneWave && (OUT == kOutAll || outputs >= 4)) {
         const int lane_bytes = C::U * (C::kReadBytes + outputs * ((C::W == MCCLX_F32 || C::kOutF32) ? 16 : 2 * C::E));
         lds = resident_lds(a.total_items * 64 * (uint64_t)lane_bytes, lane_bytes, outputs,

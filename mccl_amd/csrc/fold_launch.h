@@ -41,6 +41,11 @@ struct FewArgs {
     int32_t nseg;
     int32_t fan;        // further destinations of the result, in[k .. k+fan-1] (fan-out kernels only)
     int32_t op;         // the operator, where the kernel takes it from here (to-all kernels of MIN, MAX, PRODUCT)
+    // Fan-out and to-all kernels, where not null: the last block to end writes `mark_number` there.
+    uint64_t* mark_word;
+    uint32_t* mark_count;  // blocks that have ended, 0 between launches
+    uint64_t mark_number;
+    uint32_t mark_blocks;  // blocks of the launch
 #if MCCLX_TUNE_TIMELINE
     TimelineRecord* timeline;  // this launch's records, one per block (x fastest, then y), or null
 #endif
@@ -67,7 +72,16 @@ struct PlanKey {
     int dtype, io, k, topo, op, acc;
 };
 
+// A launch that tells the host of its own end (mcclx_queue_wait's word), if it has few enough blocks.
+struct LaunchMark {
+    uint64_t* word;
+    uint32_t* count;
+    uint64_t number;
+    bool taken = false;
+};
+
 struct LaunchParams {
+    LaunchMark* mark = nullptr;
     const FewArgs* few = nullptr;      // exactly one of few / table is set
     const TableArgs* table = nullptr;
     uint32_t max_blocks = 0;           // cap on the grid (persistent sizing)

@@ -123,6 +123,7 @@ struct mcclx_ctx {
     uint64_t* word = nullptr;
     uint64_t* word_dev = nullptr;  // the same memory as the device addresses it
     hipEvent_t word_ev = nullptr;
+    uint32_t* mark_count = nullptr;  // device memory: blocks of a marked launch that have ended (LaunchMark)
     std::chrono::steady_clock::time_point last_wait{};  // of the newest mcclx_queue_wait (under away_mu)
     uint64_t word_number = 0;      // the last number handed out (under away_mu)
     std::atomic<bool> exposed{false};  // the caller holds the queue's HIP stream (mcclx_queue_stream, mcclx_init_on_stream)
@@ -158,6 +159,13 @@ bool records(hipStream_t s) {
     return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
 }
 
+// Set while a call that waits for its launches issues them: each launch that can, marks its own end.
+struct MarkRequest {
+    uint64_t number = 0;  // what the newest launch writes, 0 = it does not mark its end
+    uint64_t upto = 0;    // `issued` of the context then
+};
+thread_local MarkRequest* g_mark = nullptr;
+
 // The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its
 // place.  As an argument it lives until the call that enqueues the operation has returned, so that
 // no other thread finds the queue idle in between and launches beside it.
@@ -177,6 +185,7 @@ QueueUse queue_of(mcclx_ctx* ctx) {
         ctx->away.store(false, std::memory_order_release);
     }
     ctx->issued.fetch_add(1, std::memory_order_relaxed);
+    if (g_mark) g_mark->number = 0;
     return {std::move(lk), ctx->stream};
 }
 
@@ -580,8 +589,19 @@ int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, in
     a.has_scale = has_scale;
     a.nseg = (int32_t)nseg;
     lp.few = &a;
+    mcclx::LaunchMark mark;
+    if (g_mark && ctx->mark_count) {  // (the caller holds away_mu: numbers are handed out in the queue's order)
+        mark.word = ctx->word_dev;
+        mark.count = ctx->mark_count;
+        mark.number = ctx->word_number + 1;
+        lp.mark = &mark;
+    }
     hipError_t e = mcclx::launch_fold(st, key, lp);
     if (e != hipSuccess) return launch_error(e, key);
+    if (mark.taken) {
+        g_mark->number = ++ctx->word_number;
+        g_mark->upto = ctx->issued.load(std::memory_order_relaxed);
+    }
     ++ctx->launches;
     if (held) ++ctx->hold_launches;
     return MCCLX_OK;
@@ -859,6 +879,13 @@ int make_ctx(int device, hipStream_t borrowed, bool borrow, mcclx_ctx** out) {
     if (hipHostMalloc(&w, 64, hipHostMallocMapped | hipHostMallocPortable) == hipSuccess &&
         hipHostGetDevicePointer(&wd, w, 0) == hipSuccess &&
         hipEventCreateWithFlags(&ctx->word_ev, hipEventDisableTiming) == hipSuccess) {
+        void* count = nullptr;  // (without it no launch marks its own end; nothing is put on a caller's stream here)
+        if (!borrow && hipMalloc(&count, sizeof(uint64_t)) == hipSuccess) {
+            // cleared on the queue, in front of every launch that uses it (a blocking copy would wait for the default stream)
+            if (mcclx::launch_word(ctx->stream, static_cast<uint64_t*>(count), 0) == hipSuccess) ctx->mark_count = static_cast<uint32_t*>(count);
+            else (void)hipFree(count);
+        }
+        (void)hipGetLastError();
         ctx->word = static_cast<uint64_t*>(w);
         ctx->word_dev = static_cast<uint64_t*>(wd);
         *ctx->word = 0;
@@ -926,6 +953,7 @@ int mcclx_destroy(mcclx_ctx* ctx) {
     for (auto& kv : ctx->host_allocs) (void)hipHostFree(kv.first);
     if (ctx->word) (void)hipHostFree(ctx->word);
     if (ctx->word_ev) (void)hipEventDestroy(ctx->word_ev);
+    if (ctx->mark_count) (void)hipFree(ctx->mark_count);
     if (ctx->stage_send) (void)hipHostFree(ctx->stage_send);
     for (int i = 0; i < 2; ++i) {
         if (ctx->stage_recv[i]) (void)hipHostFree(ctx->stage_recv[i]);
@@ -1372,24 +1400,28 @@ int mcclx_queue_drain(mcclx_ctx* ctx) {
 // into pinned host memory, and a host that watches it, get there sooner, and the second launch is issued
 // while the first runs: a 20 us kernel, from the launch call to the return, 31.5 -> 27.8 us, an empty one 11.6 -> 9.8.
 // The queue's order ends and publishes the launches before that wave starts, as for any kernel behind them.
-int mcclx_queue_wait(mcclx_ctx* ctx, uint32_t spin_us) {
-    if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
-    REFUSE_WHILE_RECORDING(ctx, "queue_wait");
+static int queue_wait(mcclx_ctx* ctx, uint32_t spin_us, const MarkRequest& mark) {
     DeviceGuard guard(ctx->device);
     if (spin_us && ctx->word && !ctx->away.load(std::memory_order_acquire) && !records(ctx->stream)) {
-        uint64_t upto, number;
+        uint64_t upto = mark.upto, number = mark.number;
         {
-            QueueUse use = queue_of(ctx);
-            upto = ctx->issued.load(std::memory_order_relaxed);
-            number = ++ctx->word_number;
-            HIP_TRY(mcclx::launch_word(use, ctx->word_dev, number));
+            std::unique_lock<std::mutex> lk(ctx->away_mu);
+            hipStream_t st = ctx->stream;
+            if (number == 0) {
+                lk.unlock();
+                QueueUse use = queue_of(ctx);
+                upto = ctx->issued.load(std::memory_order_relaxed);
+                number = ++ctx->word_number;
+                HIP_TRY(mcclx::launch_word(use, ctx->word_dev, number));
+                lk = std::move(use.lk);
+            }
             // A device-wide or stream synchronisation behind this call waits for a completion signal of
             // its own, 6 us sooner if one is under way already.  Calls in quick succession leave it out:
             // it would be in front of the next launch (metrics of 4 KB, back to back, 11.5 -> 12..16.5 us).
             const auto now = std::chrono::steady_clock::now();
             if (now - ctx->last_wait > std::chrono::microseconds(200)) {
-                HIP_TRY(hipEventRecord(ctx->word_ev, use));
-                ctx->marked.store(upto, std::memory_order_release);
+                HIP_TRY(hipEventRecord(ctx->word_ev, st));
+                ctx->marked.store(ctx->issued.load(std::memory_order_relaxed), std::memory_order_release);
             }
             ctx->last_wait = now;
         }
@@ -1409,6 +1441,25 @@ int mcclx_queue_wait(mcclx_ctx* ctx, uint32_t spin_us) {
     }
     HIP_TRY(drain(ctx));  // also what reports a launch that failed
     return MCCLX_OK;
+}
+
+int mcclx_queue_wait(mcclx_ctx* ctx, uint32_t spin_us) {
+    if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
+    REFUSE_WHILE_RECORDING(ctx, "queue_wait");
+    return queue_wait(ctx, spin_us, MarkRequest{});
+}
+
+int mcclx_allreduce_replay_wait(mcclx_ctx* ctx, const mcclx_replay* replays, uint32_t n, uint32_t spin_us) {
+    if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
+    REFUSE_WHILE_RECORDING(ctx, "allreduce_replay_wait");
+    MarkRequest mark;
+    if (spin_us && !records(ctx->stream)) g_mark = &mark;
+    const int rc = mcclx_allreduce_replay_many(ctx, replays, n);
+    g_mark = nullptr;
+    const std::string why = rc ? g_err : std::string();
+    const int waited = queue_wait(ctx, spin_us, mark);
+    if (rc) g_err = why;
+    return rc ? rc : waited;
 }
 
 static int stream_wait(mcclx_ctx* ctx, hipStream_t waiter, hipStream_t producer) {

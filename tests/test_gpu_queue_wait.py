@@ -150,3 +150,76 @@ def test_every_wait_holds_whether_or_not_the_stream_was_asked(env, streams, drai
             assert y.cpu().eq(2 * (i + 1)).all(), i
     finally:
         q.close()
+
+
+def test_making_a_queue_does_not_wait_for_the_default_stream(env):
+    _, K = env
+    K.ReduceQueue(0).close()  # what a process does once is done
+    torch.cuda.synchronize()
+    torch.cuda._sleep(400_000_000)
+    busy = torch.cuda.Event()
+    busy.record()
+    q = K.ReduceQueue(0)
+    still = not busy.query()
+    torch.cuda.synchronize()
+    q.close()
+    assert still
+
+
+@pytest.mark.parametrize("world,dtype", [(2, "fp32"), (3, "bf16"), (4, "wire"), (5, "fp16"), (8, "fp32"), (8, "wire")])
+def test_small_allreduces_that_tell_of_their_own_end(env, world, dtype):
+    """Launches of few blocks write the word themselves, others have a wave behind them for it: in turn,
+    on tensors that change, each call returns with its result in place for a copy to the host, a kernel on
+    another stream and the next call."""
+    L, K = env
+    from mccl_amd import harness as H
+    K.hip_kernels_init(0)
+    dt = {"fp32": torch.float32, "wire": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
+    side = torch.cuda.Stream()
+    sizes = [world, 63, 255, 1_000, 4_097, 8_192 * world, 300_000, 16_385, 2_047, 70_001, 500, 32_768, 33_000]
+    for op in ("sum", "max"):
+        for rep in range(3):
+            for n in sizes:
+                ts = [((torch.arange(n, device="cuda") * (r + 2) + rep) % 9 - 4).to(dt) for r in range(world)]
+                stack = torch.stack([t.float() for t in ts])
+                want = stack.sum(0) if op == "sum" else stack.amax(0)
+                H.allreduce_replay(ts, op, L.ALGO_BUTTERFLY if n >= world else L.ALGO_TREE, wire_bf16=dtype == "wire", mode=L.REPLAY_DIRECT)
+                with torch.cuda.stream(side):
+                    doubled = [t.float() * 2 for t in ts]
+                host = [t.cpu().float() for t in ts]
+                side.synchronize()
+                want = want.cpu()
+                for r in range(world):
+                    assert torch.equal(host[r], want), (op, n, r)
+                    assert torch.equal(doubled[r].cpu(), 2 * want), (op, n, r)
+    assert L.lib().mcclx_allreduce_replay_wait(C.c_void_p(None), None, 0, 1000) == L.ERR_STATE
+
+
+def test_marked_calls_from_threads_on_queues_of_their_own_and_on_one(env):
+    L, K = env
+    from mccl_amd import harness as H
+    shared = K.ReduceQueue(0)
+    wrong = []
+
+    def work(i):
+        torch.cuda.set_device(0)
+        q = shared if i % 2 else K.ReduceQueue(0)
+        a = torch.zeros(3_000, device="cuda")
+        b = torch.ones(3_000, device="cuda")
+        torch.cuda.current_stream().synchronize()
+        for rep in range(150):
+            b.fill_(1)
+            torch.cuda.current_stream().synchronize()
+            H.allreduce_replay([a, b], "sum", L.ALGO_TREE, mode=L.REPLAY_DIRECT, queue=q)
+            if rep % 30 == 29 and not (a.cpu().eq(rep + 1).all() and b.cpu().eq(rep + 1).all()):
+                wrong.append((i, rep))
+        if q is not shared:
+            q.close()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    shared.close()
+    assert not wrong
