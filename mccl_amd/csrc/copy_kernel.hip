@@ -233,7 +233,7 @@ hipError_t launch_copy_few_n(hipStream_t st, const CopyFew& a) {
     // waves that copies of three destinations get are right for every mixture tried (67 MB from nine
     // ranks to all nine, eight destinations and one in turn, 1465 -> 1065 us; twelve ranks, eight and
     // four, 609 -> 450).
-    const uint32_t lds = resident_lds(moved, MIXED ? 16 * (3 + 1) : 16 * (N + 1), N, kLaneBytesCopy);
+    const uint32_t lds = resident_lds(moved, MIXED ? 16 * (3 + 1) : 16 * (N + 1), N, kLaneBytesCopy, kResidentMinBytesCopy);
     if (four)
         copy_few_kernel<N, kFourWaves, MIXED><<<grid, dim3(kFourWaves), lds, st>>>(a);
     else

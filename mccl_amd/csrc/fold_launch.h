@@ -139,12 +139,16 @@ hipError_t launch_fold(hipStream_t st, const PlanKey& key, const LaunchParams& l
 //
 // A launch that ends soon needs its waves to get going: the limit pays from 160 MB moved on
 // (200 MB, eight operands into one: 36.2 -> 35.4 us; 80 MB: 5.5 TB/s without it, 5.1 with),
-// and not where 20 waves or more would be left of a launch with one output.
+// and not where 20 waves or more would be left of a launch with one output.  Copies, whose waves have
+// nothing to do between load and store, gain from 90 MB on (eight to eight, 144 MB: 30.5 -> 28.6 us, 86 MB
+// level; two to two, 96 MB: 17.9 -> 16.8).
 constexpr uint64_t kResidentMinBytes = 160'000'000;
+constexpr uint64_t kResidentMinBytesCopy = 90'000'000;
 constexpr int kLaneBytes = 1160, kLaneBytesInPlace = 1280, kLaneBytesCopy = 1020;
-inline uint32_t resident_lds(uint64_t launch_bytes, int lane_bytes, int outputs, int budget = kLaneBytes) {
+inline uint32_t resident_lds(uint64_t launch_bytes, int lane_bytes, int outputs, int budget = kLaneBytes,
+                             uint64_t min_bytes = kResidentMinBytes) {
     int waves = budget / lane_bytes;
-    if (launch_bytes < kResidentMinBytes || (outputs == 1 && waves >= 20)) return 0;
+    if (launch_bytes < min_bytes || (outputs == 1 && waves >= 20)) return 0;
     waves = waves > 18 ? 18 : waves < 3 ? 3 : waves;  // three blocks reserve 53 KiB each: a launch may ask for 64 KiB
     return 163840u / (uint32_t)waves / 1280u * 1280u;
 }
