@@ -95,7 +95,8 @@ __global__ void __launch_bounds__(kBlock) stream_probe_kernel(uint8_t* buf, uint
 }
 
 // The mark of mcclx_queue_wait: the number travels in the arguments, so the one wave that runs reads
-// no memory (a 4-byte copy in its place, with a copy's descriptors, took 3.8 us on the device).
+// no memory.  Bound by the store's way over the link (4 us in a trace, to its acknowledgement; the host
+// sees the number before that).
 __global__ void __launch_bounds__(64) word_kernel(uint64_t* word, uint64_t number) {
     if (threadIdx.x == 0) __hip_atomic_store(word, number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
