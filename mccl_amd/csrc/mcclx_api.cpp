@@ -490,7 +490,8 @@ int ensure_slot(mcclx_ctx* ctx, TableSlot& sl, size_t need) {
     if (sl.dev) HIP_TRY(hipFree(sl.dev));
     sl.host = sl.dev = nullptr;
     sl.cap = 0;
-    HIP_TRY(hipHostMalloc(&sl.host, cap, hipHostMallocMapped));
+    // (coherent whatever the environment says: a slot is written again while the device may hold lines of it)
+    HIP_TRY(hipHostMalloc(&sl.host, cap, hipHostMallocMapped | hipHostMallocCoherent));
     HIP_TRY(hipHostGetDevicePointer(&sl.host_dev, sl.host, 0));
     HIP_TRY(hipMalloc(&sl.dev, cap));
     // (it tells the host that `host` has been read: nothing the device wrote has to be published)
@@ -876,7 +877,7 @@ int make_ctx(int device, hipStream_t borrowed, bool borrow, mcclx_ctx** out) {
     }
     void* w = nullptr;  // (without it mcclx_queue_wait drains)
     void* wd = nullptr;
-    if (hipHostMalloc(&w, 64, hipHostMallocMapped | hipHostMallocPortable) == hipSuccess &&
+    if (hipHostMalloc(&w, 64, hipHostMallocMapped | hipHostMallocPortable | hipHostMallocCoherent) == hipSuccess &&
         hipHostGetDevicePointer(&wd, w, 0) == hipSuccess &&
         hipEventCreateWithFlags(&ctx->word_ev, hipEventDisableTiming) == hipSuccess) {
         void* count = nullptr;  // (without it no launch marks its own end; nothing is put on a caller's stream here)
