@@ -31,8 +31,12 @@ extern "C" int mcclx_fail(int code, const char* fmt, ...) {
     va_start(ap, fmt);
     vsnprintf(buf, sizeof buf, fmt, ap);
     va_end(ap);
-    // same prefix as the reference's MCCLError (csrc/common/Errors.hpp:9-13)
-    g_err = std::string("[MCCL] ") + buf;
+    try {
+        // same prefix as the reference's MCCLError (csrc/common/Errors.hpp:9-13)
+        g_err = std::string("[MCCL] ") + buf;
+    } catch (const std::exception&) {  // no memory for the words either
+        g_err.clear();
+    }
     return code;
 }
 
@@ -165,6 +169,10 @@ struct MarkRequest {
     uint64_t upto = 0;    // `issued` of the context then
 };
 thread_local MarkRequest* g_mark = nullptr;
+struct MarkScope {
+    explicit MarkScope(MarkRequest* m) { g_mark = m; }
+    ~MarkScope() { g_mark = nullptr; }
+};
 
 // The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its
 // place.  As an argument it lives until the call that enqueues the operation has returned, so that
@@ -625,7 +633,7 @@ bool even_enough(const mcclx::PlanKey& key, const mcclx_seg* segs, uint32_t nseg
     return longest * nseg <= 4 * total + 64;
 }
 
-int fold_impl(mcclx_ctx* ctx, const mcclx_plan* plan, const mcclx_seg* segs, uint32_t nseg) {
+int fold_checked(mcclx_ctx* ctx, const mcclx_plan* plan, const mcclx_seg* segs, uint32_t nseg) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     mcclx::PlanKey key;
     float scale_f;
@@ -695,6 +703,10 @@ int fold_impl(mcclx_ctx* ctx, const mcclx_plan* plan, const mcclx_seg* segs, uin
     if (e != hipSuccess) return launch_error(e, key);
     ++ctx->launches;
     return MCCLX_OK;
+}
+
+int fold_impl(mcclx_ctx* ctx, const mcclx_plan* plan, const mcclx_seg* segs, uint32_t nseg) {
+    return mcclx_entry([&] { return fold_checked(ctx, plan, segs, nseg); });
 }
 
 // The hold form's gate follows the device.  Its model -- no store before
@@ -1268,7 +1280,7 @@ int mcclx_copy(mcclx_ctx* ctx, void* dst, const void* src, uint64_t nbytes) {
     return MCCLX_OK;
 }
 
-int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n) {
+static int copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     if (n == 0) return MCCLX_OK;
     if (!descs) return fail(MCCLX_ERR_INVALID, "copy_batched: descriptor array is null");
@@ -1370,6 +1382,10 @@ int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n)
     return MCCLX_OK;
 }
 
+int mcclx_copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n) {
+    return mcclx_entry([&] { return copy_batched(ctx, descs, n); });
+}
+
 int mcclx_batch_begin(mcclx_ctx* ctx, const char* label) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     if (ctx->batch_active) return fail(MCCLX_ERR_STATE, "batch already active");  // MetalKernels.mm:562
@@ -1454,12 +1470,15 @@ int mcclx_allreduce_replay_wait(mcclx_ctx* ctx, const mcclx_replay* replays, uin
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     REFUSE_WHILE_RECORDING(ctx, "allreduce_replay_wait");
     MarkRequest mark;
-    if (spin_us && !records(ctx->stream)) g_mark = &mark;
-    const int rc = mcclx_allreduce_replay_many(ctx, replays, n);
-    g_mark = nullptr;
-    const std::string why = rc ? g_err : std::string();
-    const int waited = queue_wait(ctx, spin_us, mark);
-    if (rc) g_err = why;
+    int rc;
+    {
+        const MarkScope scope(spin_us && !records(ctx->stream) ? &mark : nullptr);
+        rc = mcclx_allreduce_replay_many(ctx, replays, n);
+    }
+    std::string why;
+    if (rc) why.swap(g_err);
+    const int waited = queue_wait(ctx, spin_us, mark);  // in any case: the caller's workspace is still read
+    if (rc) g_err.swap(why);
     return rc ? rc : waited;
 }
 

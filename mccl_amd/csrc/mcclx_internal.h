@@ -1,12 +1,27 @@
 // mcclx_internal.h -- shared by the translation units of libmcclx.so only.
 #pragma once
 
+#include <exception>
+#include <new>
+
 #include "mcclx.h"
 
 // Records the calling thread's error message (what mcclx_last_error() returns)
 // and hands back `code`.
 extern "C" __attribute__((visibility("hidden"))) int mcclx_fail(int code, const char* fmt, ...)
     __attribute__((format(printf, 2, 3)));
+
+// The body of a C entry that allocates: no exception leaves it.
+template <class F>
+int mcclx_entry(F&& body) {
+    try {
+        return body();
+    } catch (const std::bad_alloc&) {
+        return mcclx_fail(MCCLX_ERR_NOMEM, "out of host memory");
+    } catch (const std::exception& e) {  // (a vector asked for more than it can ever hold)
+        return mcclx_fail(MCCLX_ERR_STATE, "%s", e.what());
+    }
+}
 
 // Is `p` pinned host memory?  (Link traffic, where everything else is the device's own.)
 extern "C" __attribute__((visibility("hidden"))) bool mcclx_in_host_memory(mcclx_ctx* ctx, const void* p);

@@ -715,57 +715,7 @@ bool same_plan(const mcclx_replay* a, const mcclx_replay* b) {
            (a->wire_bf16 != 0) == (b->wire_bf16 != 0) && a->acc == b->acc && a->mode == b->mode;
 }
 
-}  // namespace
-
-extern "C" {
-
-int mcclx_chunkize(int64_t numel, uint64_t elem_size, int world, mcclx_chunk* out) {
-    if (world < 1 || numel < 0 || !out) return bad("chunkize: bad argument");
-    const int64_t per = (numel + world - 1) / world;  // AllreduceAlgos.cpp:23
-    for (int i = 0; i < world; ++i) {
-        int64_t lo = (int64_t)i * per, hi = lo + per;
-        lo = lo < numel ? lo : numel;
-        hi = hi < numel ? hi : numel;
-        out[i] = mcclx_chunk{lo, hi - lo, (uint64_t)lo * elem_size, (uint64_t)(hi - lo) * elem_size};
-    }
-    return MCCLX_OK;
-}
-
-int mcclx_select_algo(const char* env_algo, int64_t tree_below, uint64_t wire_nbytes,
-                      int64_t numel, int world) {
-    std::string alg = env_algo ? env_algo : "auto";  // ProcessGroupMCCL.cpp:134-135
-    int algo = MCCLX_ALGO_TREE;                     // any unknown name runs the tree (:173-176)
-    if (alg == "auto") {
-        uint64_t below = tree_below < 0 ? 256ull * 1024 : (uint64_t)tree_below;  // :137-139
-        algo = wire_nbytes <= below ? MCCLX_ALGO_TREE : MCCLX_ALGO_RING;        // :140
-    } else if (alg == "ring") {
-        algo = MCCLX_ALGO_RING;
-    } else if (alg == "butterfly") {
-        algo = MCCLX_ALGO_BUTTERFLY;
-    }
-    if (algo == MCCLX_ALGO_RING && numel < world) algo = MCCLX_ALGO_TREE;  // :143
-    if (algo == MCCLX_ALGO_BUTTERFLY && (world < 2 || numel < world)) algo = MCCLX_ALGO_TREE;  // :144-145
-    return algo;
-}
-
-uint64_t mcclx_replay_workspace_bytes(const mcclx_replay* r) {
-    if (!r || r->world < 1) return 0;
-    uint64_t need = layout_of(r).total;
-    if (r->mode != MCCLX_REPLAY_STEPWISE && r->algo == MCCLX_ALGO_TREE &&
-        r->world > MCCLX_MAX_INPUTS * MCCLX_MAX_INPUTS) {  // runs the stepwise schedule (check_replay)
-        mcclx_replay s = *r;
-        s.mode = MCCLX_REPLAY_STEPWISE;
-        const uint64_t step = layout_of(&s).total;
-        need = step > need ? step : need;
-    }
-    return need;
-}
-
-int mcclx_allreduce_replay(mcclx_ctx* ctx, const mcclx_replay* r) {
-    return mcclx_allreduce_replay_many(ctx, r, 1);
-}
-
-int mcclx_allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t n) {
+int allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t n) {
     if (n && !rs) return bad("replay: null argument");
     uint32_t i = 0;
     while (i < n) {
@@ -823,9 +773,9 @@ int mcclx_allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t
     return MCCLX_OK;
 }
 
-int mcclx_reduce_scatter_shares(mcclx_ctx* ctx, int world, void* const* outs,
-                                const void* const* shares, int dtype, uint64_t chunk_numel, int op,
-                                int mode, int acc) {
+int reduce_scatter_shares(mcclx_ctx* ctx, int world, void* const* outs,
+                          const void* const* shares, int dtype, uint64_t chunk_numel, int op,
+                          int mode, int acc) {
     if (!ctx || !outs || !shares || world < 1) return bad("reduce_scatter: bad argument");
     auto share = [&](int r, int p) { return shares[(size_t)r * (size_t)world + (size_t)p]; };
     const uint64_t cb = chunk_numel * esize(dtype);
@@ -879,19 +829,19 @@ int mcclx_reduce_scatter_shares(mcclx_ctx* ctx, int world, void* const* outs,
     return MCCLX_OK;
 }
 
-int mcclx_reduce_scatter_replay(mcclx_ctx* ctx, int world, void* const* outs,
-                                const void* const* ins, int dtype, uint64_t chunk_numel, int op,
-                                int mode, int acc) {
+int reduce_scatter_replay(mcclx_ctx* ctx, int world, void* const* outs,
+                          const void* const* ins, int dtype, uint64_t chunk_numel, int op,
+                          int mode, int acc) {
     if (!ctx || !outs || !ins || world < 1) return bad("reduce_scatter: bad argument");
     const uint64_t cb = chunk_numel * esize(dtype);
     std::vector<const void*> shares((size_t)world * (size_t)world);
     for (int r = 0; r < world; ++r)
         for (int p = 0; p < world; ++p) shares[(size_t)r * world + p] = at(ins[p], (uint64_t)r * cb);
-    return mcclx_reduce_scatter_shares(ctx, world, outs, shares.data(), dtype, chunk_numel, op, mode, acc);
+    return reduce_scatter_shares(ctx, world, outs, shares.data(), dtype, chunk_numel, op, mode, acc);
 }
 
-int mcclx_allgather_replay(mcclx_ctx* ctx, int world, void* const* outs, const void* const* ins,
-                           uint64_t chunk_nbytes) {
+int allgather_replay(mcclx_ctx* ctx, int world, void* const* outs, const void* const* ins,
+                     uint64_t chunk_nbytes) {
     if (!ctx || !outs || !ins || world < 1) return bad("allgather: bad argument");
     std::vector<mcclx_copy_desc> copies;
     copies.reserve((size_t)world * (size_t)world);
@@ -899,6 +849,77 @@ int mcclx_allgather_replay(mcclx_ctx* ctx, int world, void* const* outs, const v
         for (int r = 0; r < world; ++r)  // ProcessGroupMCCL.cpp:256-270
             copies.push_back(mcclx_copy_desc{at(outs[r], (uint64_t)p * chunk_nbytes), ins[p], chunk_nbytes});
     return mcclx_copy_batched(ctx, copies.data(), (uint32_t)copies.size());
+}
+
+}  // namespace
+
+extern "C" {
+
+int mcclx_chunkize(int64_t numel, uint64_t elem_size, int world, mcclx_chunk* out) {
+    if (world < 1 || numel < 0 || !out) return bad("chunkize: bad argument");
+    const int64_t per = (numel + world - 1) / world;  // AllreduceAlgos.cpp:23
+    for (int i = 0; i < world; ++i) {
+        int64_t lo = (int64_t)i * per, hi = lo + per;
+        lo = lo < numel ? lo : numel;
+        hi = hi < numel ? hi : numel;
+        out[i] = mcclx_chunk{lo, hi - lo, (uint64_t)lo * elem_size, (uint64_t)(hi - lo) * elem_size};
+    }
+    return MCCLX_OK;
+}
+
+int mcclx_select_algo(const char* env_algo, int64_t tree_below, uint64_t wire_nbytes,
+                      int64_t numel, int world) {
+    std::string alg = env_algo ? env_algo : "auto";  // ProcessGroupMCCL.cpp:134-135
+    int algo = MCCLX_ALGO_TREE;                     // any unknown name runs the tree (:173-176)
+    if (alg == "auto") {
+        uint64_t below = tree_below < 0 ? 256ull * 1024 : (uint64_t)tree_below;  // :137-139
+        algo = wire_nbytes <= below ? MCCLX_ALGO_TREE : MCCLX_ALGO_RING;        // :140
+    } else if (alg == "ring") {
+        algo = MCCLX_ALGO_RING;
+    } else if (alg == "butterfly") {
+        algo = MCCLX_ALGO_BUTTERFLY;
+    }
+    if (algo == MCCLX_ALGO_RING && numel < world) algo = MCCLX_ALGO_TREE;  // :143
+    if (algo == MCCLX_ALGO_BUTTERFLY && (world < 2 || numel < world)) algo = MCCLX_ALGO_TREE;  // :144-145
+    return algo;
+}
+
+uint64_t mcclx_replay_workspace_bytes(const mcclx_replay* r) {
+    if (!r || r->world < 1) return 0;
+    uint64_t need = layout_of(r).total;
+    if (r->mode != MCCLX_REPLAY_STEPWISE && r->algo == MCCLX_ALGO_TREE &&
+        r->world > MCCLX_MAX_INPUTS * MCCLX_MAX_INPUTS) {  // runs the stepwise schedule (check_replay)
+        mcclx_replay s = *r;
+        s.mode = MCCLX_REPLAY_STEPWISE;
+        const uint64_t step = layout_of(&s).total;
+        need = step > need ? step : need;
+    }
+    return need;
+}
+
+int mcclx_allreduce_replay(mcclx_ctx* ctx, const mcclx_replay* r) {
+    return mcclx_allreduce_replay_many(ctx, r, 1);
+}
+
+int mcclx_allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t n) {
+    return mcclx_entry([&] { return allreduce_replay_many(ctx, rs, n); });
+}
+
+int mcclx_reduce_scatter_shares(mcclx_ctx* ctx, int world, void* const* outs,
+                                const void* const* shares, int dtype, uint64_t chunk_numel, int op,
+                                int mode, int acc) {
+    return mcclx_entry([&] { return reduce_scatter_shares(ctx, world, outs, shares, dtype, chunk_numel, op, mode, acc); });
+}
+
+int mcclx_reduce_scatter_replay(mcclx_ctx* ctx, int world, void* const* outs,
+                                const void* const* ins, int dtype, uint64_t chunk_numel, int op,
+                                int mode, int acc) {
+    return mcclx_entry([&] { return reduce_scatter_replay(ctx, world, outs, ins, dtype, chunk_numel, op, mode, acc); });
+}
+
+int mcclx_allgather_replay(mcclx_ctx* ctx, int world, void* const* outs, const void* const* ins,
+                           uint64_t chunk_nbytes) {
+    return mcclx_entry([&] { return allgather_replay(ctx, world, outs, ins, chunk_nbytes); });
 }
 
 }  // extern "C"

@@ -2,15 +2,58 @@
 // the kernel layer (null_mcclx.cpp): launches per list, results of fp32 sums, workspace sizes.
 #include <atomic>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
+#include <new>
 #include <vector>
 
 #include "mcclx.h"
 
 extern "C" std::atomic<long> null_memory_questions;
 
+// The calling thread's allocation number `g_fail_at` fails, once.
+thread_local long g_fail_at = -1;
+void* operator new(size_t n) {
+    if (g_fail_at >= 0 && g_fail_at-- == 0) throw std::bad_alloc();
+    if (void* p = malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
+
 namespace {
 int g_bad = 0;
+
+// A call whose k-th allocation fails, for every k it has: an error code and no exception, and the
+// call goes through as soon as nothing fails any more.
+template <class F>
+void without_memory(mcclx_ctx* ctx, const char* what, F&& call) {
+    int refused = 0;
+    for (long k = 0;; ++k) {
+        int rc = MCCLX_OK;
+        bool threw = false;
+        g_fail_at = k;
+        try {
+            rc = call();
+        } catch (...) {
+            threw = true;
+        }
+        const bool met = g_fail_at < 0;
+        g_fail_at = -1;
+        mcclx_queue_drain(ctx);
+        if (threw || (met && rc != MCCLX_ERR_NOMEM) || (!met && rc != MCCLX_OK)) {
+            printf("FAILED: %s, allocation %ld: %s, code %d\n", what, k, threw ? "an exception" : "returned", rc);
+            ++g_bad;
+            return;
+        }
+        if (!met) break;
+        ++refused;
+    }
+    if (!refused) {
+        printf("FAILED: %s allocates nothing\n", what);
+        ++g_bad;
+    }
+}
 
 mcclx_replay replay(int world, int algo, int op, int wire, int mode, uint64_t numel, void* const* tensors) {
     mcclx_replay r;
@@ -91,6 +134,19 @@ int main() {
     if (asked || !null_memory_questions) {
         printf("FAILED: %ld questions about small workspaces, %ld in all\n", asked, null_memory_questions.load());
         ++g_bad;
+    }
+    {
+        std::vector<std::vector<float>> data(12, std::vector<float>(4096, 1.f));
+        std::vector<void*> p;
+        for (auto& d : data) p.push_back(d.data());
+        std::vector<mcclx_replay> reps;
+        for (int e = 0; e < 4; ++e) reps.push_back(replay(3, MCCLX_ALGO_TREE, MCCLX_AVG, 0, MCCLX_REPLAY_FUSED, 4096, &p[size_t(3 * e)]));
+        without_memory(ctx, "a list", [&] { return mcclx_allreduce_replay_many(ctx, reps.data(), 4); });
+        without_memory(ctx, "one allreduce", [&] { return mcclx_allreduce_replay(ctx, &reps[1]); });
+        without_memory(ctx, "reduce_scatter", [&] {
+            return mcclx_reduce_scatter_replay(ctx, 3, &p[0], &p[3], MCCLX_F32, 1024, MCCLX_AVG, MCCLX_REPLAY_FUSED, MCCLX_ACC_STEP);
+        });
+        without_memory(ctx, "allgather", [&] { return mcclx_allgather_replay(ctx, 3, &p[0], &p[3], 4 * 1024); });
     }
     // what a replay needs does not fall as it grows: sized once for the largest, enough for all
     for (int world = 2; world <= 20; ++world)
