@@ -128,7 +128,10 @@ struct mcclx_ctx {
     uint64_t* word_dev = nullptr;  // the same memory as the device addresses it
     hipEvent_t word_ev = nullptr;
     uint32_t* mark_count = nullptr;  // device memory: blocks of a marked launch that have ended (LaunchMark)
-    std::chrono::steady_clock::time_point last_wait{};  // of the newest mcclx_queue_wait (under away_mu)
+    // When mcclx_queue_wait last returned (steady clock, ns), whether nothing has been put on the queue since, and
+    // whether what came next came within kQuickNs.  A hint: a wait is right either way.
+    std::atomic<int64_t> waited_at{0};
+    std::atomic<bool> resting{false}, quick{false};
     uint64_t word_number = 0;      // the last number handed out (under away_mu)
     std::atomic<bool> exposed{false};  // the caller holds the queue's HIP stream (mcclx_queue_stream, mcclx_init_on_stream)
     hipStream_t upload_stream = nullptr;  // blocking table uploads while the queue is recording
@@ -174,6 +177,22 @@ struct MarkScope {
     ~MarkScope() { g_mark = nullptr; }
 };
 
+// A call that returns early (mcclx_queue_wait) leaves an event behind its launches, in which a device-wide or
+// stream synchronisation of the caller's finds the completion signal it waits for (without one it puts a marker on
+// the queue then: 11 us instead of 5.5).  The event takes the queue some 3 us, so it is left out where the
+// next call starts at once, as this one did: within kQuickNs of the return before it.  Calls back to back start
+// after 1.4-3.6 us, behind a synchronisation after 6.5-15.  A maximum of 4 KB over eight ranks (us): back to back 13.6
+// with the event always, 10.8 never, 10.8 by this rule; each with a synchronisation behind it 15.5, 21.6 and 15.5 (through
+// hipStreamSynchronize and no word 14.2 and 17.4).
+constexpr int64_t kQuickNs = 5000;
+int64_t now_ns() {
+    return std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+void note_start(mcclx_ctx* ctx) {
+    if (ctx->resting.load(std::memory_order_relaxed) && ctx->resting.exchange(false, std::memory_order_relaxed))
+        ctx->quick.store(now_ns() - ctx->waited_at.load(std::memory_order_relaxed) < kQuickNs, std::memory_order_relaxed);
+}
+
 // The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its
 // place.  As an argument it lives until the call that enqueues the operation has returned, so that
 // no other thread finds the queue idle in between and launches beside it.
@@ -183,6 +202,7 @@ struct QueueUse {
     operator hipStream_t() const { return stream; }
 };
 QueueUse queue_of(mcclx_ctx* ctx) {
+    note_start(ctx);
     std::unique_lock<std::mutex> lk(ctx->away_mu);
     if (ctx->away.load(std::memory_order_relaxed)) {
         const hipEvent_t ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
@@ -1432,15 +1452,10 @@ static int queue_wait(mcclx_ctx* ctx, uint32_t spin_us, const MarkRequest& mark)
                 HIP_TRY(mcclx::launch_word(use, ctx->word_dev, number));
                 lk = std::move(use.lk);
             }
-            // A device-wide or stream synchronisation behind this call waits for a completion signal of
-            // its own, 6 us sooner if one is under way already.  Calls in quick succession leave it out:
-            // it would be in front of the next launch (metrics of 4 KB, back to back, 11.5 -> 12..16.5 us).
-            const auto now = std::chrono::steady_clock::now();
-            if (now - ctx->last_wait > std::chrono::microseconds(200)) {
+            if (!ctx->quick.load(std::memory_order_relaxed)) {  // see kQuickNs
                 HIP_TRY(hipEventRecord(ctx->word_ev, st));
                 ctx->marked.store(ctx->issued.load(std::memory_order_relaxed), std::memory_order_release);
             }
-            ctx->last_wait = now;
         }
         const volatile uint64_t* word = ctx->word;
         const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(spin_us);
@@ -1450,6 +1465,8 @@ static int queue_wait(mcclx_ctx* ctx, uint32_t spin_us, const MarkRequest& mark)
                     std::atomic_thread_fence(std::memory_order_acquire);
                     note_finished(ctx, upto);
                     ctx->host_caught_up.store(true, std::memory_order_relaxed);
+                    ctx->waited_at.store(now_ns(), std::memory_order_relaxed);
+                    ctx->resting.store(true, std::memory_order_relaxed);
                     return MCCLX_OK;
                 }
                 __builtin_ia32_pause();
@@ -1485,6 +1502,7 @@ int mcclx_allreduce_replay_wait(mcclx_ctx* ctx, const mcclx_replay* replays, uin
 static int stream_wait(mcclx_ctx* ctx, hipStream_t waiter, hipStream_t producer) {
     if (waiter == producer) return MCCLX_OK;
     REFUSE_WHILE_RECORDING(ctx, "cross-stream ordering");
+    if (waiter == ctx->stream) note_start(ctx);  // where a collective starts
     DeviceGuard guard(ctx->device);
     // A producer that has nothing in flight needs no event: everything enqueued on it so far is
     // complete, which is all the wait would establish (an event record plus a stream wait cost
