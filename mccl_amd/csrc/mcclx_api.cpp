@@ -161,6 +161,16 @@ struct DeviceGuard {
     }
 };
 
+// While it lives, this thread may allocate and wait although a stream records in a mode that forbids it
+// (torch's default one ends the recording at such a call of any thread).
+struct BesideRecordings {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    bool ok = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    ~BesideRecordings() {
+        if (ok) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+};
+
 bool records(hipStream_t s) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone;
@@ -840,6 +850,7 @@ int make_ctx(int device, hipStream_t borrowed, bool borrow, mcclx_ctx** out) {
         return fail(MCCLX_ERR_INVALID, "device %d out of range (%d visible)", device, n);
     DeviceGuard guard(device);
     if (!guard.ok) return fail(MCCLX_ERR_HIP, "hipSetDevice(%d) failed", device);
+    const BesideRecordings beside;  // allocations follow, and what is measured once per device
     auto* ctx = new mcclx_ctx();
     ctx->device = device;
     hipDeviceProp_t prop;
@@ -971,6 +982,7 @@ int mcclx_init_on_stream(int device, void* hip_stream, mcclx_ctx** out) {
 int mcclx_destroy(mcclx_ctx* ctx) {
     if (!ctx) return MCCLX_OK;
     DeviceGuard guard(ctx->device);
+    const BesideRecordings beside;
     (void)drain(ctx);
     for (auto& kv : ctx->tickets) (void)hipEventDestroy(kv.second.ev);
     for (auto ev : ctx->free_events) (void)hipEventDestroy(ev);
@@ -1556,11 +1568,8 @@ int mcclx_stream_wait_queue(mcclx_ctx* ctx, void* consumer_stream) {
         if (ctx->away.load(std::memory_order_relaxed)) {
             const hipEvent_t ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
             if (records(consumer)) {  // it cannot wait for what its recording does not hold: the host does
-                hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (a blocking call beside a recording)
-                HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
-                const hipError_t done = hipEventSynchronize(ev);
-                HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
-                HIP_TRY(done);
+                const BesideRecordings beside;
+                HIP_TRY(hipEventSynchronize(ev));
                 ctx->away.store(false, std::memory_order_release);
             } else {
                 HIP_TRY(hipStreamWaitEvent(consumer, ev, 0));

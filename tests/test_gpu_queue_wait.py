@@ -196,6 +196,51 @@ def test_making_a_queue_does_not_wait_for_the_default_stream(env):
     assert still
 
 
+@pytest.mark.parametrize("borrowed", [False, True])
+@pytest.mark.parametrize("thread", ["the recording one", "another"])
+def test_a_queue_made_and_one_closed_while_a_stream_records(env, thread, borrowed):
+    """The memory that a queue sets up for its waits is allocated and given back in a way that a recording in
+    the strictest mode survives, on the thread that records and on others."""
+    L, K = env
+    K.ReduceQueue(0).close()  # what a process does once is done
+    x = torch.zeros(1000, device="cuda")
+    side, other = torch.cuda.Stream(), torch.cuda.Stream()
+    made, old = [], K.ReduceQueue(0)
+
+    def make():
+        torch.cuda.set_device(0)
+        with torch.cuda.stream(other):
+            made.append(K.ReduceQueue(0, on_torch_stream=borrowed))
+            old.close()
+
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=side):  # capture_error_mode="global"
+        x.add_(1)
+        if thread == "another":
+            t = threading.Thread(target=make)
+            t.start()
+            t.join()
+        else:
+            make()
+        x.mul_(2)
+    want = 0.0
+    q = made[0]
+    try:
+        for rep in range(3):
+            g.replay()
+            torch.cuda.synchronize()
+            want = 2 * (want + 1)
+            assert x.cpu().eq(want).all()
+            y = torch.full((5_000,), float(rep), device="cuda")
+            torch.cuda.synchronize()
+            L.check(L.lib().mcclx_reduce(q.handle, y.data_ptr(), y.data_ptr(), L.F32, y.numel(), L.SUM))
+            q.wait_results()
+            assert y.cpu().eq(2.0 * rep).all()
+    finally:
+        q.close()
+
+
 @pytest.mark.parametrize("world,dtype", [(2, "fp32"), (3, "bf16"), (4, "wire"), (5, "fp16"), (8, "fp32"), (8, "wire")])
 def test_small_allreduces_that_tell_of_their_own_end(env, world, dtype):
     """Launches of few blocks write the word themselves, others have a wave behind them for it: in turn,
