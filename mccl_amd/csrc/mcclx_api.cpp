@@ -119,9 +119,9 @@ struct mcclx_ctx {
     std::atomic<uint64_t> issued{0}, finished{0};
     std::atomic<uint64_t> marked{0};  // `issued` when an event was last recorded on the queue
     // The stream that was last asked whether it is idle and was not, and for how many further waits it
-    // is taken to be busy without being asked (under mu).  A hint: a wait is right either way.
-    hipStream_t busy_stream = nullptr;
-    int busy_for = 0;
+    // is taken to be busy without being asked.  A hint: a wait is right either way.
+    std::atomic<hipStream_t> busy_stream{nullptr};
+    std::atomic<int> busy_for{0};
     std::atomic<bool> host_caught_up{false};  // the queue has been drained since
     // mcclx_queue_wait: the last number the device has written, in pinned host memory
     uint64_t* word = nullptr;
@@ -1523,19 +1523,21 @@ static int stream_wait(mcclx_ctx* ctx, hipStream_t waiter, hipStream_t producer)
     // finds the stream busy every time: one that was is not asked again for the next seven waits,
     // unless the host has caught up with the queue in between (the two orderings around a fold of 12 us,
     // back to back: 44.6 us a pass with both queries, 33.4 with neither).
-    if (producer == ctx->stream && queue_idle(ctx)) return MCCLX_OK;
-    std::lock_guard<std::mutex> lk(ctx->mu);
-    if (producer != ctx->stream) {
-        if (ctx->host_caught_up.exchange(false, std::memory_order_relaxed)) ctx->busy_for = 0;
-        if (ctx->busy_for > 0 && ctx->busy_stream == producer) {
-            --ctx->busy_for;
+    // All of that without mu, which mcclx_stage_for_send holds through a whole copy.
+    if (producer == ctx->stream) {
+        if (queue_idle(ctx)) return MCCLX_OK;
+    } else {
+        if (ctx->host_caught_up.exchange(false, std::memory_order_relaxed)) ctx->busy_for.store(0, std::memory_order_relaxed);
+        if (ctx->busy_for.load(std::memory_order_relaxed) > 0 && ctx->busy_stream.load(std::memory_order_relaxed) == producer) {
+            ctx->busy_for.fetch_sub(1, std::memory_order_relaxed);
         } else {
             if (hipStreamQuery(producer) == hipSuccess) return MCCLX_OK;
             (void)hipGetLastError();  // hipErrorNotReady, or a state the record below reports properly
-            ctx->busy_stream = producer;
-            ctx->busy_for = 7;
+            ctx->busy_stream.store(producer, std::memory_order_relaxed);
+            ctx->busy_for.store(7, std::memory_order_relaxed);
         }
     }
+    std::lock_guard<std::mutex> lk(ctx->mu);
     hipEvent_t& ev = ctx->xev[ctx->xnext];
     ctx->xnext = (ctx->xnext + 1) % 16;
     if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));

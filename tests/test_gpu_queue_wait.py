@@ -154,6 +154,36 @@ def test_every_wait_holds_whether_or_not_the_stream_was_asked(env, streams, drai
         q.close()
 
 
+def test_a_wait_for_an_idle_stream_does_not_stand_behind_a_staging_copy(env):
+    """mcclx_stage_for_send holds the context's lock while 512 MB come off the device (10 ms): a wait for an
+    idle stream on another thread needs nothing of what it guards."""
+    L, K = env
+    q = K.ReduceQueue(0)
+    try:
+        big = torch.ones(128 << 20, device="cuda")
+        side = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        host = C.c_void_p()
+        stage = lambda: L.check(L.lib().mcclx_stage_for_send(q.handle, big.data_ptr(), 4 * big.numel(), C.byref(host)))
+        stage()  # the pinned buffer is there from now on
+        longest = []
+        for _ in range(3):
+            copying = threading.Thread(target=stage)
+            started = time.perf_counter()
+            copying.start()
+            waits = [0.0]
+            while copying.is_alive():
+                t = time.perf_counter()
+                q.wait_torch_stream(side)
+                waits.append(time.perf_counter() - t)
+                time.sleep(1e-4)
+            longest.append(max(waits) / (time.perf_counter() - started))
+            copying.join()
+        assert min(longest) < 0.3, longest
+    finally:
+        q.close()
+
+
 @pytest.mark.parametrize("what", ["allreduce", "reduce_scatter", "allgather"])
 def test_a_synchronisation_behind_each_call_finds_a_signal_to_wait_for(env, what):
     """A device synchronisation behind a call takes as long in a run of such calls as behind one that
