@@ -653,6 +653,12 @@ int check_replay(mcclx_ctx* ctx, const mcclx_replay* r, Layout* L, bool* fused, 
     return MCCLX_OK;
 }
 
+// The same for an entry of a list with the plan of the entry before it, whose size may be the same too.
+int check_next(mcclx_ctx* ctx, const mcclx_replay* r, Layout* L, bool* fused, bool* nothing_to_do) {
+    if (r->tensors && r->reserved == 0 && r->numel == r[-1].numel) return check_memory(r, *L);
+    return check_replay(ctx, r, L, fused, nothing_to_do);
+}
+
 int run_stepwise(mcclx_ctx* ctx, const mcclx_replay* r) {
     mcclx_replay s = *r;
     s.mode = MCCLX_REPLAY_STEPWISE;
@@ -717,7 +723,7 @@ bool same_plan(const mcclx_replay* a, const mcclx_replay* b) {
 
 int allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t n) {
     if (n && !rs) return bad("replay: null argument");
-    uint32_t i = 0;
+    uint32_t i = 0, checked = 0;  // entries known to be sound
     while (i < n) {
         bool fused, nothing;
         Layout L;
@@ -743,14 +749,17 @@ int allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t n) {
         while (i < n) {
             if (&rs[i] != first) {
                 // a long list goes out in pieces: see kPieceEntries
-                if (&rs[i] - first >= kPieceEntries && moved >= kPieceBytes) break;
-                if (!same_plan(first, &rs[i])) break;
-                if (rs[i].tensors && rs[i].reserved == 0 && rs[i].numel == rs[i - 1].numel) {
-                    TRY(check_memory(&rs[i], L));  // all else is as in the entry before
-                } else {
-                    TRY(check_replay(ctx, &rs[i], &L, &fused, &nothing));
-                    if (!fused || nothing) break;
+                if (&rs[i] - first >= kPieceEntries && moved >= kPieceBytes) {
+                    // (what is wrong with an entry of its other pieces is said before this one is issued)
+                    for (checked = checked > i ? checked : i; checked < n && same_plan(first, &rs[checked]); ++checked) {
+                        TRY(check_next(ctx, &rs[checked], &L, &fused, &nothing));
+                        if (!fused || nothing) break;
+                    }
+                    break;
                 }
+                if (!same_plan(first, &rs[i])) break;
+                TRY(check_next(ctx, &rs[i], &L, &fused, &nothing));
+                if (!fused || nothing) break;
             } else if (first->algo == MCCLX_ALGO_TREE) {
                 plan_phases(first, L, ph);
                 ph.folds[0].segs.reserve(n - i < (uint32_t)kPieceEntries ? n - i : (uint32_t)kPieceEntries);

@@ -135,6 +135,26 @@ int main() {
         printf("FAILED: %ld questions about small workspaces, %ld in all\n", asked, null_memory_questions.load());
         ++g_bad;
     }
+    {   // a list long enough for three pieces with one bad entry is refused whole, wherever that entry is
+        const int entries = 5000;
+        std::vector<float> a(size_t(entries) * 4100, 1.f), b(a.size(), 1.f);
+        for (int wrong : {0, 2047, 2048, 3000, 4999}) {
+            std::vector<void*> p;
+            std::vector<mcclx_replay> reps;
+            for (int e = 0; e < entries; ++e) {
+                p.push_back(&a[size_t(e) * 4100]);
+                p.push_back(e == wrong ? nullptr : &b[size_t(e) * 4100]);
+            }
+            for (int e = 0; e < entries; ++e) reps.push_back(replay(2, MCCLX_ALGO_TREE, MCCLX_SUM, 0, MCCLX_REPLAY_FUSED, e % 3 ? 4100 : 4096, &p[size_t(2 * e)]));
+            const unsigned long long before = mcclx_launch_count(ctx);
+            const int rc = mcclx_allreduce_replay_many(ctx, reps.data(), uint32_t(entries));
+            mcclx_queue_drain(ctx);
+            if (rc != MCCLX_ERR_INVALID || mcclx_launch_count(ctx) != before || a[0] != 1.f) {
+                printf("FAILED: a bad entry at %d: code %d, %llu launches\n", wrong, rc, static_cast<unsigned long long>(mcclx_launch_count(ctx) - before));
+                ++g_bad;
+            }
+        }
+    }
     {
         std::vector<std::vector<float>> data(12, std::vector<float>(4096, 1.f));
         std::vector<void*> p;
