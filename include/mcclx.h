@@ -135,6 +135,10 @@ MCCLX_API uint64_t mcclx_launch_count(mcclx_ctx* ctx);
 MCCLX_API int mcclx_set_hold(mcclx_ctx* ctx, int enabled);
 /* Diagnostic: launches of this context that took the hold form. */
 MCCLX_API uint64_t mcclx_hold_launch_count(mcclx_ctx* ctx);
+/* Diagnostic: launches of this context that wrote mcclx_queue_wait's word themselves, and by-value fold
+ * launches that ran in blocks of four wavefronts. */
+MCCLX_API uint64_t mcclx_marked_launch_count(mcclx_ctx* ctx);
+MCCLX_API uint64_t mcclx_four_wave_launch_count(mcclx_ctx* ctx);
 /* Diagnostic: the model behind that time -- no store before `latency_ticks` +
  * bytes read / `bytes_per_tick` ticks of a 100 MHz clock after a block's start.
  * The rate is measured on the device when the first context of a process is made

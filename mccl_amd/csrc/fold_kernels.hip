@@ -41,7 +41,7 @@ namespace mcclx {
 namespace {
 
 // Launch shapes, each measured on MI355X.  By-value launches run one-wavefront blocks of one
-// packet per lane (Cfg::FEW_U, kSmallShape, four_waves): a block of eight wavefronts keeps its slots until
+// packet per lane (Cfg::FEW_U, kSmallShape, launch_few): a block of eight wavefronts keeps its slots until
 // the last of its loads is back, one-wavefront blocks turn them over one by one (operands of
 // 128-512 MiB: one fp32 operand scaled 84.5 -> 80.9 us, own fp32 + one bf16 peer 106 -> 99.6,
 // + two peers 124 -> 119.5, copy 82.6 -> 80.6; 25 MiB operands: 10.3 -> 9.5, 12.5 -> 11.4,
@@ -1009,19 +1009,6 @@ static bool off_lines(const FewArgs& a) {
     return false;
 }
 
-// Blocks of four wavefronts for a by-value launch of `waves` one-wavefront tiles whose streams share one
-// element size?  Such launches take one-wavefront blocks (C::BLOCK) because those turn their slots over
-// one by one; one that one generation of waves covers turns nothing over, and four waves of a block spread over a
-// CU's four SIMDs where blocks of one pile up on some.  Cold, blocks of one and of four (us): 8 ranks of
-// 1 M bf16 in place (1950 waves) 9.3 and 7.8, of 0.5 M fp32 9.1 and 7.6, eight bf16 operands into one (4000)
-// 9.0 and 8.0, (6000) 11.6 and 10.8; two operands into one (5000) 4.6 and 4.1, two ranks in place (5500) 5.7 and
-// 5.0; four ranks (1400) 4.5 and 4.1, (5000) 9.2 and 8.9.  In between and above, blocks of one again: three or four
-// ranks (2500) 5.5 and 5.7, eight (8000) 26.4 and 27.8, two operands into one (12000) 7.7 and 8.1.
-static bool four_waves(uint64_t waves, int k) {
-    if (k >= 5) return waves >= 480 && waves < 6144;
-    return (waves >= 960 && waves < 2048) || (waves >= 4608 && waves < (k == 2 ? 7680u : 6144u));
-}
-
 // A by-value launch: one block per tile of the longest segment, the hold form where it applies.
 template <class C, int OUT>
 static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchParams& lp) {
@@ -1048,6 +1035,7 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
         const uint64_t gx = (maxc + span - 1) / span;
         if (gx * B >> 32) return hipErrorInvalidValue;  // (see few_fits)
         const dim3 grid((uint32_t)gx, (uint32_t)a.nseg);
+        if (B == kFourWaves && lp.four) *lp.four = true;
         if (OUT != kOutOne && lp.mark && gx * (uint64_t)a.nseg <= kMarkBlocks) {
             a.mark_word = lp.mark->word;
             a.mark_count = lp.mark->count;
@@ -1075,8 +1063,18 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
         if constexpr (C::BLOCK == kBlock)
             if (off_lines<C, OUT>(a))
                 return go(std::integral_constant<int, kBlock>{}, std::integral_constant<int, C::U>{}, 0);
-    } else if (four_waves(waves, C::K) || (OUT != kOutOne && lp.mark && waves > kMarkBlocks && waves <= 4 * kMarkBlocks)) {
-        return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
+    } else {
+        // Streams of one element size: one-wavefront blocks turn their slots over one by one.  Blocks of four are
+        // four times as few to hand out, but a CU more or less of them is four waves: 1.25 blocks a CU take up to 30 %
+        // longer than five waves (eight 16-bit operands into one 4.3 and 5.6 us), 4.25 no longer.  Five operands or more into
+        // one therefore take them from four blocks a CU on: 4096 to 49152 waves 0.95-1.13 times as fast, 3 % on average
+        // (eight fp32 operands, 6144 waves, 12.5 -> 11.2 us), below that 0.76-1.06; folds in place or to several gain nothing on
+        // average at any size (0.98-1.03), nor do up to four operands.  Not beside resident_lds, which counts blocks of one.
+        if (OUT == kOutOne && C::K >= 5 && lds == 0 && waves >= 16 * (uint64_t)lp.cus)
+            return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
+        // few enough blocks of four to tell of their end (kMarkBlocks), too many of one
+        if (OUT != kOutOne && lp.mark && waves > kMarkBlocks && waves <= 4 * kMarkBlocks)
+            return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
     }
     return go(std::integral_constant<int, kOneWave>{}, Few{}, lds);
 }

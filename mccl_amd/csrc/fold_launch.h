@@ -93,6 +93,7 @@ struct LaunchParams {
     // wall clock have passed since its block started.
     int cus = 0;
     bool* held = nullptr;              // set when the launch took that form (diagnostic)
+    bool* four = nullptr;              // set when a by-value launch took blocks of four wavefronts (diagnostic)
     uint64_t hold_min_read_bytes = 0;
     uint32_t hold_latency_ticks = 40;
     uint32_t hold_bytes_per_tick = 72000;

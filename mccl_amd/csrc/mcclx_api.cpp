@@ -89,7 +89,7 @@ struct mcclx_ctx {
     uint32_t wall_khz = 100000;                                      // the device's wall clock
     bool hold_measured = false;        // the gate's rate was measured on this device (not the default)
     std::atomic<bool> hold_enabled{true};  // a completer thread may switch it while ranks launch
-    std::atomic<uint64_t> hold_launches{0};
+    std::atomic<uint64_t> hold_launches{0}, four_launches{0}, marked_launches{0};
     bool batch_active = false;
     std::string batch_label;
     std::mutex mu;
@@ -617,6 +617,8 @@ int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, in
     lp.cus = ctx->cus;
     bool held = false;
     lp.held = &held;
+    bool four = false;
+    lp.four = &four;
     lp.hold_min_read_bytes = ctx->hold_enabled.load(std::memory_order_relaxed) ? ctx->hold_min_read_bytes : 0;
     lp.hold_latency_ticks = (uint32_t)((uint64_t)ctx->hold_latency_ticks * ctx->wall_khz / 100000);
     lp.hold_bytes_per_tick = (uint32_t)((uint64_t)ctx->hold_bytes_per_tick * 100000 / ctx->wall_khz);
@@ -640,9 +642,11 @@ int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, in
     if (mark.taken) {
         g_mark->number = ++ctx->word_number;
         g_mark->upto = ctx->issued.load(std::memory_order_relaxed);
+        ++ctx->marked_launches;
     }
     ++ctx->launches;
     if (held) ++ctx->hold_launches;
+    if (four) ++ctx->four_launches;
     return MCCLX_OK;
 }
 
@@ -1019,6 +1023,8 @@ void* mcclx_queue_stream(mcclx_ctx* ctx) {
 int mcclx_device_cus(mcclx_ctx* ctx) { return ctx ? ctx->cus : 0; }
 uint64_t mcclx_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->launches.load() : 0; }
 uint64_t mcclx_hold_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->hold_launches.load() : 0; }
+uint64_t mcclx_marked_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->marked_launches.load() : 0; }
+uint64_t mcclx_four_wave_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->four_launches.load() : 0; }
 int mcclx_hold_model(mcclx_ctx* ctx, uint32_t* latency_ticks, uint32_t* bytes_per_tick) {
     if (!ctx) return 0;
     if (latency_ticks) *latency_ticks = ctx->hold_latency_ticks;

@@ -205,6 +205,14 @@ class ReduceQueue:
         writes once the reads are through (diagnostic)."""
         return int(L.lib().mcclx_hold_launch_count(self.handle))
 
+    def marked_launch_count(self) -> int:
+        """Launches of this queue that told the host of their own end (diagnostic)."""
+        return int(L.lib().mcclx_marked_launch_count(self.handle))
+
+    def four_wave_launch_count(self) -> int:
+        """Fold launches of this queue in blocks of four wavefronts (diagnostic)."""
+        return int(L.lib().mcclx_four_wave_launch_count(self.handle))
+
     def set_hold(self, enabled: bool) -> None:
         """Switch the hold form of fold launches off (a queue whose launches overlap with other
         work on the GPU) or on again."""

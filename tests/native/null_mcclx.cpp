@@ -162,6 +162,8 @@ void* mcclx_queue_stream(mcclx_ctx* c) { return c; }
 int mcclx_device_cus(mcclx_ctx*) { return 256; }
 uint64_t mcclx_launch_count(mcclx_ctx* c) { return c ? c->launches.load() : 0; }
 uint64_t mcclx_hold_launch_count(mcclx_ctx*) { return 0; }
+uint64_t mcclx_marked_launch_count(mcclx_ctx*) { return 0; }
+uint64_t mcclx_four_wave_launch_count(mcclx_ctx*) { return 0; }
 int mcclx_set_hold(mcclx_ctx*, int) { return MCCLX_OK; }
 int mcclx_hold_model(mcclx_ctx*, uint32_t* a, uint32_t* b) {
     if (a) *a = 40;
