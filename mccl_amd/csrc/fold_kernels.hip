@@ -1116,22 +1116,22 @@ static hipError_t launch_table(hipStream_t st, const TableArgs& args, const Laun
     TableArgs a = args;
     const uint32_t grid = (uint32_t)(a.total_items < lp.max_blocks ? a.total_items : lp.max_blocks);
     if (grid == 0) return hipSuccess;
-    // Fewer waves resident (resident_lds) only for launches that write to four places or more, or
+    // Fewer waves resident (resident_lds) only for launches that write to three places or more, or
     // back into all operands: a block fetches its work item and its descriptor before its operands,
     // and with one output or two the waves that are left do not hide that.  Without the limit and
     // with it, 4096 messages of 64 KB: three operands into one 167 and 181 us, eight 393 and 414,
-    // two operands to two 172 and 192, three to three 266 and 267; four to four 377 and 351.
+    // two operands to two 172 and 192; four to four 377 and 351.
     // In place, 1024 messages: three ranks 72 and 68 us, five 123 and 113, eight 206 and 187.
-    // Three operands to three, 16 waves resident: 1.6 GB 261 and 248 us, 0.8 GB 130 and 126, 0.5 GB 86 and 86.
+    // To three, as many waves as resident_lds leaves at most.  Three operands, lists of 200 MB to 3.2 GB in messages of 4 to
+    // 256 KB, the time without the limit over the time with 12 / 16 / 18 / 20 waves: fp32 0.94-1.04 / 1.00-1.06 / 1.00-1.05 /
+    // 1.00-1.03, the wire form 0.91-1.04 / 0.99-1.05 / 0.99-1.03 / 0.99-1.03, bf16 0.87-1.01 / 0.97-1.05 / 0.99-1.04 /
+    // 0.99-1.01, fp16 0.93-1.06 / 0.99-1.05 / 0.99-1.03 / 1.00-1.02; most where much is moved (1.6 GB of fp32 265 -> 253 us).
     uint32_t lds = 0;
     const int outputs = OUT == kOutAll ? C::K : 1 + a.fan;
-    if (C::BLOCK == kOneWave && OUT == kOutFan && outputs == 3 && C::E == 4 && C::K == 3 &&
-        a.total_items * 64 * (uint64_t)(C::U * (C::kReadBytes + 48)) >= 600'000'000)
-        lds = 163840u / 16u / 1280u * 1280u;
-    if (C::BLOCK == kOneWave && (OUT == kOutAll || outputs >= 4)) {
+    if (C::BLOCK == kOneWave && (OUT == kOutAll || outputs >= 3)) {
         const int lane_bytes = C::U * (C::kReadBytes + outputs * ((C::W == MCCLX_F32 || C::kOutF32) ? 16 : 2 * C::E));
         lds = resident_lds(a.total_items * 64 * (uint64_t)lane_bytes, lane_bytes, outputs,
-                           OUT == kOutAll ? kLaneBytesInPlace : kLaneBytes);
+                           OUT == kOutAll ? kLaneBytesInPlace : outputs == 3 ? kMostResident * lane_bytes : kLaneBytes);
     }
     if constexpr (OUT == kOutAll)
         fold_table_all_kernel<C><<<dim3(grid), dim3(C::BLOCK), lds, st>>>(a);

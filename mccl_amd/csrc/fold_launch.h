@@ -146,11 +146,12 @@ hipError_t launch_fold(hipStream_t st, const PlanKey& key, const LaunchParams& l
 constexpr uint64_t kResidentMinBytes = 160'000'000;
 constexpr uint64_t kResidentMinBytesCopy = 90'000'000;
 constexpr int kLaneBytes = 1160, kLaneBytesInPlace = 1280, kLaneBytesCopy = 1020;
+constexpr int kMostResident = 18;
 inline uint32_t resident_lds(uint64_t launch_bytes, int lane_bytes, int outputs, int budget = kLaneBytes,
                              uint64_t min_bytes = kResidentMinBytes) {
     int waves = budget / lane_bytes;
     if (launch_bytes < min_bytes || (outputs == 1 && waves >= 20)) return 0;
-    waves = waves > 18 ? 18 : waves < 3 ? 3 : waves;  // three blocks reserve 53 KiB each: a launch may ask for 64 KiB
+    waves = waves > kMostResident ? kMostResident : waves < 3 ? 3 : waves;  // three blocks reserve 53 KiB each: a launch may ask for 64 KiB
     return 163840u / (uint32_t)waves / 1280u * 1280u;
 }
 

@@ -191,10 +191,10 @@ struct MarkScope {
 // stream synchronisation of the caller's finds the completion signal it waits for (without one it puts a marker on
 // the queue then: 11 us instead of 5.5).  The event takes the queue some 3 us, so it is left out where the
 // next call starts at once, as this one did: within kQuickNs of the return before it.  Calls back to back start
-// after 1.4-3.6 us, behind a synchronisation after 6.5-15.  A maximum of 4 KB over eight ranks (us): back to back 13.6
+// after 1.4-6 us, behind a synchronisation after 6.5-15.  A maximum of 4 KB over eight ranks (us): back to back 13.6
 // with the event always, 10.8 never, 10.8 by this rule; each with a synchronisation behind it 15.5, 21.6 and 15.5 (through
 // hipStreamSynchronize and no word 14.2 and 17.4).
-constexpr int64_t kQuickNs = 5000;
+constexpr int64_t kQuickNs = 6000;
 int64_t now_ns() {
     return std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
