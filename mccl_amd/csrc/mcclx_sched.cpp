@@ -17,6 +17,7 @@
 // kernels would, so both modes give bit-identical tensors.
 
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -653,9 +654,12 @@ int check_replay(mcclx_ctx* ctx, const mcclx_replay* r, Layout* L, bool* fused, 
     return MCCLX_OK;
 }
 
-// The same for an entry of a list with the plan of the entry before it, whose size may be the same too.
+// Does the entry of a list ask for what the entry before it does, of tensors of the same size?
+bool alike(const mcclx_replay* r) { return memcmp(r, r - 1, offsetof(mcclx_replay, tensors)) == 0; }
+
+// The same for an entry with the plan of the entry before it.
 int check_next(mcclx_ctx* ctx, const mcclx_replay* r, Layout* L, bool* fused, bool* nothing_to_do) {
-    if (r->tensors && r->reserved == 0 && r->numel == r[-1].numel) return check_memory(r, *L);
+    if (r->tensors && alike(r)) return check_memory(r, *L);
     return check_replay(ctx, r, L, fused, nothing_to_do);
 }
 
@@ -751,13 +755,13 @@ int allreduce_replay_many(mcclx_ctx* ctx, const mcclx_replay* rs, uint32_t n) {
                 // a long list goes out in pieces: see kPieceEntries
                 if (&rs[i] - first >= kPieceEntries && moved >= kPieceBytes) {
                     // (what is wrong with an entry of its other pieces is said before this one is issued)
-                    for (checked = checked > i ? checked : i; checked < n && same_plan(first, &rs[checked]); ++checked) {
+                    for (checked = checked > i ? checked : i; checked < n && (alike(&rs[checked]) || same_plan(first, &rs[checked])); ++checked) {
                         TRY(check_next(ctx, &rs[checked], &L, &fused, &nothing));
                         if (!fused || nothing) break;
                     }
                     break;
                 }
-                if (!same_plan(first, &rs[i])) break;
+                if (!alike(&rs[i]) && !same_plan(first, &rs[i])) break;
                 TRY(check_next(ctx, &rs[i], &L, &fused, &nothing));
                 if (!fused || nothing) break;
             } else if (first->algo == MCCLX_ALGO_TREE) {
