@@ -93,10 +93,8 @@ int run(mcclx_ctx* ctx, int device, std::vector<mcclx_replay>& reps) {
     void* stream = dev::current_stream(device);
     py::gil_scoped_release unlocked;
     // The call waits in any case: the workspace goes back to the allocator.  Tensors and workspace are device
-    // memory, so the end of the queue may be seen early (mcclx_queue_wait); not for a list nor for a call that
-    // moves more than 500 MB, where that gains nothing (1000 messages of 20 KB 105 us against 101, 3.5 GB level) and
-    // a synchronisation of the caller's behind it would take 10-30 us.
-    const bool early = reps.size() == 1 && static_cast<uint64_t>(reps[0].world) * reps[0].numel * (reps[0].dtype == MCCLX_F32 ? 8u : 4u) < 500'000'000;
+    // memory, so the end of the queue may be seen early (mcclx_queue_wait); not for a list, where that gains nothing.
+    const bool early = reps.size() == 1;
     const int rc = mcclx_queue_wait_stream(ctx, stream);
     if (rc != MCCLX_OK) return rc;  // nothing has been issued
     return mcclx_allreduce_replay_wait(ctx, reps.data(), static_cast<uint32_t>(reps.size()), early ? kWaitSpinUs : 0);
