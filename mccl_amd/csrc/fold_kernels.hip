@@ -232,16 +232,19 @@ struct Cfg {
     }();
     // Bytes under way per CU that a large launch is held to (resident_lds).  The longer a wave computes
     // between its loads and its stores, the more waves it takes to keep as many under way: bf16 rounds
-    // after every operand, fp16 in one instruction, the wire form once more on the way in, fp32 never.
-    // Eight ranks in place, 3 / 4 / 5 waves per CU (us): bf16 12.5 M 80.5 / 71.3 / 67.8, fp16 50 M 249 / 252 /
-    // 263, the wire form 8 M 86.8 / 80.9 / 83.4, fp32 40 M 407 / 414 / 425; five ranks of 40 M, 5 / 6 / 7 / 8:
-    // the wire form 261 / 249 / 249 / 251, fp32 246 / 250 / 252 / 254.
-    static constexpr int kInPlaceBudget = W == MCCLX_F32 ? (K >= 5 ? 800 : kLaneBytesInPlace)
-                                          : W == MCCLX_F16 ? 1024
+    // after every operand, fp16 in one instruction, the wire form once more on the way in, fp32 never; the kernels of
+    // MIN, MAX and PRODUCT choose their operator for every operand (kAnyOp).
+    // Sums of eight ranks in place, 3 / 4 / 5 waves per CU, 0.8 GB moved (us): fp32 133 / 136 / 138, fp16 135 / 136 / 138,
+    // the wire form 146 / 138 / 137, bf16 165 / 145 / 137; of seven fp32 ranks 137 / 133 / 136.  MAX of eight fp32 ranks
+    // 161 / 141 / 138, of seven 170 / 144 / 136, of seven fp16 ranks 186 / 156 / 143.
+    static constexpr int kInPlaceBudget = OP == kAnyOp       ? kLaneBytesInPlace
+                                          : W == MCCLX_F32   ? (K >= 5 ? 900 : kLaneBytesInPlace)
+                                          : W == MCCLX_F16   ? 1024
                                           : IO == MCCLX_IO_ALL_F32 ? 1130 : kLaneBytesInPlace;
     // (fan-out of 100 M elements, 7 / 8 / 9 / 10 / 12 waves: four ranks over the wire form 496 / 496 / 504 / 513 / 511,
-    // three 398 / 378 / 367 / 367 / 375, four of bf16 268 / 251 / 246 / 248 / 257)
-    static constexpr int kFanBudget = (W == MCCLX_F32 || IO == MCCLX_IO_ALL_F32) ? 1024 : kLaneBytes;
+    // three 398 / 378 / 367 / 367 / 375, four of bf16 268 / 251 / 246 / 248 / 257; two fp32 ranks of 188 M, 14 / 16 / 18 waves
+    // 467 / 464 / 460)
+    static constexpr int kFanBudget = K >= 3 && (W == MCCLX_F32 || IO == MCCLX_IO_ALL_F32) ? 1024 : kLaneBytes;
     // bytes a lane reads per packet
     static constexpr int kReadBytes = [] {
         int b = 0;
