@@ -306,6 +306,11 @@ MCCLX_API int mcclx_queue_drain(mcclx_ctx* ctx);
  * polls a word that the queue's end writes, for spin_us microseconds; if it has not come by then, or with
  * spin_us = 0, the call drains. */
 MCCLX_API int mcclx_queue_wait(mcclx_ctx* ctx, uint32_t spin_us);
+/* A stream or device synchronisation behind mcclx_queue_wait is 5 us shorter if the call has left an event behind
+ * the launches, and the next launch some 3 us later.  A call leaves one unless it began within gap_us of the
+ * last one's return, where the next is expected to follow as soon (default 6; a queue that several threads use
+ * in turn wants more). */
+MCCLX_API int mcclx_set_wait_gap(mcclx_ctx* ctx, uint32_t gap_us);
 /* The queue waits (on the device, host not blocked) for everything enqueued so
  * far on `producer_stream`.  Replaces mps_stream_sync (MPSInterop.mm:308-310)
  * and mps_event_sync_nonblocking + wait_for_mps (:336-356, EventSync.mm:112-132). */

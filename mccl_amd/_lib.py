@@ -99,6 +99,7 @@ SIGNATURES = {
     "mcclx_copy_batched": (_i, [_vp, C.POINTER(CopyDesc), C.c_uint32]),
     "mcclx_queue_drain": (_i, [_vp]),
     "mcclx_queue_wait": (_i, [_vp, C.c_uint32]),
+    "mcclx_set_wait_gap": (_i, [_vp, C.c_uint32]),
     "mcclx_queue_wait_stream": (_i, [_vp, _vp]),
     "mcclx_stream_wait_queue": (_i, [_vp, _vp]),
     "mcclx_event_record": (_i, [_vp, C.POINTER(C.c_uint64)]),

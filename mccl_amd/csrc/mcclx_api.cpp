@@ -129,7 +129,8 @@ struct mcclx_ctx {
     hipEvent_t word_ev = nullptr;
     uint32_t* mark_count = nullptr;  // device memory: blocks of a marked launch that have ended (LaunchMark)
     // When mcclx_queue_wait last returned (steady clock, ns), whether nothing has been put on the queue since, and
-    // whether what came next came within kQuickNs.  A hint: a wait is right either way.
+    // whether what came next came within quick_ns.  A hint: a wait is right either way.
+    std::atomic<int64_t> quick_ns{6000};
     std::atomic<int64_t> waited_at{0};
     std::atomic<bool> resting{false}, quick{false};
     uint64_t word_number = 0;      // the last number handed out (under away_mu)
@@ -190,17 +191,16 @@ struct MarkScope {
 // A call that returns early (mcclx_queue_wait) leaves an event behind its launches, in which a device-wide or
 // stream synchronisation of the caller's finds the completion signal it waits for (without one it puts a marker on
 // the queue then: 11 us instead of 5.5).  The event takes the queue some 3 us, so it is left out where the
-// next call starts at once, as this one did: within kQuickNs of the return before it.  Calls back to back start
+// next call starts at once, as this one did: within quick_ns of the return before it.  Calls back to back start
 // after 1.4-6 us, behind a synchronisation after 6.5-15.  A maximum of 4 KB over eight ranks (us): back to back 13.6
 // with the event always, 10.8 never, 10.8 by this rule; each with a synchronisation behind it 15.5, 21.6 and 15.5 (through
 // hipStreamSynchronize and no word 14.2 and 17.4).
-constexpr int64_t kQuickNs = 6000;
 int64_t now_ns() {
     return std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 void note_start(mcclx_ctx* ctx) {
     if (ctx->resting.load(std::memory_order_relaxed) && ctx->resting.exchange(false, std::memory_order_relaxed))
-        ctx->quick.store(now_ns() - ctx->waited_at.load(std::memory_order_relaxed) < kQuickNs, std::memory_order_relaxed);
+        ctx->quick.store(now_ns() - ctx->waited_at.load(std::memory_order_relaxed) < ctx->quick_ns.load(std::memory_order_relaxed), std::memory_order_relaxed);
 }
 
 // The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its
@@ -1470,7 +1470,7 @@ static int queue_wait(mcclx_ctx* ctx, uint32_t spin_us, const MarkRequest& mark)
                 HIP_TRY(mcclx::launch_word(use, ctx->word_dev, number));
                 lk = std::move(use.lk);
             }
-            if (!ctx->quick.load(std::memory_order_relaxed)) {  // see kQuickNs
+            if (!ctx->quick.load(std::memory_order_relaxed)) {  // see note_start
                 HIP_TRY(hipEventRecord(ctx->word_ev, st));
                 ctx->marked.store(ctx->issued.load(std::memory_order_relaxed), std::memory_order_release);
             }
@@ -1492,6 +1492,12 @@ static int queue_wait(mcclx_ctx* ctx, uint32_t spin_us, const MarkRequest& mark)
         } while (std::chrono::steady_clock::now() < until);
     }
     HIP_TRY(drain(ctx));  // also what reports a launch that failed
+    return MCCLX_OK;
+}
+
+int mcclx_set_wait_gap(mcclx_ctx* ctx, uint32_t gap_us) {
+    if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
+    ctx->quick_ns.store((int64_t)gap_us * 1000, std::memory_order_relaxed);
     return MCCLX_OK;
 }
 

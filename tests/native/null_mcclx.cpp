@@ -165,6 +165,7 @@ uint64_t mcclx_hold_launch_count(mcclx_ctx*) { return 0; }
 uint64_t mcclx_marked_launch_count(mcclx_ctx*) { return 0; }
 uint64_t mcclx_four_wave_launch_count(mcclx_ctx*) { return 0; }
 int mcclx_set_hold(mcclx_ctx*, int) { return MCCLX_OK; }
+int mcclx_set_wait_gap(mcclx_ctx*, uint32_t) { return MCCLX_OK; }
 int mcclx_hold_model(mcclx_ctx*, uint32_t* a, uint32_t* b) {
     if (a) *a = 40;
     if (b) *b = 72000;

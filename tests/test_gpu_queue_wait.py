@@ -212,6 +212,29 @@ def test_a_synchronisation_behind_each_call_finds_a_signal_to_wait_for(env, what
     assert min(median_sync(0) for _ in range(3)) < 1.5 * alone
 
 
+@pytest.mark.parametrize("gap_us", [0, 6, 10_000_000])
+def test_results_hold_with_any_gap(env, gap_us):
+    """An event behind every call, behind some and behind none."""
+    L, K = env
+    from mccl_amd import harness as H
+    q = K.ReduceQueue(0)
+    try:
+        L.check(L.lib().mcclx_set_wait_gap(q.handle, gap_us))
+        for n in (1_000, 100_001):
+            a, b = torch.zeros(n, device="cuda"), torch.ones(n, device="cuda")
+            for rep in range(20):
+                b.fill_(1)
+                H.allreduce_replay([a, b], "sum", L.ALGO_TREE, queue=q)
+                if rep % 3 == 0:
+                    torch.cuda.synchronize()
+                K.hip_accumulate_chunk(a, b, queue=q)
+                a.sub_(b)
+            assert a.cpu().eq(20).all()
+        assert L.lib().mcclx_set_wait_gap(C.c_void_p(None), 1) == L.ERR_STATE
+    finally:
+        q.close()
+
+
 def test_making_a_queue_does_not_wait_for_the_default_stream(env):
     _, K = env
     K.ReduceQueue(0).close()  # what a process does once is done
@@ -281,14 +304,18 @@ def test_small_allreduces_that_tell_of_their_own_end(env, world, dtype):
     K.hip_kernels_init(0)
     dt = {"fp32": torch.float32, "wire": torch.float32, "bf16": torch.bfloat16, "fp16": torch.float16}[dtype]
     side = torch.cuda.Stream()
-    sizes = [world, 63, 255, 1_000, 4_097, 8_192 * world, 300_000, 16_385, 2_047, 70_001, 500, 32_768, 33_000]
+    q = K._q(None)
+    sizes = [1, world, 63, 255, 1_000, 4_097, 8_192 * world, 300_000, 16_385, 2_047, 70_001, 500, 32_768, 33_000]
     for op in ("sum", "max"):
         for rep in range(3):
             for n in sizes:
                 ts = [((torch.arange(n, device="cuda") * (r + 2) + rep) % 9 - 4).to(dt) for r in range(world)]
                 stack = torch.stack([t.float() for t in ts])
                 want = stack.sum(0) if op == "sum" else stack.amax(0)
+                told = q.marked_launch_count()
                 H.allreduce_replay(ts, op, L.ALGO_BUTTERFLY if n >= world else L.ALGO_TREE, wire_bf16=dtype == "wire", mode=L.REPLAY_DIRECT)
+                told = q.marked_launch_count() - told
+                assert told == 1 if n <= 4_097 else told == 0 if n >= 70_001 else told <= 1, n
                 with torch.cuda.stream(side):
                     doubled = [t.float() * 2 for t in ts]
                 host = [t.cpu().float() for t in ts]
