@@ -1459,6 +1459,7 @@ static int queue_wait(mcclx_ctx* ctx, uint32_t spin_us, const MarkRequest& mark)
     DeviceGuard guard(ctx->device);
     if (spin_us && ctx->word && !ctx->away.load(std::memory_order_acquire) && !records(ctx->stream)) {
         uint64_t upto = mark.upto, number = mark.number;
+        bool coming = true;  // the number; what fails here leaves the wait to the drain
         {
             std::unique_lock<std::mutex> lk(ctx->away_mu);
             hipStream_t st = ctx->stream;
@@ -1467,17 +1468,19 @@ static int queue_wait(mcclx_ctx* ctx, uint32_t spin_us, const MarkRequest& mark)
                 QueueUse use = queue_of(ctx);
                 upto = ctx->issued.load(std::memory_order_relaxed);
                 number = ++ctx->word_number;
-                HIP_TRY(mcclx::launch_word(use, ctx->word_dev, number));
+                coming = mcclx::launch_word(use, ctx->word_dev, number) == hipSuccess;
                 lk = std::move(use.lk);
             }
-            if (!ctx->quick.load(std::memory_order_relaxed)) {  // see note_start
-                HIP_TRY(hipEventRecord(ctx->word_ev, st));
-                ctx->marked.store(ctx->issued.load(std::memory_order_relaxed), std::memory_order_release);
+            if (coming && !ctx->quick.load(std::memory_order_relaxed)) {  // see note_start
+                if (hipEventRecord(ctx->word_ev, st) == hipSuccess)
+                    ctx->marked.store(ctx->issued.load(std::memory_order_relaxed), std::memory_order_release);
+                else
+                    (void)hipGetLastError();
             }
         }
         const volatile uint64_t* word = ctx->word;
         const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(spin_us);
-        do {
+        while (coming) {
             for (int k = 0; k < 64; ++k) {
                 if (*word >= number) {  // numbers are written in the order they are handed out
                     std::atomic_thread_fence(std::memory_order_acquire);
@@ -1489,7 +1492,8 @@ static int queue_wait(mcclx_ctx* ctx, uint32_t spin_us, const MarkRequest& mark)
                 }
                 __builtin_ia32_pause();
             }
-        } while (std::chrono::steady_clock::now() < until);
+            coming = std::chrono::steady_clock::now() < until;
+        }
     }
     HIP_TRY(drain(ctx));  // also what reports a launch that failed
     return MCCLX_OK;
