@@ -21,6 +21,8 @@ typedef u32x4 Packet __attribute__((aligned(1)));
 constexpr int kBlock = 256;
 
 constexpr int kOneWave = 64, kFourWaves = 256;  // threads per block of a launch by value, see kOneWaveBlocksFrom
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kSpreadTile = kFourWaves * 32;  // bytes a block of copy_spread_kernel moves
 
 // Up to kFewCopies copies with their descriptors in the kernel arguments:
 // blockIdx.y picks the copy, blockIdx.x one tile of B packets of 16 bytes, one
@@ -70,6 +72,53 @@ __global__ void __launch_bounds__(B) copy_few_kernel(CopyFew a) {
         for (uint32_t i = threadIdx.x; i < head; i += B) byte(i);
         const uint64_t i = head + P * 16 + threadIdx.x;  // fewer than 16 bytes remain
         if (i < nbytes) byte(i);
+    }
+}
+
+// One source to N destinations, one destination after another.  copy_few_kernel reads a packet once and
+// stores it N times: N + 1 streams at a time, and the memory channels switch rows between them.  Here a
+// piece of the source goes to its first destination, then to the next, and then the next piece
+// follows: the first pass brings the piece into the L2 caches, the others read it there (ordinary loads; a
+// tile's number within the piece decides its XCD, for every destination alike), and memory sees one
+// stream of writes.  Bound by those: writes alone run at 6.6-7.2 TB/s, eight streams of them beside one read
+// at 6.2.  Eight to eight, us: 8 x 1 MiB 15.9 -> 12.6, 8 x 8 MiB 105 -> 90, 8 x 16 MiB 212 -> 183, 8 x 64 MiB 774 -> 744.
+// blockIdx.x is the tile of the piece, blockIdx.y copy and destination, blockIdx.z the piece.  An XCD takes
+// 2^group tiles in a row (blocks go to the XCDs in turn): 64 tiles, 512 KiB, 737 us, in turn 773.
+template <int N>
+__global__ void __launch_bounds__(kFourWaves) copy_spread_kernel(CopyFew a, uint64_t piece, uint32_t group) {
+    const uint32_t c = blockIdx.y / N, f = blockIdx.y - c * N;
+    const void* src = a.d[c].src;
+    void* dst = a.d[c].dst[f];
+    uint64_t nbytes = a.d[c].nbytes;
+    asm volatile("" : "+s"(src), "+s"(dst), "+s"(nbytes), "+s"(piece), "+s"(group));
+    const uint32_t xcd = blockIdx.x % kXcds, n = blockIdx.x / kXcds;
+    const uint32_t tile = (((n >> group) * kXcds + xcd) << group) + (n & ((1u << group) - 1));
+    const uint32_t mis = (0u - (uint32_t)reinterpret_cast<uintptr_t>(dst)) & 127u;  // packets start on a line of this destination
+    const uint32_t head = nbytes < mis ? (uint32_t)nbytes : mis;
+    const uint64_t whole = (nbytes - head) / 16 * 16;
+    const uint64_t first = blockIdx.z * piece + (uint64_t)tile * kSpreadTile;
+    const MCCLX_GLOBAL uint8_t* gs = (const MCCLX_GLOBAL uint8_t*)src;
+    MCCLX_GLOBAL uint8_t* gd = (MCCLX_GLOBAL uint8_t*)dst;
+    if (first < whole) {
+        const MCCLX_GLOBAL uint8_t* ps = gs + head + first;
+        MCCLX_GLOBAL uint8_t* pd = gd + head + first;
+        constexpr uint32_t half = kSpreadTile / 2;
+        const uint32_t off = threadIdx.x * 16u;
+        if (whole - first >= kSpreadTile) {
+            const u32x4 v0 = *(const MCCLX_GLOBAL Packet*)(ps + off), v1 = *(const MCCLX_GLOBAL Packet*)(ps + half + off);
+            COPY_ST((MCCLX_GLOBAL Packet*)(pd + off), v0);
+            COPY_ST((MCCLX_GLOBAL Packet*)(pd + half + off), v1);
+        } else {
+            const uint32_t left = (uint32_t)(whole - first);
+            if (off < left) COPY_ST((MCCLX_GLOBAL Packet*)(pd + off), *(const MCCLX_GLOBAL Packet*)(ps + off));
+            if (half + off < left)
+                COPY_ST((MCCLX_GLOBAL Packet*)(pd + half + off), *(const MCCLX_GLOBAL Packet*)(ps + half + off));
+        }
+    }
+    if (blockIdx.x == 0 && blockIdx.z == 0) {
+        if (threadIdx.x < head) gd[threadIdx.x] = gs[threadIdx.x];
+        const uint64_t i = head + whole + threadIdx.x;  // fewer than 16 bytes remain
+        if (i < nbytes) gd[i] = gs[i];
     }
 }
 
@@ -241,12 +290,68 @@ hipError_t launch_copy_few_n(hipStream_t st, const CopyFew& a) {
         copy_few_kernel<N, kOneWave, MIXED><<<grid, dim3(kOneWave), lds, st>>>(a);
     return hipGetLastError();
 }
+
+// Four blocks a CU: their writes lie close together (16 / 12 / 8 waves a CU, 8 x 64 MiB to eight: 735 / 734 / 763 us, two
+// copies of 8 MiB to two 8.7 / 8.9 / 9.3).
+constexpr uint32_t kSpreadLds = 163840 / 4;
+
+// Pieces of 8 to 12 MiB (1 to 1.5 MiB of each XCD's L2; 8 x 64 MiB to eight with 4 / 8 / 16 MiB: 755 / 737 / 735 us, 4 x 32 MiB
+// to four 97.0 / 95.2 / 95.2).  A source is cut where all pieces have one length and the XCDs take long runs of tiles, with at
+// most one block in sixteen without work.
+constexpr uint64_t kSpreadTiles = (8u << 20) / kSpreadTile;
+struct SpreadShape {
+    uint64_t pieces, tiles;  // tiles of a piece
+    uint32_t group;
+};
+SpreadShape spread_shape(uint64_t need) {  // tiles of the longest source, one at least
+    constexpr uint32_t kGroup = 6;
+    if (need > 16 * kSpreadTiles) return {(need + kSpreadTiles - 1) / kSpreadTiles, kSpreadTiles, kGroup};
+    const uint64_t most = (need + kSpreadTiles - 1) / kSpreadTiles, least = (2 * need + 3 * kSpreadTiles - 1) / (3 * kSpreadTiles);
+    for (uint32_t g = kGroup;; --g)
+        for (uint64_t p = most; p >= least; --p) {
+            const uint64_t step = kXcds << g, tiles = ((need + p - 1) / p + step - 1) / step * step;
+            if (g == 0 || (p * tiles - need) * 16 <= need) return {p, tiles, g};
+        }
+}
+// To two or three, pieces pay while the launch is small: 50 / 100 / 200 / 400 MB moved to two 1.2 / 1.12 / 0.95 / 0.94 times as
+// fast, to three 1.19 / 1.19 / 0.99 / 1.0; to four and more 1.0-1.26 times at every size from 100 KB to 5.6 GB (one of the 60
+// tried 0.98).
+constexpr uint64_t kSpreadToThree = 150'000'000;
+
+bool spread_pays(const CopyFew& a, bool local_sources) {
+    if (!local_sources || a.d[0].n < 2) return false;
+    uint64_t moved = 0;
+    for (uint32_t i = 0; i < a.n; ++i) moved += a.d[i].nbytes * (1 + a.d[i].n);
+    return a.d[0].n >= 4 || moved < kSpreadToThree;
+}
+
+template <int N>
+hipError_t launch_copy_spread(hipStream_t st, const CopyFew& a) {
+    uint64_t longest = 0;
+    for (uint32_t i = 0; i < a.n; ++i) longest = a.d[i].nbytes > longest ? a.d[i].nbytes : longest;
+    if (longest == 0) return hipSuccess;
+    const SpreadShape p = spread_shape((longest + kSpreadTile - 1) / kSpreadTile);
+    if (p.pieces > 65535) return hipErrorInvalidValue;
+    copy_spread_kernel<N><<<dim3((uint32_t)p.tiles, N * a.n, (uint32_t)p.pieces), dim3(kFourWaves), kSpreadLds, st>>>(
+        a, p.tiles * kSpreadTile, p.group);
+    return hipGetLastError();
+}
 }  // namespace
 
-hipError_t launch_copy_few(hipStream_t st, const CopyFew& a) {
+hipError_t launch_copy_few(hipStream_t st, const CopyFew& a, bool local_sources) {
     if (a.n == 0 || a.n > (uint32_t)kFewCopies) return a.n ? hipErrorInvalidValue : hipSuccess;
     for (uint32_t i = 1; i < a.n; ++i)
         if (a.d[i].n != a.d[0].n) return launch_copy_few_n<kCopyDsts, true>(st, a);
+    if (spread_pays(a, local_sources)) switch (a.d[0].n) {
+        case 2: return launch_copy_spread<2>(st, a);
+        case 3: return launch_copy_spread<3>(st, a);
+        case 4: return launch_copy_spread<4>(st, a);
+        case 5: return launch_copy_spread<5>(st, a);
+        case 6: return launch_copy_spread<6>(st, a);
+        case 7: return launch_copy_spread<7>(st, a);
+        case 8: return launch_copy_spread<8>(st, a);
+        default: return hipErrorInvalidValue;
+    }
     switch (a.d[0].n) {
         case 1: return launch_copy_few_n<1>(st, a);
         case 2: return launch_copy_few_n<2>(st, a);
@@ -264,7 +369,7 @@ hipError_t launch_copy(hipStream_t st, void* dst, const void* src, uint64_t nbyt
     CopyFew a;
     a.d[0] = CopyDesc{src, nbytes, 1, {dst}};
     a.n = 1;
-    return launch_copy_few(st, a);
+    return launch_copy_few(st, a, false);
 }
 
 }  // namespace mcclx

@@ -186,7 +186,9 @@ struct CopyFew {
     CopyDesc d[kFewCopies];
     uint32_t n;
 };
-hipError_t launch_copy_few(hipStream_t st, const CopyFew& copies);
+// `local_sources`: every source lies in this device's own memory, which its caches hold (a copy to several
+// destinations may then read it more than once).
+hipError_t launch_copy_few(hipStream_t st, const CopyFew& copies, bool local_sources);
 // Work items (tiles) one copy of nbytes splits into.
 uint64_t copy_items(uint64_t nbytes);
 // `most`: the largest number of destinations any descriptor of the launch has.

@@ -440,6 +440,16 @@ int check_range(const void* p, uint64_t nbytes, const char* what, uint32_t seg) 
     return MCCLX_OK;
 }
 
+// Is `p` memory of the context's own device?  (0.06 us)
+bool in_device_memory(const mcclx_ctx* ctx, const void* p) {
+    hipPointerAttribute_t attr;
+    if (hipPointerGetAttributes(&attr, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return attr.type == hipMemoryTypeDevice && attr.device == ctx->device;
+}
+
 int check_segs(mcclx_ctx* ctx, const mcclx::PlanKey& key, const mcclx_seg* segs, uint32_t nseg, int fan) {
     if (!segs && nseg) return fail(MCCLX_ERR_INVALID, "segment array is null");
     const bool out_f32 = key.dtype == MCCLX_F32 || key.io != MCCLX_IO_PURE;
@@ -1364,7 +1374,9 @@ static int copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n
         uint64_t longest = 0, sum = 0;
         auto flush = [&]() -> int {
             if (few.n == 0) return MCCLX_OK;
-            hipError_t e = mcclx::launch_copy_few(queue_of(ctx), few);
+            bool local = true;
+            for (uint32_t i = 0; local && i < few.n; ++i) local = few.d[i].n < 2 || in_device_memory(ctx, few.d[i].src);
+            hipError_t e = mcclx::launch_copy_few(queue_of(ctx), few, local);
             if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy_batched launch failed: %s", hipGetErrorString(e));
             ++ctx->launches;
             few.n = 0;

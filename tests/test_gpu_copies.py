@@ -60,3 +60,49 @@ def test_allgather_of_odd_chunks(world, in_place):
         H.allgather_replay(outs, ins)
         want = torch.cat(parts)
         assert all(torch.equal(o.view(torch.int16), want.view(torch.int16)) for o in outs), chunk
+
+
+# A block moves 8 KiB, an XCD takes up to 64 of them in a row, a piece of the source is at most 8 MiB.
+PIECE = 8 << 20
+
+
+@pytest.mark.parametrize("fan", [2, 3, 4, 8])
+@pytest.mark.parametrize("nbytes", [8191, 8192 * 8 + 1, 8192 * 512, 8192 * 512 + 15, PIECE - 1, PIECE + 34, 2 * PIECE + 8192, 3 * PIECE + 1])
+def test_destination_after_destination_at_the_edges_of_tiles_and_pieces(fan, nbytes):
+    from mccl_amd import kernels as K
+    q = K.hip_kernels_init(0)
+    assert deliver(q, nbytes, fan, 0, [0]) == 1
+    assert deliver(q, nbytes, fan, 2, [6, 100, 129]) == 1
+
+
+def test_sources_of_many_lengths_share_a_launch_of_several_destinations():
+    from mccl_amd import kernels as K
+    q = K.hip_kernels_init(0)
+    lengths = [9_000_001, 8_999_987, 6_000_000, 1, 4_000_003, 16, 8192 * 700]
+    srcs = [torch.randint(0, 256, (n,), dtype=torch.uint8, device="cuda") for n in lengths]
+    outs = [[torch.full((n + 64,), 0xA5, dtype=torch.uint8, device="cuda") for _ in range(5)] for n in lengths]
+    torch.cuda.synchronize()
+    q.copy_batched([(o.data_ptr() + 3 * f, s.data_ptr(), n) for s, group, n in zip(srcs, outs, lengths)
+                    for f, o in enumerate(group)])
+    q.drain()
+    for s, group, n in zip(srcs, outs, lengths):
+        for f, o in enumerate(group):
+            assert torch.equal(o[3 * f:3 * f + n], s), (n, f)
+            assert bool((o[:3 * f] == 0xA5).all()) and bool((o[3 * f + n:] == 0xA5).all()), (n, f)
+
+
+@pytest.mark.parametrize("fan", [2, 4])
+def test_a_source_in_pinned_host_memory_goes_to_several_destinations(fan):
+    import ctypes
+    from mccl_amd import kernels as K
+    q = K.hip_kernels_init(0)
+    n = 5_000_003
+    host, dev = q.host_alloc(n)
+    data = np.random.default_rng(7).integers(0, 256, n, dtype=np.uint8)
+    ctypes.memmove(host, data.ctypes.data, n)
+    outs = [torch.zeros(n, dtype=torch.uint8, device="cuda") for _ in range(fan)]
+    torch.cuda.synchronize()
+    q.copy_batched([(o.data_ptr(), dev, n) for o in outs])
+    q.drain()
+    q.host_free(host)
+    assert all(np.array_equal(o.cpu().numpy(), data) for o in outs)
