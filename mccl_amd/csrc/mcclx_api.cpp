@@ -114,6 +114,9 @@ struct mcclx_ctx {
     uint64_t away_number = 0;  // counts those launches; launch i marks its end in away_ev[i % kAwayEvents]
     static constexpr uint64_t kAwayEvents = 4;
     hipEvent_t away_ev[kAwayEvents] = {};
+    // ... or writes this number to `word`; 0 = it does not.  The event is then recorded only where somebody
+    // has to wait on the device before the number is there (away_event).
+    std::atomic<uint64_t> away_word{0};
     // Operations enqueued on the queue, and how many of them are known to have finished (counted while
     // away_mu is held).  Equal: the queue is idle, and nothing has to be asked of the runtime.
     std::atomic<uint64_t> issued{0}, finished{0};
@@ -127,7 +130,10 @@ struct mcclx_ctx {
     uint64_t* word = nullptr;
     uint64_t* word_dev = nullptr;  // the same memory as the device addresses it
     hipEvent_t word_ev = nullptr;
-    uint32_t* mark_count = nullptr;  // device memory: blocks of a marked launch that have ended (LaunchMark)
+    // Device memory: blocks of a marked launch that have ended (LaunchMark), one counter for the queue's
+    // launches and, 8 bytes on, one for those on the default stream in its place, cleared there before the first.
+    uint32_t* mark_count = nullptr;
+    bool away_count_cleared = false;  // (under away_mu)
     // When mcclx_queue_wait last returned (steady clock, ns), whether nothing has been put on the queue since, and
     // whether what came next came within quick_ns.  A hint: a wait is right either way.
     std::atomic<int64_t> quick_ns{6000};
@@ -181,6 +187,7 @@ bool records(hipStream_t s) {
 struct MarkRequest {
     uint64_t number = 0;  // what the newest launch writes, 0 = it does not mark its end
     uint64_t upto = 0;    // `issued` of the context then
+    bool away = false;    // the launch runs in the queue's place
 };
 thread_local MarkRequest* g_mark = nullptr;
 struct MarkScope {
@@ -203,6 +210,40 @@ void note_start(mcclx_ctx* ctx) {
         ctx->quick.store(now_ns() - ctx->waited_at.load(std::memory_order_relaxed) < ctx->quick_ns.load(std::memory_order_relaxed), std::memory_order_relaxed);
 }
 
+// Is the newest launch that ran in the queue's place over, as far as its number tells?
+bool away_word_seen(const mcclx_ctx* ctx) {
+    const uint64_t number = ctx->away_word.load(std::memory_order_relaxed);
+    if (!number || *static_cast<const volatile uint64_t*>(ctx->word) < number) return false;
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return true;
+}
+// The same, watched for a while.
+bool away_word_comes(const mcclx_ctx* ctx, uint32_t spin_us) {
+    if (!ctx->away_word.load(std::memory_order_relaxed)) return false;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(spin_us);
+    do {
+        for (int k = 0; k < 64; ++k) {
+            if (away_word_seen(ctx)) return true;
+            __builtin_ia32_pause();
+        }
+    } while (std::chrono::steady_clock::now() < until);
+    return false;
+}
+// The event behind that launch; caller holds away_mu.  Where the launch left none it is recorded here,
+// behind everything that the default stream has been given since.
+hipError_t away_event(mcclx_ctx* ctx, hipEvent_t* ev) {
+    *ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
+    if (!ctx->away_word.load(std::memory_order_relaxed)) return hipSuccess;
+    const BesideRecordings beside;
+    const hipError_t e = hipEventRecord(*ev, nullptr);
+    if (e == hipSuccess) ctx->away_word.store(0, std::memory_order_relaxed);
+    return e;
+}
+
+// How long a host that waits watches for the number: what it waits for otherwise is the end of all that the
+// caller has put on the default stream behind the launch.
+constexpr uint32_t kAwayDrainUs = 1000;
+
 // The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its
 // place.  As an argument it lives until the call that enqueues the operation has returned, so that
 // no other thread finds the queue idle in between and launches beside it.
@@ -215,10 +256,15 @@ QueueUse queue_of(mcclx_ctx* ctx) {
     note_start(ctx);
     std::unique_lock<std::mutex> lk(ctx->away_mu);
     if (ctx->away.load(std::memory_order_relaxed)) {
-        const hipEvent_t ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
-        if (hipStreamWaitEvent(ctx->stream, ev, 0) != hipSuccess) {
-            (void)hipGetLastError();
-            (void)hipEventSynchronize(ev);
+        if (!away_word_seen(ctx)) {
+            hipEvent_t ev;
+            if (away_event(ctx, &ev) != hipSuccess) {
+                (void)hipGetLastError();
+                (void)hipStreamSynchronize(nullptr);
+            } else if (hipStreamWaitEvent(ctx->stream, ev, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                (void)hipEventSynchronize(ev);
+            }
         }
         ctx->away.store(false, std::memory_order_release);
     }
@@ -257,16 +303,21 @@ hipError_t drain(mcclx_ctx* ctx) {
         upto = ctx->issued.load(std::memory_order_relaxed);
     }
     if (ctx->away.load(std::memory_order_acquire)) {
-        hipEvent_t ev;
         uint64_t number;
         {
             std::lock_guard<std::mutex> lk(ctx->away_mu);
             number = ctx->away_number;
-            ev = ctx->away_ev[number % mcclx_ctx::kAwayEvents];
         }
         // (a thread that launches again meanwhile makes this wait longer, never shorter)
-        if (ev)
-            if (hipError_t e = hipEventSynchronize(ev); e != hipSuccess) return e;
+        if (!away_word_comes(ctx, kAwayDrainUs)) {
+            hipEvent_t ev;
+            {
+                std::lock_guard<std::mutex> lk(ctx->away_mu);
+                if (hipError_t e = away_event(ctx, &ev); e != hipSuccess) return e;
+            }
+            if (ev)
+                if (hipError_t e = hipEventSynchronize(ev); e != hipSuccess) return e;
+        }
         std::lock_guard<std::mutex> lk(ctx->away_mu);
         if (ctx->away_number == number) ctx->away.store(false, std::memory_order_release);
     }
@@ -643,7 +694,7 @@ int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, in
     mcclx::LaunchMark mark;
     if (g_mark && ctx->mark_count) {  // (the caller holds away_mu: numbers are handed out in the queue's order)
         mark.word = ctx->word_dev;
-        mark.count = ctx->mark_count;
+        mark.count = ctx->mark_count + (g_mark->away ? 2 : 0);
         mark.number = ctx->word_number + 1;
         lp.mark = &mark;
     }
@@ -938,7 +989,7 @@ int make_ctx(int device, hipStream_t borrowed, bool borrow, mcclx_ctx** out) {
         hipHostGetDevicePointer(&wd, w, 0) == hipSuccess &&
         hipEventCreateWithFlags(&ctx->word_ev, hipEventDisableTiming) == hipSuccess) {
         void* count = nullptr;  // (without it no launch marks its own end; nothing is put on a caller's stream here)
-        if (!borrow && hipMalloc(&count, sizeof(uint64_t)) == hipSuccess) {
+        if (!borrow && hipMalloc(&count, 2 * sizeof(uint64_t)) == hipSuccess) {
             // cleared on the queue, in front of every launch that uses it (a blocking copy would wait for the default stream)
             if (mcclx::launch_word(ctx->stream, static_cast<uint64_t*>(count), 0) == hipSuccess) ctx->mark_count = static_cast<uint32_t*>(count);
             else (void)hipFree(count);
@@ -1240,7 +1291,9 @@ int mcclx_decode_bf16(mcclx_ctx* ctx, void* dst_f32, const void* src_bf16, uint6
 // mcclx_stream_wait_queue): no cross-stream event and none of the two hand-overs between
 // hardware queues, which bound a sequence of such calls (events and launch 31 us a call, the
 // launch and its mark 7; 4097 bf16 values reduced through Python 50 -> 11 us, 25 MiB encoded and
-// decoded 110 -> 25 us).  The mark is an event record and not the kernel's own stop event: after
+// decoded 110 -> 25 us).  A launch of up to 32 blocks into device memory tells of its end itself (LaunchMark),
+// and no event is recorded behind it: the device takes 4 us for a kernel's event, 6.6 us a kernel and
+// event, 2.4 a kernel.  For the others the mark is an event record and not the kernel's own stop event: after
 // thousands of launches with one, the next calls on the stream took three times as long.
 // Everything else takes the two orderings: a queue with work in flight, a queue whose HIP stream
 // the caller holds (what they put there would not see a launch made elsewhere), a recording, and
@@ -1265,11 +1318,21 @@ static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
                 // (a launch before this one that is still away lies on the same stream, in front of it)
                 hipEvent_t& ev = ctx->away_ev[(ctx->away_number + 1) % mcclx_ctx::kAwayEvents];
                 if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-                if (int rc = launch_by_value(ctx, key, scale_f, has_scale, &l.seg, 1, fan, st)) return rc;
-                if (hipError_t e = hipEventRecord(ev, st); e != hipSuccess) {  // no mark to order by: the host waits
-                    HIP_TRY(hipStreamSynchronize(st));
-                    return MCCLX_OK;
+                MarkRequest mark;
+                mark.away = true;
+                {
+                    if (ctx->mark_count && !ctx->away_count_cleared)
+                        ctx->away_count_cleared = mcclx::launch_word(st, reinterpret_cast<uint64_t*>(ctx->mark_count + 2), 0) == hipSuccess;
+                    const bool device = ctx->away_count_cleared && in_device_memory(ctx, l.seg.out ? l.seg.out : l.seg.wire_out);
+                    const MarkScope scope(device ? &mark : nullptr);
+                    if (int rc = launch_by_value(ctx, key, scale_f, has_scale, &l.seg, 1, fan, st)) return rc;
                 }
+                if (mark.number == 0)
+                    if (hipError_t e = hipEventRecord(ev, st); e != hipSuccess) {  // no mark to order by: the host waits
+                        HIP_TRY(hipStreamSynchronize(st));
+                        return MCCLX_OK;
+                    }
+                ctx->away_word.store(mark.number, std::memory_order_relaxed);
                 ++ctx->away_number;
                 ctx->away.store(true, std::memory_order_release);
                 return MCCLX_OK;
@@ -1595,13 +1658,19 @@ int mcclx_stream_wait_queue(mcclx_ctx* ctx, void* consumer_stream) {
     if (ctx->away.load(std::memory_order_acquire) && !ctx->capturing) {
         DeviceGuard guard(ctx->device);
         std::lock_guard<std::mutex> lk(ctx->away_mu);
-        if (ctx->away.load(std::memory_order_relaxed)) {
-            const hipEvent_t ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
+        if (away_word_seen(ctx)) {
+            ctx->away.store(false, std::memory_order_release);
+        } else if (ctx->away.load(std::memory_order_relaxed) && consumer != nullptr) {  // (the launch lies on the default stream)
+            hipEvent_t ev;
             if (records(consumer)) {  // it cannot wait for what its recording does not hold: the host does
-                const BesideRecordings beside;
-                HIP_TRY(hipEventSynchronize(ev));
+                if (!away_word_comes(ctx, kAwayDrainUs)) {
+                    HIP_TRY(away_event(ctx, &ev));
+                    const BesideRecordings beside;
+                    HIP_TRY(hipEventSynchronize(ev));
+                }
                 ctx->away.store(false, std::memory_order_release);
             } else {
+                HIP_TRY(away_event(ctx, &ev));
                 HIP_TRY(hipStreamWaitEvent(consumer, ev, 0));
             }
         }

@@ -174,3 +174,84 @@ def test_a_recording_stream_may_wait_for_an_idle_queue(which):
         K.hip_reduce_op(dst, src, "sum", queue=q)
         assert torch.equal(dst, torch.full_like(dst, 5.0))
     q.close()
+
+
+# A launch of up to 32 blocks of 256 lanes tells of its own end and leaves no event behind it.
+@pytest.mark.parametrize("dtype,most", [(torch.float32, 32 * 256 * 4), (torch.bfloat16, 32 * 256 * 8), (torch.float16, 32 * 256 * 8)])
+@pytest.mark.parametrize("consumer", ["torch", "queue", "other_stream", "ticket", "drain", "wait", "exposed"])
+@pytest.mark.parametrize("behind", ["nothing", "a_running_kernel"])
+def test_small_launches_that_tell_of_their_own_end(dtype, most, consumer, behind):
+    q = K.ReduceQueue(0)
+    other = torch.cuda.Stream()
+    for n in (1, 4_097, most - 1, most, most + 1, 4 * most + 3):
+        dst = torch.full((n,), 3.0, device="cuda", dtype=dtype)
+        src = torch.full((n,), 2.0, device="cuda", dtype=dtype)
+        got = torch.zeros_like(dst)
+        torch.cuda.synchronize()
+        marked = q.marked_launch_count()
+        if behind == "a_running_kernel":
+            torch.cuda._sleep(300_000)
+        src.add_(1)
+        K.hip_reduce_op(dst, src, "sum", queue=q)
+        K.hip_scale_inplace(dst, 0.5, queue=q)
+        if n <= most and (consumer != "exposed" or n == 1):  # (once its stream is out, the queue runs everything itself)
+            assert q.marked_launch_count() - marked == 2
+        if consumer == "torch":
+            got.copy_(dst)
+        elif consumer == "queue":
+            q.copy(got.data_ptr(), dst.data_ptr(), n * dst.element_size())
+            q.drain()
+        elif consumer == "other_stream":
+            q.torch_stream_wait(other)
+            with torch.cuda.stream(other):
+                got.copy_(dst)
+            other.synchronize()
+        else:
+            if consumer == "ticket":
+                q.wait(q.record())
+            elif consumer == "drain":
+                q.drain()
+            elif consumer == "wait":
+                q.wait_results()
+            else:
+                torch.cuda.ExternalStream(q.stream).synchronize()
+            with torch.cuda.stream(other):
+                got.copy_(dst)
+            other.synchronize()
+        torch.cuda.synchronize()
+        assert bool((got == 3.0).all()), n
+    q.close()
+
+
+def test_codec_and_scaling_at_the_last_size_that_tells_of_its_end():
+    q = K.ReduceQueue(0)
+    for blocks in (1, 2, 31, 32, 33):
+        for extra in (-1, 0, 1):
+            n = blocks * 256 * 4 + extra
+            x = torch.randn(n, device="cuda")
+            w = K.encode_bf16(x, queue=q)
+            assert torch.equal(w.view(torch.int16), x.to(torch.bfloat16).view(torch.int16))
+            assert torch.equal(K.decode_bf16(w, queue=q), w.float())
+            y = x.clone()
+            assert torch.equal(K.hip_accumulate_and_scale(y, x, 0.25, queue=q), (x + x) * 0.25)
+    assert q.marked_launch_count() > 0
+    q.close()
+
+
+def test_a_host_that_waits_for_a_small_launch_does_not_wait_for_what_came_behind_it():
+    import time
+    q = K.ReduceQueue(0)
+    dst, src = torch.zeros(4_097, device="cuda"), torch.ones(4_097, device="cuda")
+    K.hip_reduce_op(dst, src, "sum", queue=q)
+    torch.cuda.synchronize()
+    K.hip_reduce_op(dst, src, "sum", queue=q)
+    torch.cuda._sleep(100_000_000)  # some 50 ms
+    t = time.perf_counter()
+    q.drain()
+    waited = time.perf_counter() - t
+    t = time.perf_counter()
+    torch.cuda.synchronize()
+    slept = time.perf_counter() - t
+    assert waited < slept / 2, (waited, slept)
+    assert bool((dst == 2.0).all())
+    q.close()
