@@ -77,6 +77,7 @@ SIGNATURES = {
     "mcclx_launch_count": (_u64, [_vp]),
     "mcclx_hold_launch_count": (_u64, [_vp]),
     "mcclx_marked_launch_count": (_u64, [_vp]),
+    "mcclx_away_launch_count": (_u64, [_vp]),
     "mcclx_four_wave_launch_count": (_u64, [_vp]),
     "mcclx_set_hold": (_i, [_vp, _i]),
     "mcclx_hold_model": (_i, [_vp, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32)]),

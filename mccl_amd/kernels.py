@@ -209,6 +209,10 @@ class ReduceQueue:
         """Launches of this queue that told the host of their own end (diagnostic)."""
         return int(L.lib().mcclx_marked_launch_count(self.handle))
 
+    def away_launch_count(self) -> int:
+        """Launches that ran on the default stream in this queue's place (diagnostic)."""
+        return int(L.lib().mcclx_away_launch_count(self.handle))
+
     def four_wave_launch_count(self) -> int:
         """Fold launches of this queue in blocks of four wavefronts (diagnostic)."""
         return int(L.lib().mcclx_four_wave_launch_count(self.handle))
