@@ -1017,6 +1017,11 @@ static bool off_lines(const FewArgs& a) {
     return false;
 }
 
+// The wire codec's two casts.
+template <class C>
+constexpr bool kCast = C::K == 1 && C::W == MCCLX_BF16 && C::ACC == MCCLX_ACC_STEP && C::OP == MCCLX_SUM &&
+                       (C::IO == MCCLX_IO_OWN_FIRST_F32 || C::kDecode);
+
 // A by-value launch: one block per tile of the longest segment, the hold form where it applies.
 template <class C, int OUT>
 static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchParams& lp) {
@@ -1066,6 +1071,16 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
     };
     using Few = std::integral_constant<int, C::FEW_U>;
     const uint64_t waves = (maxc + 64 * lane_elems - 1) / (64 * lane_elems) * (uint64_t)a.nseg;
+    // One tensor of the codec has a kernel of its own.  Not where the launch is to tell of its end and can, and not
+    // where a large one's streams share lines (off_lines).
+    if constexpr (kCast<C> && OUT == kOutOne) {
+        const SegArgs& s = a.seg[0];
+        void* out = C::kDecode ? s.out : s.wire_out;
+        const bool plain = a.nseg == 1 && !a.has_scale && out && !(C::kDecode ? s.wire_out : s.out) && maxc < (1ull << 33) && lp.cus > 0;
+        const bool tells = lp.mark && (waves + 3) / 4 <= kMarkBlocks;
+        if (plain && !tells && (waves < C::kOneWaveFrom || !off_lines<C, OUT>(a)))
+            return launch_cast(st, C::kDecode, out, s.in[0], maxc, lp.cus);
+    }
     if constexpr (C::kSmallShape) {
         if (waves < C::kOneWaveFrom) return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
         if constexpr (C::BLOCK == kBlock)

@@ -109,6 +109,10 @@ bool all_plan_ok(const PlanKey& key);
 bool fold_encode_ok(const PlanKey& key);
 hipError_t launch_fold_encode(hipStream_t st, const PlanKey& key, const FewArgs& few, uint32_t nfold);
 
+// One tensor to its wire form or back, as the plans of one operand without a scale give it (per-step rounding):
+// dst <- src, up to 2^33 elements.
+hipError_t launch_cast(hipStream_t st, bool decode, void* dst, const void* src, uint64_t count, int cus);
+
 // Can a segment of `count` elements be launched by value?  A grid has at most 2^32 threads, one
 // per packet there (more are dropped without an error); the table kernels loop.
 bool few_fits(const PlanKey& key, uint64_t count);
