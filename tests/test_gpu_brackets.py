@@ -159,9 +159,10 @@ def test_work_put_between_a_fold_and_the_second_ordering_runs_beside_it():
     assert q.away_launch_count() == 0
     q.wait_torch_stream()
     scale(q, x, out)
+    ticket = q.record()  # (a drain's own marker may share a hardware queue with what follows)
     torch.cuda._sleep(100_000_000)
     t = time.perf_counter()
-    q.drain()
+    q.wait(ticket)
     waited = time.perf_counter() - t
     torch.cuda.synchronize()
     assert waited < (time.perf_counter() - t) / 2
