@@ -873,6 +873,16 @@ static bool hold_launch(hipStream_t st, FewArgs& a, uint64_t packets, uint32_t g
     const uint32_t cap = hold_capacity<C, T, HB, OUT>(lp.cus);
     if (cap < (uint32_t)a.nseg) return false;
     uint32_t hx = cap / (uint32_t)a.nseg;
+    // Two tensors to two: 512 blocks per segment would put a lane's packets 4 MiB apart.  As many as three segments get
+    // where that is enough, at five packets per lane up to two fifths of the device, and the plain form beyond.
+    // Two ranks of 18 / 22 / 26.2 / 32 / 34 MB (us): 512 blocks 13.2 / 16.5 / 20.2 / 23.1 / -, these 12.6 / 15.0 / 17.8 / 21.7 / 24.3,
+    // plain 13.4 / 15.9 / 18.5 / 22.2 / 23.5.
+    if (OUT == kOutFan && a.nseg == 2) {
+        const uint64_t need = (packets + (uint64_t)HB * T - 1) / ((uint64_t)HB * T);
+        hx = cap / 3 & ~3u;
+        if (T == 5 && need > hx) hx = (uint32_t)(need + 3 < cap * 2 / 5 ? (need + 3) & ~3ull : 0);
+        if (hx == 0) return false;
+    }
     if (packets > (uint64_t)hx * HB * T) return false;
     // As many blocks as the device holds -- the more waves share the launch's loads, the sooner
     // they are through (C2 with 267 instead of 341 blocks per segment: 16 us instead of 13) --

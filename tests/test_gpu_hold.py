@@ -329,3 +329,23 @@ def test_one_operand_plans_in_the_hold_form_match_the_plain_form(env, queues, wi
                 assert torch.equal(ho.view(torch.int32), po.view(torch.int32)), f"fp32 output, counts {counts}"
             if with_wire:
                 assert torch.equal(hw.view(torch.int16), pw.view(torch.int16)), f"bf16 output, counts {counts}"
+
+
+@pytest.mark.parametrize("dtype,wire", [(torch.float32, True), (torch.float32, False), (torch.bfloat16, False)])
+@pytest.mark.parametrize("blocks_and_packets", [(340, 4), (340, 5), (408, 5)])
+def test_two_ranks_at_the_sizes_where_the_number_of_blocks_changes(dtype, wire, blocks_and_packets):
+    """An allreduce of two tensors: 340 blocks per chunk at four packets per lane, at five, then more, then
+    the plain form; one packet to either side of each, the same bits as step by step."""
+    from mccl_amd import harness as H, kernels as K, _lib as L
+    blocks, per = blocks_and_packets
+    elems = 4 if dtype == torch.float32 else 8
+    q = K.hip_kernels_init(0)
+    for extra in (-3, 1):
+        n = 2 * (blocks * 512 * per + extra) * elems + 1
+        g = torch.Generator(device="cuda").manual_seed(n)
+        ts = [torch.randn(n, generator=g, device="cuda").to(dtype) for _ in range(2)]
+        want = [t.clone() for t in ts]
+        H.allreduce_replay(ts, "avg", L.ALGO_RING, wire_bf16=wire, mode=L.REPLAY_DIRECT, queue=q)
+        H.allreduce_replay(want, "avg", L.ALGO_RING, wire_bf16=wire, mode=L.REPLAY_STEPWISE, queue=q)
+        for a, b in zip(ts, want):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16)), (n, extra)
