@@ -138,8 +138,7 @@ MCCLX_API uint64_t mcclx_hold_launch_count(mcclx_ctx* ctx);
 /* Diagnostic: launches of this context that wrote mcclx_queue_wait's word themselves, and by-value fold
  * launches that ran in blocks of four wavefronts. */
 MCCLX_API uint64_t mcclx_marked_launch_count(mcclx_ctx* ctx);
-/* Launches that ran on the default stream in the queue's place (diagnostic): see the _ordered forms and
- * mcclx_queue_wait_stream. */
+/* Launches that ran on the default stream in the queue's place (diagnostic): see the _ordered forms. */
 MCCLX_API uint64_t mcclx_away_launch_count(mcclx_ctx* ctx);
 MCCLX_API uint64_t mcclx_four_wave_launch_count(mcclx_ctx* ctx);
 /* Diagnostic: the model behind that time -- no store before `latency_ticks` +
@@ -316,10 +315,7 @@ MCCLX_API int mcclx_queue_wait(mcclx_ctx* ctx, uint32_t spin_us);
 MCCLX_API int mcclx_set_wait_gap(mcclx_ctx* ctx, uint32_t gap_us);
 /* The queue waits (on the device, host not blocked) for everything enqueued so
  * far on `producer_stream`.  Replaces mps_stream_sync (MPSInterop.mm:308-310)
- * and mps_event_sync_nonblocking + wait_for_mps (:336-356, EventSync.mm:112-132).
- * After several sequences in a row of this call for the default stream (NULL), folds of up to 32 segments and
- * mcclx_stream_wait_queue for it at once (within 20 us), the next such sequence of a context that has not handed
- * out its HIP stream runs its folds on the default stream itself; the first other call goes back to two queues. */
+ * and mps_event_sync_nonblocking + wait_for_mps (:336-356, EventSync.mm:112-132). */
 MCCLX_API int mcclx_queue_wait_stream(mcclx_ctx* ctx, void* producer_stream);
 /* `consumer_stream` waits for everything enqueued so far on the queue: the
  * non-blocking form of "queue drained before the Work completes"

@@ -117,12 +117,6 @@ struct mcclx_ctx {
     // ... or writes this number to `word`; 0 = it does not.  The event is then recorded only where somebody
     // has to wait on the device before the number is there (away_event).
     std::atomic<uint64_t> away_word{0};
-    // "The queue waits for the default stream", launches, "the default stream waits for the queue": see join.
-    std::atomic<int> bracket{0};  // 1: the first has been said and nothing since, 2: launches by value have followed
-    int64_t bracket_at = 0;       // when the last of those returned (steady clock, ns)
-    int tight = 0;                // how many of them in a row were closed at once
-    bool joined = false;          // the first has been said and is still to be carried out
-    bool join_new = false;        // ... and since the newest launch on the default stream  (all under away_mu)
     // Operations enqueued on the queue, and how many of them are known to have finished (counted while
     // away_mu is held).  Equal: the queue is idle, and nothing has to be asked of the runtime.
     std::atomic<uint64_t> issued{0}, finished{0};
@@ -253,40 +247,6 @@ hipError_t away_event(mcclx_ctx* ctx, hipEvent_t* ev) {
 // caller has put on the default stream behind the launch.
 constexpr uint32_t kAwayDrainUs = 1000;
 
-// Launches between two orderings, "the queue waits for the default stream" and "the default stream waits for the
-// queue", whose second follows at once can run on the default stream: the two hand-overs between hardware
-// queues take 10 us each.  A caller who puts work of their own on the default stream before the second ordering
-// wants the two side by side, so a context does this only while its last brackets (kTight or more in
-// a row) were closed within kTightNs of their last launch and held nothing but launches by value.  Then the first
-// ordering of an idle queue is left open (`joined`); a launch by value finds it open and goes to the default
-// stream, where the order holds by itself, and every other operation carries it out first (end_join).  A
-// hint: what comes behind what is the same either way.  A fold of three 25 MiB tensors between the two
-// takes 15.7 us a pass instead of 36, of tensors of 40 KB to 4 MB 9 to 12 instead of 24 to 33.
-constexpr int kTight = 4;
-constexpr int64_t kTightNs = 20'000;
-
-// The queue waits for the default stream, as it has been told to (caller holds away_mu).
-void end_join(mcclx_ctx* ctx) {
-    if (!ctx->joined) return;
-    ctx->joined = false;
-    const BesideRecordings beside;
-    hipEvent_t& ev = ctx->away_ev[(ctx->away_number + 1) % mcclx_ctx::kAwayEvents];
-    if ((!ev && hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) || hipEventRecord(ev, nullptr) != hipSuccess ||
-        hipStreamWaitEvent(ctx->stream, ev, 0) != hipSuccess) {
-        (void)hipGetLastError();
-        (void)hipStreamSynchronize(nullptr);
-    }
-    ++ctx->away_number;
-    ctx->away.store(false, std::memory_order_release);  // (what ran there in the queue's place came before)
-    ctx->issued.fetch_add(1, std::memory_order_relaxed);
-}
-// Something other than a launch by value or the end of a bracket.
-void no_bracket(mcclx_ctx* ctx) {
-    if (ctx->bracket.load(std::memory_order_relaxed) == 0) return;
-    ctx->bracket.store(0, std::memory_order_relaxed);
-    ctx->tight = 0;
-}
-
 // The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its
 // place.  As an argument it lives until the call that enqueues the operation has returned, so that
 // no other thread finds the queue idle in between and launches beside it.
@@ -295,11 +255,9 @@ struct QueueUse {
     hipStream_t stream;
     operator hipStream_t() const { return stream; }
 };
-QueueUse queue_of(mcclx_ctx* ctx, bool by_value = false) {
+QueueUse queue_of(mcclx_ctx* ctx) {
     note_start(ctx);
     std::unique_lock<std::mutex> lk(ctx->away_mu);
-    if (!by_value) no_bracket(ctx);
-    end_join(ctx);
     if (ctx->away.load(std::memory_order_relaxed)) {
         if (!away_word_seen(ctx)) {
             hipEvent_t ev;
@@ -345,8 +303,6 @@ hipError_t drain(mcclx_ctx* ctx) {
     uint64_t upto;
     {
         std::lock_guard<std::mutex> lk(ctx->away_mu);  // an operation is counted before it is enqueued
-        no_bracket(ctx);
-        end_join(ctx);
         upto = ctx->issued.load(std::memory_order_relaxed);
     }
     if (ctx->away.load(std::memory_order_acquire)) {
@@ -799,7 +755,6 @@ int launch_away(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, int ha
     ++ctx->away_number;
     ++ctx->away_launches;
     ctx->away_at = now_ns();
-    ctx->join_new = false;
     ctx->away.store(true, std::memory_order_release);
     return MCCLX_OK;
 }
@@ -841,25 +796,8 @@ int fold_checked(mcclx_ctx* ctx, const mcclx_plan* plan, const mcclx_seg* segs, 
 
     mcclx::LaunchParams lp;
     lp.max_blocks = ctx->max_blocks;
-    if (nseg <= ctx->few_max && even_enough(key, segs, nseg)) {
-        if (ctx->bracket.load(std::memory_order_relaxed) == 0)
-            return launch_by_value(ctx, key, scale_f, has_scale, segs, nseg, fan, queue_of(ctx, true));
-        int rc;
-        std::unique_lock<std::mutex> lk(ctx->away_mu);
-        if (ctx->joined && may_go_away(ctx)) {
-            rc = launch_away(ctx, key, scale_f, has_scale, segs, nseg, fan);
-        } else {
-            lk.unlock();
-            QueueUse use = queue_of(ctx, true);
-            rc = launch_by_value(ctx, key, scale_f, has_scale, segs, nseg, fan, use);
-            lk = std::move(use.lk);
-        }
-        if (ctx->bracket.load(std::memory_order_relaxed)) {
-            ctx->bracket.store(2, std::memory_order_relaxed);
-            ctx->bracket_at = now_ns();
-        }
-        return rc;
-    }
+    if (nseg <= ctx->few_max && even_enough(key, segs, nseg))
+        return launch_by_value(ctx, key, scale_f, has_scale, segs, nseg, fan, queue_of(ctx));
 
     // Descriptor table: segs; then, where a block cannot work out its segment by division, (segment, tile)
     // per work item, so that it finds its work with one load instead of a binary search through
@@ -1427,7 +1365,6 @@ static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
         if (!guard.ok) return fail(MCCLX_ERR_HIP, "hipSetDevice(%d) failed", ctx->device);
         std::lock_guard<std::mutex> lk(ctx->away_mu);
         if (may_go_away(ctx)) {
-            no_bracket(ctx);
             mcclx::PlanKey key;
             float scale_f;
             int has_scale, fan;
@@ -1704,25 +1641,6 @@ static int stream_wait(mcclx_ctx* ctx, hipStream_t waiter, hipStream_t producer)
     REFUSE_WHILE_RECORDING(ctx, "cross-stream ordering");
     if (waiter == ctx->stream) note_start(ctx);  // where a collective starts
     DeviceGuard guard(ctx->device);
-    {
-        std::lock_guard<std::mutex> lk(ctx->away_mu);
-        if (waiter == ctx->stream && producer == nullptr) {
-            ctx->join_new = true;
-            if (ctx->joined) {
-                ctx->bracket.store(1, std::memory_order_relaxed);
-                return MCCLX_OK;
-            }
-            if (ctx->bracket.load(std::memory_order_relaxed)) ctx->tight = 0;  // (the one before was never closed)
-            ctx->bracket.store(1, std::memory_order_relaxed);
-            if (ctx->tight >= kTight && may_go_away(ctx)) {
-                ctx->joined = true;
-                return MCCLX_OK;
-            }
-        } else {
-            if (waiter != nullptr) no_bracket(ctx);
-            end_join(ctx);
-        }
-    }
     // A producer that has nothing in flight needs no event: everything enqueued on it so far is
     // complete, which is all the wait would establish (an event record plus a stream wait cost
     // the host 10-20 us on torch's legacy stream, a query of an idle stream 0.1 us).  The query costs as
@@ -1774,21 +1692,6 @@ int mcclx_queue_wait_stream(mcclx_ctx* ctx, void* producer_stream) {
 int mcclx_stream_wait_queue(mcclx_ctx* ctx, void* consumer_stream) {
     if (!ctx) return fail(MCCLX_ERR_STATE, "context is null (mcclx_init not called)");
     const hipStream_t consumer = static_cast<hipStream_t>(consumer_stream);
-    if (consumer == nullptr && ctx->bracket.load(std::memory_order_relaxed)) {
-        std::lock_guard<std::mutex> lk(ctx->away_mu);
-        if (ctx->bracket.load(std::memory_order_relaxed) == 2) {
-            ctx->tight = now_ns() - ctx->bracket_at < kTightNs ? ctx->tight + (ctx->tight < kTight) : 0;
-            ctx->bracket.store(0, std::memory_order_relaxed);
-            // The launches lie on the default stream, and the queue gets behind them there (queue_of); a wait that
-            // another thread has asked for since the last of them stays open.
-            if (ctx->joined) {
-                ctx->joined = ctx->join_new;
-                return MCCLX_OK;
-            }
-        } else {
-            no_bracket(ctx);
-        }
-    }
     if (ctx->away.load(std::memory_order_acquire) && !ctx->capturing) {
         DeviceGuard guard(ctx->device);
         std::lock_guard<std::mutex> lk(ctx->away_mu);
