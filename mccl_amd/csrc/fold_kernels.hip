@@ -634,11 +634,6 @@ __device__ __forceinline__ void fetch_together(SegArgs& s, float& scale, int32_t
 // kernel with more starts 768 blocks at launch instead of 1024 and streams
 // 2-4 % slower.  Six registers are set aside on top of what the code uses (VCC,
 // flat scratch, XNACK mask), so the code itself has 74.
-// Launches that can tell the host of their own end: into several places in any shape, into one in blocks of
-// four wavefronts (the large launches keep the scalar registers).
-template <int OUT, int B>
-constexpr bool kMarks = OUT != kOutOne || B == kFourWaves;
-
 template <class C, int OUT, int B, int U>
 __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
 #if MCCLX_TUNE_TIMELINE
@@ -652,7 +647,7 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
     int32_t fan = 0;
     if constexpr (OUT == kOutFan) fan = a.fan;
     uint64_t* mark_word = nullptr;
-    if constexpr (kMarks<OUT, B>) {
+    if constexpr (OUT != kOutOne) {
         mark_word = a.mark_word;
         asm volatile("" : "+s"(mark_word));
     }
@@ -672,7 +667,7 @@ __device__ __forceinline__ void fold_few_body(const FewArgs& a) {
     // the last one writes the number.  Blocks that count themselves one after another cost 30 ns each, a
     // launch behind this one 2 us: 16 blocks 7.8 us from launch call to word against 9.2, 64 blocks 9.2 and 9.4,
     // 256 blocks 14.9 and 9.4 (kMarkBlocks).
-    if constexpr (kMarks<OUT, B>)
+    if constexpr (OUT != kOutOne)
         if (mark_word) {
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
             if constexpr (B > kOneWave) __syncthreads();
@@ -1059,7 +1054,7 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
         if (gx * B >> 32) return hipErrorInvalidValue;  // (see few_fits)
         const dim3 grid((uint32_t)gx, (uint32_t)a.nseg);
         if (B == kFourWaves && lp.four) *lp.four = true;
-        if (kMarks<OUT, B> && lp.mark && gx * (uint64_t)a.nseg <= kMarkBlocks) {
+        if (OUT != kOutOne && lp.mark && gx * (uint64_t)a.nseg <= kMarkBlocks) {
             a.mark_word = lp.mark->word;
             a.mark_count = lp.mark->count;
             a.mark_number = lp.mark->number;
@@ -1081,14 +1076,12 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
     };
     using Few = std::integral_constant<int, C::FEW_U>;
     const uint64_t waves = (maxc + 64 * lane_elems - 1) / (64 * lane_elems) * (uint64_t)a.nseg;
-    // One tensor of the codec has a kernel of its own.  Not where the launch is to tell of its end and can, and not
-    // where a large one's streams share lines (off_lines).
+    // One tensor of the codec has a kernel of its own.  Not where a large one's streams share lines (off_lines).
     if constexpr (kCast<C> && OUT == kOutOne) {
         const SegArgs& s = a.seg[0];
         void* out = C::kDecode ? s.out : s.wire_out;
         const bool plain = a.nseg == 1 && !a.has_scale && out && !(C::kDecode ? s.wire_out : s.out) && maxc < (1ull << 33) && lp.cus > 0;
-        const bool tells = lp.mark && (waves + 3) / 4 <= kMarkBlocks;
-        if (plain && !tells && (waves < C::kOneWaveFrom || !off_lines<C, OUT>(a)))
+        if (plain && (waves < C::kOneWaveFrom || !off_lines<C, OUT>(a)))
             return launch_cast(st, C::kDecode, out, s.in[0], maxc, lp.cus);
     }
     if constexpr (C::kSmallShape) {
@@ -1105,8 +1098,8 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
         // average at any size (0.98-1.03), nor do up to four operands.  Not beside resident_lds, which counts blocks of one.
         if (OUT == kOutOne && C::K >= 5 && lds == 0 && waves >= 16 * (uint64_t)lp.cus)
             return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
-        // few enough blocks of four to tell of their end (kMarkBlocks), too many of one, which into one place cannot
-        if (lp.mark && (OUT == kOutOne || waves > kMarkBlocks) && waves <= 4 * kMarkBlocks)
+        // few enough blocks of four to tell of their end (kMarkBlocks), too many of one
+        if (OUT != kOutOne && lp.mark && waves > kMarkBlocks && waves <= 4 * kMarkBlocks)
             return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);
     }
     return go(std::integral_constant<int, kOneWave>{}, Few{}, lds);

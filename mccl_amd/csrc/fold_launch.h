@@ -41,7 +41,7 @@ struct FewArgs {
     int32_t nseg;
     int32_t fan;        // further destinations of the result, in[k .. k+fan-1] (fan-out kernels only)
     int32_t op;         // the operator, where the kernel takes it from here (to-all kernels of MIN, MAX, PRODUCT)
-    // Where not null: the last block to end writes `mark_number` there (kernels that can, kMarks).
+    // Fan-out and to-all kernels, where not null: the last block to end writes `mark_number` there.
     uint64_t* mark_word;
     uint32_t* mark_count;  // blocks that have ended, 0 between launches
     uint64_t mark_number;

@@ -114,9 +114,6 @@ struct mcclx_ctx {
     uint64_t away_number = 0;  // counts those launches; launch i marks its end in away_ev[i % kAwayEvents]
     static constexpr uint64_t kAwayEvents = 4;
     hipEvent_t away_ev[kAwayEvents] = {};
-    // ... or writes this number to `word`; 0 = it does not.  The event is then recorded only where somebody
-    // has to wait on the device before the number is there (away_event).
-    std::atomic<uint64_t> away_word{0};
     // Operations enqueued on the queue, and how many of them are known to have finished (counted while
     // away_mu is held).  Equal: the queue is idle, and nothing has to be asked of the runtime.
     std::atomic<uint64_t> issued{0}, finished{0};
@@ -131,11 +128,7 @@ struct mcclx_ctx {
     uint64_t* word = nullptr;
     uint64_t* word_dev = nullptr;  // the same memory as the device addresses it
     hipEvent_t word_ev = nullptr;
-    // Device memory: blocks of a marked launch that have ended (LaunchMark), one counter for the queue's
-    // launches and, 8 bytes on, one for those on the default stream in its place, cleared there before the first.
-    uint32_t* mark_count = nullptr;
-    bool away_count_cleared = false;  // (under away_mu)
-    int64_t away_at = 0;              // when the last such launch returned (steady clock, ns; under away_mu)
+    uint32_t* mark_count = nullptr;  // device memory: blocks of a marked launch that have ended (LaunchMark)
     // When mcclx_queue_wait last returned (steady clock, ns), whether nothing has been put on the queue since, and
     // whether what came next came within quick_ns.  A hint: a wait is right either way.
     std::atomic<int64_t> quick_ns{6000};
@@ -189,13 +182,11 @@ bool records(hipStream_t s) {
 struct MarkRequest {
     uint64_t number = 0;  // what the newest launch writes, 0 = it does not mark its end
     uint64_t upto = 0;    // `issued` of the context then
-    bool away = false;    // the launch runs in the queue's place
 };
 thread_local MarkRequest* g_mark = nullptr;
 struct MarkScope {
-    MarkRequest* const before = g_mark;
     explicit MarkScope(MarkRequest* m) { g_mark = m; }
-    ~MarkScope() { g_mark = before; }
+    ~MarkScope() { g_mark = nullptr; }
 };
 
 // A call that returns early (mcclx_queue_wait) leaves an event behind its launches, in which a device-wide or
@@ -213,40 +204,6 @@ void note_start(mcclx_ctx* ctx) {
         ctx->quick.store(now_ns() - ctx->waited_at.load(std::memory_order_relaxed) < ctx->quick_ns.load(std::memory_order_relaxed), std::memory_order_relaxed);
 }
 
-// Is the newest launch that ran in the queue's place over, as far as its number tells?
-bool away_word_seen(const mcclx_ctx* ctx) {
-    const uint64_t number = ctx->away_word.load(std::memory_order_relaxed);
-    if (!number || *static_cast<const volatile uint64_t*>(ctx->word) < number) return false;
-    std::atomic_thread_fence(std::memory_order_acquire);
-    return true;
-}
-// The same, watched for a while.
-bool away_word_comes(const mcclx_ctx* ctx, uint32_t spin_us) {
-    if (!ctx->away_word.load(std::memory_order_relaxed)) return false;
-    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(spin_us);
-    do {
-        for (int k = 0; k < 64; ++k) {
-            if (away_word_seen(ctx)) return true;
-            __builtin_ia32_pause();
-        }
-    } while (std::chrono::steady_clock::now() < until);
-    return false;
-}
-// The event behind that launch; caller holds away_mu.  Where the launch left none it is recorded here,
-// behind everything that the default stream has been given since.
-hipError_t away_event(mcclx_ctx* ctx, hipEvent_t* ev) {
-    *ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
-    if (!ctx->away_word.load(std::memory_order_relaxed)) return hipSuccess;
-    const BesideRecordings beside;
-    const hipError_t e = hipEventRecord(*ev, nullptr);
-    if (e == hipSuccess) ctx->away_word.store(0, std::memory_order_relaxed);
-    return e;
-}
-
-// How long a host that waits watches for the number: what it waits for otherwise is the end of all that the
-// caller has put on the default stream behind the launch.
-constexpr uint32_t kAwayDrainUs = 1000;
-
 // The queue's stream, for the next operation on it: behind the launches that ran elsewhere in its
 // place.  As an argument it lives until the call that enqueues the operation has returned, so that
 // no other thread finds the queue idle in between and launches beside it.
@@ -259,15 +216,10 @@ QueueUse queue_of(mcclx_ctx* ctx) {
     note_start(ctx);
     std::unique_lock<std::mutex> lk(ctx->away_mu);
     if (ctx->away.load(std::memory_order_relaxed)) {
-        if (!away_word_seen(ctx)) {
-            hipEvent_t ev;
-            if (away_event(ctx, &ev) != hipSuccess) {
-                (void)hipGetLastError();
-                (void)hipStreamSynchronize(nullptr);
-            } else if (hipStreamWaitEvent(ctx->stream, ev, 0) != hipSuccess) {
-                (void)hipGetLastError();
-                (void)hipEventSynchronize(ev);
-            }
+        const hipEvent_t ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
+        if (hipStreamWaitEvent(ctx->stream, ev, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipEventSynchronize(ev);
         }
         ctx->away.store(false, std::memory_order_release);
     }
@@ -306,21 +258,16 @@ hipError_t drain(mcclx_ctx* ctx) {
         upto = ctx->issued.load(std::memory_order_relaxed);
     }
     if (ctx->away.load(std::memory_order_acquire)) {
+        hipEvent_t ev;
         uint64_t number;
         {
             std::lock_guard<std::mutex> lk(ctx->away_mu);
             number = ctx->away_number;
+            ev = ctx->away_ev[number % mcclx_ctx::kAwayEvents];
         }
         // (a thread that launches again meanwhile makes this wait longer, never shorter)
-        if (!away_word_comes(ctx, kAwayDrainUs)) {
-            hipEvent_t ev;
-            {
-                std::lock_guard<std::mutex> lk(ctx->away_mu);
-                if (hipError_t e = away_event(ctx, &ev); e != hipSuccess) return e;
-            }
-            if (ev)
-                if (hipError_t e = hipEventSynchronize(ev); e != hipSuccess) return e;
-        }
+        if (ev)
+            if (hipError_t e = hipEventSynchronize(ev); e != hipSuccess) return e;
         std::lock_guard<std::mutex> lk(ctx->away_mu);
         if (ctx->away_number == number) ctx->away.store(false, std::memory_order_release);
     }
@@ -697,7 +644,7 @@ int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, in
     mcclx::LaunchMark mark;
     if (g_mark && ctx->mark_count) {  // (the caller holds away_mu: numbers are handed out in the queue's order)
         mark.word = ctx->word_dev;
-        mark.count = ctx->mark_count + (g_mark->away ? 2 : 0);
+        mark.count = ctx->mark_count;
         mark.number = ctx->word_number + 1;
         lp.mark = &mark;
     }
@@ -714,47 +661,20 @@ int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, in
     return MCCLX_OK;
 }
 
-// Could a launch into these places tell of its end (LaunchMark)?  Few elements, and all of it device memory.
-bool may_mark_away(const mcclx_ctx* ctx, const mcclx::PlanKey& key, const mcclx_seg* segs, uint32_t nseg, int fan) {
-    if (!ctx->away_count_cleared || nseg > 4) return false;
-    for (uint32_t s = 0; s < nseg; ++s) {
-        const mcclx_seg& g = segs[s];
-        if (g.count > (1u << 17)) return false;
-        if ((g.out && !in_device_memory(ctx, g.out)) || (g.wire_out && !in_device_memory(ctx, g.wire_out))) return false;
-        for (int i = fan == kToAll ? 0 : key.k; i < key.k + (fan > 0 ? fan : 0); ++i)
-            if (!in_device_memory(ctx, g.in[i])) return false;
-    }
-    return true;
-}
-
-// Launches that follow one another within this time tell of their end themselves where they can; one on its own
-// has an event behind it, which a synchronisation of the caller's finds: a call of 4097 values and a device
-// synchronisation take 15.9 us with the event and 17.1 to 18.3 without, calls in a row 9.1 and 6.1.
-constexpr int64_t kAwayQuickNs = 8'000;
-
-// A launch by value on the default stream in the place of the queue: see may_go_away (caller holds away_mu).
-int launch_away(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, int has_scale, const mcclx_seg* segs, uint32_t nseg, int fan) {
+// A launch of one segment on the default stream in the place of the queue: see may_go_away (caller holds away_mu).
+// The event that marks its end is recorded at once: recorded when somebody asks, it would stand behind all that the
+// caller has put on the stream since, and who asks would wait for that too.
+int launch_away(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, int has_scale, const mcclx_seg& seg, int fan) {
     // (a launch before this one that is still away lies on the same stream, in front of it)
     hipEvent_t& ev = ctx->away_ev[(ctx->away_number + 1) % mcclx_ctx::kAwayEvents];
     if (!ev) HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-    MarkRequest mark;
-    mark.away = true;
-    if (ctx->mark_count && !ctx->away_count_cleared)
-        ctx->away_count_cleared = mcclx::launch_word(nullptr, reinterpret_cast<uint64_t*>(ctx->mark_count + 2), 0) == hipSuccess;
-    {
-        const bool at_once = now_ns() - ctx->away_at < kAwayQuickNs;
-        const MarkScope scope(at_once && may_mark_away(ctx, key, segs, nseg, fan) ? &mark : nullptr);
-        if (int rc = launch_by_value(ctx, key, scale_f, has_scale, segs, nseg, fan, nullptr)) return rc;
+    if (int rc = launch_by_value(ctx, key, scale_f, has_scale, &seg, 1, fan, nullptr)) return rc;
+    if (hipError_t e = hipEventRecord(ev, nullptr); e != hipSuccess) {  // no mark to order by: the host waits
+        HIP_TRY(hipStreamSynchronize(nullptr));
+        return MCCLX_OK;
     }
-    if (mark.number == 0)
-        if (hipError_t e = hipEventRecord(ev, nullptr); e != hipSuccess) {  // no mark to order by: the host waits
-            HIP_TRY(hipStreamSynchronize(nullptr));
-            return MCCLX_OK;
-        }
-    ctx->away_word.store(mark.number, std::memory_order_relaxed);
     ++ctx->away_number;
     ++ctx->away_launches;
-    ctx->away_at = now_ns();
     ctx->away.store(true, std::memory_order_release);
     return MCCLX_OK;
 }
@@ -1044,7 +964,7 @@ int make_ctx(int device, hipStream_t borrowed, bool borrow, mcclx_ctx** out) {
         hipHostGetDevicePointer(&wd, w, 0) == hipSuccess &&
         hipEventCreateWithFlags(&ctx->word_ev, hipEventDisableTiming) == hipSuccess) {
         void* count = nullptr;  // (without it no launch marks its own end; nothing is put on a caller's stream here)
-        if (!borrow && hipMalloc(&count, 2 * sizeof(uint64_t)) == hipSuccess) {
+        if (!borrow && hipMalloc(&count, sizeof(uint64_t)) == hipSuccess) {
             // cleared on the queue, in front of every launch that uses it (a blocking copy would wait for the default stream)
             if (mcclx::launch_word(ctx->stream, static_cast<uint64_t*>(count), 0) == hipSuccess) ctx->mark_count = static_cast<uint32_t*>(count);
             else (void)hipFree(count);
@@ -1347,10 +1267,10 @@ int mcclx_decode_bf16(mcclx_ctx* ctx, void* dst_f32, const void* src_bf16, uint6
 // mcclx_stream_wait_queue): no cross-stream event and none of the two hand-overs between
 // hardware queues, which bound a sequence of such calls (events and launch 31 us a call, the
 // launch and its mark 7; 4097 bf16 values reduced through Python 50 -> 11 us, 25 MiB encoded and
-// decoded 110 -> 25 us).  A launch of up to 32 blocks into device memory that follows another at once tells of its end
-// itself (LaunchMark), and no event is recorded behind it: the device takes 4 us for a kernel's event, 6.6 us a kernel and
-// event, 2.4 a kernel.  For the others the mark is an event record and not the kernel's own stop event: after
-// thousands of launches with one, the next calls on the stream took three times as long.
+// decoded 110 -> 25 us).  The mark is an event record and not the kernel's own stop event: after
+// thousands of launches with one, the next calls on the stream took three times as long.  An event without a system
+// fence saves a sequence of calls nothing (10.8 us a call of 4097 values either way, 7.0 without an event): the host's
+// part of the record bounds it.
 // Everything else takes the two orderings: a queue with work in flight, a queue whose HIP stream
 // the caller holds (what they put there would not see a launch made elsewhere), a recording, and
 // every `stream` but the legacy default one.  (Once handed out, the HIP stream stays the caller's to
@@ -1370,7 +1290,7 @@ static int ordered_launch(mcclx_ctx* ctx, void* stream, const OneLaunch& l) {
             int has_scale, fan;
             if (int rc = check_plan(&l.plan, &key, &scale_f, &has_scale, &fan)) return rc;
             if (int rc = check_segs(ctx, key, &l.seg, 1, fan)) return rc;
-            return launch_away(ctx, key, scale_f, has_scale, &l.seg, 1, fan);
+            return launch_away(ctx, key, scale_f, has_scale, l.seg, fan);
         }
     }
     if (int rc = mcclx_queue_wait_stream(ctx, stream)) return rc;
@@ -1695,19 +1615,13 @@ int mcclx_stream_wait_queue(mcclx_ctx* ctx, void* consumer_stream) {
     if (ctx->away.load(std::memory_order_acquire) && !ctx->capturing) {
         DeviceGuard guard(ctx->device);
         std::lock_guard<std::mutex> lk(ctx->away_mu);
-        if (away_word_seen(ctx)) {
-            ctx->away.store(false, std::memory_order_release);
-        } else if (ctx->away.load(std::memory_order_relaxed) && consumer != nullptr) {  // (the launch lies on the default stream)
-            hipEvent_t ev;
+        if (ctx->away.load(std::memory_order_relaxed) && consumer != nullptr) {  // (the launch lies on the default stream)
+            const hipEvent_t ev = ctx->away_ev[ctx->away_number % mcclx_ctx::kAwayEvents];
             if (records(consumer)) {  // it cannot wait for what its recording does not hold: the host does
-                if (!away_word_comes(ctx, kAwayDrainUs)) {
-                    HIP_TRY(away_event(ctx, &ev));
-                    const BesideRecordings beside;
-                    HIP_TRY(hipEventSynchronize(ev));
-                }
+                const BesideRecordings beside;
+                HIP_TRY(hipEventSynchronize(ev));
                 ctx->away.store(false, std::memory_order_release);
             } else {
-                HIP_TRY(away_event(ctx, &ev));
                 HIP_TRY(hipStreamWaitEvent(consumer, ev, 0));
             }
         }

@@ -176,11 +176,11 @@ def test_a_recording_stream_may_wait_for_an_idle_queue(which):
     q.close()
 
 
-# A launch of up to 32 blocks of 256 lanes tells of its own end and leaves no event behind it.
+# Small launches in a row, up to one packet a lane in 32 blocks of 256 lanes and beyond.
 @pytest.mark.parametrize("dtype,most", [(torch.float32, 32 * 256 * 4), (torch.bfloat16, 32 * 256 * 8), (torch.float16, 32 * 256 * 8)])
 @pytest.mark.parametrize("consumer", ["torch", "queue", "other_stream", "ticket", "drain", "wait", "exposed"])
 @pytest.mark.parametrize("behind", ["nothing", "a_running_kernel"])
-def test_small_launches_that_tell_of_their_own_end(dtype, most, consumer, behind):
+def test_small_launches_in_a_row(dtype, most, consumer, behind):
     q = K.ReduceQueue(0)
     other = torch.cuda.Stream()
     for n in (1, 4_097, most - 1, most, most + 1, 4 * most + 3):
@@ -217,11 +217,11 @@ def test_small_launches_that_tell_of_their_own_end(dtype, most, consumer, behind
             other.synchronize()
         torch.cuda.synchronize()
         assert bool((got == 3.0).all()), n
-    assert q.marked_launch_count() > 0  # (a launch that follows another one at once)
+    assert q.away_launch_count() > 0  # (the queue was idle, and its stream not handed out, at the first of the sizes)
     q.close()
 
 
-def test_codec_and_scaling_at_the_last_size_that_tells_of_its_end():
+def test_codec_and_scaling_at_the_edges_of_blocks():
     q = K.ReduceQueue(0)
     for blocks in (1, 2, 31, 32, 33):
         for extra in (-1, 0, 1):
@@ -233,7 +233,6 @@ def test_codec_and_scaling_at_the_last_size_that_tells_of_its_end():
             K.hip_accumulate_and_scale(y, x, 0.25, queue=q)
             assert torch.equal(w.view(torch.int16), x.to(torch.bfloat16).view(torch.int16))
             assert torch.equal(back, w.float()) and torch.equal(y, (x + x) * 0.25)
-    assert q.marked_launch_count() > 0
     q.close()
 
 
@@ -255,3 +254,48 @@ def test_a_host_that_waits_for_a_small_launch_does_not_wait_for_what_came_behind
     assert waited < slept / 2, (waited, slept)
     assert bool((dst == 4.0).all())
     q.close()
+
+
+@pytest.mark.parametrize("who", ["drain", "wait", "ticket", "queue", "other_stream"])
+def test_who_asks_for_a_launch_that_is_still_running_waits_for_it_and_no_more(who):
+    """Behind small calls in a row, the newest of which are still to run, the caller puts a long kernel on their stream:
+    the host, the queue and other streams get the results long before that kernel ends.  (Two streams may share a
+    hardware queue, where one waits for the other whatever the library does: one try of several.)"""
+    import time
+    on_time = False
+    for _ in range(8):
+        q, side = K.ReduceQueue(0), torch.cuda.Stream()
+        dst, src, got = torch.zeros(4_097, device="cuda"), torch.ones(4_097, device="cuda"), torch.zeros(4_097, device="cuda")
+        host = torch.zeros(4_097, pin_memory=True)
+        K.hip_reduce_op(dst, src, "sum", queue=q)
+        torch.cuda.synchronize()
+        torch.cuda._sleep(8_000_000)  # some 4 ms
+        for _ in range(8):
+            K.hip_reduce_op(dst, src, "sum", queue=q)
+        torch.cuda._sleep(100_000_000)  # some 50 ms
+        t = time.perf_counter()
+        if who == "drain":
+            q.drain()
+        elif who == "wait":
+            q.wait_results()
+        elif who == "ticket":
+            q.wait(q.record())
+        elif who == "queue":
+            q.copy(got.data_ptr(), dst.data_ptr(), 4 * 4_097)
+            q.wait(q.record())
+        else:
+            q.torch_stream_wait(side)
+            with torch.cuda.stream(side):
+                got.copy_(dst)
+                host.copy_(dst, non_blocking=True)
+            side.synchronize()
+            assert bool((host == 9.0).all())
+        waited = time.perf_counter() - t
+        torch.cuda.synchronize()
+        whole = time.perf_counter() - t
+        assert bool((dst == 9.0).all()) and (who not in ("queue", "other_stream") or bool((got == 9.0).all()))
+        q.close()
+        on_time = on_time or waited < whole / 2
+        if on_time:
+            break
+    assert on_time
