@@ -868,11 +868,12 @@ static bool hold_launch(hipStream_t st, FewArgs& a, uint64_t packets, uint32_t g
     const uint32_t cap = hold_capacity<C, T, HB, OUT>(lp.cus);
     if (cap < (uint32_t)a.nseg) return false;
     uint32_t hx = cap / (uint32_t)a.nseg;
-    // Two tensors to two: 512 blocks per segment would put a lane's packets 4 MiB apart.  As many as three segments get
-    // where that is enough, at five packets per lane up to two fifths of the device, and the plain form beyond.
-    // Two ranks of 18 / 22 / 26.2 / 32 / 34 MB (us): 512 blocks 13.2 / 16.5 / 20.2 / 23.1 / -, these 12.6 / 15.0 / 17.8 / 21.7 / 24.3,
-    // plain 13.4 / 15.9 / 18.5 / 22.2 / 23.5.
-    if (OUT == kOutFan && a.nseg == 2) {
+    // Two segments of two operands to two places, as the tensors of two ranks are: 512 blocks per segment put a lane's
+    // packets 4 MiB apart, which costs from more than two of them on.  As many blocks there as three segments get where
+    // that is enough, at five packets per lane up to two fifths of the device, and the plain form beyond.
+    // Two ranks of 18 / 22 / 26.2 / 32 / 34 MB (us): 512 blocks 13.2 / 16.0 / 20.4 / 23.4 / 24.3, these 13.0 / 15.4 / 18.5 / 22.9 / -,
+    // plain 13.4 / 15.9 / 18.5 / 22.2 / 23.5; of 8 / 8.3 / 11 MB (one and two packets) 512 blocks 6.8 / 7.8 / 9.5, these 7.0 / 8.3 / 9.8.
+    if (OUT == kOutFan && C::K == 2 && a.nseg == 2 && a.fan == 1 && packets > 2 * (uint64_t)hx * HB) {
         const uint64_t need = (packets + (uint64_t)HB * T - 1) / ((uint64_t)HB * T);
         hx = cap / 3 & ~3u;
         if (T == 5 && need > hx) hx = (uint32_t)(need + 3 < cap * 2 / 5 ? (need + 3) & ~3ull : 0);

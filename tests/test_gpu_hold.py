@@ -332,10 +332,11 @@ def test_one_operand_plans_in_the_hold_form_match_the_plain_form(env, queues, wi
 
 
 @pytest.mark.parametrize("dtype,wire", [(torch.float32, True), (torch.float32, False), (torch.bfloat16, False)])
-@pytest.mark.parametrize("blocks_and_packets", [(340, 4), (340, 5), (408, 5)])
+@pytest.mark.parametrize("blocks_and_packets", [(512, 2), (340, 4), (340, 5), (405, 5)])
 def test_two_ranks_at_the_sizes_where_the_number_of_blocks_changes(dtype, wire, blocks_and_packets):
-    """An allreduce of two tensors: 340 blocks per chunk at four packets per lane, at five, then more, then
-    the plain form; one packet to either side of each, the same bits as step by step."""
+    """An allreduce of two tensors on a device that holds 1024 blocks: 512 per chunk up to two packets per lane, 340 at four,
+    at five, then more, up to 408 in fours, then the plain form; some packets to either side of each, the
+    same bits as step by step."""
     from mccl_amd import harness as H, kernels as K, _lib as L
     blocks, per = blocks_and_packets
     elems = 4 if dtype == torch.float32 else 8
@@ -345,7 +346,29 @@ def test_two_ranks_at_the_sizes_where_the_number_of_blocks_changes(dtype, wire, 
         g = torch.Generator(device="cuda").manual_seed(n)
         ts = [torch.randn(n, generator=g, device="cuda").to(dtype) for _ in range(2)]
         want = [t.clone() for t in ts]
+        before = q.hold_launch_count()
         H.allreduce_replay(ts, "avg", L.ALGO_RING, wire_bf16=wire, mode=L.REPLAY_DIRECT, queue=q)
+        if q.compute_units == 256:
+            assert q.hold_launch_count() - before == (0 if blocks == 405 and extra > 0 else 1), extra
         H.allreduce_replay(want, "avg", L.ALGO_RING, wire_bf16=wire, mode=L.REPLAY_STEPWISE, queue=q)
         for a, b in zip(ts, want):
             assert torch.equal(a.view(torch.int16), b.view(torch.int16)), (n, extra)
+
+
+def test_two_messages_over_three_ranks_keep_half_the_device_each():
+    """The smaller number of blocks is for two operands to two places: two messages over three ranks hold up to
+    half of what the device holds of their kernel (768 blocks), at four packets a lane."""
+    from mccl_amd import harness as H, kernels as K, _lib as L
+    q = K.hip_kernels_init(0)
+    n = (384 * 512 * 4 - 3) * 4 + 1
+    g = torch.Generator(device="cuda").manual_seed(3)
+    groups = [[torch.randn(n, generator=g, device="cuda") for _ in range(3)] for _ in range(2)]
+    want = [[t.clone() for t in ts] for ts in groups]
+    before = q.hold_launch_count()
+    H.allreduce_replay_many(groups, "avg", L.ALGO_TREE, queue=q)
+    if q.compute_units == 256:
+        assert q.hold_launch_count() == before + 1
+    for ts, ws in zip(groups, want):
+        H.allreduce_replay(ws, "avg", L.ALGO_TREE, mode=L.REPLAY_STEPWISE, queue=q)
+        for a, b in zip(ts, ws):
+            assert torch.equal(a.view(torch.int32), b.view(torch.int32))
