@@ -140,6 +140,8 @@ MCCLX_API uint64_t mcclx_hold_launch_count(mcclx_ctx* ctx);
 MCCLX_API uint64_t mcclx_marked_launch_count(mcclx_ctx* ctx);
 /* Launches that ran on the default stream in the queue's place (diagnostic): see the _ordered forms. */
 MCCLX_API uint64_t mcclx_away_launch_count(mcclx_ctx* ctx);
+/* Copy launches that went one destination after another (diagnostic). */
+MCCLX_API uint64_t mcclx_spread_copy_count(mcclx_ctx* ctx);
 MCCLX_API uint64_t mcclx_four_wave_launch_count(mcclx_ctx* ctx);
 /* Diagnostic: the model behind that time -- no store before `latency_ticks` +
  * bytes read / `bytes_per_tick` ticks of a 100 MHz clock after a block's start.

@@ -78,6 +78,7 @@ SIGNATURES = {
     "mcclx_hold_launch_count": (_u64, [_vp]),
     "mcclx_marked_launch_count": (_u64, [_vp]),
     "mcclx_away_launch_count": (_u64, [_vp]),
+    "mcclx_spread_copy_count": (_u64, [_vp]),
     "mcclx_four_wave_launch_count": (_u64, [_vp]),
     "mcclx_set_hold": (_i, [_vp, _i]),
     "mcclx_hold_model": (_i, [_vp, C.POINTER(C.c_uint32), C.POINTER(C.c_uint32)]),

@@ -297,7 +297,7 @@ constexpr uint32_t kSpreadLds = 163840 / 4;
 
 // Pieces of 8 to 12 MiB (1 to 1.5 MiB of each XCD's L2; 8 x 64 MiB to eight with 4 / 8 / 16 MiB: 755 / 737 / 735 us, 4 x 32 MiB
 // to four 97.0 / 95.2 / 95.2).  A source is cut where all pieces have one length and the XCDs take long runs of tiles, with at
-// most one block in sixteen without work.
+// most one block in sixteen without work; the shortest, of fewer than 16 tiles, have up to seven tiles beside theirs.
 constexpr uint64_t kSpreadTiles = (8u << 20) / kSpreadTile;
 struct SpreadShape {
     uint64_t pieces, tiles;  // tiles of a piece
@@ -313,17 +313,14 @@ SpreadShape spread_shape(uint64_t need) {  // tiles of the longest source, one a
             if (g == 0 || (p * tiles - need) * 16 <= need) return {p, tiles, g};
         }
 }
+// From 6 MB moved on pieces are 0.97-1.3 times as fast on the device, one, two or a rank's number of sources to two to eight
+// destinations, 1.1 times on average; below that 0.86-1.2 times, worst where many small sources leave blocks without work
+// (eight of 16 KB to eight 2.14 and 2.46 us).  Looking up where the memory lies takes the host 0.3 to 0.7 us, so whole calls
+// gain from 20 MB on (allgathers of 8 x 20 / 128 / 256 KB 17.6 / 18.0 / 18.9 us without, 18.0 / 18.5 / 18.7 with; of 8 x 1 / 2 / 4 MB
+// 29.2 / 42.4 / 65.1 and 26.4 / 35.9 / 56.8).
 // To two or three, pieces pay while the launch is small: 50 / 100 / 200 / 400 MB moved to two 1.2 / 1.12 / 0.95 / 0.94 times as
-// fast, to three 1.19 / 1.19 / 0.99 / 1.0; to four and more 1.0-1.26 times at every size from 100 KB to 5.6 GB (one of the 60
-// tried 0.98).
-constexpr uint64_t kSpreadToThree = 150'000'000;
-
-bool spread_pays(const CopyFew& a, bool local_sources) {
-    if (!local_sources || a.d[0].n < 2) return false;
-    uint64_t moved = 0;
-    for (uint32_t i = 0; i < a.n; ++i) moved += a.d[i].nbytes * (1 + a.d[i].n);
-    return a.d[0].n >= 4 || moved < kSpreadToThree;
-}
+// fast, to three 1.19 / 1.19 / 0.99 / 1.0; to four and more 1.0-1.26 times up to 5.6 GB.
+constexpr uint64_t kSpreadFrom = 20'000'000, kSpreadToThree = 150'000'000;
 
 template <int N>
 hipError_t launch_copy_spread(hipStream_t st, const CopyFew& a) {
@@ -338,11 +335,21 @@ hipError_t launch_copy_spread(hipStream_t st, const CopyFew& a) {
 }
 }  // namespace
 
-hipError_t launch_copy_few(hipStream_t st, const CopyFew& a, bool local_sources) {
+bool copy_spread_pays(const CopyFew& a) {
+    if (a.n == 0 || a.d[0].n < 2) return false;
+    uint64_t moved = 0;
+    for (uint32_t i = 0; i < a.n; ++i) {
+        if (a.d[i].n != a.d[0].n) return false;
+        moved += a.d[i].nbytes * (1 + a.d[i].n);
+    }
+    return moved >= kSpreadFrom && (a.d[0].n >= 4 || moved < kSpreadToThree);
+}
+
+hipError_t launch_copy_few(hipStream_t st, const CopyFew& a, bool spread) {
     if (a.n == 0 || a.n > (uint32_t)kFewCopies) return a.n ? hipErrorInvalidValue : hipSuccess;
     for (uint32_t i = 1; i < a.n; ++i)
         if (a.d[i].n != a.d[0].n) return launch_copy_few_n<kCopyDsts, true>(st, a);
-    if (spread_pays(a, local_sources)) switch (a.d[0].n) {
+    if (spread) switch (a.d[0].n) {
         case 2: return launch_copy_spread<2>(st, a);
         case 3: return launch_copy_spread<3>(st, a);
         case 4: return launch_copy_spread<4>(st, a);

@@ -190,9 +190,11 @@ struct CopyFew {
     CopyDesc d[kFewCopies];
     uint32_t n;
 };
-// `local_sources`: every source lies in this device's own memory, which its caches hold (a copy to several
-// destinations may then read it more than once).
-hipError_t launch_copy_few(hipStream_t st, const CopyFew& copies, bool local_sources);
+// `spread`: one destination after another (copy_spread_pays).  For memory of this device alone: its caches hold no other
+// sources, and destinations behind links of their own want to be written side by side.
+hipError_t launch_copy_few(hipStream_t st, const CopyFew& copies, bool spread);
+// Is `spread` the faster form of these copies, where all of their memory is this device's?
+bool copy_spread_pays(const CopyFew& copies);
 // Work items (tiles) one copy of nbytes splits into.
 uint64_t copy_items(uint64_t nbytes);
 // `most`: the largest number of destinations any descriptor of the launch has.

@@ -89,7 +89,7 @@ struct mcclx_ctx {
     uint32_t wall_khz = 100000;                                      // the device's wall clock
     bool hold_measured = false;        // the gate's rate was measured on this device (not the default)
     std::atomic<bool> hold_enabled{true};  // a completer thread may switch it while ranks launch
-    std::atomic<uint64_t> hold_launches{0}, four_launches{0}, marked_launches{0}, away_launches{0};
+    std::atomic<uint64_t> hold_launches{0}, four_launches{0}, marked_launches{0}, away_launches{0}, spread_copies{0};
     bool batch_active = false;
     std::string batch_label;
     std::mutex mu;
@@ -449,6 +449,15 @@ bool in_device_memory(const mcclx_ctx* ctx, const void* p) {
         return false;
     }
     return attr.type == hipMemoryTypeDevice && attr.device == ctx->device;
+}
+
+// Do these copies lie in the context's own device's memory?  The schedules send every source to the same tensors, one per
+// rank: the first and the last stand for the others.  (What it decides is a choice between two forms of the same copies.)
+bool in_device_memory(const mcclx_ctx* ctx, const mcclx::CopyFew& copies) {
+    for (uint32_t i = 0; i < copies.n; ++i)
+        if (!in_device_memory(ctx, copies.d[i].src)) return false;
+    const mcclx::CopyDesc& d = copies.d[0];
+    return in_device_memory(ctx, d.dst[0]) && in_device_memory(ctx, d.dst[d.n - 1]);
 }
 
 int check_segs(mcclx_ctx* ctx, const mcclx::PlanKey& key, const mcclx_seg* segs, uint32_t nseg, int fan) {
@@ -1061,6 +1070,7 @@ uint64_t mcclx_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->launches.load() 
 uint64_t mcclx_hold_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->hold_launches.load() : 0; }
 uint64_t mcclx_marked_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->marked_launches.load() : 0; }
 uint64_t mcclx_away_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->away_launches.load() : 0; }
+uint64_t mcclx_spread_copy_count(mcclx_ctx* ctx) { return ctx ? ctx->spread_copies.load() : 0; }
 uint64_t mcclx_four_wave_launch_count(mcclx_ctx* ctx) { return ctx ? ctx->four_launches.load() : 0; }
 int mcclx_hold_model(mcclx_ctx* ctx, uint32_t* latency_ticks, uint32_t* bytes_per_tick) {
     if (!ctx) return 0;
@@ -1391,11 +1401,11 @@ static int copy_batched(mcclx_ctx* ctx, const mcclx_copy_desc* descs, uint32_t n
         uint64_t longest = 0, sum = 0;
         auto flush = [&]() -> int {
             if (few.n == 0) return MCCLX_OK;
-            bool local = true;
-            for (uint32_t i = 0; local && i < few.n; ++i) local = few.d[i].n < 2 || in_device_memory(ctx, few.d[i].src);
-            hipError_t e = mcclx::launch_copy_few(queue_of(ctx), few, local);
+            const bool spread = mcclx::copy_spread_pays(few) && in_device_memory(ctx, few);
+            hipError_t e = mcclx::launch_copy_few(queue_of(ctx), few, spread);
             if (e != hipSuccess) return fail(MCCLX_ERR_HIP, "copy_batched launch failed: %s", hipGetErrorString(e));
             ++ctx->launches;
+            if (spread) ++ctx->spread_copies;
             few.n = 0;
             longest = sum = 0;
             return MCCLX_OK;

@@ -213,6 +213,10 @@ class ReduceQueue:
         """Launches that ran on the default stream in this queue's place (diagnostic)."""
         return int(L.lib().mcclx_away_launch_count(self.handle))
 
+    def spread_copy_count(self) -> int:
+        """Copy launches of this queue that went one destination after another (diagnostic)."""
+        return int(L.lib().mcclx_spread_copy_count(self.handle))
+
     def four_wave_launch_count(self) -> int:
         """Fold launches of this queue in blocks of four wavefronts (diagnostic)."""
         return int(L.lib().mcclx_four_wave_launch_count(self.handle))
