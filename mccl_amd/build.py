@@ -21,7 +21,7 @@ LIB_PATH = os.path.join(HERE, "libmcclx.so")
 
 SOURCES = ["fold_kernels.hip", "copy_kernel.hip", "cast_kernel.hip", "static_table.hip", "mcclx_api.cpp", "mcclx_sched.cpp"]
 FOLD_PARTS = 9  # fold_kernels.hip is compiled once per part (-DMCCLX_PART=n), in parallel
-HEADERS = ["fold_launch.h", "mcclx_internal.h", "spans.h", os.path.join(ROOT, "include", "mcclx.h")]
+HEADERS = ["fold_launch.h", "mcclx_internal.h", "spans.h", "wire_codec.h", os.path.join(ROOT, "include", "mcclx.h")]
 
 # -ffp-contract=off / -fno-fast-math: IEEE fp32 add and mul, no FMA fusion, so
 # the kernels match the CPU oracle bit for bit.  Denormals are kept (hipcc's

@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "fold_launch.h"
+#include "wire_codec.h"
 
 namespace mcclx {
 namespace {
@@ -24,18 +25,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // element alignment is all the kernels may assume
 typedef u32x4 F32Pack __attribute__((aligned(4)));
 typedef u32x2 WirePack __attribute__((aligned(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// Round to nearest even, NaN -> 0x7FC0.
-__device__ __forceinline__ uint32_t encode1(float x) {
-    return (x != x) ? 0x7FC0u : (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)x);
-}
-__device__ __forceinline__ uint32_t encode2(float a, float b) {
-    uint32_t r = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
-    r = (a != a) ? (r & 0xFFFF0000u) | 0x7FC0u : r;
-    return (b != b) ? (r & 0x0000FFFFu) | 0x7FC00000u : r;
-}
 
 // s_waitcnt vmcnt(0), the other counters as they are: all loads of the wave are back, and its last store has arrived.
 constexpr int kVmcnt0 = 0x0F70;
@@ -58,8 +47,8 @@ __global__ void __launch_bounds__(B) cast_kernel(void* dst, const void* src, uin
             __builtin_nontemporal_store((u32x4{v[0] << 16, v[0] & 0xFFFF0000u, v[1] << 16, v[1] & 0xFFFF0000u}),
                                         (MCCLX_GLOBAL F32Pack*)(out + p * kOut));
         else
-            __builtin_nontemporal_store((u32x2{encode2(__uint_as_float(v[0]), __uint_as_float(v[1])),
-                                               encode2(__uint_as_float(v[2]), __uint_as_float(v[3]))}),
+            __builtin_nontemporal_store((u32x2{bf16_encode_pair(__uint_as_float(v[0]), __uint_as_float(v[1])),
+                                               bf16_encode_pair(__uint_as_float(v[2]), __uint_as_float(v[3]))}),
                                         (MCCLX_GLOBAL WirePack*)(out + p * kOut));
     };
     Raw v[T];
@@ -84,7 +73,7 @@ __global__ void __launch_bounds__(B) cast_kernel(void* dst, const void* src, uin
             if constexpr (DECODE)
                 ((MCCLX_GLOBAL uint32_t*)dst)[i] = (uint32_t)((const MCCLX_GLOBAL uint16_t*)src)[i] << 16;
             else
-                ((MCCLX_GLOBAL uint16_t*)dst)[i] = (uint16_t)encode1(((const MCCLX_GLOBAL float*)src)[i]);
+                ((MCCLX_GLOBAL uint16_t*)dst)[i] = (uint16_t)(bf16_round_bits(((const MCCLX_GLOBAL float*)src)[i]) >> 16);
         };
         if (threadIdx.x < head) edge((int64_t)threadIdx.x - head);
         if (threadIdx.x < tail) edge((int64_t)packets * 4 + threadIdx.x);

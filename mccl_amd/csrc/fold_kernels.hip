@@ -36,6 +36,7 @@
 #include <type_traits>
 
 #include "fold_launch.h"
+#include "wire_codec.h"
 
 namespace mcclx {
 namespace {
@@ -86,17 +87,7 @@ typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
 
 // ---------------------------------------------------------------- rounding
 
-// fp32 -> bf16 round-to-nearest-even, NaN -> 0x7FC0, result kept as the fp32
-// whose low half is zero (torch/headeronly/util/BFloat16.h:100-114).
-__device__ __forceinline__ uint32_t bf16_round_bits(float x) {
-    uint32_t r = (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)x) << 16;  // v_cvt_pk_bf16_f32
-    return (x != x) ? 0x7FC00000u : r;
-}
-
-template <int W> struct Num;  // arithmetic dtype traits
-
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+template <int W> struct Num;  // arithmetic dtype traits (bf16: wire_codec.h)
 
 // Besides the scalar rnd (round to W, NaN made canonical where W defines one),
 // every dtype has the array form the packet path uses between the operands of
@@ -118,12 +109,10 @@ template <> struct Num<MCCLX_BF16> {
     __device__ static __forceinline__ uint32_t enc(float x) { return bf16_round_bits(x) >> 16; }
     __device__ static __forceinline__ float dec(uint32_t h) { return __uint_as_float(h << 16); }
     __device__ static __forceinline__ float scaled(float x, float s) { return x * s; }
-    // two values per v_cvt_pk_bf16_f32; a NaN whose quiet bit is set (every NaN an
-    // add, a multiply or a decoded bf16 operand can hand over) converts to a NaN
     template <int E> __device__ static __forceinline__ void round_mid(float (&x)[E]) {
 #pragma unroll
         for (int j = 0; j < E; j += 2) {
-            const uint32_t u = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x[j], x[j + 1]}, bf16x2));
+            const uint32_t u = bf16_pair(x[j], x[j + 1]);
             x[j] = __uint_as_float(u << 16);
             x[j + 1] = __uint_as_float(u & 0xFFFF0000u);
         }
