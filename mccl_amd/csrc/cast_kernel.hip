@@ -94,7 +94,10 @@ hipError_t go(hipStream_t st, void* dst, const void* src, uint32_t packets, uint
 // 6.3 / 6.8, 6.5 M (3.1) 9.1 / 8.5 / 7.9 / 7.8 / 8.6, 10 M (4.8) 12.4 / 12.6 / 13.1 / 11.3 / 11.9, 14 M (6.7) 16.3 / 16.6 / 16.8 /
 // 15.7 / 15.9, 16 M (7.6) 18.0 / 18.5 / 18.7 / 17.7 / 17.4.  Encode at 1 / 2 in blocks of four and at 1 in blocks of one: 1.5 M
 // 3.1 / 3.3 / 3.6, 2.5 M (1.2) 4.4 / 3.9 / 4.5, 4 M 5.7 / 6.0 / 5.7, 6.5 M 9.2 / 8.9 / 8.4, 16 M 19.3 / 18.1 / 16.9.
-hipError_t launch_cast(hipStream_t st, bool decode, void* dst, const void* src, uint64_t count, int cus) {
+// Off the lines a decode of 1.5 M takes 3.6 us at 1 and 3.1 at 2, which are level on them: 2 from 0.6 generations on.
+// One store under way per wave is not enough for a result in host memory (6.5 M decoded into pinned memory 536 us at 2
+// in blocks of one and 561 at 8): `far`.
+hipError_t launch_cast(hipStream_t st, bool decode, void* dst, const void* src, uint64_t count, int cus, bool far) {
     // packets start on a 128-byte line of the output
     const uint32_t size = decode ? 4 : 2, mis = (uint32_t)(reinterpret_cast<uintptr_t>(dst) & 127u);
     const uint64_t peel = mis ? (128u - mis) / size : 0;
@@ -106,10 +109,10 @@ hipError_t launch_cast(hipStream_t st, bool decode, void* dst, const void* src, 
     src = static_cast<const char*>(src) + (uint64_t)head * (6 - size);
     const uint64_t waves = whole / 64, gen = 32 * (uint64_t)cus;
     if (decode) {
-        if (waves * 4 <= 3 * gen) return go<true, 256, 1>(st, dst, src, packets, head, tail);
+        if (waves * 5 <= 3 * gen) return go<true, 256, 1>(st, dst, src, packets, head, tail);
         if (waves <= 2 * gen) return go<true, 256, 2>(st, dst, src, packets, head, tail);
-        if (waves <= 3 * gen) return go<true, 256, 4>(st, dst, src, packets, head, tail);
-        if (waves <= 7 * gen) return go<true, 256, 8>(st, dst, src, packets, head, tail);
+        if (waves <= 3 * gen && !far) return go<true, 256, 4>(st, dst, src, packets, head, tail);
+        if (waves <= 7 * gen && !far) return go<true, 256, 8>(st, dst, src, packets, head, tail);
         return go<true, 64, 2>(st, dst, src, packets, head, tail);
     }
     if (waves <= gen) return go<false, 256, 1>(st, dst, src, packets, head, tail);

@@ -1072,7 +1072,7 @@ static hipError_t launch_few(hipStream_t st, const FewArgs& args, const LaunchPa
         void* out = C::kDecode ? s.out : s.wire_out;
         const bool plain = a.nseg == 1 && !a.has_scale && out && !(C::kDecode ? s.wire_out : s.out) && maxc < (1ull << 33) && lp.cus > 0;
         if (plain && (waves < C::kOneWaveFrom || !off_lines<C, OUT>(a)))
-            return launch_cast(st, C::kDecode, out, s.in[0], maxc, lp.cus);
+            return launch_cast(st, C::kDecode, out, s.in[0], maxc, lp.cus, lp.far_out);
     }
     if constexpr (C::kSmallShape) {
         if (waves < C::kOneWaveFrom) return go(std::integral_constant<int, kFourWaves>{}, Few{}, lds);

@@ -92,6 +92,7 @@ struct LaunchParams {
     // before hold_latency_ticks + read bytes / hold_bytes_per_tick ticks of the 100 MHz
     // wall clock have passed since its block started.
     int cus = 0;
+    bool far_out = false;              // a large cast's result lies outside the device's memory
     bool* held = nullptr;              // set when the launch took that form (diagnostic)
     bool* four = nullptr;              // set when a by-value launch took blocks of four wavefronts (diagnostic)
     uint64_t hold_min_read_bytes = 0;
@@ -110,8 +111,8 @@ bool fold_encode_ok(const PlanKey& key);
 hipError_t launch_fold_encode(hipStream_t st, const PlanKey& key, const FewArgs& few, uint32_t nfold);
 
 // One tensor to its wire form or back, as the plans of one operand without a scale give it (per-step rounding):
-// dst <- src, up to 2^33 elements.
-hipError_t launch_cast(hipStream_t st, bool decode, void* dst, const void* src, uint64_t count, int cus);
+// dst <- src, up to 2^33 elements.  `far`: dst lies outside the device's memory (a choice of shape).
+hipError_t launch_cast(hipStream_t st, bool decode, void* dst, const void* src, uint64_t count, int cus, bool far);
 
 // Can a segment of `count` elements be launched by value?  A grid has at most 2^32 threads, one
 // per packet there (more are dropped without an error); the table kernels loop.

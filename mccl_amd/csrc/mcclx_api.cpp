@@ -627,6 +627,9 @@ int stage_upload(mcclx_ctx* ctx, Staged* s, size_t nbytes, void** dev) {
     return MCCLX_OK;
 }
 
+// Decodes of more elements are asked where their result lies (launch_cast), 0.06 us of 5 and more.
+constexpr uint64_t kLookAtCast = 4'000'000;
+
 // Descriptors in the kernel arguments (nseg <= kFewSegs), on the queue or on `st`.
 int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, int has_scale,
                     const mcclx_seg* segs, uint32_t nseg, int fan, hipStream_t st) {
@@ -635,6 +638,8 @@ int launch_by_value(mcclx_ctx* ctx, const mcclx::PlanKey& key, float scale_f, in
     lp.fan = fan > 0 ? fan : 0;
     lp.to_all = fan == kToAll;
     lp.cus = ctx->cus;
+    if (key.io == MCCLX_IO_OUT_F32 && key.k == 1 && nseg == 1 && segs[0].count > kLookAtCast && segs[0].out)
+        lp.far_out = !in_device_memory(ctx, segs[0].out);
     bool held = false;
     lp.held = &held;
     bool four = false;
@@ -1278,9 +1283,8 @@ int mcclx_decode_bf16(mcclx_ctx* ctx, void* dst_f32, const void* src_bf16, uint6
 // hardware queues, which bound a sequence of such calls (events and launch 31 us a call, the
 // launch and its mark 7; 4097 bf16 values reduced through Python 50 -> 11 us, 25 MiB encoded and
 // decoded 110 -> 25 us).  The mark is an event record and not the kernel's own stop event: after
-// thousands of launches with one, the next calls on the stream took three times as long.  An event without a system
-// fence saves a sequence of calls nothing (10.8 us a call of 4097 values either way, 7.0 without an event): the host's
-// part of the record bounds it.
+// thousands of launches with one, the next calls on the stream took three times as long.  With it a sequence of calls
+// of 4097 values takes 7.3 or 11 us a call, from process to process, without any mark 7.0.
 // Everything else takes the two orderings: a queue with work in flight, a queue whose HIP stream
 // the caller holds (what they put there would not see a launch made elsewhere), a recording, and
 // every `stream` but the legacy default one.  (Once handed out, the HIP stream stays the caller's to

@@ -1,5 +1,5 @@
 """The wire codec on one tensor, at the sizes where the number of packets a lane takes changes (in waves of one
-packet a lane: three quarters, one, one and a half, two, three and seven generations of the device), at
+packet a lane: three fifths, three quarters, one, one and a half, two, three and seven generations of the device), at
 the edges of a tile and off the lines of memory, bit for bit: encode against torch's cast, decode against
 the bits moved up by sixteen."""
 import pytest
@@ -26,7 +26,7 @@ def special(n, offset):
 
 
 SIZES = [1, 3, 4, 63, 64, 65, 1023, 1025, 33_000, 40_001]
-SIZES += [GEN * a // b + d for a, b in ((3, 4), (1, 1), (3, 2), (2, 1), (3, 1), (7, 1)) for d in (-1, 0, 1, 259)]
+SIZES += [GEN * a // b + d for a, b in ((3, 5), (3, 4), (1, 1), (3, 2), (2, 1), (3, 1), (7, 1)) for d in (-1, 0, 1, 259)]
 
 
 @pytest.mark.parametrize("n", SIZES)
@@ -51,6 +51,24 @@ def test_casts_at_every_change_of_shape(n, src_off, dst_off):
     q.drain()
     assert torch.equal(back[src_off:src_off + n].view(torch.int32), src.view(torch.int16).to(torch.int32) << 16)
     assert bool((back[:src_off] == -5).all()) and bool((back[src_off + n:] == -5).all())
+
+
+@pytest.mark.parametrize("n", [GEN * 2 - 1, GEN * 2 + 1029, GEN * 3 + 1, GEN * 7 + 5])
+def test_decode_into_pinned_host_memory(n):
+    import ctypes
+    import numpy as np
+    q = K.hip_kernels_init(0)
+    wire = special(n, 0).to(torch.bfloat16)
+    host, dev = q.host_alloc(4 * n + 64)
+    ctypes.memset(host, 0x5A, 4 * n + 64)
+    torch.cuda.synchronize()
+    L.check(L.lib().mcclx_decode_bf16(q.handle, dev, wire.data_ptr(), n))
+    q.drain()
+    got = np.ctypeslib.as_array((ctypes.c_uint32 * (n + 16)).from_address(host))
+    want = wire.view(torch.int16).cpu().numpy().view(np.uint16).astype(np.uint32) << 16
+    same = np.array_equal(got[:n], want) and bool((got[n:] == 0x5A5A5A5A).all())
+    q.host_free(host)
+    assert same
 
 
 def test_the_same_plan_with_a_scale_or_two_outputs_is_not_taken_for_a_cast():
