@@ -299,3 +299,28 @@ def test_who_asks_for_a_launch_that_is_still_running_waits_for_it_and_no_more(wh
         if on_time:
             break
     assert on_time
+
+
+def test_a_queue_that_the_default_stream_waits_for_counts_as_idle():
+    """The launch is behind the queue's work on that stream already; what the queue is given next is behind the launch."""
+    from mccl_amd import _lib as L
+    q = K.ReduceQueue(0)
+    x, out, got = torch.zeros(N, device="cuda"), torch.zeros(N, device="cuda"), torch.zeros(N, device="cuda")
+    torch.cuda.synchronize()
+    plan = K.make_plan(L.F32, 2, scale_mode=L.SCALE_VIEW, scale=0.5)
+    for i in range(1, 9):
+        torch.cuda._sleep(300_000)
+        x.fill_(i)
+        q.wait_torch_stream()
+        q.fold(plan, [K.make_seg(out.data_ptr(), 0, [x.data_ptr(), x.data_ptr()], N)])
+        q.torch_stream_wait()
+        K.hip_scale_inplace(out, 2.0, queue=q)
+        assert q.away_launch_count() == i
+        q.copy(got.data_ptr(), out.data_ptr(), 4 * N)
+        if i % 2:
+            K.hip_scale_inplace(out, 4.0, queue=q)   # the queue's copy is still to run: through the queue
+            assert q.away_launch_count() == i
+        q.drain()
+        torch.cuda.synchronize()
+        assert bool((got == 2 * i).all()) and bool((out == (8 * i if i % 2 else 2 * i)).all()), i
+    q.close()
