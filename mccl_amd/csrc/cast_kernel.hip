@@ -95,6 +95,8 @@ hipError_t go(hipStream_t st, void* dst, const void* src, uint32_t packets, uint
 // 15.7 / 15.9, 16 M (7.6) 18.0 / 18.5 / 18.7 / 17.7 / 17.4.  Encode at 1 / 2 in blocks of four and at 1 in blocks of one: 1.5 M
 // 3.1 / 3.3 / 3.6, 2.5 M (1.2) 4.4 / 3.9 / 4.5, 4 M 5.7 / 6.0 / 5.7, 6.5 M 9.2 / 8.9 / 8.4, 16 M 19.3 / 18.1 / 16.9.
 // Off the lines a decode of 1.5 M takes 3.6 us at 1 and 3.1 at 2, which are level on them: 2 from 0.6 generations on.
+// An encode from off the lines of 3.4 / 4 M takes 5.6 / 6.1 us at 1 in blocks of one and 5.4 / 5.9 in blocks of four (on the
+// lines 5.3 / 5.7 and 5.4 / 5.8).
 // One store under way per wave is not enough for a result in host memory (6.5 M decoded into pinned memory 536 us at 2
 // in blocks of one and 561 at 8): `far`.
 hipError_t launch_cast(hipStream_t st, bool decode, void* dst, const void* src, uint64_t count, int cus, bool far) {
@@ -117,6 +119,7 @@ hipError_t launch_cast(hipStream_t st, bool decode, void* dst, const void* src, 
     }
     if (waves <= gen) return go<false, 256, 1>(st, dst, src, packets, head, tail);
     if (waves * 2 <= 3 * gen) return go<false, 256, 2>(st, dst, src, packets, head, tail);
+    if (waves <= 2 * gen && (reinterpret_cast<uintptr_t>(src) & 127u)) return go<false, 256, 1>(st, dst, src, packets, head, tail);
     return go<false, 64, 1>(st, dst, src, packets, head, tail);
 }
 
